@@ -266,7 +266,8 @@ __global__ __launch_bounds__(256, (lookup_min_waves<F, G>())) void k_lookup(Tree
                                                 const uint32_t* __restrict__ npend,
                                                 const uint32_t* __restrict__ sidx,
                                                 const BatchCounters* __restrict__ cnt,
-                                                uint32_t chunk, uint64_t* __restrict__ out_vals,
+                                                uint32_t chunk, uint32_t fill,
+                                                uint64_t* __restrict__ out_vals,
                                                 uint8_t* __restrict__ out_found,
                                                 const RouteHeader* __restrict__ rh,
                                                 const uint64_t* __restrict__ fences,
@@ -284,9 +285,11 @@ __global__ __launch_bounds__(256, (lookup_min_waves<F, G>())) void k_lookup(Tree
   const uint64_t grp0 = (blockIdx.x * (uint64_t)blockDim.x + threadIdx.x) / G;
   const uint64_t ngroups = (uint64_t)gridDim.x * blockDim.x / G;
   const uint32_t U = cnt->n_unique;
-  // Every lane group walks one contiguous span of at least `chunk` sorted groups, so its
-  // cached leaf, parent and directory cursor carry over for the whole span.
-  const uint64_t span = max<uint64_t>(chunk, (U + ngroups - 1) / ngroups);
+  // Every lane group walks one contiguous span of sorted groups, so its cached leaf, parent and
+  // directory cursor carry over for the whole span: at least `chunk` of them once there are
+  // enough to give every lane group the device holds at once (`fill`) a chunk, fewer below that.
+  const uint64_t least = min(chunk, (U + fill - 1) / fill);
+  const uint64_t span = max<uint64_t>(max<uint64_t>(least, 1u), (U + ngroups - 1) / ngroups);
   // Groups past the end skip the walk but stay for the wave's statistics reduction.
   const bool active = grp0 * span < U;
   if (desc) {
@@ -2053,32 +2056,53 @@ hipError_t launch_build_inner(const TreeView& t, const uint64_t* lows_prev, uint
                                                    first_this, level, lows_out, s));
 }
 
+// Lane groups of a lookup kernel the device holds at once (asked once per instantiation).
+template <int F, int G, bool LEARNED, bool INDEX>
+static hipError_t lookup_fill(uint32_t& fill) {
+  static std::atomic<uint32_t> groups{0};
+  uint32_t v = groups.load(std::memory_order_relaxed);
+  if (v == 0) {
+    int dev = 0, cus = 0, per_cu = 0;
+    hipError_t e = hipGetDevice(&dev);
+    if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    if (e == hipSuccess)
+      e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_lookup<F, G, LEARNED, INDEX>, 256, 0);
+    if (e != hipSuccess) return e;
+    v = (uint32_t)std::max(1, cus * per_cu) * (256u / G);
+    groups.store(v, std::memory_order_relaxed);
+  }
+  fill = v;
+  return hipSuccess;
+}
+
+template <int F, int G, bool LEARNED, bool INDEX>
+static hipError_t launch_lookup_k(const TreeView& t, const LookupArgs& a, hipStream_t s) {
+  uint32_t fill = 1;
+  hipError_t e = lookup_fill<F, G, LEARNED, INDEX>(fill);
+  if (e != hipSuccess) return e;
+  // A lane group per chunk of ops, but never fewer groups than ops or than the device holds at
+  // once: a lane group's ops are a chain of dependent node reads, so a small batch that gave each
+  // group a whole chunk ran sixteen chains' length on a mostly idle device (whole call at 1000 ops
+  // 112 -> 85 µs, at 40001 ops 165 -> 149 µs; from chunk * fill ops, 458752 at 16 lanes and
+  // chunks of 16, the spans are what they were).
+  const uint64_t groups = std::max<uint64_t>((a.n_max + a.chunk - 1) / a.chunk,
+                                             std::min<uint64_t>(a.n_max, fill));
+  // Persistent grid: at most LOOKUP_GRID_CAP workgroups; each lane group walks one contiguous span.
+  const uint32_t blocks = (uint32_t)std::min<uint64_t>((groups * G + 255) / 256, LOOKUP_GRID_CAP);
+  if (blocks == 0) return hipSuccess;
+  k_lookup<F, G, LEARNED, INDEX><<<blocks, 256, 0, s>>>(
+      t, a.ukey, a.uop, a.gstart, a.npend, a.sidx, a.counters, a.chunk, fill, a.out_vals,
+      a.out_found, LEARNED ? a.route_hdr : nullptr, LEARNED ? a.fences : nullptr,
+      LEARNED ? a.lids : nullptr, LEARNED ? a.segs : nullptr, a.desc, a.ihint, a.gval, a.fanout,
+      a.fanout_cap);
+  return hipGetLastError();
+}
+
 template <int F, int G>
 static hipError_t launch_lookup_fg(const TreeView& t, const LookupArgs& a, hipStream_t s) {
-  const uint64_t groups = (a.n_max + a.chunk - 1) / a.chunk;
-  const uint64_t threads = groups * G;
-  // Persistent grid: at most LOOKUP_GRID_CAP workgroups; each lane group walks one contiguous span.
-  const uint32_t blocks = (uint32_t)std::min<uint64_t>((threads + 255) / 256, LOOKUP_GRID_CAP);
-  if (blocks == 0) return hipSuccess;
-  if (a.route_hdr && a.index)
-    k_lookup<F, G, true, true><<<blocks, 256, 0, s>>>(t, a.ukey, a.uop, a.gstart, a.npend, a.sidx,
-                                                       a.counters, a.chunk, a.out_vals, a.out_found,
-                                                       a.route_hdr, a.fences, a.lids, a.segs, a.desc,
-                                                       a.ihint, a.gval, a.fanout,
-                                                       a.fanout_cap);
-  else if (a.route_hdr)
-    k_lookup<F, G, true, false><<<blocks, 256, 0, s>>>(t, a.ukey, a.uop, a.gstart, a.npend, a.sidx,
-                                                        a.counters, a.chunk, a.out_vals, a.out_found,
-                                                        a.route_hdr, a.fences, a.lids, a.segs, a.desc,
-                                                        a.ihint, a.gval, a.fanout,
-                                                        a.fanout_cap);
-  else
-    k_lookup<F, G, false, false><<<blocks, 256, 0, s>>>(t, a.ukey, a.uop, a.gstart, a.npend, a.sidx,
-                                                         a.counters, a.chunk, a.out_vals, a.out_found,
-                                                         nullptr, nullptr, nullptr, nullptr, a.desc,
-                                                         a.ihint, a.gval, a.fanout,
-                                                         a.fanout_cap);
-  return hipGetLastError();
+  if (a.route_hdr && a.index) return launch_lookup_k<F, G, true, true>(t, a, s);
+  if (a.route_hdr) return launch_lookup_k<F, G, true, false>(t, a, s);
+  return launch_lookup_k<F, G, false, false>(t, a, s);
 }
 
 template <int F>
