@@ -35,10 +35,13 @@ constexpr int OFF_BLOCK = 256;
 constexpr int OFF_ITEMS = 16;
 constexpr int OFF_TILE = OFF_BLOCK * OFF_ITEMS;
 constexpr uint32_t SCAN_GRID_CAP = 2048;
-// Wavefronts that share the scans of one 64-op window.  A scan is a chain of dependent leaf
-// reads, so a window holding several scans set the kernel's time when one wavefront ran them
-// all.
+// Wavefronts that share the scans of one 64-op window: at least SCAN_SPLIT, and up to one per scan
+// while the batch is too short to give the device SCAN_WAVES wavefronts otherwise.  A scan is a
+// chain of dependent leaf reads, so a window holding several scans sets the kernel's time when
+// few wavefronts run them all (4099 ops, half of them scans of 500..8000 pairs: 3.91 ms a call
+// with four wavefronts per window and no load ahead, 0.41 ms now).
 constexpr uint32_t SCAN_SPLIT = 4;
+constexpr uint32_t SCAN_WAVES = 8192;
 constexpr uint32_t SCAN_ROUND_CAP = 1u << 24;
 
 STM_DEV uint64_t scan_len(uint8_t op, uint64_t v) {
@@ -171,60 +174,122 @@ STM_DEV uint32_t lanes_below(uint64_t v, uint32_t n, uint64_t x) {
 
 STM_DEV uint64_t mask_below(uint32_t r) { return r >= 64 ? ~0ull : ((1ull << r) - 1); }
 
+// The leaf that holds key, by a root-to-leaf descent (each level one round trip: a node's keys and
+// children are loaded together).
 template <int F>
 STM_DEV uint32_t wave_find_leaf(const TreeView& t, uint64_t key) {
+  constexpr int SPL = (F + WAVE - 1) / WAVE;
   const uint32_t cap = t.capacity;
   uint32_t node = (uint32_t)min<uint64_t>(uniform64(t.hdr->root), cap - 1);
   const uint32_t height = (uint32_t)min<uint64_t>(uniform64(t.hdr->height), 64);
   const int lane = lane_id();
   for (uint32_t lvl = height; lvl > 1; --lvl) {
+    uint64_t k[SPL], v[SPL];
+#pragma unroll
+    for (int j = 0; j < SPL; ++j) {
+      const uint64_t at = (uint64_t)node * F + (uint32_t)min(j * WAVE + lane, F - 1);
+      k[j] = t.keys[at];
+      v[j] = t.vals[at];
+    }
     uint32_t cnt = 0;
 #pragma unroll
-    for (int s0 = 0; s0 < F; s0 += WAVE) {
-      const int s = s0 + lane;
-      const bool le = s < F && t.keys[(uint64_t)node * F + s] <= key;
-      cnt += (uint32_t)__popcll(ballot(le));
-    }
+    for (int j = 0; j < SPL; ++j)
+      cnt += (uint32_t)__popcll(ballot(j * WAVE + lane < F && k[j] <= key));
     const uint32_t slot = cnt ? cnt - 1 : 0;
-    node = (uint32_t)min<uint64_t>(uniform64(t.vals[(uint64_t)node * F + slot]), cap - 1);
+    uint64_t child = 0;
+#pragma unroll
+    for (int j = 0; j < SPL; ++j)
+      if ((slot >> 6) == (uint32_t)j) child = readlane64(v[j], (int)(slot & 63));
+    node = (uint32_t)min<uint64_t>(child, cap - 1);
   }
   return node;
 }
 
-template <int F>
-STM_DEV uint32_t wave_leaf_below(const TreeView& t, uint32_t leaf, uint64_t key) {
-  const int lane = lane_id();
-  uint32_t cnt = 0;
-#pragma unroll
-  for (int s0 = 0; s0 < F; s0 += WAVE) {
-    const int s = s0 + lane;
-    const bool lt = s < F && t.keys[(uint64_t)leaf * F + s] < key;
-    cnt += (uint32_t)__popcll(ballot(lt));
+// First of the n ascending keys that is not below x: every lane probes one key of the range per
+// step, so a step cuts the range 64-fold (three round trips for 2^18 keys).
+STM_DEV uint32_t wave_lower_bound(const uint64_t* __restrict__ keys, uint32_t n, uint64_t x) {
+  const uint32_t lane = (uint32_t)lane_id();
+  uint32_t lo = 0, hi = n;
+  while (hi - lo > (uint32_t)WAVE) {
+    const uint32_t step = (hi - lo + WAVE - 1) / WAVE;
+    const uint32_t at = lo + lane * step;
+    const uint32_t below = (uint32_t)__popcll(ballot(at < hi && keys[min(at, n - 1)] < x));
+    if (below == 0) return lo;
+    const uint32_t up = min(hi, lo + below * step);
+    lo += (below - 1) * step + 1;
+    hi = up;
   }
-  return cnt;
+  const uint32_t at = lo + lane;
+  return lo + (n ? (uint32_t)__popcll(ballot(at < hi && keys[min(at, n - 1)] < x)) : 0u);
 }
 
-// The entries of leaf `leaf` (the first `count` slots; a leaf's entries are unordered) in key
-// order: position p = j * WAVE + lane holds key sk[j] from slot ss[j] (KEY_EMPTY past count).
-// A bitonic sorting network over the wavefront's N = WAVE * SPL elements (element j * WAVE +
+// A leaf on its way into registers: slot j * WAVE + lane of its keys and values, and its right
+// sibling.  Free slots hold KEY_EMPTY, so the entry count need not be known to load it.
+template <int F>
+struct LeafLoad {
+  static constexpr int SPL = (F + WAVE - 1) / WAVE;
+  uint64_t k[SPL], v[SPL];
+  uint64_t next;
+};
+
+template <int F>
+STM_DEV void load_leaf(const TreeView& t, uint32_t leaf, LeafLoad<F>& b) {
+  const int lane = lane_id();
+  b.next = t.meta[leaf].next;
+#pragma unroll
+  for (int j = 0; j < LeafLoad<F>::SPL; ++j) {
+    const int sl = j * WAVE + lane;
+    const uint64_t at = (uint64_t)leaf * F + (uint32_t)min(sl, F - 1);
+    const uint64_t k = t.keys[at];
+    b.v[j] = t.vals[at];
+    b.k[j] = sl < F ? k : KEY_EMPTY;
+  }
+}
+
+// Element p (lane-dependent, p < F) of a leaf held in registers.
+template <int F, typename T>
+STM_DEV T at_position(const T (&x)[(F + WAVE - 1) / WAVE], uint32_t p) {
+  T r = x[0];
+#pragma unroll
+  for (int j = 0; j < (F + WAVE - 1) / WAVE; ++j) {
+    T v;
+    if constexpr (sizeof(T) == 8) v = shfl64(x[j], (int)(p & 63));
+    else v = (T)__shfl((int)x[j], (int)(p & 63), WAVE);
+    if ((p >> 6) == (uint32_t)j) r = v;
+  }
+  return r;
+}
+
+// The entries of a loaded leaf in key order: position j * WAVE + lane holds key b.k[j] and value
+// b.v[j] (KEY_EMPTY past the last).  A bulk-built leaf and both halves of a split are in key order
+// until an insert is appended, which one comparison with the next slot shows; others go through
+// a bitonic sorting network over the wavefront's N = WAVE * SPL elements (element j * WAVE +
 // lane in register j): 21 compare-exchange steps for N = 64, 28 for 128, each a lane shuffle of
 // the key and slot (or, at distance 64, the lane's other register).  The keys are distinct and
-// KEY_EMPTY pads past count, so the order is exact.  (Ranking each entry with two wave-uniform
+// KEY_EMPTY pads past the last, so the order is exact.  (Ranking each entry with two wave-uniform
 // passes over the entries took a serving batch's scan kernel from 49 to 115 µs.)
 template <int F>
-STM_DEV void leaf_in_key_order(const TreeView& t, uint32_t leaf, uint32_t count,
-                               uint64_t (&sk)[(F + WAVE - 1) / WAVE],
-                               uint32_t (&ss)[(F + WAVE - 1) / WAVE]) {
-  constexpr int SPL = (F + WAVE - 1) / WAVE;
+STM_DEV void leaf_in_key_order(LeafLoad<F>& b) {
+  constexpr int SPL = LeafLoad<F>::SPL;
   constexpr uint32_t N = (uint32_t)(WAVE * SPL);
   static_assert(SPL == 1 || SPL == 2, "one or two slots per lane");
   const uint32_t lane = (uint32_t)lane_id();
+  bool in_order = true;
 #pragma unroll
   for (int j = 0; j < SPL; ++j) {
-    const uint32_t sl = (uint32_t)j * WAVE + lane;
-    sk[j] = sl < count ? t.keys[(uint64_t)leaf * F + sl] : KEY_EMPTY;
-    ss[j] = sl;
+    const uint64_t right = shfl64(b.k[j], (int)min(lane + 1, (uint32_t)WAVE - 1));
+    uint64_t next = right;
+    if constexpr (SPL == 2) {
+      const uint64_t first = readlane64(b.k[1], 0);
+      next = lane == WAVE - 1 ? (j == 0 ? first : KEY_EMPTY) : right;
+    }
+    in_order = in_order && b.k[j] <= next;
   }
+  if (ballot(!in_order) == 0) return;
+  uint64_t (&sk)[SPL] = b.k;
+  uint32_t ss[SPL];
+#pragma unroll
+  for (int j = 0; j < SPL; ++j) ss[j] = (uint32_t)j * WAVE + lane;
 #pragma unroll
   for (uint32_t size = 2; size <= N; size <<= 1) {
 #pragma unroll
@@ -261,60 +326,64 @@ STM_DEV void leaf_in_key_order(const TreeView& t, uint32_t leaf, uint32_t count,
       }
     }
   }
-}
-
-// Entry at key-order position p (lane-dependent, p < F) of a leaf_in_key_order view.
-template <int F, typename T>
-STM_DEV T at_position(const T (&x)[(F + WAVE - 1) / WAVE], uint32_t p) {
-  T r = x[0];
+  uint64_t sv[SPL];
 #pragma unroll
-  for (int j = 0; j < (F + WAVE - 1) / WAVE; ++j) {
-    T v;
-    if constexpr (sizeof(T) == 8) v = shfl64(x[j], (int)(p & 63));
-    else v = (T)__shfl((int)x[j], (int)(p & 63), WAVE);
-    if ((p >> 6) == (uint32_t)j) r = v;
-  }
-  return r;
+  for (int j = 0; j < SPL; ++j) sv[j] = at_position<F>(b.v, ss[j]);
+#pragma unroll
+  for (int j = 0; j < SPL; ++j) b.v[j] = sv[j];
 }
 
-// One scan op, run by the whole wavefront; returns the pairs written.
+// One scan op, run by the whole wavefront; returns the pairs written.  The leaf chain is walked one
+// leaf ahead: the right sibling's load goes out before the current leaf is ordered and written, so
+// a step costs the longer of the two instead of their sum.  Bound by that chain's latency (about
+// 1 µs a leaf), not by bytes.
 template <int F>
 STM_DEV uint32_t run_scan(const TreeView& t, const ScanArgs& a, const ScanIn& in, uint32_t U,
                           uint64_t k, uint32_t i, uint32_t L, uint64_t off) {
   const int lane = lane_id();
   const uint32_t cap = t.capacity;
   constexpr int SPL = (F + WAVE - 1) / WAVE;
-  uint32_t tl = wave_find_leaf<F>(t, k);
-  uint32_t tcount = min(meta_count(uniform64(t.meta[tl].info)), (uint32_t)F);
-  uint64_t tsk[SPL];  // the current leaf in key order
-  uint32_t tss[SPL];
-  leaf_in_key_order<F>(t, tl, tcount, tsk, tss);
-  uint32_t ts = wave_leaf_below<F>(t, tl, k);
-  bool t_done = false;
+  LeafLoad<F> cur, ahead;
+  load_leaf<F>(t, wave_find_leaf<F>(t, k), cur);
   // First group with key >= k (groups are in ascending key order).
-  uint32_t bg;
-  {
-    uint32_t lo = 0, hi = U;
-    while (lo < hi) {
-      const uint32_t mid = (lo + hi) >> 1;
-      if (a.ukey[mid] < k) lo = mid + 1;
-      else hi = mid;
-    }
-    bg = uniform32(lo);
-  }
+  uint32_t bg = wave_lower_bound(a.ukey, U, k);
   uint32_t cnt = 0;
+  uint32_t tl = NODE_NONE;  // the next leaf of the chain, NODE_NONE at its end
+  bool loaded = false;      // `ahead` holds it
+  uint32_t ts = 0, tcount = 0;  // key-order positions [ts, tcount) of cur are left
+  bool t_done = false;
+  // Makes the leaf in `cur` current: its entries into key order, its right sibling under way when
+  // the scan will go past it.
+  auto enter = [&](uint64_t from) {
+    const uint64_t nx = uniform64(cur.next);
+    tl = nx < cap ? (uint32_t)nx : NODE_NONE;
+    tcount = 0;
+    ts = 0;
+#pragma unroll
+    for (int j = 0; j < SPL; ++j) {
+      tcount += (uint32_t)__popcll(ballot(cur.k[j] != KEY_EMPTY));
+      ts += (uint32_t)__popcll(ballot(cur.k[j] < from));
+    }
+    loaded = tl != NODE_NONE && L - cnt > tcount - ts;
+    if (loaded) load_leaf<F>(t, tl, ahead);
+    leaf_in_key_order<F>(cur);
+  };
+  enter(k);
+  // The groups [bg, bg + 64) as the scan sees them, loaded when bg moves: key, whether the group
+  // inserts before op i, and the value it then holds.
+  uint32_t bn = 0, bg_at = NODE_NONE;
+  uint64_t bk = KEY_EMPTY, bval = 0;
+  bool bv = false, vis = false;
   // Every round consumes a whole chunk of one stream; the caps only guard a corrupt pool.
   for (uint32_t round = 0; cnt < L && round < SCAN_ROUND_CAP; ++round) {
     // Next non-empty leaf chunk.
     for (uint32_t hop = 0; !t_done && ts >= tcount; ++hop) {
-      const uint64_t nx = uniform64(t.meta[tl].next);
-      if (nx == NODE_NONE || nx >= cap || hop >= SCAN_ROUND_CAP) {
+      if (tl == NODE_NONE || hop >= SCAN_ROUND_CAP) {
         t_done = true;
       } else {
-        tl = (uint32_t)nx;
-        tcount = min(meta_count(uniform64(t.meta[tl].info)), (uint32_t)F);
-        leaf_in_key_order<F>(t, tl, tcount, tsk, tss);
-        ts = 0;
+        if (!loaded) load_leaf<F>(t, tl, ahead);
+        cur = ahead;
+        enter(0);
       }
     }
     if (t_done && bg >= U) break;
@@ -323,38 +392,52 @@ STM_DEV uint32_t run_scan(const TreeView& t, const ScanArgs& a, const ScanIn& in
     // Key-order position ts + lane, read from every lane (the shuffles need their sources
     // active) and then selected.
     const uint32_t tp = min(ts + (uint32_t)lane, (uint32_t)F - 1);
-    const uint64_t tk_at = at_position<F>(tsk, tp);
-    const uint64_t tslot = (uint64_t)tl * F + at_position<F>(tss, tp);
+    const uint64_t tk_at = at_position<F>(cur.k, tp);
+    const uint64_t tval = at_position<F>(cur.v, tp);
     const uint64_t tk = tv ? tk_at : KEY_EMPTY;
-    const bool t_more = !t_done && (ts + tn < tcount || uniform64(t.meta[tl].next) != NODE_NONE);
+    const bool t_more = !t_done && (ts + tn < tcount || tl != NODE_NONE);
     const uint64_t lastT = t_more ? readlane64(tk, (int)tn - 1) : KEY_EMPTY;
 
-    const uint32_t bn = bg < U ? min(U - bg, (uint32_t)WAVE) : 0u;
-    const bool bv = (uint32_t)lane < bn;
-    uint64_t bk = KEY_EMPTY;
-    uint64_t bval = 0;
-    bool vis = false;
-    if (bv) {
-      const uint32_t g = bg + lane;
-      bk = a.ukey[g];
-      if (a.uop[g] == OP_INSERT) {
-        const uint32_t gs = a.gstart[g];
-        const uint32_t fi = gs + max(a.npend[g], 1u) - 1;  // sorted index of the first insert
-        const uint32_t ge = (g + 1 < U) ? a.gstart[g + 1] : in.n;
-        if (pos_of(a.sidx[fi]) < i) {
-          uint32_t lo = fi, hi = ge;  // sidx[lo] < i; the last such entry lies in [lo, hi)
-          while (hi - lo > 1) {
-            const uint32_t mid = (lo + hi) >> 1;
-            if (pos_of(a.sidx[mid]) < i) lo = mid;
-            else hi = mid;
-          }
-          const int32_t li = a.lastins[lo];
-          if (li >= 0) {
-            vis = true;
-            bval = in.vals[pos_of(a.sidx[li])];
+    if (bg != bg_at) {
+      bg_at = bg;
+      bn = bg < U ? min(U - bg, (uint32_t)WAVE) : 0u;
+      bv = (uint32_t)lane < bn;
+      bk = KEY_EMPTY;
+      bval = 0;
+      vis = false;
+      if (bv) {
+        const uint32_t g = bg + lane;
+        bk = a.ukey[g];
+        if (a.uop[g] == OP_INSERT) {
+          const uint32_t gs = a.gstart[g];
+          const uint32_t fi = gs + max(a.npend[g], 1u) - 1;  // sorted index of the first insert
+          const uint32_t ge = (g + 1 < U) ? a.gstart[g + 1] : in.n;
+          if (pos_of(a.sidx[fi]) < i) {
+            uint32_t lo = fi, hi = ge;  // sidx[lo] < i; the last such entry lies in [lo, hi)
+            while (hi - lo > 1) {
+              const uint32_t mid = (lo + hi) >> 1;
+              if (pos_of(a.sidx[mid]) < i) lo = mid;
+              else hi = mid;
+            }
+            const int32_t li = a.lastins[lo];
+            if (li >= 0) {
+              vis = true;
+              bval = in.vals[pos_of(a.sidx[li])];
+            }
           }
         }
       }
+    }
+    const uint32_t room = L - cnt;
+    if (tn && (bn == 0 || readlane64(bk, 0) > lastT)) {
+      // No group of the batch falls into this chunk: its entries as they are.
+      if (tv && (uint32_t)lane < room) {
+        in.scan_keys[off + cnt + lane] = tk;
+        in.scan_vals[off + cnt + lane] = tval;
+      }
+      cnt += min(tn, room);
+      ts += tn;
+      continue;
     }
     const bool b_more = bg + bn < U;
     const uint64_t lastB = b_more ? readlane64(bk, (int)bn - 1) : KEY_EMPTY;
@@ -371,13 +454,12 @@ STM_DEV uint32_t run_scan(const TreeView& t, const ScanArgs& a, const ScanIn& in
     const uint64_t tM = ballot(t_el);
     const uint32_t rT = lanes_below(tk, tn, bk);  // tree keys below this group key
     const uint64_t lt = lanemask_lt();
-    const uint32_t room = L - cnt;
     if (t_el && !shadow) {
       const uint32_t p = (uint32_t)lane - (uint32_t)__popcll(shM & lt) +
                          (uint32_t)__popcll(visM & mask_below(rB));
       if (p < room) {
         in.scan_keys[off + cnt + p] = tk;
-        in.scan_vals[off + cnt + p] = t.vals[tslot];
+        in.scan_vals[off + cnt + p] = tval;
       }
     }
     if (b_el) {
@@ -398,7 +480,7 @@ STM_DEV uint32_t run_scan(const TreeView& t, const ScanArgs& a, const ScanIn& in
 // One wavefront per window of 64 input positions: the window's scan ops run one after the
 // other, each by the whole wavefront.  soff[i] becomes the pair count of scan op i.
 template <int F>
-__global__ __launch_bounds__(256) void k_range_scan(TreeView t, ScanArgs a) {
+__global__ __launch_bounds__(256) void k_range_scan(TreeView t, ScanArgs a, uint32_t split) {
   const ScanIn in = scan_in(a);
   const uint32_t U = a.counters->n_unique;
   const int lane = lane_id();
@@ -406,16 +488,16 @@ __global__ __launch_bounds__(256) void k_range_scan(TreeView t, ScanArgs a) {
   const uint64_t nwaves = (uint64_t)gridDim.x * blockDim.x / WAVE;
   const uint64_t nwin = ((uint64_t)in.n + WAVE - 1) / WAVE;
   const uint64_t lt = lanemask_lt();
-  // Work item p = (window p / SCAN_SPLIT, share p % SCAN_SPLIT): the wavefront runs the scans
-  // of the window whose rank among the window's scans is p % SCAN_SPLIT modulo SCAN_SPLIT, so
-  // a window with several scans spreads them over SCAN_SPLIT wavefronts.
-  for (uint64_t p = wave0; p < nwin * SCAN_SPLIT; p += nwaves) {
-    const uint64_t w = p / SCAN_SPLIT;
-    const uint32_t share = (uint32_t)(p % SCAN_SPLIT);
+  // Work item p = (window p / split, share p % split): the wavefront runs the scans of the window
+  // whose rank among the window's scans is p % split modulo split, so a window with several scans
+  // spreads them over split wavefronts.
+  for (uint64_t p = wave0; p < nwin * split; p += nwaves) {
+    const uint64_t w = p / split;
+    const uint32_t share = (uint32_t)(p % split);
     const uint64_t i_l = w * WAVE + lane;
     const bool is_scan = i_l < in.n && in.ops[i_l] == OP_RANGE;
     const uint32_t rank = (uint32_t)__popcll(ballot(is_scan) & lt);
-    const bool mine = is_scan && rank % SCAN_SPLIT == share;
+    const bool mine = is_scan && rank % split == share;
     uint64_t todo = ballot(mine);
     uint64_t k_l = 0, v_l = 0, off_l = 0;
     if (mine) {
@@ -471,9 +553,12 @@ hipError_t launch_scan_offsets(const ScanArgs& a, hipStream_t s) {
 
 template <int F>
 static hipError_t launch_range_scan_f(const TreeView& t, const ScanArgs& a, hipStream_t s) {
-  const uint64_t waves = ((uint64_t)a.n + WAVE - 1) / WAVE * SCAN_SPLIT;
+  const uint64_t windows = ((uint64_t)a.n + WAVE - 1) / WAVE;
+  uint32_t split = SCAN_SPLIT;
+  while (split < (uint32_t)WAVE && windows * split < SCAN_WAVES) split *= 2;
+  const uint64_t waves = windows * split;
   const uint32_t blocks = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((waves + 3) / 4, SCAN_GRID_CAP));
-  k_range_scan<F><<<blocks, 256, 0, s>>>(t, a);
+  k_range_scan<F><<<blocks, 256, 0, s>>>(t, a, split);
   return hipGetLastError();
 }
 

@@ -152,3 +152,30 @@ def test_scan_bad_length_rejected():
                                  np.array([3], dtype=np.uint8))
             assert e.value.code == 1
         assert t.check() == 0
+
+
+@pytest.mark.parametrize("n", [1, 64, 65, 1000, 33000])
+@pytest.mark.parametrize("fanout", [32, 64, 128])
+def test_scan_batch_sizes_over_unordered_leaves(oracle_mod, n, fanout):
+    """Few ops (a wavefront per scan) to many (four per 64-op window), over leaves in key order
+    (just built), leaves with appended entries and split ones, with scans that end inside a leaf,
+    at its last entry and past the key space."""
+    rng = np.random.default_rng(n + fanout)
+    load = rng.integers(0, 1 << 62, 30000, dtype=np.uint64)
+    o = oracle_mod.Oracle()
+    o.bulk_load(load, load)
+    with tree(fanout=fanout) as t:
+        t.bulk_load(load, load)
+        for part in (0.0, 0.3):
+            keys = rng.integers(0, 1 << 62, n, dtype=np.uint64)
+            keys[0] = (1 << 62) - 1
+            ops = rng.choice(np.array([0, 1, 3], dtype=np.uint8), n, p=[part, 0.6 - part, 0.4])
+            ops[0] = 3
+            vals = rng.integers(0, 1 << 40, n, dtype=np.uint64)
+            s = ops == 3
+            vals[s] = rng.integers(1, 4 * fanout, int(s.sum()))
+            check_scan_batch(t, o, keys, vals, ops, f"n={n} inserts={part}")
+            more = rng.integers(0, 1 << 62, 9000, dtype=np.uint64)  # appended entries, some splits
+            zero = np.zeros(more.size, dtype=np.uint8)
+            assert np.array_equal(t.run_batch(more, more, zero)[0], o.run_batch(more, more, zero)[0])
+        assert t.check() == 0
