@@ -26,6 +26,7 @@ ARCH = os.environ.get("STM_OFFLOAD_ARCH", "gfx950")
 HIP_SOURCES = [
     "stm_sort.hip",
     "stm_fold.hip",
+    "stm_front.hip",
     "stm_tree.hip",
     "stm_learned.hip",
     "stm_scan.hip",

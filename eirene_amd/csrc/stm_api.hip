@@ -60,10 +60,10 @@ struct StreamAcc {
   unsigned long long bad;      // ops rejected for the reserved key
   unsigned long long batches;  // batches that ran
   unsigned long long skipped;  // batches skipped after an error
-  unsigned long long sort_stalls;  // batches whose sort gave up a look-back wait
+  unsigned long long sort_stalls;  // batches whose sort gave up a grid-barrier wait
   unsigned long long fallbacks;    // batches whose normalized sort fell back to the exact passes
   unsigned long long leaf_splits;  // leaves the batches split
-  unsigned long long pad[1];
+  unsigned long long retries;      // a batch whose small-batch sort overflowed a bucket
 };
 
 constexpr uint32_t DESC_TABLE = 4096;  // descriptors uploaded per window of a stream
@@ -78,7 +78,7 @@ __global__ void k_advance(const BatchDesc* __restrict__ table, uint32_t* __restr
   if (threadIdx.x != 0) return;
   const uint32_t c = cursor[0];
   BatchDesc d = table[c];
-  if (acc->bad || acc->sort_stalls || hdr->error) d.n = 0;
+  if (acc->bad || acc->sort_stalls || acc->retries || hdr->error) d.n = 0;
   *live = d;
   cursor[0] = c + 1;
 }
@@ -89,6 +89,10 @@ __global__ void k_epilogue(const BatchCounters* __restrict__ cnt, const BatchDes
   if (threadIdx.x != 0) return;
   if (live->n == 0) {
     acc->skipped += 1;
+    return;
+  }
+  if (cnt->sort_retry) {  // ran empty: the host runs it again and resumes the stream after it
+    acc->retries += 1;
     return;
   }
   acc->unique += cnt->n_unique;
@@ -106,7 +110,7 @@ __global__ void k_gate(const StreamAcc* __restrict__ acc, const TreeHeader* __re
                        BatchDesc* __restrict__ live, BatchCounters* __restrict__ cnt) {
   if (threadIdx.x != 0) return;
   if (live->n == 0) return;
-  if (acc->bad || acc->sort_stalls || hdr->error) {
+  if (acc->bad || acc->sort_stalls || acc->retries || hdr->error) {
     live->n = 0;
     cnt->n_unique = 0;
     cnt->n_upserts = 0;
@@ -134,6 +138,7 @@ struct Scratch {
   uint64_t *skeys_tmp = nullptr, *skeys = nullptr;
   uint32_t *sidx_tmp = nullptr, *sidx = nullptr;
   uint32_t* hist = nullptr;
+  uint32_t* front = nullptr;  // front half of small batches (front_scratch_words)
   void* fold_tiles = nullptr;
   uint64_t *ukey = nullptr, *uval = nullptr;
   uint8_t* uop = nullptr;
@@ -167,6 +172,7 @@ struct Scratch {
     }
     A_(skeys_tmp, cap); A_(skeys, cap); A_(sidx_tmp, cap); A_(sidx, cap);
     A_(hist, sort_hist_words(cap));
+    A_(front, front_scratch_words());
     uint8_t* ft = nullptr;
     A_(ft, fold_scratch_bytes(cap));
     fold_tiles = ft;
@@ -208,7 +214,7 @@ struct Scratch {
   }
   void release() {
     void* ps[] = {in_keys, in_vals, out_vals, in_ops, out_found, skeys_tmp, skeys, sidx_tmp, sidx,
-                  hist, fold_tiles, ukey, uval, uop, gstart, npend, dlist, ihint, slist, scount, ilist, fanout, counters,
+                  hist, front, fold_tiles, ukey, uval, uop, gstart, npend, dlist, ihint, slist, scount, ilist, fanout, counters,
                   desc_table, desc_live, cursor, acc, soff, lastins, scan_tiles};
     for (void* p : ps)
       if (p) (void)hipFree(p);
@@ -254,9 +260,14 @@ struct stm_tree {
   // sort had to fall back (long buckets of distinct keys: hot keys with neighbours) makes the
   // next EXACT_HOLD batches use the eight exact passes directly.  graphs_exact: the form the
   // captured graphs hold.
+  // A smaller batch is sorted by the front half's own sort unless front_hold > 0: one that
+  // overflowed a bucket there makes the next EXACT_HOLD of them use the exact passes too
+  // (graphs_front_exact: the form the captured graphs of those sizes hold).
   uint32_t exact_left = 0;
   bool graphs_exact = false;
-  uint64_t sort_fallbacks = 0;  // batches whose normalized sort fell back (stm_stats)
+  uint32_t front_hold = 0;
+  bool graphs_front_exact = false;
+  uint64_t sort_fallbacks = 0;  // batches sorted again with the exact passes (stm_stats)
 };
 
 namespace {
@@ -476,11 +487,6 @@ hipError_t enqueue_front(stm_tree* t, Scratch& s, const PipeIn& in, bool timed, 
                          hipStream_t st) {
   hipError_t e;
   if (timed) phase_begin(t, STM_PHASE_SORT);
-  e = radix_sort_pairs_desc(in.keys, in.ops, in.desc, in.n, s.skeys_tmp, s.skeys, s.sidx_tmp, s.sidx, 0,
-                            64, s.hist, (int)t->cfg.sort_tile_items, exact, st);
-  if (e != hipSuccess) return e;
-  if (timed) phase_switch(t, STM_PHASE_SORT, STM_PHASE_MERGE);
-
   FoldArgs fa{};
   fa.skeys = s.skeys;
   fa.sidx = s.sidx;
@@ -499,6 +505,19 @@ hipError_t enqueue_front(stm_tree* t, Scratch& s, const PipeIn& in, bool timed, 
   fa.tile_scratch = s.fold_tiles;
   fa.lastins = in.scans ? s.lastins : nullptr;
   fa.ilist = s.ilist;
+  if (in.n <= FRONT_MAX_OPS && !exact) {
+    const FrontArgs fr{in.keys, in.ops, fa, s.skeys_tmp, s.sidx_tmp, s.front};
+    if ((e = front_batch(fr, st)) != hipSuccess) return e;
+    if (timed) {  // sort and fold in one phase
+      phase_switch(t, STM_PHASE_SORT, STM_PHASE_MERGE);
+      phase_switch(t, STM_PHASE_MERGE, STM_PHASE_LOOKUP);
+    }
+    return hipSuccess;
+  }
+  e = radix_sort_pairs_desc(in.keys, in.ops, in.desc, in.n, s.skeys_tmp, s.skeys, s.sidx_tmp, s.sidx, 0,
+                            64, s.hist, (int)t->cfg.sort_tile_items, exact, st);
+  if (e != hipSuccess) return e;
+  if (timed) phase_switch(t, STM_PHASE_SORT, STM_PHASE_MERGE);
   fa.sort_stall = sort_stall_word(s.hist);
   fa.sort_exact = sort_exact_word(s.hist);
   if ((e = fold_batch(fa, st)) != hipSuccess) return e;
@@ -648,20 +667,30 @@ int run_chunk(stm_tree* t, const uint64_t* keys, const uint64_t* vals, const uin
   } else {
     in.host_counters = s.h_counters;  // the scan answers kernel runs after the upsert kernels
   }
-  const bool exact = t->exact_left > 0;
-  HIP_TRY(enqueue_pipeline(t, s, in, true, exact));
-  // One readback per batch, into pinned memory: counters and the tree's error bits.
-  if (so)
-    HIP_TRY(hipMemcpyAsync(s.h_counters, s.counters, sizeof(BatchCounters), hipMemcpyDeviceToHost, st));
-  HIP_TRY(hipStreamSynchronize(st));
-  const BatchCounters bc = *s.h_counters;
+  const bool small = n <= FRONT_MAX_OPS;
+  uint32_t& hold = small ? t->front_hold : t->exact_left;
+  bool exact = hold > 0;
+  BatchCounters bc;
+  for (;;) {
+    HIP_TRY(enqueue_pipeline(t, s, in, true, exact));
+    // One readback per batch, into pinned memory: counters and the tree's error bits.
+    if (so)
+      HIP_TRY(hipMemcpyAsync(s.h_counters, s.counters, sizeof(BatchCounters), hipMemcpyDeviceToHost, st));
+    HIP_TRY(hipStreamSynchronize(st));
+    bc = *s.h_counters;
+    if (!bc.sort_retry || exact) break;
+    // The small-batch sort overflowed a bucket and the batch ran empty: once more, exactly.
+    exact = true;
+    hold = EXACT_HOLD + 1;  // this batch and the next EXACT_HOLD
+    t->sort_fallbacks += 1;
+  }
   phase_collect(t);
-  if (bc.sort_stall) return fail(STM_ERR_DEVICE, "batch sort: a look-back wait gave up");
+  if (bc.sort_stall) return fail(STM_ERR_DEVICE, "batch sort: a grid-barrier wait gave up");
   if (bc.sort_fallback) {
     t->exact_left = EXACT_HOLD;
     t->sort_fallbacks += 1;
   } else if (exact) {
-    t->exact_left -= 1;
+    hold -= 1;
   }
   t->st.batches += 1;
   t->st.ops += n;
@@ -725,7 +754,8 @@ int capture_pair(stm_tree* t, int c, int k) {
     if (half == 0) {
       k_advance<<<1, 64, 0, st>>>(s0.desc_table, s0.cursor, s.desc_live, s0.acc, t->view.hdr);
       e = hipGetLastError();
-      if (e == hipSuccess) e = enqueue_front(t, s, in, false, t->graphs_exact, st);
+      const bool exact = in.n <= FRONT_MAX_OPS ? t->graphs_front_exact : t->graphs_exact;
+      if (e == hipSuccess) e = enqueue_front(t, s, in, false, exact, st);
     } else {
       k_gate<<<1, 64, 0, st>>>(s0.acc, t->view.hdr, s.desc_live, s.counters);
       e = hipGetLastError();
@@ -755,31 +785,22 @@ int capture_class(stm_tree* t, int c) {
   return rc;
 }
 
-int run_stream(stm_tree* t, const uint64_t* keys, const uint64_t* vals, const uint8_t* ops,
-               const uint64_t* offsets, size_t nb, uint64_t* out_vals, uint8_t* out_found) {
+// Replays the graphs of descs[at..]; ran = how many of them ran.  Fewer than all with STM_OK: the
+// next one's small-batch sort overflowed a bucket, and it and the later ones ran empty.
+int replay_stream(stm_tree* t, const std::vector<BatchDesc>& descs, const std::vector<uint8_t>& cls,
+                  size_t at, size_t& ran) {
   Scratch& s = t->scr;
   hipStream_t st = t->stream;
-  const uint64_t mb = t->cfg.max_batch;
-  // Batches cut into chunks of at most max_batch ops, in order.
-  std::vector<BatchDesc> descs;
-  std::vector<uint8_t> cls;
-  for (size_t b = 0; b < nb; ++b) {
-    for (uint64_t off = offsets[b]; off < offsets[b + 1]; off += mb) {
-      const uint32_t m = (uint32_t)std::min<uint64_t>(mb, offsets[b + 1] - off);
-      descs.push_back(BatchDesc{keys + off, vals + off, ops + off, out_vals + off, out_found + off, m,
-                                0, nullptr, nullptr, 0});
-      cls.push_back((uint8_t)class_of(t, m));
-    }
-  }
-  if (descs.empty()) return STM_OK;
+  ran = 0;
   int rc = maybe_retrain(t);  // learned routing: the router's buffers exist before capture
   if (rc) return rc;
-  if (t->graphs_exact != (t->exact_left > 0)) {  // graphs of the other sort form
-    drop_graphs(t);
+  if (t->graphs_exact != (t->exact_left > 0) || t->graphs_front_exact != (t->front_hold > 0)) {
+    drop_graphs(t);  // graphs of the other sort form
     t->graphs_exact = t->exact_left > 0;
+    t->graphs_front_exact = t->front_hold > 0;
   }
-  for (uint8_t c : cls) {
-    rc = capture_class(t, c);
+  for (size_t i = at; i < descs.size(); ++i) {
+    rc = capture_class(t, cls[i]);
     if (rc) return rc;
   }
   // Batch i runs on scratch set i % 2: its front half on stream_front once the back half of
@@ -789,7 +810,7 @@ int run_stream(stm_tree* t, const uint64_t* keys, const uint64_t* vals, const ui
   hipStream_t sf = t->stream_front;
   bool used[2] = {false, false};
   HIP_TRY(hipMemsetAsync(s.acc, 0, sizeof(StreamAcc), st));
-  for (size_t w0 = 0; w0 < descs.size(); w0 += DESC_TABLE) {
+  for (size_t w0 = at; w0 < descs.size(); w0 += DESC_TABLE) {
     const size_t w1 = std::min<size_t>(descs.size(), w0 + DESC_TABLE);
     // The window's table and cursor are replaced once every front half of the previous window
     // has taken its descriptor.
@@ -821,13 +842,20 @@ int run_stream(stm_tree* t, const uint64_t* keys, const uint64_t* vals, const ui
   HIP_TRY(hipStreamWaitEvent(st, t->ev_sync, 0));
   HIP_TRY(hipMemcpyAsync(&acc, s.acc, sizeof(acc), hipMemcpyDeviceToHost, st));
   HIP_TRY(hipStreamSynchronize(st));
+  ran = (size_t)acc.batches;
+  if (acc.retries) {  // the failing batch and those after it did not run: taken out again
+    for (size_t i = at + ran; i < descs.size(); ++i) t->st.ops -= descs[i].n;
+    t->st.batches -= descs.size() - at - ran;
+    t->batches_since_train -= (uint32_t)std::min<uint64_t>(t->batches_since_train, descs.size() - at - ran);
+  }
   t->st.unique_ops += acc.unique;
   t->sort_fallbacks += acc.fallbacks;
   t->splits_since_train += acc.leaf_splits;
   if (acc.fallbacks) t->exact_left = EXACT_HOLD;
   else if (t->graphs_exact) t->exact_left -= (uint32_t)std::min<uint64_t>(t->exact_left, acc.batches);
+  if (t->graphs_front_exact) t->front_hold -= (uint32_t)std::min<uint64_t>(t->front_hold, acc.batches);
   if (acc.sort_stalls)
-    return fail(STM_ERR_DEVICE, "a batch sort gave up a look-back wait (%llu later batches skipped)",
+    return fail(STM_ERR_DEVICE, "a batch sort gave up a grid-barrier wait (%llu later batches skipped)",
                 acc.skipped);
   if (acc.bad)
     return fail(STM_ERR_INVALID, "a batch holds the reserved key 0xffffffffffffffff (%llu later batches skipped)",
@@ -839,6 +867,37 @@ int run_stream(stm_tree* t, const uint64_t* keys, const uint64_t* vals, const ui
     g_last_error += buf;
   }
   return rc;
+}
+
+int run_stream(stm_tree* t, const uint64_t* keys, const uint64_t* vals, const uint8_t* ops,
+               const uint64_t* offsets, size_t nb, uint64_t* out_vals, uint8_t* out_found) {
+  const uint64_t mb = t->cfg.max_batch;
+  // Batches cut into chunks of at most max_batch ops, in order.
+  std::vector<BatchDesc> descs;
+  std::vector<uint8_t> cls;
+  for (size_t b = 0; b < nb; ++b) {
+    for (uint64_t off = offsets[b]; off < offsets[b + 1]; off += mb) {
+      const uint32_t m = (uint32_t)std::min<uint64_t>(mb, offsets[b + 1] - off);
+      descs.push_back(BatchDesc{keys + off, vals + off, ops + off, out_vals + off, out_found + off, m,
+                                0, nullptr, nullptr, 0});
+      cls.push_back((uint8_t)class_of(t, m));
+    }
+  }
+  for (size_t at = 0; at < descs.size();) {
+    size_t ran = 0;
+    int rc = replay_stream(t, descs, cls, at, ran);
+    if (rc) return rc;
+    at += ran;
+    if (at >= descs.size()) break;
+    // One batch's small-batch sort overflowed: it runs on its own with the exact sort (as do the
+    // next EXACT_HOLD batches), then the stream goes on.
+    t->front_hold = EXACT_HOLD + 1;
+    t->sort_fallbacks += 1;
+    const BatchDesc& d = descs[at++];
+    rc = run_chunk(t, d.keys, d.vals, d.ops, d.n, d.out_vals, d.out_found);
+    if (rc) return rc;
+  }
+  return STM_OK;
 }
 
 int validate_host_batch(const uint64_t* keys, const uint8_t* ops, size_t n, bool need_vals,
@@ -907,7 +966,7 @@ int build_from_device(stm_tree* t, const uint64_t* keys, const uint64_t* vals, s
         rc = fail(STM_ERR_DEVICE, "bulk-load counters");
         break;
       }
-      if (bc.sort_stall) { rc = fail(STM_ERR_DEVICE, "bulk-load sort: a look-back wait gave up"); break; }
+      if (bc.sort_stall) { rc = fail(STM_ERR_DEVICE, "bulk-load sort: a grid-barrier wait gave up"); break; }
       if (bc.n_bad) { rc = fail(STM_ERR_INVALID, "bulk load holds the reserved key"); break; }
       U = bc.n_unique;
     }
@@ -989,8 +1048,7 @@ constexpr int NOALLOC_DEVICES = 64;
 NoAllocSlot g_noalloc[NOALLOC_DEVICES];
 
 // Lays the batch scratch out in the device's copy of `scratch` (set up on the first call on
-// the device: address lookup, then the sort's control words cleared so its look-back status
-// starts untagged).  Nothing is allocated.  The caller has made the tree's device current.
+// the device: address lookup, then the sort's control words cleared).  Nothing is allocated.  The caller has made the tree's device current.
 int noalloc_scratch(stm_tree* t, Scratch& s) {
   const int dev = t->cfg.device;
   if (dev < 0 || dev >= NOALLOC_DEVICES)
@@ -1487,7 +1545,7 @@ int stm_dump(stm_tree* t, uint64_t* keys, uint64_t* vals, size_t cap, size_t* n)
   if (hipMemcpyAsync(&stalled, sort_stall_word(hist), 4, hipMemcpyDeviceToHost, st) != hipSuccess ||
       hipStreamSynchronize(st) != hipSuccess)
     return err(STM_ERR_DEVICE, "leaf order");
-  if (stalled) return err(STM_ERR_DEVICE, "leaf order: a sort look-back wait gave up");
+  if (stalled) return err(STM_ERR_DEVICE, "leaf order: a sort grid-barrier wait gave up");
   std::vector<uint32_t> hc(n_leaves);
   if (n_leaves && (hipMemcpyAsync(hc.data(), counts, 4ull * n_leaves, hipMemcpyDeviceToHost, st) != hipSuccess ||
                    hipStreamSynchronize(st) != hipSuccess))

@@ -22,6 +22,7 @@
 // each group up to and including its first insert waits for the tree ("npend" ops from
 // "gstart").
 #include "stm_common.hpp"
+#include "stm_fold.hpp"
 #include "stm_internal.hpp"
 
 namespace stm {
@@ -31,34 +32,6 @@ constexpr int FOLD_WAVES = FOLD_BLOCK / WAVE;
 constexpr int FOLD_ROUNDS = 8;                     // rounds of WAVE elements per wavefront
 constexpr int FOLD_CHUNK = FOLD_ROUNDS * WAVE;     // elements of one wavefront
 constexpr int FOLD_TILE = FOLD_WAVES * FOLD_CHUNK;  // elements of one block
-
-struct Acc {
-  uint32_t c;    // group heads in the range
-  int32_t head;  // position of the last head (-1 if none)
-  int32_t ins;   // position of the last INSERT (-1 if none)
-};
-
-STM_DEV Acc acc_identity() { return Acc{0u, -1, -1}; }
-STM_DEV Acc acc_combine(const Acc& a, const Acc& b) {
-  return Acc{a.c + b.c, max(a.head, b.head), max(a.ins, b.ins)};
-}
-
-// Position of the highest lane set in m within a round starting at rb, or `none`.
-STM_DEV int32_t last_set(uint64_t m, uint32_t rb, int32_t none) {
-  return m ? (int32_t)(rb + 63u - (uint32_t)__clzll((long long)m)) : none;
-}
-
-// With a batch descriptor the element count and the caller's arrays come from device memory
-// (one launch sequence serves every batch size).
-STM_DEV void fold_resolve(FoldArgs& a) {
-  const BatchDesc* d = a.desc;
-  if (!d) return;
-  a.n = d->n;
-  a.vals = d->vals;
-  a.ops = d->ops;
-  a.out_vals = d->out_vals;
-  a.out_found = d->out_found;
-}
 
 // A wavefront's chunk: element r * WAVE + lane of the chunk in k[r], sx[r] of that lane.
 struct Chunk {
@@ -190,7 +163,7 @@ __global__ __launch_bounds__(FOLD_BLOCK) void k_fold_scan_tiles(Acc* tile_agg, F
     run = acc_combine(run, t);
   }
   if (threadIdx.x == 0) {
-    // A sort that gave up a look-back wait may have mis-ordered the batch: the batch then has
+    // A sort that gave up a grid-barrier wait may have mis-ordered the batch: the batch then has
     // no groups, so the fold, lookup, scan and upsert kernels do nothing and the tree keeps
     // its state from before the batch.
     const uint32_t stalled = a.sort_stall ? *a.sort_stall : 0u;
@@ -202,6 +175,7 @@ __global__ __launch_bounds__(FOLD_BLOCK) void k_fold_scan_tiles(Acc* tile_agg, F
     counters->n_fanout = 0;
     counters->sort_stall = stalled;
     counters->sort_fallback = a.sort_exact ? *a.sort_exact : 0u;
+    counters->sort_retry = 0;
     counters->leaf_splits = 0;
   }
 }

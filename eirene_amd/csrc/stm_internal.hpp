@@ -34,15 +34,13 @@ __host__ __device__ inline uint32_t op_of(uint32_t payload) { return payload >> 
 // ------------------------------------------------------------------ radix sort (stm_sort.hip)
 // Words of scratch (u32) the sort needs for n elements.
 size_t sort_hist_words(uint64_t n);
-// Prepares freshly allocated sort scratch (synchronous): the single-sweep look-back status
-// must start with no valid tag.
+// Prepares freshly allocated sort scratch (synchronous).
 hipError_t sort_scratch_init(uint32_t* words);
-// Non-zero after a sort whose look-back gave up waiting (its output is then wrong); cleared
-// when the next sort on the same scratch starts.
+// Non-zero after a sort one of whose grid barriers gave up waiting (its output is then wrong);
+// cleared when the next sort on the same scratch starts.
 const uint32_t* sort_stall_word(const uint32_t* words);
-// The three-kernel region of the scratch (at least n/8 words for scratch sized for n), which
-// single-sweep sorts leave alone and three-kernel sorts write before they read: free for other
-// kernels between sorts.
+// The histogram region of the scratch (at least n/8 words for scratch sized for n), which every
+// sort writes before it reads: free for other kernels between sorts.
 uint32_t* sort_spare_words(uint32_t* words);
 // Stable ascending sort of keys[begin_bit, end_bit) with the original index as payload.
 // keys_in is not modified; results land in keys_out / idx_out.
@@ -54,8 +52,8 @@ hipError_t radix_sort_pairs(const uint64_t* keys_in, uint64_t* keys_tmp, uint64_
 // With desc the keys, op codes and their count are read from the device-side descriptor
 // (keys_in and ops_in unused) and n_max only bounds that count (grid and scratch sizing);
 // without it keys_in holds n_max keys.
-// Above 2^18 keys the normalized-key form runs unless `exact` asks for the eight-pass form
-// (the library asks for it after a batch whose normalized sort had to fall back).
+// The normalized-key form runs unless `exact` asks for the eight-pass form (the library asks for
+// it after a batch whose normalized sort had to fall back).
 hipError_t radix_sort_pairs_desc(const uint64_t* keys_in, const uint8_t* ops_in,
                                  const BatchDesc* desc, uint32_t n_max,
                                  uint64_t* keys_tmp, uint64_t* keys_out, uint32_t* idx_tmp,
@@ -76,12 +74,14 @@ struct BatchCounters {
   uint32_t n_bad;       // ops rejected (reserved key)
   uint32_t scan_bad;    // scan ops rejected (length or output area)
   uint64_t scan_total;  // sum of the scan lengths (pairs the output area must hold)
-  uint32_t sort_stall;  // the batch's sort gave up a look-back wait
+  uint32_t sort_stall;  // the batch's sort gave up a grid-barrier wait
   uint32_t n_fanout;    // answer chunks of hot GET groups queued for k_fanout
   uint64_t hdr_error;   // the tree's sticky error bits after the batch (one readback per batch)
   uint32_t sort_fallback;  // the batch's normalized sort fell back to the exact passes
   uint32_t leaf_splits;    // leaves the batch's transactions split
-  uint32_t pad[2];
+  uint32_t sort_retry;     // a bucket of the small-batch sort overflowed: the batch ran empty and
+                           // is to be run again with the exact sort
+  uint32_t pad;
 };
 static_assert(sizeof(BatchCounters) == 64, "one 64-byte block");
 
@@ -109,6 +109,24 @@ struct FoldArgs {
   const uint32_t* sort_stall;  // optional: the sort's stall word, copied into the counters
   const uint32_t* sort_exact;  // optional: the sort's fallback word, copied into the counters
 };
+// ------------------------------------------------------------------ front half of small batches
+// (stm_front.hip): sort and fold of at most FRONT_MAX_OPS ops in one or three launches, with the
+// results of the radix sort and fold_batch.  A whole call on 2^22 uniform keys, with the radix
+// form and the lookup's longer spans in parentheses: 1000 ops 37 µs (113), 16384 ops 60 (123), 2^16
+// ops 73 (144), 2^18 ops 119 (171).  Above
+// 2^18 ops a workgroup's sample sort and the buckets' comparison sorts grow past what they save.
+constexpr uint32_t FRONT_MAX_OPS = 1u << 18;
+struct FrontArgs {
+  const uint64_t* keys;  // the batch (or fold.desc)
+  const uint8_t* ops;
+  FoldArgs fold;         // fold.skeys and fold.sidx are written here; fold.tile_scratch is unused
+  uint64_t* tmp_keys;    // scratch of the batch's size
+  uint32_t* tmp_ties;
+  uint32_t* words;       // front_scratch_words()
+};
+size_t front_scratch_words();
+hipError_t front_batch(const FrontArgs& a, hipStream_t stream);
+
 constexpr uint8_t UOP_SKIP = 0xff;
 constexpr uint8_t OP_RANGE = 3;
 constexpr uint32_t SCAN_MAX_LEN = 65536;  // longest scan (pairs)

@@ -120,9 +120,11 @@ typedef struct stm_stats {
     uint64_t leaf_steps;      /* right-sibling steps taken along the leaf level (learned and index
                                  routing after leaf splits; the reference's leaf traversal steps,
                                  src/gpu-stm-tree-v38/bpt-gpustm.cpp:142-160) */
-    uint64_t sort_fallbacks;  /* batches above 2^18 ops whose sort of normalized keys met a long
-                                 run of close, distinct keys (hot keys with neighbours) and re-sorted
-                                 with the exact passes; the next 16 batches then sort exactly */
+    uint64_t sort_fallbacks;  /* batches sorted a second time with the exact passes: above 2^18
+                                 ops, one whose normalized keys met a long run of close, distinct
+                                 keys (hot keys with neighbours); up to there, one whose keys
+                                 misled the sample its buckets are cut by.  The next 16 such
+                                 batches then sort exactly at once */
 } stm_stats;
 
 typedef struct stm_tree stm_tree;
@@ -154,9 +156,9 @@ int stm_run_batch(stm_tree* tree, const uint64_t* keys, const uint64_t* vals, co
 
 /* Same with device-resident inputs and outputs (d_vals is required).  Work is queued on
  * the tree's stream (stm_get_stream); the call returns after the batch has completed.
- * Batches of at most 2^18 ops are sorted in a single sweep whose waits between workgroups are
- * bounded; a sort that gives up such a wait fails the call with STM_ERR_DEVICE, and that batch
- * then leaves the tree unchanged (its lookups, scans and inserts do not run). */
+ * The exact re-sort of a batch (stm_stats.sort_fallbacks) waits between workgroups, for a bounded
+ * time; a sort that gives up such a wait fails the call with STM_ERR_DEVICE, and that batch then
+ * leaves the tree unchanged (its lookups, scans and inserts do not run). */
 int stm_run_batch_device(stm_tree* tree, const uint64_t* d_keys, const uint64_t* d_vals,
                          const uint8_t* d_ops, size_t n, uint64_t* d_out_vals, uint8_t* d_out_found);
 

@@ -8,7 +8,8 @@ import pytest
 
 pytestmark = pytest.mark.gpu
 
-SIZES = [1, 2, 63, 65, 255, 1000, 2047, 2048, 2049, 4097, 16384, 16385, 28673, 65537, 114689]
+SIZES = [1, 2, 63, 65, 255, 1000, 1024, 1025, 2047, 2048, 2049, 4097, 16384, 16385, 28673, 32769,
+         65536, 65537, 114689, 262144, 262145]
 
 
 def batch(rng, dist, n, load):
@@ -38,7 +39,7 @@ def test_batch_sizes(oracle_mod, n, dist, route, fanout, lanes):
     lv = rng.integers(0, 1 << 63, load.size, dtype=np.uint64)
     o = oracle_mod.Oracle()
     o.bulk_load(load, lv)
-    with StmTree(StmConfig(max_keys=1 << 20, max_batch=1 << 17, route=route, fanout=fanout,
+    with StmTree(StmConfig(max_keys=1 << 20, max_batch=1 << 19, route=route, fanout=fanout,
                            lanes_per_op=lanes, train_steps=20)) as t:
         t.bulk_load(load, lv)
         keys, vals, ops = batch(rng, dist, n, load)
@@ -49,4 +50,50 @@ def test_batch_sizes(oracle_mod, n, dist, route, fanout, lanes):
         k, v = t.dump()
         ek, ev = o.dump()
         assert np.array_equal(k, ek) and np.array_equal(v, ev)
+        assert t.check() == 0
+
+
+def sample_positions(n, s):
+    """Input positions the small-batch sort samples: a hashed place in each of s equal stretches."""
+    def h(x):
+        x = np.uint32(x)
+        x = np.uint32(((int(x) ^ (int(x) >> 16)) * 0x7FEB352D) & 0xFFFFFFFF)
+        x = np.uint32(((int(x) ^ (int(x) >> 15)) * 0x846CA68B) & 0xFFFFFFFF)
+        return int(x) ^ (int(x) >> 16)
+    lo = [j * n // s for j in range(s + 1)]
+    return np.array([lo[j] + ((h(j) * (lo[j + 1] - lo[j])) >> 32) for j in range(s)])
+
+
+@pytest.mark.parametrize("stream", [False, True])
+def test_misleading_sample_sorts_again(oracle_mod, stream):
+    """A batch whose sampled ops all hold low keys puts the rest into one bucket of the small-batch
+    sort: it is sorted again exactly (sort_fallbacks = 1), the batches after it at once."""
+    from eirene_amd import DeviceBuffer, StmConfig, StmTree
+    rng = np.random.default_rng(5)
+    n = 20000
+    load = np.unique(rng.integers(0, 1 << 62, 30000, dtype=np.uint64))
+    o = oracle_mod.Oracle()
+    o.bulk_load(load, load)
+    with StmTree(StmConfig(max_keys=1 << 20, max_batch=1 << 16)) as t:
+        t.bulk_load(load, load)
+        keys, vals, ops = batch(rng, "spread", 4 * n, load)
+        for s in (512, 1024):  # the bucket counts of a 20000-op call and of its replayed size class
+            low = sample_positions(n, s) + n
+            keys[low] = np.sort(rng.choice(1 << 40, low.size, replace=False).astype(np.uint64))
+        rest = np.setdiff1d(np.arange(n, 2 * n), np.concatenate(
+            [sample_positions(n, s) + n for s in (512, 1024)]))
+        keys[rest] = load[100] + rng.integers(0, 1 << 30, rest.size, dtype=np.uint64)
+        offsets = np.arange(0, 4 * n + 1, n).astype(np.uint64)
+        want = [o.run_batch(keys[a:a + n], vals[a:a + n], ops[a:a + n]) for a in range(0, 4 * n, n)]
+        bufs = [DeviceBuffer.from_array(x) for x in (keys, vals, ops)]
+        ov, of = DeviceBuffer(4 * n, np.uint64), DeviceBuffer(4 * n, np.uint8)
+        if stream:
+            t.run_batches_device(*bufs, ov, of, offsets)
+        else:
+            for b in range(4):
+                t.run_batch_device(*bufs, ov, of, n=n, offset=b * n)
+        assert np.array_equal(ov.download(), np.concatenate([w[0] for w in want]))
+        assert np.array_equal(of.download(), np.concatenate([w[1] for w in want]))
+        st = t.stats()
+        assert st["sort_fallbacks"] == 1 and st["batches"] == 4 and st["ops"] == 4 * n
         assert t.check() == 0
