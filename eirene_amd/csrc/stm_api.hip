@@ -131,8 +131,23 @@ __global__ __launch_bounds__(256) void k_copy16(uint4* __restrict__ dst, const u
     dst[i] = src[i];
 }
 
+// Where an array of a slab goes: arrays lie back to back, 256-byte aligned.  One allocation holds
+// them all (a tree has about sixty arrays; each hipMalloc and hipFree of its own cost 10-300 µs,
+// 12 of the 17 ms that creating, loading, using and closing a tree of 2^20 keys took).
+struct SlabCursor {
+  uint8_t* base;  // null: only count
+  size_t at = 0;
+  void* take(size_t bytes) {
+    at = (at + 255) / 256 * 256;
+    void* p = base ? base + at : nullptr;
+    at += std::max<size_t>(bytes, 1);
+    return p;
+  }
+};
+
 struct Scratch {
   uint64_t n = 0;
+  void* slab = nullptr;  // the allocation that holds every device array (null: a fixed region does)
   uint64_t *in_keys = nullptr, *in_vals = nullptr, *out_vals = nullptr;
   uint8_t *in_ops = nullptr, *out_found = nullptr;
   uint64_t *skeys_tmp = nullptr, *skeys = nullptr;
@@ -159,14 +174,15 @@ struct Scratch {
   uint32_t* cursor = nullptr;       // next desc_table entry
   StreamAcc* acc = nullptr;
 
-  // Every device array of the scratch for batches of up to cap ops, in one fixed order:
-  // take(&pointer, bytes) provides each one (allocation, or a place in a fixed region).
-  template <typename Take>
-  hipError_t layout(uint64_t cap, bool staging, Take&& take) {
+  // What a scratch is for: a tree's synchronous calls (host staging and stream control too), the
+  // second set of a batch stream, or one bulk load (sort and fold only).
+  enum Use { CALLS, STREAM, LOAD };
+
+  // Every device array of the scratch for batches of up to cap ops, in one fixed order.
+  void layout(uint64_t cap, Use use, SlabCursor& cur) {
     n = cap;
-    hipError_t e;
-#define A_(p, c) \
-    if ((e = take((void**)&p, sizeof(*p) * std::max<uint64_t>((uint64_t)(c), 1))) != hipSuccess) return e
+#define A_(p, c) p = static_cast<decltype(p)>(cur.take(sizeof(*p) * (size_t)(c)))
+    const bool staging = use == CALLS;
     if (staging) {
       A_(in_keys, cap); A_(in_vals, cap); A_(in_ops, cap); A_(out_vals, cap); A_(out_found, cap);
     }
@@ -176,48 +192,47 @@ struct Scratch {
     uint8_t* ft = nullptr;
     A_(ft, fold_scratch_bytes(cap));
     fold_tiles = ft;
-    A_(ukey, cap); A_(uval, cap); A_(uop, cap); A_(gstart, cap); A_(npend, cap);
+    A_(ukey, cap); A_(uval, cap); A_(uop, cap);
+    A_(counters, 1);
+    if (use == LOAD) return;
+    A_(gstart, cap); A_(npend, cap);
     A_(dlist, cap);
     A_(ihint, cap);
     A_(slist, cap);
     A_(scount, FAST_WAVES_MAX);
     A_(ilist, cap);
     A_(fanout, fanout_capacity(cap));
-    A_(counters, 1);
     A_(desc_live, 1);
     if (staging) {
       A_(desc_table, DESC_TABLE); A_(cursor, 1); A_(acc, 1);
       A_(soff, cap); A_(lastins, cap); A_(scan_tiles, scan_tile_words(cap));
     }
 #undef A_
-    return hipSuccess;
   }
 
-  hipError_t alloc(uint64_t cap, bool staging) {
-    hipError_t e = layout(cap, staging, [](void** p, size_t bytes) { return hipMalloc(p, bytes); });
-    if (e != hipSuccess) return e;
-    if ((e = sort_scratch_init(hist)) != hipSuccess) return e;
+  hipError_t alloc(uint64_t cap, Use use) {
+    SlabCursor size{nullptr};
+    layout(cap, use, size);
+    hipError_t e = hipMalloc(&slab, size.at);
+    if (e != hipSuccess) {
+      *this = Scratch();
+      return e;
+    }
+    SlabCursor place{static_cast<uint8_t*>(slab)};
+    layout(cap, use, place);
+    if ((e = sort_scratch_init(hist)) != hipSuccess || use != CALLS) return e;
     return hipHostMalloc((void**)&h_counters, sizeof(BatchCounters), hipHostMallocCoherent);
   }
 
-  // Lays the arrays out back to back (256-byte aligned) from base; with base null only
-  // counts.  Returns the bytes the layout spans.
+  // Lays the arrays out from base (a fixed region); with base null only counts.  Returns the bytes
+  // the layout spans.
   size_t carve(uint64_t cap, uint8_t* base) {
-    size_t at = 0;
-    (void)layout(cap, false, [&](void** p, size_t bytes) {
-      at = (at + 255) / 256 * 256;
-      *p = base ? base + at : nullptr;
-      at += bytes;
-      return hipSuccess;
-    });
-    return at;
+    SlabCursor cur{base};
+    layout(cap, STREAM, cur);
+    return cur.at;
   }
   void release() {
-    void* ps[] = {in_keys, in_vals, out_vals, in_ops, out_found, skeys_tmp, skeys, sidx_tmp, sidx,
-                  hist, front, fold_tiles, ukey, uval, uop, gstart, npend, dlist, ihint, slist, scount, ilist, fanout, counters,
-                  desc_table, desc_live, cursor, acc, soff, lastins, scan_tiles};
-    for (void* p : ps)
-      if (p) (void)hipFree(p);
+    if (slab) (void)hipFree(slab);
     if (h_counters) (void)hipHostFree(h_counters);
     *this = Scratch();
   }
@@ -229,6 +244,7 @@ struct stm_tree {
   stm_config cfg{};
   hipStream_t stream = nullptr;
   TreeView view{};
+  void* pool = nullptr;  // the allocation behind view's arrays
   uint64_t capacity = 0;
   Scratch scr;
   stm_stats st{};
@@ -238,6 +254,7 @@ struct stm_tree {
   bool phase_used[STM_NUM_PHASES] = {};
   // learned routing
   RouteState route;
+  void* route_slab = nullptr;  // the allocation behind route's arrays
   bool route_alloc = false;
   bool route_valid = false;       // directory + model describe a recent tree
   bool route_warm = false;        // the segment models were trained on this tree
@@ -392,12 +409,22 @@ int alloc_router(stm_tree* t) {
   if (t->route_alloc) return STM_OK;
   RouteState& r = t->route;
   const uint64_t cap = t->capacity;
-  if (dalloc(&r.hdr, 1) || dalloc(&r.fences, cap + 1) || dalloc(&r.lids, cap) ||
-      dalloc(&r.segs, ROUTE_SEGMENTS) || dalloc(&r.dir, cap + 1) || dalloc(&r.rank_of, cap) ||
-      dalloc(&r.lows, cap) || dalloc(&r.lows_tmp, cap) || dalloc(&r.sorted_lows, cap) ||
-      dalloc(&r.order, cap) || dalloc(&r.order_tmp, cap) || dalloc(&r.hist, sort_hist_words(cap)) ||
-      dalloc(&r.dir_alt, cap + 1))
+  auto layout = [&](SlabCursor& cur) {
+#define A_(p, c) p = static_cast<decltype(p)>(cur.take(sizeof(*p) * (size_t)(c)))
+    A_(r.hdr, 1); A_(r.fences, cap + 1); A_(r.lids, cap); A_(r.segs, ROUTE_SEGMENTS);
+    A_(r.dir, cap + 1); A_(r.rank_of, cap); A_(r.lows, cap); A_(r.lows_tmp, cap);
+    A_(r.sorted_lows, cap); A_(r.order, cap); A_(r.order_tmp, cap); A_(r.hist, sort_hist_words(cap));
+    A_(r.dir_alt, cap + 1);
+#undef A_
+  };
+  SlabCursor size{nullptr};
+  layout(size);
+  if (hipMalloc(&t->route_slab, size.at) != hipSuccess) {
+    t->route_slab = nullptr;
     return fail(STM_ERR_NOMEM, "learned-routing buffers for %llu nodes", (unsigned long long)cap);
+  }
+  SlabCursor place{static_cast<uint8_t*>(t->route_slab)};
+  layout(place);
   if (sort_scratch_init(r.hist) != hipSuccess) return fail(STM_ERR_DEVICE, "learned-routing sort scratch");
   t->route_alloc = true;
   t->view.rank_of = r.rank_of;
@@ -407,11 +434,8 @@ int alloc_router(stm_tree* t) {
 }
 
 void free_router(stm_tree* t) {
-  RouteState& r = t->route;
-  void* ps[] = {r.hdr, r.fences, r.lids, r.segs, r.dir, r.rank_of, r.lows, r.lows_tmp,
-                r.sorted_lows, r.order, r.order_tmp, r.hist, r.dir_alt};
-  for (void* p : ps)
-    if (p) (void)hipFree(p);
+  if (t->route_slab) (void)hipFree(t->route_slab);
+  t->route_slab = nullptr;
   t->route = RouteState();
   t->view.rank_of = nullptr;
   t->view.dir = nullptr;
@@ -723,7 +747,7 @@ int class_of(const stm_tree* t, uint32_t n) {
 // The second scratch set, the front stream and the pipeline's events, made on first use.
 int ensure_pipeline(stm_tree* t) {
   if (t->scr2_alloc) return STM_OK;
-  hipError_t e = t->scr2.alloc(t->cfg.max_batch, false);
+  hipError_t e = t->scr2.alloc(t->cfg.max_batch, Scratch::STREAM);
   if (e == hipSuccess) e = hipStreamCreate(&t->stream_front);
   for (int k = 0; k < 2 && e == hipSuccess; ++k) {
     e = hipEventCreateWithFlags(&t->ev_front[k], hipEventDisableTiming);
@@ -933,12 +957,15 @@ int build_from_device(stm_tree* t, const uint64_t* keys, const uint64_t* vals, s
   hipStream_t st = t->stream;
   const uint32_t fill = t->cfg.leaf_fill;
   if (n > 0x7fffffffull) return fail(STM_ERR_INVALID, "bulk load of %zu keys exceeds 2^31-1", n);
-  Scratch tmp;
-  hipError_t e = tmp.alloc(std::max<uint64_t>(n, 1), false);
+  // The tree's own scratch when it is large enough, else one for this load.
+  Scratch own;
+  const bool fits = n <= t->scr.n;
+  hipError_t e = fits ? hipSuccess : own.alloc(n, Scratch::LOAD);
   if (e != hipSuccess) {
-    tmp.release();
+    own.release();
     return fail(STM_ERR_NOMEM, "bulk-load scratch for %zu keys: %s", n, hipGetErrorString(e));
   }
+  Scratch& tmp = fits ? t->scr : own;
   int rc = STM_OK;
   do {
     uint32_t U = 0;
@@ -982,12 +1009,8 @@ int build_from_device(stm_tree* t, const uint64_t* keys, const uint64_t* vals, s
                 (unsigned long long)total, (unsigned long long)t->capacity);
       break;
     }
-    uint64_t *lows_a = nullptr, *lows_b = nullptr;
-    if (dalloc(&lows_a, L) != hipSuccess || dalloc(&lows_b, L) != hipSuccess) {
-      if (lows_a) (void)hipFree(lows_a);
-      rc = fail(STM_ERR_NOMEM, "bulk-load fence arrays");
-      break;
-    }
+    // The levels' low fences ping-pong between the sort's key buffers, which the fold is done with.
+    uint64_t *lows_a = tmp.skeys_tmp, *lows_b = tmp.skeys;
     hipError_t r2 = hipMemsetAsync(t->view.meta, 0, sizeof(NodeMeta) * t->capacity, st);
     if (r2 == hipSuccess)
       r2 = launch_build_leaves(t->view, tmp.ukey, tmp.uval, U, fill, (uint32_t)L, lows_a, st);
@@ -1019,12 +1042,10 @@ int build_from_device(stm_tree* t, const uint64_t* keys, const uint64_t* vals, s
       t->route_valid = false;  // the router describes the previous tree
       t->route_warm = false;
     }
-    (void)hipFree(lows_a);
-    (void)hipFree(lows_b);
     if (r2 != hipSuccess) rc = fail(STM_ERR_DEVICE, "bulk build: %s", hipGetErrorString(r2));
   } while (0);
   (void)hipStreamSynchronize(st);
-  tmp.release();
+  own.release();
   return rc;
 }
 
@@ -1163,16 +1184,24 @@ int stm_create(const stm_config* cfg_in, stm_tree** out) {
   if (hipStreamCreate(&t->stream) != hipSuccess) return bail(fail(STM_ERR_DEVICE, "hipStreamCreate"));
   const uint32_t F = cfg.fanout;
   hipError_t e = hipSuccess;
-  if ((e = dalloc(&t->view.keys, cap * F)) != hipSuccess ||
-      (e = dalloc(&t->view.vals, cap * F)) != hipSuccess ||
-      (e = dalloc(&t->view.meta, cap)) != hipSuccess ||
-      (e = dalloc(&t->view.hdr, 1)) != hipSuccess ||
-      (e = dalloc(&t->view.stats, (size_t)STATS_WORDS)) != hipSuccess)
+  auto pool_layout = [&](SlabCursor& cur) {
+    t->view.keys = (uint64_t*)cur.take(sizeof(uint64_t) * cap * F);
+    t->view.vals = (uint64_t*)cur.take(sizeof(uint64_t) * cap * F);
+    t->view.meta = (NodeMeta*)cur.take(sizeof(NodeMeta) * cap);
+    t->view.hdr = (TreeHeader*)cur.take(sizeof(TreeHeader));
+    t->view.stats = (unsigned long long*)cur.take(sizeof(unsigned long long) * STATS_WORDS);
+  };
+  SlabCursor pool_size{nullptr};
+  pool_layout(pool_size);
+  if ((e = hipMalloc(&t->pool, pool_size.at)) == hipSuccess) {
+    SlabCursor pool_place{(uint8_t*)t->pool};
+    pool_layout(pool_place);
+  } else
     return bail(fail(STM_ERR_NOMEM, "node pool of %llu nodes: %s", (unsigned long long)cap,
                      hipGetErrorString(e)));
   t->view.capacity = (uint32_t)cap;
   t->view.fanout = F;
-  if ((e = t->scr.alloc(cfg.max_batch, true)) != hipSuccess)
+  if ((e = t->scr.alloc(cfg.max_batch, Scratch::CALLS)) != hipSuccess)
     return bail(fail(STM_ERR_NOMEM, "batch scratch for %llu ops: %s",
                      (unsigned long long)cfg.max_batch, hipGetErrorString(e)));
   if (hipMemsetAsync(t->view.meta, 0, sizeof(NodeMeta) * cap, t->stream) != hipSuccess ||
@@ -1205,9 +1234,7 @@ int stm_destroy(stm_tree* t) {
   }
   if (t->ev_sync) (void)hipEventDestroy(t->ev_sync);
   if (t->stream_front) (void)hipStreamDestroy(t->stream_front);
-  void* ps[] = {t->view.keys, t->view.vals, t->view.meta, t->view.hdr, t->view.stats};
-  for (void* p : ps)
-    if (p) (void)hipFree(p);
+  if (t->pool) (void)hipFree(t->pool);
   for (int p = 0; p < STM_NUM_PHASES; ++p) {
     if (t->ev_a[p]) (void)hipEventDestroy(t->ev_a[p]);
     if (t->ev_b[p]) (void)hipEventDestroy(t->ev_b[p]);
