@@ -158,9 +158,11 @@ struct Scratch {
   uint64_t *ukey = nullptr, *uval = nullptr;
   uint8_t* uop = nullptr;
   uint32_t *gstart = nullptr, *npend = nullptr, *dlist = nullptr;
-  uint32_t* slist = nullptr;  // merged INSERTs the fast path hands back
-  uint32_t* scount = nullptr;  // per fast-path wavefront: how many it handed back
-  uint32_t* ilist = nullptr;  // merged INSERTs of the batch
+  uint32_t *rlist = nullptr, *rlen = nullptr;  // pieces of runs that need a split (UpsertArgs)
+  uint32_t *rfirst = nullptr, *rcount = nullptr;  // per wavefront of k_upsert_runs
+  SplitState* split = nullptr;  // leaves split without a lock, and the parents to update
+  uint32_t *plist = nullptr, *plist2 = nullptr;
+  uint32_t* ilist = nullptr;  // merged INSERTs of the batch, in key order
   InsHint* ihint = nullptr;   // the lookup kernel's record of every merged INSERT
   uint64_t* fanout = nullptr; // answer chunks of hot GET groups (fanout_capacity(n))
   BatchCounters* counters = nullptr;
@@ -198,8 +200,9 @@ struct Scratch {
     A_(gstart, cap); A_(npend, cap);
     A_(dlist, cap);
     A_(ihint, cap);
-    A_(slist, cap);
-    A_(scount, FAST_WAVES_MAX);
+    A_(rlist, cap); A_(rlen, cap);
+    A_(rfirst, RUN_WAVES_MAX); A_(rcount, RUN_WAVES_MAX);
+    A_(split, 1); A_(plist, cap); A_(plist2, cap);
     A_(ilist, cap);
     A_(fanout, fanout_capacity(cap));
     A_(desc_live, 1);
@@ -601,6 +604,7 @@ hipError_t enqueue_back(stm_tree* t, Scratch& s, const PipeIn& in, bool timed) {
   la.gval = s.uval;  // GET groups carry no merged value: a hot group's value goes there
   la.fanout = s.fanout;
   la.fanout_cap = fanout_capacity(in.n);
+  la.split = s.split;
   if ((e = launch_lookup(t->view, la, st)) != hipSuccess) return e;
 
   if (in.scans) {  // on the tree as it was before the batch: before the upsert kernel
@@ -615,14 +619,13 @@ hipError_t enqueue_back(stm_tree* t, Scratch& s, const PipeIn& in, bool timed) {
   UpsertArgs ua{};
   ua.ukey = s.ukey;
   ua.uval = s.uval;
-  ua.uop = s.uop;
   ua.gstart = s.gstart;
   ua.npend = s.npend;
   ua.sidx = s.sidx;
   ua.counters = s.counters;
   ua.dlist = s.dlist;
   ua.max_attempts = t->cfg.max_attempts;
-  // Each wavefront owns the groups of upsert_ops_per_wave batch slots; at most 8192 wavefronts
+  // The transactions' grid: upsert_ops_per_wave batch ops per wavefront, at most 8192 wavefronts
   // (every SIMD of the chip fully occupied).
   const uint64_t waves = ((uint64_t)in.n + t->cfg.upsert_ops_per_wave - 1) / t->cfg.upsert_ops_per_wave;
   ua.blocks = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((waves + 3) / 4, 2048));
@@ -631,9 +634,15 @@ hipError_t enqueue_back(stm_tree* t, Scratch& s, const PipeIn& in, bool timed) {
   ua.desc = in.desc;
   ua.ihint = s.ihint;
   ua.ilist = s.ilist;
-  ua.slist = s.slist;
-  ua.scount = s.scount;
-  ua.lanes = t->cfg.upsert_lanes;
+  ua.n_max = in.n;
+  ua.piece = t->cfg.upsert_ops_per_wave;
+  ua.split = s.split;
+  ua.plist = s.plist;
+  ua.plist2 = s.plist2;
+  ua.rlist = s.rlist;
+  ua.rlen = s.rlen;
+  ua.rfirst = s.rfirst;
+  ua.rcount = s.rcount;
   ua.fanout = s.fanout;
   ua.fanout_cap = fanout_capacity(in.n);
   ua.gval = s.uval;
@@ -1156,8 +1165,7 @@ int stm_create(const stm_config* cfg_in, stm_tree** out) {
   if (cfg.sort_tile_items == 0) cfg.sort_tile_items = 16;
   if (cfg.sort_tile_items != 8 && cfg.sort_tile_items != 16)
     return fail(STM_ERR_INVALID, "sort_tile_items %u not in {8, 16}", cfg.sort_tile_items);
-  // Automatic: 8 lanes (8 inserts per wavefront round) while that keeps the leaf in at most 8
-  // elements per lane (measured 0.186 vs 0.206 ms per batch at fanout 64), 16 above.
+  // Kept for callers that set it; no kernel reads it.
   if (cfg.upsert_lanes == 0) cfg.upsert_lanes = cfg.fanout <= 64 ? 8u : 16u;
   if (!(cfg.upsert_lanes == 8 || cfg.upsert_lanes == 16 || cfg.upsert_lanes == 32) ||
       cfg.upsert_lanes > cfg.fanout)

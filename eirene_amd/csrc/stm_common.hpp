@@ -34,7 +34,10 @@ struct alignas(64) NodeMeta {
   uint64_t low;    // inclusive low fence
   uint64_t high;   // exclusive high fence, KEY_EMPTY = +inf
   uint64_t next;   // right sibling id at the same level, NODE_NONE at the right edge
-  uint64_t pad[3];
+  uint64_t made;   // right siblings an unlocked split of this batch made and the parent does not
+                   // list yet: first id (bits 0..31) | number (bits 32..63); 0 between batches
+  uint64_t dirty;  // 1: on the batch's list of parents with such children; 0 between batches
+  uint64_t pad;
 };
 static_assert(sizeof(NodeMeta) == 64, "meta record must be one 64-byte sector");
 
@@ -118,15 +121,13 @@ struct TreeView {
 // invalidate (buffer_inv sc1), which only matter for non-atomic accesses.  The read-only
 // lookup kernel uses plain loads and runs only when no writer is active; kernel boundaries
 // order it against the transactional kernels.
-// One exception inside the transactional kernels: the lane-group fast path of k_upsert_fast
-// (fast_leaf_upserts in stm_tree.hip) reads and writes a leaf's fences, keys and values with
-// plain loads and stores.  That is safe only because a group touches a leaf solely when it owns
-// the leaf in that launch (no other merged INSERT of the batch lies between the leaf's low fence
-// and its key, which the batch's sorted order proves) and the leaf's lock word still holds the
-// version the lookup kernel recorded: then no other group of the launch reads or writes that
-// leaf, so the plain loads return what earlier kernels left, and the launch boundary publishes
-// the plain stores.  A change that lets a group of that kernel touch a leaf it does not own
-// must use the agent-scope accesses and the lock word instead, as k_upsert does.
+// Two exceptions among the upsert kernels read and write nodes with plain loads and stores:
+// k_upsert_runs, where a leaf belongs to the lanes of one wavefront in that launch (the batch's
+// inserts into a leaf are neighbours in its sorted list), and the kernels that bring the new
+// leaves to their parents (one wavefront per parent, one launch or one workgroup step per level).
+// No other wavefront of the launch reads or writes those nodes, so the plain loads return what
+// earlier kernels left, and the launch boundary publishes the plain stores.  Metadata words, which
+// share lines with other nodes' words, are stored at agent scope there too.
 // Plain load through a pointer known to address device global memory.  Pointers read from
 // memory (a batch descriptor's) are generic to the compiler, which then emits flat loads; this
 // lets it use global loads with a scalar base and immediate offsets.
@@ -136,6 +137,9 @@ STM_DEV T gload(const T* p) {
 }
 
 STM_DEV uint64_t ld_relaxed(const uint64_t* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+STM_DEV uint32_t ld_relaxed32(const uint32_t* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
 STM_DEV void st_relaxed(uint64_t* p, uint64_t v) {

@@ -14,9 +14,11 @@
 // prefix: the number of group heads, the position of the last head and the position of the
 // last INSERT.  For element i with head h(i), the latest earlier insert of its key is the
 // prefix's last insert if it is >= h(i); the group's merged op is INSERT iff the last insert
-// up to its end is >= its head.  A wavefront owns 512 consecutive elements as 8 rounds of
-// 64 (coalesced loads and group outputs); within a round the three values of every lane's
-// prefix come from two ballots (heads, inserts): a popcount and a highest set bit.  Three
+// up to its end is >= its head.  A fourth value, the number of groups with an INSERT, is the
+// place of such a group in the batch's insert list, which so comes out in key order.  A wavefront
+// owns 512 consecutive elements as 8 rounds of
+// 64 (coalesced loads and group outputs); within a round the values of every lane's
+// prefix come from two ballots (heads, inserts): popcounts and highest set bits.  Three
 // kernels: tile reduce, scan of the tile aggregates, apply.  Ops that the fold answers (an
 // earlier insert of the same key exists) are written to the outputs here; the first op of
 // each group up to and including its first insert waits for the tree ("npend" ops from
@@ -67,7 +69,7 @@ STM_DEV void round_flags(const FoldArgs& a, const Chunk& ch, int r, bool& valid,
   const uint64_t next_first = r + 1 < FOLD_ROUNDS ? readlane64(ch.k[r + 1 < FOLD_ROUNDS ? r + 1 : r], 0) : ch.nk;
   next = lane < WAVE - 1 ? down : next_first;
   head = valid && (i == 0 || ch.k[r] != prev);
-  ins = valid && op_of(ch.sx[r]) == OP_INSERT;
+  ins = valid && op_of(ch.sx[r]) == OP_INSERT && ch.k[r] != KEY_EMPTY;
 }
 
 // The chunk's aggregate (wave-uniform).
@@ -78,11 +80,7 @@ STM_DEV Acc chunk_acc(const FoldArgs& a, const Chunk& ch) {
     bool valid, head, ins;
     uint64_t next;
     round_flags(a, ch, r, valid, head, ins, next);
-    const uint32_t rb = ch.c0 + (uint32_t)r * WAVE;
-    const uint64_t hm = ballot(head), im = ballot(ins);
-    t.c += (uint32_t)__popcll(hm);
-    t.head = last_set(hm, rb, t.head);
-    t.ins = last_set(im, rb, t.ins);
+    t = acc_round(t, ballot(head), ballot(ins), ch.c0 + (uint32_t)r * WAVE);
   }
   return t;
 }
@@ -126,10 +124,11 @@ STM_DEV Acc block_exclusive_acc(const Acc& v, Acc* s_w /*[FOLD_WAVES]*/, Acc& to
 #pragma unroll
   for (int off = 1; off < WAVE; off <<= 1) {
     const Acc y{(uint32_t)__shfl_up((int)x.c, off, WAVE), __shfl_up(x.head, off, WAVE),
-                __shfl_up(x.ins, off, WAVE)};
+                __shfl_up(x.ins, off, WAVE), (uint32_t)__shfl_up((int)x.m, off, WAVE)};
     if (lane >= off) x = acc_combine(y, x);
   }
-  Acc ex{(uint32_t)__shfl_up((int)x.c, 1, WAVE), __shfl_up(x.head, 1, WAVE), __shfl_up(x.ins, 1, WAVE)};
+  Acc ex{(uint32_t)__shfl_up((int)x.c, 1, WAVE), __shfl_up(x.head, 1, WAVE),
+         __shfl_up(x.ins, 1, WAVE), (uint32_t)__shfl_up((int)x.m, 1, WAVE)};
   if (lane == 0) ex = acc_identity();
   if (lane == WAVE - 1) s_w[wave] = x;
   __syncthreads();
@@ -168,7 +167,7 @@ __global__ __launch_bounds__(FOLD_BLOCK) void k_fold_scan_tiles(Acc* tile_agg, F
     // its state from before the batch.
     const uint32_t stalled = a.sort_stall ? *a.sort_stall : 0u;
     counters->n_unique = stalled ? 0u : total.c;
-    counters->n_upserts = 0;
+    counters->n_upserts = stalled ? 0u : total.m & ~ACC_LEAD;
     counters->n_deferred = 0;
     counters->queue_head = 0;
     counters->n_bad = 0;
@@ -182,8 +181,6 @@ __global__ __launch_bounds__(FOLD_BLOCK) void k_fold_scan_tiles(Acc* tile_agg, F
 
 __global__ __launch_bounds__(FOLD_BLOCK) void k_fold_apply(FoldArgs a, const Acc* tile_prefix) {
   __shared__ Acc s_w[FOLD_WAVES];
-  __shared__ uint32_t s_ins[FOLD_TILE];  // the tile's merged INSERT groups
-  __shared__ uint32_t s_nins, s_base;
   fold_resolve(a);
   if (a.counters->sort_stall) return;  // the batch runs empty (k_fold_scan_tiles)
   const uint32_t ntiles = (a.n + FOLD_TILE - 1) / FOLD_TILE;
@@ -191,11 +188,10 @@ __global__ __launch_bounds__(FOLD_BLOCK) void k_fold_apply(FoldArgs a, const Acc
   const uint64_t lt = lanemask_lt();
   const uint64_t le = lt | (1ull << lane_id());
   for (uint32_t b = blockIdx.x; b < ntiles; b += gridDim.x) {
-    if (threadIdx.x == 0) s_nins = 0;
     Chunk ch;
     load_chunk(a, b * FOLD_TILE + wave * FOLD_CHUNK, ch);
     Acc total;
-    // State before this wavefront's chunk (block_wave_prefix syncs s_nins too).
+    // State before this wavefront's chunk.
     Acc carry = acc_combine(tile_prefix[b], block_wave_prefix(chunk_acc(a, ch), s_w, total));
     // The rounds in halves of HALF, each in three phases, so that the gathers of a half share
     // two round trips: the vector memory counter also counts stores, so a gather after a
@@ -206,7 +202,7 @@ __global__ __launch_bounds__(FOLD_BLOCK) void k_fold_apply(FoldArgs a, const Acc
 #pragma unroll
     for (int h = 0; h < FOLD_ROUNDS; h += HALF) {
     // Phase 1, registers only: each round's flags, group index, head and latest earlier insert.
-    uint32_t fl[HALF], gg[HALF];
+    uint32_t fl[HALF], gg[HALF], ge[HALF];
     int32_t hd[HALF], lb[HALF];
 #pragma unroll
     for (int q = 0; q < HALF; ++q) {
@@ -223,11 +219,12 @@ __global__ __launch_bounds__(FOLD_BLOCK) void k_fold_apply(FoldArgs a, const Acc
       const int32_t ins_before = last_set(im & lt, rb, carry.ins);
       lb[q] = ins_before >= hd[q] ? ins_before : -1;  // latest earlier insert of the key
       gg[q] = c_incl - 1;
+      // groups with an INSERT up to and including this lane's, less one: its place in the list
+      const uint64_t fm = first_inserts(hm, im, acc_open_insert(carry));
+      ge[q] = (carry.m & ~ACC_LEAD) + (uint32_t)__popcll(fm & le) - 1;
       const bool group_end = valid && (i + 1 == a.n || next != ch.k[r]);
       fl[q] = (valid ? F_VALID : 0u) | (is_ins ? F_INS : 0u) | (group_end ? F_END : 0u);
-      carry.c += (uint32_t)__popcll(hm);
-      carry.head = last_set(hm, rb, carry.head);
-      carry.ins = last_set(im, rb, carry.ins);
+      carry = acc_round(carry, hm, im, rb);
     }
     // Phase 2: input positions of the earlier inserts, then the values.  va = the latest
     // earlier insert's value (an op's answer, or the merged value of a group ending in a
@@ -247,7 +244,7 @@ __global__ __launch_bounds__(FOLD_BLOCK) void k_fold_apply(FoldArgs a, const Acc
       va[q] = need_a ? a.vals[pos_of(ia[q])] : 0ull;
       vb[q] = need_b ? a.vals[pos_of(ch.sx[r])] : 0ull;
     }
-    // Phase 3: the outputs and the tile's insert list.
+    // Phase 3: the outputs and the insert list.
 #pragma unroll
     for (int q = 0; q < HALF; ++q) {
       const int r = h + q;
@@ -256,7 +253,6 @@ __global__ __launch_bounds__(FOLD_BLOCK) void k_fold_apply(FoldArgs a, const Acc
       const int32_t head = hd[q];
       const int32_t last_before = lb[q];
       const uint32_t g = gg[q];
-      bool append = false;
       if (valid) {
         const uint64_t key = ch.k[r];
         if (a.lastins) a.lastins[i] = is_ins ? i : last_before;
@@ -278,7 +274,7 @@ __global__ __launch_bounds__(FOLD_BLOCK) void k_fold_apply(FoldArgs a, const Acc
           } else if (last_in >= 0) {
             op = OP_INSERT;
             a.uval[g] = is_ins ? vb[q] : va[q];
-            append = true;
+            if (a.ilist) a.ilist[ge[q]] = g;
           } else {
             op = OP_GET;
             if (a.gstart) a.npend[g] = (uint32_t)(i - head + 1);
@@ -286,20 +282,8 @@ __global__ __launch_bounds__(FOLD_BLOCK) void k_fold_apply(FoldArgs a, const Acc
           a.uop[g] = op;
         }
       }
-      const uint64_t want = ballot(append);
-      uint32_t wb = 0;
-      if (lane_id() == 0 && want) wb = atomicAdd(&s_nins, (uint32_t)__popcll(want));  // LDS
-      wb = (uint32_t)__shfl((int)wb, 0, WAVE);
-      if (append) s_ins[wb + (uint32_t)__popcll(want & lt)] = g;
     }
     }  // halves
-    // One counter update per tile (a hot atomic per wavefront round would serialize the
-    // kernel on one L2 channel), then the tile's INSERT groups go to the batch's list.
-    __syncthreads();
-    if (threadIdx.x == 0) s_base = s_nins ? atomicAdd(&a.counters->n_upserts, s_nins) : 0u;
-    __syncthreads();
-    if (a.ilist)
-      for (uint32_t k = threadIdx.x; k < s_nins; k += FOLD_BLOCK) a.ilist[s_base + k] = s_ins[k];
     __syncthreads();
   }  // tiles
 }

@@ -48,13 +48,12 @@ constexpr uint32_t TILES_MAX = FRONT_MAX_OPS / (2 * FT);
 // summary, then per tile the first element of every bucket within the tile.
 struct BucketSum {
   uint32_t start;  // sorted position of the bucket's first element
-  uint32_t heads;  // group heads among its elements after the first
-  int32_t head;    // the last of them (-1 if none)
-  int32_t ins;     // its last INSERT (-1 if none)
+  Acc acc;         // its elements, the first one not counted as a head
 };
+static_assert(sizeof(BucketSum) == 20, "five words");
 constexpr uint32_t FRONT_RETRY = 0;
 constexpr uint32_t FRONT_SUMS = 64;
-constexpr uint32_t FRONT_OFFS = FRONT_SUMS + 4 * BUCKETS_MAX;
+constexpr uint32_t FRONT_OFFS = FRONT_SUMS + 5 * BUCKETS_MAX;
 constexpr uint32_t FRONT_WORDS = FRONT_OFFS + TILES_MAX * (BUCKETS_MAX + 1);
 size_t front_scratch_words() { return FRONT_WORDS; }
 
@@ -152,6 +151,7 @@ struct FoldElem {
   bool valid, ins, end;  // in the batch; an INSERT; the last element of its group
   int32_t i, head, lb;   // sorted position, its group's head, the latest earlier insert of the key (-1)
   uint32_t g;            // group index
+  uint32_t e;            // the group's place in the insert list (a group with an INSERT)
   uint64_t key;
   uint32_t pos, lb_pos;  // input positions of the element and of lb
   uint64_t va, vb;       // lb's value, the element's own (loaded where needed)
@@ -165,47 +165,54 @@ STM_DEV void fold_gather(const FoldArgs& a, FoldElem& x) {
   x.vb = need_b ? a.vals[x.pos] : 0ull;
 }
 
-// Writes the element's outputs; true when its group is a merged INSERT that goes on the batch's
-// list.  Ops with the reserved key are added to bad.
-STM_DEV bool fold_store(const FoldArgs& a, const FoldElem& x, uint32_t* bad) {
-  if (!x.valid) return false;
+// Writes the element's outputs.  Ops with the reserved key are added to bad.
+STM_DEV void fold_store(const FoldArgs& a, const FoldElem& x, uint32_t* bad) {
+  if (!x.valid) return;
   if (a.lastins) a.lastins[x.i] = x.ins ? x.i : x.lb;
   if (x.lb >= 0) {
     a.out_vals[x.pos] = x.va;
     a.out_found[x.pos] = 1;
   }
   if (x.ins && x.lb < 0) a.npend[x.g] = (uint32_t)(x.i - x.head + 1);
-  if (!x.end) return false;
+  if (!x.end) return;
   a.ukey[x.g] = x.key;
   a.gstart[x.g] = (uint32_t)x.head;
   const int32_t last_in = x.ins ? x.i : x.lb;  // the group's last insert
   if (x.key == KEY_EMPTY) {
     a.uop[x.g] = UOP_SKIP;
     atomicAdd(bad, (uint32_t)(x.i - x.head + 1));
-    return false;
-  }
-  if (last_in >= 0) {
+  } else if (last_in >= 0) {
     a.uop[x.g] = OP_INSERT;
     a.uval[x.g] = x.ins ? x.vb : x.va;
-    return true;
+    a.ilist[x.e] = x.g;
+  } else {
+    a.uop[x.g] = OP_GET;
+    a.npend[x.g] = (uint32_t)(x.i - x.head + 1);
   }
-  a.uop[x.g] = OP_GET;
-  a.npend[x.g] = (uint32_t)(x.i - x.head + 1);
-  return false;
 }
 
-// Head, insert and group fields of this thread's element from the state before its wavefront's
-// 64 elements (which start at sorted position rb); returns the state after them.
-STM_DEV Acc fold_flags(FoldElem& x, bool is_head, uint32_t rb, const Acc& before) {
+// Head, insert, group and list fields of this thread's element from the state before its
+// wavefront's 64 elements, which start at sorted position rb and have heads hm and INSERTs im.
+STM_DEV void fold_place(FoldElem& x, uint64_t hm, uint64_t im, uint32_t rb, const Acc& before) {
   const uint64_t lt = lanemask_lt();
   const uint64_t le = lt | (1ull << lane_id());
-  const uint64_t hm = ballot(is_head), im = ballot(x.ins);
   x.head = last_set(hm & le, rb, before.head);
   const int32_t ins_before = last_set(im & lt, rb, before.ins);
   x.lb = ins_before >= x.head ? ins_before : -1;
   x.g = before.c + (uint32_t)__popcll(hm & le) - 1;
-  return Acc{before.c + (uint32_t)__popcll(hm), last_set(hm, rb, before.head),
-             last_set(im, rb, before.ins)};
+  const uint64_t fm = first_inserts(hm, im, acc_open_insert(before));
+  x.e = (before.m & ~ACC_LEAD) + (uint32_t)__popcll(fm & le) - 1;
+}
+
+// Combination, in lane order, of the 64 lanes' states (complete in lane 0).
+STM_DEV Acc wave_combine(Acc v) {
+#pragma unroll
+  for (int off = 1; off < WAVE; off <<= 1) {
+    const Acc o{(uint32_t)__shfl_down((int)v.c, off, WAVE), __shfl_down(v.head, off, WAVE),
+                __shfl_down(v.ins, off, WAVE), (uint32_t)__shfl_down((int)v.m, off, WAVE)};
+    if (lane_id() + off < WAVE) v = acc_combine(v, o);
+  }
+  return v;
 }
 
 struct FrontIn {
@@ -243,7 +250,7 @@ __global__ __launch_bounds__(FT) void k_front_small(FrontArgs fa) {
   __shared__ uint64_t s_k[N];
   __shared__ uint32_t s_p[N];
   __shared__ Acc s_acc[CHUNKS];
-  __shared__ uint32_t s_ins, s_bad;
+  __shared__ uint32_t s_bad;
   const FrontIn in = front_in(fa);
   FoldArgs a = fa.fold;
   fold_resolve(a);
@@ -268,13 +275,10 @@ __global__ __launch_bounds__(FT) void k_front_small(FrontArgs fa) {
     s_k[tid * E + r] = k[r];
     s_p[tid * E + r] = p[r];
   }
-  if (tid == 0) {
-    s_ins = 0;
-    s_bad = 0;
-  }
+  if (tid == 0) s_bad = 0;
   __syncthreads();
   FoldElem x[E];
-  bool head[E];
+  uint64_t hm[E], im[E];
 #pragma unroll
   for (int r = 0; r < E; ++r) {
     const uint32_t i = (uint32_t)r * FT + tid;
@@ -283,13 +287,12 @@ __global__ __launch_bounds__(FT) void k_front_small(FrontArgs fa) {
     x[r].key = s_k[i];
     const uint32_t tie = s_p[i];
     x[r].pos = tie >> 2;
-    x[r].ins = x[r].valid && (tie & 3u) == OP_INSERT;
-    head[r] = x[r].valid && (i == 0 || s_k[i > 0 ? i - 1 : 0] != x[r].key);
+    x[r].ins = x[r].valid && (tie & 3u) == OP_INSERT && x[r].key != KEY_EMPTY;
+    hm[r] = ballot(x[r].valid && (i == 0 || s_k[i > 0 ? i - 1 : 0] != x[r].key));
+    im[r] = ballot(x[r].ins);
     x[r].end = x[r].valid && (i + 1 >= n || s_k[min(i + 1, N - 1)] != x[r].key);
-    const uint32_t rb = i - lane_id();
-    FoldElem tmp = x[r];
-    const Acc own = fold_flags(tmp, head[r], rb, acc_identity());
-    if (lane_id() == 0) s_acc[rb / WAVE] = own;
+    const uint32_t rb = (uint32_t)r * FT + wave * WAVE;
+    if (lane_id() == 0) s_acc[rb / WAVE] = acc_round(acc_identity(), hm[r], im[r], rb);
     if (x[r].valid) const_cast<uint32_t*>(a.sidx)[i] = payload_of(tie);
   }
   __syncthreads();
@@ -300,7 +303,7 @@ __global__ __launch_bounds__(FT) void k_front_small(FrontArgs fa) {
 #pragma unroll
     for (int r = 0; r < E; ++r)
       if ((uint32_t)c == (uint32_t)r * FW + wave)
-        (void)fold_flags(x[r], head[r], (uint32_t)c * WAVE, run);
+        fold_place(x[r], hm[r], im[r], (uint32_t)c * WAVE, run);
     run = acc_combine(run, t);
   }
 #pragma unroll
@@ -309,16 +312,9 @@ __global__ __launch_bounds__(FT) void k_front_small(FrontArgs fa) {
     fold_gather(a, x[r]);
   }
 #pragma unroll
-  for (int r = 0; r < E; ++r) {
-    const bool append = fold_store(a, x[r], &s_bad);
-    const uint64_t want = ballot(append);
-    uint32_t at = 0;
-    if (lane_id() == 0 && want) at = atomicAdd(&s_ins, (uint32_t)__popcll(want));
-    at = (uint32_t)__shfl((int)at, 0, WAVE);
-    if (append) a.ilist[at + (uint32_t)__popcll(want & lanemask_lt())] = x[r].g;
-  }
+  for (int r = 0; r < E; ++r) fold_store(a, x[r], &s_bad);
   __syncthreads();
-  if (tid == 0) reset_counters(a.counters, run.c, s_ins, s_bad);
+  if (tid == 0) reset_counters(a.counters, run.c, run.m & ~ACC_LEAD, s_bad);
 }
 
 // ------------------------------------------------------------------ split
@@ -439,7 +435,7 @@ __global__ __launch_bounds__(FT) void k_front_split(FrontArgs fa) {
 // from position start, and back to s_k for the summary.
 template <int E>
 STM_DEV void sort_bucket(const FrontArgs& fa, uint32_t m, uint32_t start, uint64_t* s_k, uint32_t* s_p,
-                         BucketSum& sum, uint32_t* s_red) {
+                         BucketSum& sum, Acc* s_acc) {
   const uint32_t tid = threadIdx.x;
   uint64_t k[E];
   uint32_t p[E];
@@ -468,20 +464,13 @@ STM_DEV void sort_bucket(const FrontArgs& fa, uint32_t m, uint32_t start, uint64
       const_cast<uint32_t*>(fa.fold.sidx)[start + i] = payload_of(tie);
     }
     const uint64_t hm = ballot(v && i > 0 && s_k[i > 0 ? i - 1 : 0] != key);
-    const uint64_t im = ballot(v && (tie & 3u) == OP_INSERT);
-    if (lane_id() == 0) {
-      const uint32_t rb = start + i;
-      if (hm) {
-        atomicAdd(&s_red[0], (uint32_t)__popcll(hm));
-        atomicMax(&s_red[1], (uint32_t)last_set(hm, rb, -1) + 1u);
-      }
-      if (im) atomicMax(&s_red[2], (uint32_t)last_set(im, rb, -1) + 1u);
-    }
+    const uint64_t im = ballot(v && (tie & 3u) == OP_INSERT && key != KEY_EMPTY);
+    const uint32_t c = (uint32_t)r * FW + tid / WAVE;
+    if (lane_id() == 0) s_acc[c] = acc_round(acc_identity(), hm, im, start + c * WAVE);
   }
   __syncthreads();
-  sum.heads = s_red[0];
-  sum.head = (int32_t)s_red[1] - 1;
-  sum.ins = (int32_t)s_red[2] - 1;
+  if (tid < (uint32_t)WAVE)
+    sum.acc = wave_combine(tid < (uint32_t)(FW * E) ? s_acc[tid] : acc_identity());
 }
 
 // Bucket blockIdx.x of B: its pieces, one per tile of tile_ops elements, into LDS, sorted there.
@@ -490,14 +479,14 @@ __global__ __launch_bounds__(FT) void k_front_bucket(FrontArgs fa, uint32_t tile
   __shared__ uint32_t s_p[BUCKET_CAP];
   __shared__ uint32_t s_src[TILES_MAX], s_dst[TILES_MAX], s_len[TILES_MAX];
   __shared__ uint32_t s_w[2][2];
-  __shared__ uint32_t s_red[3];
+  __shared__ Acc s_acc[BUCKET_CAP / WAVE];
+  static_assert(BUCKET_CAP / WAVE <= WAVE, "one wavefront combines a bucket's states");
   static_assert(TILES_MAX <= 2 * WAVE, "the tiles fit two wavefronts");
   const uint32_t n = front_in(fa).n;
   const uint32_t b = blockIdx.x;
   const uint32_t tid = threadIdx.x;
   const uint32_t tiles = (n + tile_ops - 1) / tile_ops;
   BucketSum* sums = reinterpret_cast<BucketSum*>(fa.words + FRONT_SUMS);
-  if (tid < 3) s_red[tid] = 0;
   uint32_t o0 = 0, len = 0, x = 0, y = 0;
   if (tid < 2 * WAVE) {
     if (tid < tiles) {
@@ -529,7 +518,7 @@ __global__ __launch_bounds__(FT) void k_front_bucket(FrontArgs fa, uint32_t tile
     s_len[tid] = len;
   }
   __syncthreads();
-  BucketSum sum{start, 0u, -1, -1};
+  BucketSum sum{start, acc_identity()};
   if (m > BUCKET_CAP) {
     if (tid == 0) fa.words[FRONT_RETRY] = 1;
   } else if (m > 0) {
@@ -542,9 +531,9 @@ __global__ __launch_bounds__(FT) void k_front_bucket(FrontArgs fa, uint32_t tile
       }
     }
     __syncthreads();
-    if (m <= FT) sort_bucket<1>(fa, m, start, s_k, s_p, sum, s_red);
-    else if (m <= 2 * FT) sort_bucket<2>(fa, m, start, s_k, s_p, sum, s_red);
-    else sort_bucket<4>(fa, m, start, s_k, s_p, sum, s_red);
+    if (m <= FT) sort_bucket<1>(fa, m, start, s_k, s_p, sum, s_acc);
+    else if (m <= 2 * FT) sort_bucket<2>(fa, m, start, s_k, s_p, sum, s_acc);
+    else sort_bucket<4>(fa, m, start, s_k, s_p, sum, s_acc);
   }
   if (tid == 0) sums[b] = sum;
 }
@@ -552,8 +541,6 @@ __global__ __launch_bounds__(FT) void k_front_bucket(FrontArgs fa, uint32_t tile
 // ------------------------------------------------------------------ fold of a bucket
 __global__ __launch_bounds__(FT) void k_front_fold(FrontArgs fa, uint32_t B) {
   __shared__ Acc s_acc[FW];
-  __shared__ uint32_t s_list[FT];
-  __shared__ uint32_t s_nins, s_base;
   FoldArgs a = fa.fold;
   fold_resolve(a);
   const uint32_t n = a.n;
@@ -575,31 +562,30 @@ __global__ __launch_bounds__(FT) void k_front_fold(FrontArgs fa, uint32_t B) {
     const BucketSum q = sums[tid];
     const uint32_t qe = tid + 1 < B ? sums[tid + 1].start : n;
     if (qe > q.start) {
-      const bool first = q.start == 0 || a.skeys[q.start > 0 ? q.start - 1 : 0] != a.skeys[q.start];
-      v.c = q.heads + (first ? 1u : 0u);
-      v.head = q.head >= 0 ? q.head : (first ? (int32_t)q.start : -1);
-      v.ins = q.ins;
+      v = q.acc;
+      if (q.start == 0 || a.skeys[q.start > 0 ? q.start - 1 : 0] != a.skeys[q.start]) {
+        v.c += 1;
+        v.head = v.head >= 0 ? v.head : (int32_t)q.start;
+        v.m &= ~ACC_LEAD;
+      }
     }
   }
-#pragma unroll
-  for (int off = 1; off < WAVE; off <<= 1) {
-    const Acc o{(uint32_t)__shfl_xor((int)v.c, off, WAVE), __shfl_xor(v.head, off, WAVE),
-                __shfl_xor(v.ins, off, WAVE)};
-    v = acc_combine(v, o);
-  }
+  v = wave_combine(v);
   if (lane_id() == 0) s_acc[wave] = v;
   __syncthreads();
   Acc carry = acc_identity();
 #pragma unroll
   for (int w = 0; w < (int)(BUCKETS_MAX / WAVE); ++w) carry = acc_combine(carry, s_acc[w]);
   if (b == 0) {
-    if (tid == 0) a.counters->n_unique = carry.c;
+    if (tid == 0) {
+      a.counters->n_unique = carry.c;
+      a.counters->n_upserts = carry.m & ~ACC_LEAD;
+    }
     carry = acc_identity();
   }
   __syncthreads();
   for (uint32_t r0 = start; r0 < end; r0 += FT) {
     const uint32_t i = r0 + tid;
-    if (tid == 0) s_nins = 0;
     FoldElem x;
     x.valid = i < end;
     x.i = (int32_t)i;
@@ -609,13 +595,11 @@ __global__ __launch_bounds__(FT) void k_front_fold(FrontArgs fa, uint32_t B) {
     x.key = a.skeys[ic];
     const uint32_t pl = a.sidx[ic];
     x.pos = pos_of(pl);
-    x.ins = x.valid && op_of(pl) == OP_INSERT;
-    const bool head = x.valid && (i == 0 || prev != x.key);
+    x.ins = x.valid && op_of(pl) == OP_INSERT && x.key != KEY_EMPTY;
     x.end = x.valid && (i + 1 == n || next != x.key);
+    const uint64_t hm = ballot(x.valid && (i == 0 || prev != x.key)), im = ballot(x.ins);
     const uint32_t rb = r0 + wave * WAVE;
-    FoldElem tmp = x;
-    const Acc own = fold_flags(tmp, head, rb, acc_identity());
-    if (lane_id() == 0) s_acc[wave] = own;
+    if (lane_id() == 0) s_acc[wave] = acc_round(acc_identity(), hm, im, rb);
     __syncthreads();
     Acc before = carry;
 #pragma unroll
@@ -624,19 +608,10 @@ __global__ __launch_bounds__(FT) void k_front_fold(FrontArgs fa, uint32_t B) {
       if ((uint32_t)w < wave) before = acc_combine(before, t);
       carry = acc_combine(carry, t);
     }
-    (void)fold_flags(x, head, rb, before);
+    fold_place(x, hm, im, rb, before);
     x.lb_pos = x.valid && x.lb >= 0 ? pos_of(a.sidx[x.lb]) : 0u;
     fold_gather(a, x);
-    const bool append = fold_store(a, x, &a.counters->n_bad);
-    const uint64_t want = ballot(append);
-    uint32_t at = 0;
-    if (lane_id() == 0 && want) at = atomicAdd(&s_nins, (uint32_t)__popcll(want));
-    at = (uint32_t)__shfl((int)at, 0, WAVE);
-    if (append) s_list[at + (uint32_t)__popcll(want & lanemask_lt())] = x.g;
-    __syncthreads();
-    if (tid == 0) s_base = s_nins ? atomicAdd(&a.counters->n_upserts, s_nins) : 0u;
-    __syncthreads();
-    if (tid < s_nins) a.ilist[s_base + tid] = s_list[tid];
+    fold_store(a, x, &a.counters->n_bad);
     __syncthreads();
   }
 }

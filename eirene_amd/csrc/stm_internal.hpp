@@ -104,8 +104,8 @@ struct FoldArgs {
   void* tile_scratch;     // fold_scratch_bytes(n)
   int32_t* lastins;       // scan mode: per sorted entry, the latest insert of its key at or
                           // before it (sorted index), -1 if none; null otherwise
-  uint32_t* ilist;        // optional: the groups whose merged op is INSERT (n_upserts of them,
-                          // key order within each fold tile)
+  uint32_t* ilist;        // optional: the groups whose merged op is INSERT (n_upserts of them, in
+                          // key order)
   const uint32_t* sort_stall;  // optional: the sort's stall word, copied into the counters
   const uint32_t* sort_exact;  // optional: the sort's fallback word, copied into the counters
 };

@@ -8,10 +8,15 @@
 // they commute):
 //   * merged GETs run first in k_lookup on a tree no one writes, walking the sorted keys
 //     in chunks with the last inner node and leaf cached in registers;
-//   * merged INSERTs then run in k_upsert as transactions on 64-lane wavefronts:
-//     begin (root + version), optimistic reads validated by fences and lock versions,
-//     try-lock commit of the write set with 64-bit CAS, abort and retry with backoff,
-//     preemptive split of full inner nodes on the way down
+//   * merged INSERTs then run leaf by leaf: in key order the inserts of a leaf are neighbours, so
+//     k_upsert_runs gives each leaf's run to the lanes of one wavefront and k_upsert_long the long
+//     ones to a workgroup; leaves that overfill are split there, and k_upsert_parents and
+//     k_upsert_upper bring the new nodes to their parents level by level;
+//   * what that leaves (a pool that is all but full; every long run when upsert_ops_per_wave asks
+//     for less than a wavefront's worth of ops) runs as transactions on 64-lane wavefronts
+//     (k_upsert, k_upsert_serial): begin (root + version), optimistic reads validated by fences and
+//     lock versions, try-lock commit of the write set with 64-bit CAS, abort and retry with
+//     backoff, preemptive split of full inner nodes on the way down
 //     (reference: src/gpu-stm-tree-v38/bpt-gpustm-kernel.cu:162-181).
 #include <atomic>
 #include "stm_common.hpp"
@@ -22,6 +27,9 @@
 namespace stm {
 
 constexpr uint32_t LOOKUP_GRID_CAP = 8192;
+constexpr uint32_t LONG_BLOCKS = 256;        // workgroups of k_upsert_long
+constexpr uint32_t PARENT_BLOCKS = 512;      // workgroups of k_upsert_parents
+constexpr uint32_t FEW_INSERTS = 1u << 14;   // batches of at most this many ops skip that launch
 
 // ================================================================== bulk build
 template <int F>
@@ -277,8 +285,14 @@ __global__ __launch_bounds__(256, (lookup_min_waves<F, G>())) void k_lookup(Tree
                                                 InsHint* __restrict__ ihint,
                                                 uint64_t* __restrict__ gval,
                                                 uint64_t* __restrict__ fanout,
-                                                uint64_t fanout_cap) {
+                                                uint64_t fanout_cap,
+                                                SplitState* __restrict__ split) {
   constexpr int K = F / G;
+  if (blockIdx.x == 0 && threadIdx.x == 0) {
+    SplitState z{};
+    z.refused = NODE_NONE;
+    *split = z;
+  }
   const int lane = lane_id();
   const int g = lane & (G - 1);
   const int gbase = lane - g;
@@ -439,21 +453,17 @@ __global__ __launch_bounds__(256, (lookup_min_waves<F, G>())) void k_lookup(Tree
     }
     // The sub-chunk's tail loads go out together, before any of its stores (the vector memory
     // counter counts stores too, so a load issued after a store also waits for the store):
-    // the version and entry count of an INSERT group's leaf, the value a GET group returns.
+    // the entry count of an INSERT group's leaf, the value a GET group returns.
     const bool hint = walk && !mine;
-    uint64_t ver = 1ull, info = 0;
-    if (hint && leaf_l < t.capacity) {
-      ver = t.meta[leaf_l].lock;
-      info = t.meta[leaf_l].info;
-    }
+    uint64_t info = 0;
+    if (hint && leaf_l < t.capacity) info = t.meta[leaf_l].info;
     const uint64_t val = (mine && found_l) ? t.vals[vidx_l] : 0;
     if (hint) {
-      // The record for the upsert kernels: the op's answer range and leaf, the leaf's version
-      // and entry count now (no writer runs during this kernel), the key's slot in it and the
-      // level-1 node last used for routing.
+      // The record for the upsert kernels: the op's answer range and leaf, the leaf's entry count
+      // now (no writer runs during this kernel), the key's slot in it and the level-1 node last
+      // used for routing.
       // field by field, so that the fields need not be live together (registers)
       InsHint* h = ihint + j;
-      h->ver = ver;
       h->leaf = leaf_l;
       h->pos = (uint32_t)(vidx_l - (uint64_t)leaf_l * F) | (found_l ? UPOS_FOUND : 0u) |
                (min(meta_count(info), 255u) << UPOS_COUNT_SHIFT);
@@ -1404,124 +1414,10 @@ STM_DEV void flush_counters(const TreeView& t, const TxCounters& c, BatchCounter
   flush_counters(t, c);
 }
 
-// Lane-group fast path: NG = 64 / G merged INSERTs of one wavefront at once, each by G lanes.
-// It is the leaf-only transaction of the wave-wide path (update in place, or append at the
-// leaf's count: a leaf's entries are unordered), commit with version + 2, run for NG ops in
-// lock-step, started from the leaf, slot and entry count the lookup kernel found for the key,
-// and it runs only for the op that owns its leaf in this launch: the first merged INSERT of the
-// leaf in key order.  Groups are sorted by key, so an op owns its leaf when none of the groups
-// between the leaf's low fence and its own key is an INSERT; lane g of the op's lane group reads
-// group gi - 1 - g (key and merged op), and ownership is proven when one of those G keys lies
-// below the fence (or the batch starts).  No other group of the launch then writes the leaf, and
-// no writer ran since the lookup kernel read it, so the hint is exact and no lock is taken.  An
-// op that does not own its leaf (another INSERT of the batch precedes it there, or more than G
-// groups of the leaf do), whose leaf is full or whose hint disagrees with the leaf's version,
-// count or fences is handed back to the wave-wide path, which runs after this launch.  A found
-// key reads and writes its one value; a new key writes one key and one value.  (Measured with
-// sorted leaves, whose inserts shifted the slots above the key: 97 µs per 2^22-op batch, ≈56 of
-// them the shifted slots' stores; with the leaf's test-and-set instead of the ownership test
-// before that, 131 µs.)
-// src = round lane of this group's op (-1: none).  Returns the round lanes whose op committed.
-template <int F, int G>
-STM_DEV uint64_t fast_leaf_upserts(const TreeView& t, int src, uint64_t k_l, uint64_t v_l,
-                                   uint32_t leaf_l, uint64_t ver_l, uint32_t up_l, uint32_t gi_l,
-                                   const uint64_t* __restrict__ ukey,
-                                   const uint8_t* __restrict__ uop, uint32_t gs_l,
-                                   uint32_t np_l, uint32_t p0_l, const uint32_t* __restrict__ sidx,
-                                   uint64_t* __restrict__ out_vals,
-                                   uint8_t* __restrict__ out_found, TxCounters& c) {
-  const int lane = lane_id();
-  const int g = lane & (G - 1);
-  const int gbase = lane - g;
-  const int sl = src >= 0 ? src : 0;
-  const uint64_t key = shfl64(k_l, sl);
-  const uint64_t val = shfl64(v_l, sl);
-  const uint32_t leaf = (uint32_t)__shfl((int)leaf_l, sl, WAVE);
-  const uint32_t gs = (uint32_t)__shfl((int)gs_l, sl, WAVE);
-  const uint32_t np = (uint32_t)__shfl((int)np_l, sl, WAVE);
-  const uint32_t p0 = (uint32_t)__shfl((int)p0_l, sl, WAVE);
-  const uint32_t up = (uint32_t)__shfl((int)up_l, sl, WAVE);
-  const uint32_t gi = (uint32_t)__shfl((int)gi_l, sl, WAVE);
-  const uint64_t ver = shfl64(ver_l, sl);
-  const uint32_t pos = up & UPOS_SLOT;  // the key's slot when found
-  const bool hfound = (up & UPOS_FOUND) != 0;
-  const uint32_t hcount = up >> UPOS_COUNT_SHIFT;
-  // A hint out of range (never written by the lookup kernel) is not acted on.
-  const bool act = src >= 0 && leaf < t.capacity && hcount <= (uint32_t)F &&
-                   (!hfound || pos < hcount);
-  const size_t base = (size_t)(act ? leaf : 0u) * F;
-  NodeMeta* m = t.meta + (act ? leaf : 0u);
-  uint64_t info = 0, low = 0, high = 0, word = 0, old = 0;
-  // The leaf's metadata line, the found key's value and the G groups before the op go out
-  // together.
-  const bool has_prev = act && (uint32_t)g < gi;
-  uint64_t pkey = 0;
-  uint8_t pop = UOP_SKIP;
-  if (act) {
-    word = m->lock;
-    info = m->info;
-    low = m->low;
-    high = m->high;
-    if (has_prev) {
-      pkey = ukey[gi - 1 - (uint32_t)g];
-      pop = uop[gi - 1 - (uint32_t)g];
-    }
-    if (hfound && g == 0) old = t.vals[base + pos];
-  }
-  old = shfl64(old, gbase);
-  // Keys fall as g grows, so the groups inside the leaf's range are a prefix of the G read.
-  const bool in_leaf = has_prev && pkey >= low;
-  const uint64_t gmask = (G == WAVE ? ~0ull : ((1ull << G) - 1)) << gbase;
-  const uint64_t inside = ballot(in_leaf) & gmask;
-  const bool owner = (ballot(in_leaf && pop == OP_INSERT) & gmask) == 0 && inside != gmask;
-  const bool held = act && owner && !(word & 1ull);
-  const bool fresh = held && word == ver;
-  const uint32_t count = meta_count(info);
-  const bool fits = fresh && meta_level(info) == 0 && count == hcount && key >= low && key < high;
-  const bool found = fits && hfound;
-  const bool insert = fits && !hfound && count < (uint32_t)F;
-  const bool commit = found || insert;
-  if (found) {
-    if (g == 0) t.vals[base + pos] = val;
-  } else {
-    old = 0;
-  }
-  if (insert && g == 0) {  // slot count is free (KEY_EMPTY)
-    t.keys[base + count] = key;
-    t.vals[base + count] = val;
-  }
-  if (insert && g == 1 % G) st_relaxed(&m->info, make_info(count + 1, 0));
-  if (commit && g == 0) st_relaxed(&m->lock, word + 2);
-  if (commit) {
-    for (uint32_t p = (uint32_t)g; p < np; p += G) {
-      const uint32_t pos_o = p == 0 ? p0 : pos_of(sidx[gs + p]);
-      out_vals[pos_o] = old;
-      out_found[pos_o] = found ? 1 : 0;
-    }
-  }
-  const uint64_t leaders = ballot(commit && g == 0);
-  const uint64_t news = ballot(insert && g == 0);
-  c.commits += (uint32_t)__popcll(leaders);
-  c.new_keys += (uint32_t)__popcll(news);
-  c.node_reads += (uint32_t)__popcll(ballot(act && g == 0));
-  uint64_t done = 0;
-#pragma unroll
-  for (int q = 0; q < WAVE / G; ++q) {
-    const int sq = __builtin_amdgcn_readlane(src, q * G);
-    if ((leaders >> (q * G)) & 1ull) done |= 1ull << sq;
-  }
-  return done;
-}
-
-// Fast-path kernel over the batch's merged INSERTs (ilist, n_upserts entries): each wavefront
-// owns a contiguous part and runs it NG ops at a time on the lane-group fast path.  The ops it
-// hands back go to the same part of slist, from its start, and their number to scount[wave]:
-// no counter is shared (one hot address took an atomic from every wavefront at once, at the
-// end of the launch).
 // Answers of the hot GET groups the lookup kernel queued (more than FANOUT_DIRECT waiting
 // ops): chunk c of the queue is op range [first, first + FANOUT_CHUNK) of group g's waiting
-// ops, written by one workgroup, chunks spread over the grid.  Runs at the start of the upsert
-// fast path, whose writes (INSERT groups' answers) never touch a GET group's ops.  Reference:
+// ops, written by one workgroup, chunks spread over the grid.  Runs at the start of k_upsert_runs,
+// whose writes (INSERT groups' answers) never touch a GET group's ops.  Reference:
 // the per-op answer write-back, writebackAns (src/gpu-stm-tree-v38/bpt-gpustm-kernel-aux.cuh:46-56).
 STM_DEV void fanout_answers(const uint64_t* __restrict__ fanout, uint64_t cap,
                             const BatchCounters* cnt, const uint32_t* __restrict__ gstart,
@@ -1545,98 +1441,16 @@ STM_DEV void fanout_answers(const uint64_t* __restrict__ fanout, uint64_t cap,
   }
 }
 
-template <int F, int G>
-__global__ __launch_bounds__(256) void k_upsert_fast(TreeView t, const uint64_t* __restrict__ ukey,
-                                                     const uint64_t* __restrict__ uval,
-                                                     const uint8_t* __restrict__ uop,
-                                                     const uint32_t* __restrict__ gstart,
-                                                     const uint32_t* __restrict__ npend,
-                                                     const uint32_t* __restrict__ sidx,
-                                                     const uint32_t* __restrict__ ilist,
-                                                     const InsHint* __restrict__ ihint,
-                                                     BatchCounters* cnt, uint32_t* __restrict__ slist,
-                                                     uint32_t* __restrict__ scount,
-                                                     uint64_t* __restrict__ out_vals,
-                                                     uint8_t* __restrict__ out_found,
-                                                     const BatchDesc* __restrict__ desc,
-                                                     const uint64_t* __restrict__ fanout,
-                                                     uint64_t fanout_cap,
-                                                     const uint64_t* __restrict__ gval) {
-  constexpr int NG = WAVE / G;
-  const uint32_t N = cnt->n_upserts;
-  if (desc) {
-    out_vals = desc->out_vals;
-    out_found = desc->out_found;
-  }
-  if (fanout) fanout_answers(fanout, fanout_cap, cnt, gstart, npend, gval, sidx, out_vals, out_found);
-  const uint32_t nw = gridDim.x * (blockDim.x / WAVE);
-  const uint32_t w = uniform32((blockIdx.x * blockDim.x + threadIdx.x) / WAVE);
-  const uint32_t per = (N + nw - 1) / nw;
-  const uint32_t e0 = min(w * per, N);
-  const uint32_t e1 = min(e0 + per, N);
-  TxCounters c;
-  uint32_t upserts = 0;
-  uint32_t handed = 0;  // ops handed back so far (slist[e0 .. e0 + handed))
-  for (uint32_t base = e0; base < e1; base += WAVE) {
-    const uint32_t e = base + lane_id();
-    const bool mine = e < e1;
-    // Unconditional loads from an index clamped into the range (e1 > base), selected
-    // afterwards, so the gathers issue together.
-    const uint32_t gi = ilist[mine ? e : e1 - 1];
-    uint64_t todo = ballot(mine);
-    const InsHint h = ihint[gi];
-    const uint64_t v_raw = uval[gi];
-    const uint64_t k_raw = ukey[gi];
-    const uint32_t gs_raw = h.gs;
-    const uint32_t np_raw = h.np;
-    const uint32_t leaf_raw = h.leaf;
-    const uint64_t ver_raw = h.ver;
-    const uint32_t up_raw = h.pos;
-    const uint64_t k_l = mine ? k_raw : 0;
-    const uint64_t v_l = mine ? v_raw : 0;
-    const uint32_t gs_l = mine ? gs_raw : 0;
-    const uint32_t np_l = mine ? np_raw : 0;
-    const uint32_t leaf_l = mine ? leaf_raw : NODE_NONE;
-    const uint64_t ver_l = mine ? ver_raw : 1ull;
-    const uint32_t up_l = mine ? up_raw : 0u;
-    // The first answered op's input position, loaded with the op data rather than inside
-    // the round (gs_l is a sorted position of the batch).
-    const uint32_t sx_raw = sidx[gs_l];
-    const uint32_t p0_l = (mine && np_l) ? pos_of(sx_raw) : 0u;
-    for (uint64_t rest = todo; rest;) {
-      // group q takes the q-th remaining op of the round
-      int my_src = -1;
-#pragma unroll
-      for (int q = 0; q < NG; ++q) {
-        const int l = rest ? __builtin_ctzll(rest) : -1;
-        if (l >= 0) rest &= rest - 1;
-        if (lane_id() / G == q) my_src = l;
-      }
-      const uint64_t done = fast_leaf_upserts<F, G>(t, my_src, k_l, v_l, leaf_l, ver_l, up_l, gi,
-                                                    ukey, uop, gs_l, np_l, p0_l, sidx, out_vals,
-                                                    out_found, c);
-      upserts += (uint32_t)__popcll(done);
-      todo &= ~done;
-    }
-    if ((todo >> lane_id()) & 1ull)  // handed back
-      slist[e0 + handed + (uint32_t)__popcll(todo & lanemask_lt())] = gi;
-    handed += (uint32_t)__popcll(todo);
-  }
-  if (lane_id() == 0) scount[w] = handed;
-  flush_counters(t, c);
-  if (lane_id() == 0) stat_add(t.stats, ST_UPSERTS, wave_stripe(), upserts);
-}
-
 // Answers of the committed ops of a round (lanes with ans): a lane writes its own group's few
-// waiting ops (np of them from sorted position gs); a group with many (a hot key) is written by
-// the whole wavefront.  Called by every lane of the wavefront.
+// waiting ops (np of them from sorted position gs, p0 the first one's input position); a group
+// with many (a hot key) is written by the whole wavefront.  Called by every lane of the wavefront.
 STM_DEV void write_upsert_answers(bool ans, bool found, uint64_t old, uint32_t gs, uint32_t np,
-                                  const uint32_t* __restrict__ sidx,
+                                  uint32_t p0, const uint32_t* __restrict__ sidx,
                                   uint64_t* __restrict__ out_vals, uint8_t* __restrict__ out_found) {
   const bool many = ans && np > 8;
   if (ans && !many) {
     for (uint32_t p = 0; p < np; ++p) {
-      const uint32_t pos = pos_of(sidx[gs + p]);
+      const uint32_t pos = p == 0 ? p0 : pos_of(sidx[gs + p]);
       out_vals[pos] = old;
       out_found[pos] = found ? 1 : 0;
     }
@@ -1655,148 +1469,839 @@ STM_DEV void write_upsert_answers(bool ans, bool found, uint64_t old, uint32_t g
   }
 }
 
-// Wave-wide transactions for the ops the fast path handed back, or for every merged INSERT
-// of the batch when slist is null.  The handed-back ops lie in the insert list's index range
-// [0, n_upserts): fast-path wavefront f owned [f * per_f, (f + 1) * per_f) and wrote its
-// scount[f] ops from the start of that range.  Each wavefront here owns a contiguous part of
-// the index range (key order within a part), so consecutive upserts mostly reuse the cached
-// parent.
+// Leaf of insert-list entry e as the lookup kernel routed it.
+STM_DEV uint32_t entry_leaf(const uint32_t* __restrict__ ilist, const InsHint* __restrict__ ihint,
+                            uint32_t e) {
+  return ihint[ilist[e]].leaf;
+}
+
+// First entry after `from` whose leaf differs from the leaf of `from` (N if none): entries of a
+// leaf are neighbours in the list, and every lane probes one entry of the range per step.
+STM_DEV uint32_t run_end(const uint32_t* __restrict__ ilist, const InsHint* __restrict__ ihint,
+                         uint32_t from, uint32_t N, uint32_t leaf) {
+  const uint32_t lane = (uint32_t)lane_id();
+  uint32_t lo = from + 1, hi = N;  // the answer lies in [lo, hi]
+  while (hi - lo > (uint32_t)WAVE) {
+    const uint32_t step = (hi - lo + WAVE - 1) / WAVE;
+    const uint32_t at = lo + lane * step;
+    const uint32_t same = (uint32_t)__popcll(
+        ballot(at < hi && entry_leaf(ilist, ihint, min(at, N - 1)) == leaf));
+    if (same == 0) return lo;
+    const uint32_t up = min(hi, lo + same * step);
+    lo += (same - 1) * step + 1;
+    hi = up;
+  }
+  const uint32_t at = lo + lane;
+  return lo + (uint32_t)__popcll(ballot(at < hi && entry_leaf(ilist, ihint, min(at, N - 1)) == leaf));
+}
+
+// The node at `level` (1 or more) whose range holds key, by a descent from the root; NODE_NONE if
+// the tree is not that high.  For kernels in which no node above that level is being written.
+template <int F>
+STM_DEV uint32_t find_at_level(const TreeView& t, uint64_t key, uint32_t level) {
+  constexpr int SPL = WNode<F>::SPL;
+  uint32_t node = (uint32_t)uniform64(t.hdr->root);
+  const uint32_t height = (uint32_t)min<uint64_t>(uniform64(t.hdr->height), 64);
+  if (height <= level) return NODE_NONE;
+  for (uint32_t lvl = height - 1; lvl > level && node < t.capacity; --lvl) {
+    uint64_t k[SPL], v[SPL];
+#pragma unroll
+    for (int j = 0; j < SPL; ++j) {
+      const int sl = j * WAVE + lane_id();
+      const size_t at = (size_t)node * F + (size_t)min(sl, F - 1);
+      const uint64_t kk = t.keys[at];
+      v[j] = t.vals[at];
+      k[j] = sl < F ? kk : KEY_EMPTY;
+    }
+    const uint32_t cle = wave_count_le<F>(k, key);
+    node = (uint32_t)wave_at<F>(v, cle ? cle - 1 : 0);
+  }
+  return node < t.capacity ? node : NODE_NONE;
+}
+
+// How the T entries of an overfull node are spread over nl nodes: node j gets entries [bound(j),
+// bound(j + 1)) in key order, one more in the first T mod nl nodes.  Node 0 is the old one, node
+// j > 0 has id base + j - 1.
+struct Spread {
+  uint32_t node, base, nl, per, more;
+  STM_DEV Spread(uint32_t T, uint32_t nl_, uint32_t node_, uint32_t base_)
+      : node(node_), base(base_), nl(nl_), per(T / nl_), more(T % nl_) {}
+  STM_DEV uint32_t bound(uint32_t j) const { return j * per + min(j, more); }
+  STM_DEV uint32_t id(uint32_t j) const { return j == 0 ? node : base + j - 1; }
+  // Node of the entry of rank r.
+  STM_DEV uint32_t part(uint32_t r) const {
+    const uint32_t q = more * (per + 1);
+    return r < q ? r / (per + 1) : more + (r - q) / per;
+  }
+};
+
+// Nodes an overfull node of T entries is spread over: three quarters full each, as built.
+template <int F>
+STM_DEV uint32_t spread_nodes(uint32_t T) {
+  constexpr uint32_t PER = F - F / 4;
+  return (T + PER - 1) / PER;
+}
+
+// One entry to its place; the first entry of a new node is its low fence and the high fence of the
+// node before it.
+template <int F>
+STM_DEV void spread_entry(const TreeView& t, const Spread& sp, uint32_t r, uint64_t k, uint64_t v) {
+  const uint32_t j = sp.part(r);
+  const uint32_t slot = r - sp.bound(j);
+  const size_t at = (size_t)sp.id(j) * F + slot;
+  t.keys[at] = k;
+  t.vals[at] = v;
+  if (slot == 0 && j > 0) {
+    st_relaxed(&t.meta[sp.id(j)].low, k);
+    st_relaxed(&t.meta[sp.id(j - 1)].high, k);
+  }
+}
+
+// The rest of a spread, by `waves` wavefronts of which this is the wave-th: free slots, counts,
+// sibling links, the last node's high fence, and the note for the parent.  used: entries the old
+// node held.
+template <int F>
+STM_DEV void spread_finish(const TreeView& t, const Spread& sp, uint32_t level, uint32_t used,
+                           uint64_t high, uint64_t next, uint32_t wave = 0, uint32_t waves = 1) {
+  const uint32_t lane = (uint32_t)lane_id();
+  for (uint32_t j = wave; j < sp.nl; j += waves) {
+    const uint32_t n = sp.bound(j + 1) - sp.bound(j);
+    const uint32_t end = j == 0 ? used : (uint32_t)F;
+    for (uint32_t sl = n + lane; sl < end; sl += WAVE) {
+      t.keys[(size_t)sp.id(j) * F + sl] = KEY_EMPTY;
+      t.vals[(size_t)sp.id(j) * F + sl] = 0;
+    }
+  }
+  for (uint32_t j = wave * WAVE + lane; j < sp.nl; j += waves * WAVE) {
+    NodeMeta* m = t.meta + sp.id(j);
+    const bool last = j + 1 == sp.nl;
+    st_relaxed(&m->info, make_info(sp.bound(j + 1) - sp.bound(j), level));
+    st_relaxed(&m->next, last ? next : (uint64_t)sp.id(j + 1));
+    if (last) st_relaxed(&m->high, high);
+    if (j == 0 && sp.nl > 1) st_relaxed(&m->made, (uint64_t)sp.base | ((uint64_t)(sp.nl - 1) << 32));
+  }
+}
+
+// Splits the overfull leaf of a run (entries unordered, `newm` the lanes with new keys, in key
+// order) over nl nodes.  The leaf belongs to this wavefront; nothing is locked and the parent is
+// not touched.
+template <int F>
+STM_DEV void split_run(const TreeView& t, uint32_t leaf, uint32_t base, uint32_t nl, uint64_t newm,
+                       uint64_t key, uint64_t val) {
+  constexpr int SPL = WNode<F>::SPL;
+  const uint32_t lane = (uint32_t)lane_id();
+  const uint64_t high = uniform64(t.meta[leaf].high), next = uniform64(t.meta[leaf].next);
+  const uint32_t count = meta_count(uniform64(t.meta[leaf].info));
+  uint64_t k[SPL], v[SPL];
+#pragma unroll
+  for (int j = 0; j < SPL; ++j) {
+    const int sl = j * WAVE + (int)lane;
+    const size_t at = (size_t)leaf * F + (size_t)min(sl, F - 1);
+    const uint64_t kk = t.keys[at];
+    v[j] = t.vals[at];
+    k[j] = sl < F ? kk : KEY_EMPTY;
+  }
+  const Spread sp(count + (uint32_t)__popcll(newm), nl, leaf, base);
+  // Places in key order: the old entries below plus the new keys below.
+  uint32_t r[SPL];
+#pragma unroll
+  for (int j = 0; j < SPL; ++j) r[j] = 0;
+  uint32_t rn = (uint32_t)__popcll(newm & lanemask_lt());
+  for (uint32_t i = 0; i < count; ++i) {
+    const uint64_t ki = wave_at<F>(k, i);
+#pragma unroll
+    for (int j = 0; j < SPL; ++j) r[j] += ki < k[j] ? 1u : 0u;
+    rn += ki < key ? 1u : 0u;
+  }
+  for (uint64_t rest = newm; rest; rest &= rest - 1) {
+    const uint64_t ki = readlane64(key, __builtin_ctzll(rest));
+#pragma unroll
+    for (int j = 0; j < SPL; ++j) r[j] += ki < k[j] ? 1u : 0u;
+  }
+#pragma unroll
+  for (int j = 0; j < SPL; ++j)
+    if ((uint32_t)(j * WAVE) + lane < count) spread_entry<F>(t, sp, r[j], k[j], v[j]);
+  if ((newm >> lane) & 1ull) spread_entry<F>(t, sp, rn, key, val);
+  spread_finish<F>(t, sp, 0, count, high, next);
+  if (t.rank_of && lane == 0) {
+    const uint32_t q = t.rank_of[leaf];
+    if (q != NODE_NONE) t.dir[q].pflags |= DIR_SPLIT;
+  }
+}
+
+// First id of n new inner nodes (after the batch's new leaves; the pool holds them, see the request
+// in k_upsert_runs).
+STM_DEV uint32_t new_inner(const TreeView& t, SplitState* split, uint32_t n) {
+  uint32_t at = 0;
+  if (lane_id() == 0) at = atomicAdd(&split->inner, n);
+  return (uint32_t)uniform64(t.hdr->n_nodes) + min(uniform32(split->made), uniform32(split->refused)) +
+         uniform32(at);
+}
+
+// Brings the new children of inner node id (each child's `made`) into it; run by one wavefront.
+// A node that overfills is spread over several like a leaf.  Returns whether it was.
+template <int F>
+STM_DEV bool absorb_children(const TreeView& t, SplitState* split, uint32_t id, TxCounters& c) {
+  constexpr int SPL = WNode<F>::SPL;
+  const uint32_t lane = (uint32_t)lane_id();
+  NodeMeta* m = t.meta + id;
+  // Agent-scope loads where an earlier level of the same launch may have written.
+  const uint64_t info = uniform64(ld_relaxed(&m->info)), high = uniform64(ld_relaxed(&m->high));
+  const uint64_t next = uniform64(ld_relaxed(&m->next));
+  const uint32_t count = min(meta_count(info), (uint32_t)F);
+  uint64_t k[SPL], v[SPL], made[SPL];
+#pragma unroll
+  for (int j = 0; j < SPL; ++j) {
+    const int sl = j * WAVE + (int)lane;
+    const size_t at = (size_t)id * F + (size_t)min(sl, F - 1);
+    k[j] = t.keys[at];
+    v[j] = t.vals[at];
+  }
+  uint32_t r[SPL], total = 0;
+#pragma unroll
+  for (int j = 0; j < SPL; ++j) {
+    const uint32_t sl = (uint32_t)(j * WAVE) + lane;
+    made[j] = sl < count && v[j] < t.capacity ? ld_relaxed(&t.meta[v[j]].made) : 0;
+    const uint32_t x = (uint32_t)(made[j] >> 32);
+    if (x) st_relaxed(&t.meta[v[j]].made, 0ull);
+    uint32_t incl = x;
+#pragma unroll
+    for (int off = 1; off < WAVE; off <<= 1) {
+      const uint32_t y = __shfl_up(incl, off, WAVE);
+      if ((int)lane >= off) incl += y;
+    }
+    r[j] = sl + total + incl - x;
+    total += (uint32_t)__builtin_amdgcn_readlane((int)incl, WAVE - 1);
+  }
+  if (lane == 0) st_relaxed(&m->dirty, 0ull);
+  if (total == 0) return false;
+  const uint32_t T = count + total;
+  const uint32_t nl = T <= (uint32_t)F ? 1u : spread_nodes<F>(T);
+  const Spread sp(T, nl, id, nl > 1 ? new_inner(t, split, nl - 1) : 0u);
+#pragma unroll
+  for (int j = 0; j < SPL; ++j) {
+    const uint32_t sl = (uint32_t)(j * WAVE) + lane;
+    if (sl < count) {
+      if (nl > 1 || r[j] != sl) spread_entry<F>(t, sp, r[j], k[j], v[j]);
+    }
+    // The new children: a lane those of its own child, the whole wavefront where there are many.
+    const uint32_t x = (uint32_t)(made[j] >> 32), b = (uint32_t)made[j];
+    const bool many = x > 8;
+    for (uint32_t q = 0; q < (many ? 0u : x); ++q)
+      spread_entry<F>(t, sp, r[j] + 1 + q, ld_relaxed(&t.meta[b + q].low), (uint64_t)(b + q));
+    for (uint64_t mm = ballot(many); mm; mm &= mm - 1) {
+      const int l = __builtin_ctzll(mm);
+      const uint32_t xl = (uint32_t)__builtin_amdgcn_readlane((int)x, l);
+      const uint32_t bl = (uint32_t)__builtin_amdgcn_readlane((int)b, l);
+      const uint32_t rl = (uint32_t)__builtin_amdgcn_readlane((int)r[j], l);
+      for (uint32_t q = lane; q < xl; q += WAVE)
+        spread_entry<F>(t, sp, rl + 1 + q, ld_relaxed(&t.meta[bl + q].low), (uint64_t)(bl + q));
+    }
+  }
+  c.node_reads++;
+  if (nl == 1) {
+    if (lane == 0) st_relaxed(&m->info, make_info(T, meta_level(info)));
+    return false;
+  }
+  spread_finish<F>(t, sp, meta_level(info), count, high, next);
+  c.inner_splits += nl - 1;
+  c.commits++;
+  return true;
+}
+
+// Puts inner node id on the list of parents with new children, once.
+STM_DEV void list_parent(const TreeView& t, uint32_t id, uint32_t* __restrict__ list, uint32_t* n) {
+  if (atomicOr((unsigned long long*)&t.meta[id].dirty, 1ull) == 0) list[atomicAdd(n, 1u)] = id;
+}
+
+// Parents of split leaves: one wavefront per level-1 node.  A node that is itself split is listed
+// for the level above (k_upsert_upper), by its parent; the root is noted instead.
+template <int F>
+STM_DEV void absorb_and_list(const TreeView& t, SplitState* split, uint32_t id, uint32_t level,
+                             uint32_t* __restrict__ list, uint32_t* n, TxCounters& c) {
+  const uint64_t low = uniform64(t.meta[id].low);
+  if (!absorb_children<F>(t, split, id, c)) return;
+  if ((uint32_t)uniform64(t.hdr->root) == id) {
+    if (lane_id() == 0)
+      __hip_atomic_store(&split->root, id + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  } else {
+    const uint32_t up = find_at_level<F>(t, low, level + 1);
+    if (up != NODE_NONE && lane_id() == 0) list_parent(t, up, list, n);
+  }
+}
+
+template <int F>
+__global__ __launch_bounds__(256) void k_upsert_parents(TreeView t, SplitState* split,
+                                                        const uint32_t* __restrict__ plist,
+                                                        uint32_t* __restrict__ plist2) {
+  const uint32_t n = split->n_dirty;
+  const uint32_t nw = gridDim.x * (blockDim.x / WAVE);
+  const uint32_t w = uniform32((blockIdx.x * blockDim.x + threadIdx.x) / WAVE);
+  if (w >= n) return;
+  TxCounters c;
+  for (uint32_t i = w; i < n; i += nw)
+    absorb_and_list<F>(t, split, uniform32(plist[i]), 1, plist2, &split->n_dirty2, c);
+  flush_counters(t, c);
+}
+
+// The levels above: one workgroup, level by level (a level lists at most one node per split node
+// of the level below, a 48th of them in the mean), then a new root if the root was split.  Takes
+// level 1 too when first_level is 1 (few inserts: the list is short and a launch is saved).
+template <int F>
+__global__ __launch_bounds__(1024) void k_upsert_upper(TreeView t, SplitState* split,
+                                                       uint32_t* plist, uint32_t* plist2,
+                                                       uint32_t first_level) {
+  __shared__ uint32_t s_n[2];
+  const uint32_t wave = uniform32(threadIdx.x / WAVE);
+  if (split->made == 0) return;
+  if (threadIdx.x == 0) {
+    s_n[0] = first_level == 1 ? split->n_dirty : split->n_dirty2;
+    s_n[1] = 0;
+  }
+  __syncthreads();
+  TxCounters c;
+  uint32_t* from = first_level == 1 ? plist : plist2;
+  uint32_t* to = first_level == 1 ? plist2 : plist;
+  uint32_t cur = 0;
+  for (uint32_t level = first_level; level < 64; ++level) {
+    const uint32_t n = s_n[cur];
+    if (n == 0) break;
+    for (uint32_t i = wave; i < n; i += 1024 / WAVE)
+      absorb_and_list<F>(t, split, uniform32(ld_relaxed32(from + i)), level, to, &s_n[cur ^ 1], c);
+    __syncthreads();  // the level's nodes and the next level's list are written
+    if (threadIdx.x == 0) s_n[cur] = 0;
+    cur ^= 1;
+    uint32_t* x = from;
+    from = to;
+    to = x;
+    __syncthreads();
+  }
+  __syncthreads();
+  if (wave == 0) {
+    const uint32_t lane = (uint32_t)lane_id();
+    const uint32_t r1 = uniform32(ld_relaxed32(&split->root));
+    if (r1) {
+      // The split root and its new siblings become the children of a new root, over as many
+      // levels as they take (one, unless a batch put tens of thousands of keys into the tree's
+      // only leaf).
+      uint32_t node = r1 - 1, made = 0;  // the top level: node, then made siblings from base on
+      uint32_t base = 0;
+      const uint64_t m0 = uniform64(ld_relaxed(&t.meta[node].made));
+      base = (uint32_t)m0;
+      made = (uint32_t)(m0 >> 32);
+      uint32_t level = meta_level(uniform64(ld_relaxed(&t.meta[node].info)));
+      while (made) {
+        const uint32_t T = made + 1;
+        const uint32_t nl = T <= (uint32_t)F ? 1u : spread_nodes<F>(T);
+        const uint32_t q = new_inner(t, split, nl);
+        const Spread sp(T, nl, q, q + 1);
+        level += 1;
+        for (uint32_t r = lane; r < T; r += WAVE) {
+          const uint32_t child = r == 0 ? node : base + r - 1;
+          spread_entry<F>(t, sp, r, r == 0 ? 0ull : ld_relaxed(&t.meta[child].low), (uint64_t)child);
+        }
+        spread_finish<F>(t, sp, level, (uint32_t)F, KEY_EMPTY, (uint64_t)NODE_NONE);
+        if (lane == 0) {
+          st_relaxed(&t.meta[q].low, 0ull);
+          st_relaxed(&t.meta[q].made, 0ull);
+          st_relaxed(&t.meta[node].made, 0ull);
+          t.hdr->root = q;
+          t.hdr->height = level + 1;
+        }
+        wave_order();  // the next level reads these nodes' fences
+        node = q;
+        base = q + 1;
+        made = nl - 1;
+        c.root_splits++;
+      }
+    }
+    if (lane == 0)
+      t.hdr->n_nodes += min(split->made, split->refused) + ld_relaxed32(&split->inner);
+  }
+  flush_counters(t, c);
+}
+
+// New leaves for a request of n: the first id, or NODE_NONE if the pool could not also hold every
+// inner node that may follow.  The ids start at the header's n_nodes, which no kernel moves
+// before k_upsert_upper.  A split leaves every node at least half full, so new inner nodes number
+// at most one per F / 2 - 1 nodes; nor are there more than one per new leaf and level.  By one lane.
+template <int F>
+STM_DEV uint32_t new_leaves(const TreeView& t, SplitState* split, uint32_t n) {
+  const uint32_t at = atomicAdd(&split->made, n);
+  const uint64_t nodes = t.hdr->n_nodes, made = (uint64_t)at + n;
+  const uint64_t inner = min(made * (t.hdr->height + 1), (nodes + made) / (F / 2 - 1));
+  if (nodes + made + inner + 64 <= t.capacity) return (uint32_t)nodes + at;
+  atomicMin(&split->refused, at);
+  return NODE_NONE;
+}
+
+// Exclusive count, over a workgroup of 1024 threads, of the threads with p, and their total.
+STM_DEV uint32_t block_rank_1024(bool p, uint32_t* s_w /*[16]*/, uint32_t& total) {
+  const uint32_t wave = threadIdx.x / WAVE;
+  const uint64_t m = ballot(p);
+  if (lane_id() == 0) s_w[wave] = (uint32_t)__popcll(m);
+  __syncthreads();
+  uint32_t before = 0;
+  total = 0;
+#pragma unroll
+  for (uint32_t q = 0; q < 1024 / WAVE; ++q) {
+    const uint32_t x = s_w[q];
+    before += q < wave ? x : 0u;
+    total += x;
+  }
+  __syncthreads();
+  return before + (uint32_t)__popcll(m & lanemask_lt());
+}
+
+// Number of the n ascending keys below x.
+STM_DEV uint32_t count_below(const uint64_t* s, uint32_t n, uint64_t x) {
+  uint32_t lo = 0, hi = n;
+  while (lo < hi) {
+    const uint32_t mid = (lo + hi) >> 1;
+    if (s[mid] < x) lo = mid + 1;
+    else hi = mid;
+  }
+  return lo;
+}
+
+// Runs of more than 64 ops: one workgroup takes a run 1024 ops at a time.  The first pass answers
+// the ops, stores the values of keys the leaf holds and counts the new keys; the second merges the
+// new keys (in order already) with the leaf's entries by rank and writes each to its place in the
+// old leaf or one of the new ones.  As in split_run nothing is locked and the parent learns of the
+// new leaves from the next launches.  (Transactions of up to 64 keys each, one after the other
+// since they share a leaf, took 20 µs apiece: the first batch of 2^21 ops at 50/50 beside Zipf-hot
+// keys, a quarter of its inserts in one leaf, took 75 ms that way and takes 3.1 ms.)
+template <int F>
+__global__ __launch_bounds__(1024) void k_upsert_long(TreeView t, const uint64_t* __restrict__ ukey,
+                                                      const uint64_t* __restrict__ uval,
+                                                      const uint32_t* __restrict__ sidx,
+                                                      const uint32_t* __restrict__ ilist,
+                                                      const InsHint* __restrict__ ihint,
+                                                      BatchCounters* cnt, SplitState* split,
+                                                      uint32_t* __restrict__ plist,
+                                                      const uint32_t* __restrict__ rlist,
+                                                      const uint32_t* __restrict__ rlen,
+                                                      uint32_t* __restrict__ dlist,
+                                                      uint64_t* __restrict__ out_vals,
+                                                      uint8_t* __restrict__ out_found,
+                                                      const BatchDesc* __restrict__ desc) {
+  constexpr uint32_t BT = 1024;
+  __shared__ uint64_t s_raw[F], s_xk[F], s_xv[F];
+  __shared__ uint64_t s_new[BT];
+  __shared__ uint32_t s_w[BT / WAVE];
+  __shared__ uint32_t s_base;
+  const uint32_t runs = split->n_long;
+  if (blockIdx.x >= runs) return;
+  if (desc) {
+    out_vals = desc->out_vals;
+    out_found = desc->out_found;
+  }
+  const uint32_t tid = threadIdx.x;
+  const uint32_t wave = uniform32(tid / WAVE);
+  TxCounters c;
+  uint32_t upserts = 0, deferred = 0;
+  for (uint32_t q = blockIdx.x; q < runs; q += gridDim.x) {
+    const uint32_t e0 = rlist[q], len = rlen[q];
+    const InsHint h0 = ihint[ilist[e0]];
+    const uint64_t key0 = ukey[ilist[e0]];
+    const uint32_t leaf = h0.leaf;
+    const uint32_t count = h0.pos >> UPOS_COUNT_SHIFT;
+    const size_t nb = (size_t)leaf * F;
+    uint32_t news = 0;
+    for (uint32_t b = 0; b < len; b += BT) {
+      const bool in = b + tid < len;
+      const uint32_t gi = ilist[e0 + min(b + tid, len - 1)];
+      const InsHint h = ihint[gi];
+      const bool found = (h.pos & UPOS_FOUND) != 0;
+      const uint32_t p0 = pos_of(sidx[h.gs]);
+      uint64_t old = 0;
+      if (in && found) {
+        const size_t at = nb + (h.pos & UPOS_SLOT);
+        old = t.vals[at];
+        t.vals[at] = uval[gi];
+      }
+      write_upsert_answers(in, found, old, h.gs, h.np, p0, sidx, out_vals, out_found);
+      uint32_t total;
+      (void)block_rank_1024(in && !found, s_w, total);
+      news += total;
+    }
+    const uint32_t T = count + news;
+    const uint32_t nl = T <= (uint32_t)F ? 1u : spread_nodes<F>(T);
+    if (tid == 0) s_base = nl > 1 ? new_leaves<F>(t, split, nl - 1) : 0u;
+    __builtin_amdgcn_s_waitcnt(0);  // the values stored above are read below
+    __syncthreads();
+    const uint32_t base = s_base;
+    const uint64_t high = t.meta[leaf].high, next = t.meta[leaf].next;
+    uint64_t xk = 0, xv = 0;
+    if (tid < count) {
+      xk = t.keys[nb + tid];
+      xv = t.vals[nb + tid];
+      s_raw[tid] = xk;
+    }
+    __syncthreads();
+    uint32_t xr = 0;  // new keys below the thread's entry
+    if (tid < count) {
+      uint32_t r = 0;
+      for (uint32_t i = 0; i < count; ++i) r += s_raw[i] < xk ? 1u : 0u;
+      s_xk[r] = xk;
+      s_xv[r] = xv;
+    }
+    __syncthreads();
+    if (tid < count) {
+      xk = s_xk[tid];
+      xv = s_xv[tid];
+    }
+    const Spread sp(T, nl, leaf, base);
+    uint32_t before = 0;
+    for (uint32_t b = 0; b < len; b += BT) {
+      const bool in = b + tid < len;
+      const uint32_t gi = ilist[e0 + min(b + tid, len - 1)];
+      const bool fresh = in && !(ihint[gi].pos & UPOS_FOUND);
+      const uint64_t key = ukey[gi], val = uval[gi];
+      uint32_t total;
+      const uint32_t idx = block_rank_1024(fresh, s_w, total);
+      if (base == NODE_NONE) {  // the pool is all but full: the serial pass takes the new keys
+        if (fresh) dlist[atomicAdd(&cnt->n_deferred, 1u)] = gi;
+        continue;
+      }
+      if (fresh) s_new[idx] = key;
+      __syncthreads();
+      if (fresh) spread_entry<F>(t, sp, before + idx + count_below(s_xk, count, key), key, val);
+      if (tid < count) xr += count_below(s_new, total, xk);
+      before += total;
+      __syncthreads();
+    }
+    if (base != NODE_NONE) {
+      if (tid < count) spread_entry<F>(t, sp, tid + xr, xk, xv);
+      spread_finish<F>(t, sp, 0, count, high, next, wave, BT / WAVE);
+    }
+    __syncthreads();  // LDS is the next run's
+    if (wave == 0) {
+      upserts += len;
+      c.node_reads += len;
+      c.commits++;
+      if (base == NODE_NONE) {
+        deferred += news;
+      } else {
+        c.new_keys += news;
+        c.leaf_splits += nl - 1;
+      }
+      if (nl > 1 && base != NODE_NONE) {
+        uint32_t par = NODE_NONE;
+        const uint32_t p = h0.par;
+        if (p < t.capacity && meta_level(uniform64(t.meta[p].info)) == 1 &&
+            key0 >= uniform64(t.meta[p].low) && key0 < uniform64(t.meta[p].high))
+          par = p;
+        if (par == NODE_NONE) par = find_at_level<F>(t, key0, 1);
+        if (lane_id() == 0) {
+          if (par == NODE_NONE) split->root = leaf + 1;  // the leaf is the root
+          else list_parent(t, par, plist, &split->n_dirty);
+          if (t.rank_of) {
+            const uint32_t r = t.rank_of[leaf];
+            if (r != NODE_NONE) t.dir[r].pflags |= DIR_SPLIT;
+          }
+        }
+      }
+    }
+  }
+  if (wave == 0) {
+    flush_counters(t, c, cnt);
+    if (lane_id() == 0) {
+      stat_add(t.stats, ST_UPSERTS, blockIdx.x, upserts);
+      stat_add(t.stats, ST_DEFERRED, blockIdx.x, deferred);
+    }
+  }
+}
+
+// The batch's merged INSERTs, one lane per op.  The insert list is in key order,
+// so the ops of a leaf are neighbours in it: a run.  A wavefront owns the runs that start in its
+// part of the list, and the lanes of a run are the only ones in the launch that touch its leaf, so
+// no lock is taken and the lookup kernel's hint (leaf, slot, entry count) is exact: no writer ran
+// since.  The r-th new key of a run is appended at slot count + r (a ballot; leaf entries are
+// unordered), a present key takes its value in place, and the run's first lane writes the new
+// count.  A run that overfills its leaf is split here (split_run) into new leaves that only the
+// sibling chain knows; the parents are brought up to date by the next two launches, one
+// wavefront per parent, so that the splits under one parent do not queue for its lock.
+// Runs too long for a window go to k_upsert_long (split->n_long of them, from the start of rlist and
+// rlen).  With piece below 64 (upsert_ops_per_wave: fewer ops per wavefront than a window holds),
+// runs of more than `piece` ops go to the transactions of k_upsert instead, cut into pieces of that
+// many: wavefront w records them at rlist (first entry) and rlen (ops) from index rfirst[w] on,
+// rcount[w] of them; that is the index of the first run it owns, so no two wavefronts' records
+// meet.
+// Bound by the gathers and scattered stores of an op (its record, key, value, the leaf's slot and
+// its answer, each a line of its own), all of which are in flight at once for 64 ops.  In the form
+// before, lane groups of eight proved by reading eight earlier groups that an op was the first of
+// its leaf, every other op of a leaf took a test-and-set of its lock, and every split a transaction
+// through its parent's lock.  Upsert kernels per batch, before / now: 2^22 ops at 95/5 (210 K
+// inserts) 73 / 57 µs; 2^19 ops at 50/50 (262 K inserts, most leaves split) 517 / 99 µs; 2^14 ops
+// at 50/50 beside Zipf-hot keys 830 / 72 µs.
+template <int F>
+__global__ __launch_bounds__(256) void k_upsert_runs(TreeView t, const uint64_t* __restrict__ ukey,
+                                                     const uint64_t* __restrict__ uval,
+                                                     const uint32_t* __restrict__ gstart,
+                                                     const uint32_t* __restrict__ npend,
+                                                     const uint32_t* __restrict__ sidx,
+                                                     const uint32_t* __restrict__ ilist,
+                                                     const InsHint* __restrict__ ihint,
+                                                     BatchCounters* cnt, uint32_t piece,
+                                                     SplitState* split,
+                                                     uint32_t* __restrict__ plist,
+                                                     uint32_t* __restrict__ rlist,
+                                                     uint32_t* __restrict__ rlen,
+                                                     uint32_t* __restrict__ rfirst,
+                                                     uint32_t* __restrict__ rcount,
+                                                     uint32_t* __restrict__ dlist,
+                                                     uint64_t* __restrict__ out_vals,
+                                                     uint8_t* __restrict__ out_found,
+                                                     const BatchDesc* __restrict__ desc,
+                                                     const uint64_t* __restrict__ fanout,
+                                                     uint64_t fanout_cap,
+                                                     const uint64_t* __restrict__ gval) {
+  const uint32_t N = cnt->n_upserts;
+  if (desc) {
+    out_vals = desc->out_vals;
+    out_found = desc->out_found;
+  }
+  if (fanout) fanout_answers(fanout, fanout_cap, cnt, gstart, npend, gval, sidx, out_vals, out_found);
+  const uint32_t nw = gridDim.x * (blockDim.x / WAVE);
+  const uint32_t w = uniform32((blockIdx.x * blockDim.x + threadIdx.x) / WAVE);
+  const uint32_t per = max((N + nw - 1) / nw, (uint32_t)WAVE);
+  const uint32_t e0 = (uint32_t)min<uint64_t>((uint64_t)w * per, N);
+  const uint32_t e1 = min(e0 + per, N);
+  const uint32_t lane = (uint32_t)lane_id();
+  const uint64_t lt = lanemask_lt();
+  TxCounters c;
+  uint32_t upserts = 0, deferred = 0;
+  uint32_t first = NODE_NONE;  // the first run owned
+  uint32_t recs = 0;
+  uint32_t base = e0;
+  uint32_t left = e0 > 0 && e0 < e1 ? uniform32(entry_leaf(ilist, ihint, e0 - 1)) : NODE_NONE;
+  while (base < e1) {
+    const uint32_t e = base + lane;
+    const bool in = e < N;
+    const uint32_t gi = ilist[min(e, N - 1)];
+    const uint32_t over = base + WAVE;  // the entry after the window
+    const uint32_t gi_over = ilist[min(over, N - 1)];
+    const InsHint h = ihint[gi];
+    const uint64_t key = ukey[gi];
+    const uint64_t val = uval[gi];
+    const uint32_t leaf_over = uniform32(ihint[gi_over].leaf);
+    const uint32_t p0 = pos_of(sidx[h.gs]);
+    const uint32_t leaf = h.leaf;
+    const uint32_t up = (uint32_t)__shfl((int)leaf, (int)(lane > 0 ? lane - 1 : 0), WAVE);
+    const uint32_t prev = lane > 0 ? up : left;
+    const uint64_t hm = ballot(in && (leaf != prev || e == 0));
+    const uint32_t last_leaf = (uint32_t)__builtin_amdgcn_readlane((int)leaf, WAVE - 1);
+    // The window's last run is whole when the list ends with it or the next entry has another leaf.
+    const bool whole = over >= N || leaf_over != last_leaf;
+    const uint64_t up_to = hm & (lt | (1ull << lane));
+    const uint32_t hl = up_to ? 63u - (uint32_t)__clzll((long long)up_to) : 0u;  // my run's first lane
+    const uint64_t above = hm & ~(lt | (1ull << lane));
+    const bool is_last = above == 0;
+    const uint32_t last_head = hm ? 63u - (uint32_t)__clzll((long long)hm) : 0u;
+    if (first == NODE_NONE && hm && base + (uint32_t)__builtin_ctzll(hm) < e1)
+      first = base + (uint32_t)__builtin_ctzll(hm);
+    // The ops to run now: of a whole run that starts in this wavefront's part.
+    const bool mine = in && up_to && base + hl < e1 && (!is_last || whole);
+    const uint64_t run = ballot(mine) & (~0ull << hl) &
+                         (above ? (above & (0 - above)) - 1 : ~0ull);
+    const bool hfound = (h.pos & UPOS_FOUND) != 0;
+    const uint32_t slot = h.pos & UPOS_SLOT;
+    const uint32_t count = h.pos >> UPOS_COUNT_SHIFT;
+    // Hints out of range (never written by the lookup kernel) are not acted on.
+    const bool sane = leaf < t.capacity && count <= (uint32_t)F && (!hfound || slot < count);
+    const uint64_t badm = ballot(mine && !sane);
+    const uint64_t newm = ballot(mine && !hfound) & run;
+    const uint32_t news = (uint32_t)__popcll(newm);
+    const bool fits = mine && !(badm & run) && count + news <= (uint32_t)F;
+    // Overfull runs to split here: new leaves for all of them from one request.
+    const uint32_t len = (uint32_t)__popcll(run);
+    const uint32_t nl = spread_nodes<F>(count + news);
+    const uint32_t want = mine && !fits && !(badm & run) && len <= piece && lane == hl ? nl - 1 : 0u;
+    uint64_t splitm = ballot(want != 0);
+    uint32_t nb0 = 0;  // first new leaf of the run (its first lane)
+    if (splitm) {
+      uint32_t incl = want;
+#pragma unroll
+      for (int off = 1; off < WAVE; off <<= 1) {
+        const uint32_t y = __shfl_up(incl, off, WAVE);
+        if ((int)lane >= off) incl += y;
+      }
+      const uint32_t total = (uint32_t)__builtin_amdgcn_readlane((int)incl, WAVE - 1);
+      uint32_t at = 0;
+      if (lane == 0) at = new_leaves<F>(t, split, total);
+      at = uniform32(at);
+      if (at == NODE_NONE) splitm = 0;
+      nb0 = at + incl - want;
+    }
+    const bool splits = mine && ((splitm >> hl) & 1ull);
+    const size_t nb = (size_t)(fits || splits ? leaf : 0u) * F;
+    uint64_t old = 0;
+    if (fits || splits) {
+      if (hfound) {
+        old = t.vals[nb + slot];
+        t.vals[nb + slot] = val;
+      } else if (fits) {
+        const uint32_t at = count + (uint32_t)__popcll(newm & lt);
+        t.keys[nb + at] = key;
+        t.vals[nb + at] = val;
+      }
+      if (fits && lane == hl && news) st_relaxed(&t.meta[leaf].info, make_info(count + news, 0));
+    }
+    write_upsert_answers(fits || splits, hfound, old, h.gs, h.np, p0, sidx, out_vals, out_found);
+    const uint64_t okm = ballot(fits || splits);
+    c.commits += (uint32_t)__popcll(okm & hm);
+    c.new_keys += (uint32_t)__popcll(ballot((fits || splits) && !hfound));
+    c.node_reads += (uint32_t)__popcll(okm);
+    upserts += (uint32_t)__popcll(okm);
+    if (splitm) {
+      wave_order();  // the values above are in place before the leaves are read
+      // The parents, by every run's first lane at once: the level-1 node the lookup kernel routed
+      // through when its fences hold the key, else by a descent below.
+      uint32_t par = NODE_NONE;
+      if ((splitm >> lane) & 1ull) {
+        const uint32_t p = h.par;
+        const NodeMeta* pm = t.meta + (p < t.capacity ? p : 0u);
+        const uint64_t pinfo = pm->info, plow = pm->low, phigh = pm->high;
+        if (p < t.capacity && meta_level(pinfo) == 1 && key >= plow && key < phigh) par = p;
+      }
+      for (uint64_t sm = splitm; sm; sm &= sm - 1) {
+        const int l = __builtin_ctzll(sm);
+        const uint32_t lf = (uint32_t)__builtin_amdgcn_readlane((int)leaf, l);
+        const uint32_t n = (uint32_t)__builtin_amdgcn_readlane((int)nl, l);
+        split_run<F>(t, lf, (uint32_t)__builtin_amdgcn_readlane((int)nb0, l), n, readlane64(newm, l),
+                     key, val);
+        c.leaf_splits += n - 1;
+        if ((uint32_t)__builtin_amdgcn_readlane((int)par, l) == NODE_NONE) {
+          const uint32_t p = find_at_level<F>(t, readlane64(key, l), 1);
+          if (p == NODE_NONE) {  // the leaf is the root
+            if (lane == 0) split->root = lf + 1;
+          } else if ((int)lane == l) {
+            par = p;
+          }
+        }
+      }
+      if (par != NODE_NONE) list_parent(t, par, plist, &split->n_dirty);
+    }
+    // A run that did not fit its leaf as it is: the attempt in place is given up and the run done
+    // again (a split here, or by one of the kernels after this one).
+    const uint64_t again = ballot(mine && !fits);
+    c.aborts += (uint32_t)__popcll(again & hm);
+    const uint64_t leave = ballot(mine && !fits && !splits);
+    if (piece >= (uint32_t)WAVE) {
+      // Refused by the pool (or a hint out of range): op by op in the serial pass.
+      if (leave) {
+        uint32_t at = 0;
+        if (lane == 0) at = atomicAdd(&cnt->n_deferred, (uint32_t)__popcll(leave));
+        at = uniform32(at);
+        if ((leave >> lane) & 1ull) dlist[at + (uint32_t)__popcll(leave & lt)] = gi;
+        deferred += (uint32_t)__popcll(leave);
+        upserts += (uint32_t)__popcll(leave);
+      }
+    } else {
+      for (uint64_t lm = leave & hm; lm; lm &= lm - 1) {
+        const int l = __builtin_ctzll(lm);
+        const uint32_t n = (uint32_t)__builtin_amdgcn_readlane((int)len, l);
+        const uint32_t pieces = (n + piece - 1) / piece;
+        if (lane < pieces) {
+          rlist[first + recs + lane] = base + (uint32_t)l + lane * piece;
+          rlen[first + recs + lane] = min(piece, n - lane * piece);
+        }
+        recs += pieces;
+      }
+    }
+    uint32_t next;  // lane of the first entry not dealt with (WAVE: the next window)
+    if (hm == 0 || whole || base + last_head >= e1) {
+      next = WAVE;
+    } else if (last_head > 0) {
+      next = last_head;
+    } else {
+      // A run longer than the window.
+      const uint32_t end = run_end(ilist, ihint, base + WAVE - 1, N, last_leaf);
+      const uint32_t n = end - base;
+      c.aborts++;
+      if (piece >= (uint32_t)WAVE) {
+        if (lane == 0) {
+          const uint32_t at = atomicAdd(&split->n_long, 1u);
+          rlist[at] = base;
+          rlen[at] = n;
+        }
+      } else {
+        const uint32_t pieces = (n + piece - 1) / piece;
+        for (uint32_t q = lane; q < pieces; q += WAVE) {
+          rlist[first + recs + q] = base + q * piece;
+          rlen[first + recs + q] = min(piece, n - q * piece);
+        }
+        recs += pieces;
+      }
+      left = last_leaf;
+      base = end;
+      continue;
+    }
+    left = (uint32_t)__builtin_amdgcn_readlane((int)leaf, (int)next - 1);
+    base += next;
+  }
+  if (lane == 0) {
+    rfirst[w] = first;
+    rcount[w] = recs;
+  }
+  flush_counters(t, c, cnt);
+  if (lane == 0) {
+    stat_add(t.stats, ST_UPSERTS, wave_stripe(), upserts);
+    stat_add(t.stats, ST_DEFERRED, wave_stripe(), deferred);
+  }
+}
+
+// Wave-wide transactions for the runs that k_upsert_runs left: many inserts into one leaf.
+// Wavefront f of that kernel recorded rcount[f] pieces from index rfirst[f] of rlist / rlen on.
+// With r = nw / run_waves wavefronts here per wavefront there, each takes every r-th of its pieces;
+// with fewer, wavefront w takes all pieces of wavefronts w, w + nw, ...  A piece is the ops of one
+// leaf in key order, so the ops of a round mostly commit in one transaction, and only the parent is
+// shared with other wavefronts (and the leaf, when its run was cut into pieces).
 template <int F>
 __global__ __launch_bounds__(256) void k_upsert(TreeView t, const uint64_t* __restrict__ ukey,
                                                 const uint64_t* __restrict__ uval,
-                                                const uint8_t* __restrict__ uop,
-                                                const uint32_t* __restrict__ gstart,
-                                                const uint32_t* __restrict__ npend,
                                                 const uint32_t* __restrict__ sidx,
-                                                const uint32_t* __restrict__ slist,
-                                                const uint32_t* __restrict__ scount,
-                                                uint32_t fast_waves,
+                                                const uint32_t* __restrict__ ilist,
+                                                const uint32_t* __restrict__ rlist,
+                                                const uint32_t* __restrict__ rlen,
+                                                const uint32_t* __restrict__ rfirst,
+                                                const uint32_t* __restrict__ rcount,
+                                                uint32_t run_waves,
                                                 const InsHint* __restrict__ ihint,
                                                 BatchCounters* cnt, uint32_t* __restrict__ dlist,
                                                 uint32_t max_attempts,
                                                 uint64_t* __restrict__ out_vals,
                                                 uint8_t* __restrict__ out_found,
                                                 const BatchDesc* __restrict__ desc) {
-  const uint32_t U = slist ? cnt->n_upserts : cnt->n_unique;
-  if (U == 0) return;
-  const uint32_t per_f = slist ? (U + fast_waves - 1) / fast_waves : 1u;
+  if (cnt->n_upserts == 0) return;
   if (desc) {
     out_vals = desc->out_vals;
     out_found = desc->out_found;
   }
   const uint32_t nw = gridDim.x * (blockDim.x / WAVE);
   const uint32_t w = uniform32((blockIdx.x * blockDim.x + threadIdx.x) / WAVE);
+  const uint32_t r = max(nw / run_waves, 1u);
   TxCounters c;
   ParentCache<F> pc;
   uint32_t upserts = 0, deferred = 0;
-  // The wavefront's share, as ranges [s0, s1) of the group index (no slist) or of slist.
-  // Without slist: an equal contiguous part of the groups.  With slist: fast-path wavefront f
-  // handed back scount[f] ops at slist[f * per_f ...]; with r = nw / fast_waves wavefronts per
-  // such range each takes a contiguous r-th of it (so the hand-backs, which sit at the start of
-  // each range, spread over all wavefronts), with fewer wavefronts than ranges wavefront w takes
-  // ranges w, w + nw, ...
-  for (uint32_t f = w;; f += nw) {
-    uint32_t s0, s1;
-    if (!slist) {
-      if (f != w) break;
-      const uint32_t per = (U + nw - 1) / nw;
-      s0 = min(w * per, U);
-      s1 = min(s0 + per, U);
-    } else if (nw >= fast_waves) {
-      if (f != w) break;
-      const uint32_t r = nw / fast_waves;
-      const uint32_t fi = w / r, q = w % r;
-      if (fi >= fast_waves) break;
-      const uint32_t n_f = uniform32(scount[fi]);
-      const uint32_t chunk = (n_f + r - 1) / r;
-      s0 = fi * per_f + min(q * chunk, n_f);
-      s1 = fi * per_f + min((q + 1) * chunk, n_f);
-    } else {
-      if (f >= fast_waves) break;
-      s0 = f * per_f;
-      s1 = s0 + uniform32(scount[f]);
-    }
+  for (uint32_t f = w / r; f < run_waves; f += nw / r) {
+  const uint32_t pieces = uniform32(rcount[f]);
+  const uint32_t at = uniform32(rfirst[f]);
+  for (uint32_t q = w % r; q < pieces; q += r) {
+  const uint32_t s0 = uniform32(rlist[at + q]);
+  const uint32_t s1 = s0 + uniform32(rlen[at + q]);
   for (uint32_t base = s0; base < s1; base += WAVE) {
     // Op data of the round's upserts, loaded together and read lane by lane.
     const uint32_t e = base + lane_id();
-    const bool in = e < s1;
-    const uint32_t gi = in ? (slist ? slist[e] : e) : 0;
-    const bool mine = in && (slist || uop[gi] == OP_INSERT);
+    const bool mine = e < s1;
+    const uint32_t gi = ilist[min(e, s1 - 1)];
     uint64_t todo = ballot(mine);
-    // The op: from the lookup kernel's record when there is one, else from the fold's arrays
-    // (then without leaf hints).
-    uint64_t k_l = 0, v_l = 0;
-    uint32_t gs_l = 0, np_l = 0, par_l = NODE_NONE, leaf_l = NODE_NONE, up_l = 0;
-    if (ihint) {
-      const InsHint h = ihint[gi];
-      const uint64_t k = ukey[gi];
-      const uint64_t v = uval[gi];
-      if (mine) {
-        k_l = k;
-        v_l = v;
-        gs_l = h.gs;
-        np_l = h.np;
-        par_l = h.par;
-        leaf_l = h.leaf;
-        up_l = h.pos;
-      }
-    } else if (mine) {
-      k_l = ukey[gi];
-      v_l = uval[gi];
-      gs_l = gstart[gi];
-      np_l = npend[gi];
-    }
-    if (ihint) {
-      // Every lane at once: its own leaf transaction on the hinted leaf, for an op that needs no
-      // split (leaf entries are unordered, so a new key is one append and a found key one value
-      // store).  Test-and-set of the leaf's lock word; under the lock the leaf must still be a
-      // leaf holding the key in its fences (a split by a transaction of this launch moves keys
-      // out), a found key must still sit at its hinted slot (a split rewrites the slots in key
-      // order) and a new key needs a free slot.  The same lock word serializes these with the
-      // wave-wide transactions below, which take every op that fails here.
-      bool held = false, ok = false, fnd = false;
-      uint64_t w = 0, info = 0, low = 0, high = 0, kat = 0, old = 0;
-      const uint32_t pos = up_l & UPOS_SLOT;
-      const bool hfound = (up_l & UPOS_FOUND) != 0;
-      NodeMeta* m = t.meta + (leaf_l < t.capacity ? leaf_l : 0u);
-      const size_t nb = (size_t)(leaf_l < t.capacity ? leaf_l : 0u) * F;
-      if (mine && leaf_l < t.capacity && (!hfound || pos < (uint32_t)F)) {
-        w = __hip_atomic_fetch_or(&m->lock, 1ull, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-        held = !(w & 1ull);
-      }
-      wave_order();  // the leaf's content is read only after its lock is held
-      if (held) {
-        info = ld_relaxed(&m->info);
-        low = ld_relaxed(&m->low);
-        high = ld_relaxed(&m->high);
-        if (hfound) {
-          kat = ld_relaxed(t.keys + nb + pos);
-          old = ld_relaxed(t.vals + nb + pos);
-        }
-      }
-      const uint32_t count = meta_count(info);
-      if (held && meta_level(info) == 0 && count <= (uint32_t)F && k_l >= low && k_l < high) {
-        if (hfound) {
-          ok = kat == k_l;
-          fnd = ok;
-          if (ok) st_relaxed(t.vals + nb + pos, v_l);
-        } else if (count < (uint32_t)F) {
-          ok = true;
-          st_relaxed(t.keys + nb + count, k_l);
-          st_relaxed(t.vals + nb + count, v_l);
-          st_relaxed(&m->info, make_info(count + 1, 0));
-        }
-      }
-      wave_order();  // the content stores are acknowledged before the lock word changes
-      if (held) st_relaxed(&m->lock, ok ? w + 2 : w);
-      const uint64_t adone = ballot(ok);
-      write_upsert_answers(ok, fnd, fnd ? old : 0ull, gs_l, np_l, sidx, out_vals, out_found);
-      c.commits += (uint32_t)__popcll(adone);
-      c.new_keys += (uint32_t)__popcll(ballot(ok && !fnd));
-      c.node_reads += (uint32_t)__popcll(ballot(held));
-      upserts += (uint32_t)__popcll(adone);
-      todo &= ~adone;
-    }
+    const InsHint h = ihint[gi];
+    const uint64_t k_l = ukey[gi];
+    const uint64_t v_l = uval[gi];
+    const uint32_t gs_l = h.gs, np_l = h.np, par_l = h.par, leaf_l = h.leaf;
+    const uint32_t p0_l = pos_of(sidx[gs_l]);
     // Ops of the round whose keys share a leaf commit together (tx_merge_attempt): a hot
     // leaf takes one transaction per round instead of one per op.
     while (todo) {
@@ -1845,13 +2350,14 @@ __global__ __launch_bounds__(256) void k_upsert(TreeView t, const uint64_t* __re
         todo &= ~(1ull << l);
         continue;
       }
-      write_upsert_answers(((done >> lane_id()) & 1ull) != 0, found_l, old_l, gs_l, np_l, sidx,
+      write_upsert_answers(((done >> lane_id()) & 1ull) != 0, found_l, old_l, gs_l, np_l, p0_l, sidx,
                            out_vals, out_found);
       upserts += (uint32_t)__popcll(done);
       todo &= ~done;
     }
   }
-  }  // ranges
+  }  // pieces
+  }  // wavefronts of k_upsert_runs
   flush_counters(t, c, cnt);
   if (lane_id() == 0) {
     stat_add(t.stats, ST_UPSERTS, wave_stripe(), upserts);
@@ -1859,7 +2365,8 @@ __global__ __launch_bounds__(256) void k_upsert(TreeView t, const uint64_t* __re
   }
 }
 
-// Serial pass over the ops that exhausted their attempts: one wavefront, no competitors,
+// Serial pass over the ops that exhausted their attempts or that the all but full pool refused as
+// a run: one wavefront, no competitors,
 // so every transaction commits on its first attempt.
 template <int F>
 __global__ __launch_bounds__(64) void k_upsert_serial(TreeView t, const uint64_t* __restrict__ ukey,
@@ -1880,7 +2387,11 @@ __global__ __launch_bounds__(64) void k_upsert_serial(TreeView t, const uint64_t
   }
   TxCounters c;
   ParentCache<F> pc;
-  for (uint32_t e = 0; e < n; ++e) {
+  // Once the pool is full the batch fails; the rest then gets a bounded number of tries (an op that
+  // needs no node still succeeds), so that a long list cannot hold the device for seconds.
+  uint32_t tries = 4096;
+  for (uint32_t e = 0; e < n && tries; ++e) {
+    if (uniform64(ld_relaxed(&t.hdr->error)) & ERR_POOL_FULL) --tries;
     const uint32_t g = dlist[e];
     if (!run_upsert<F>(t, ukey[g], uval[g], gstart[g], npend[g], sidx, out_vals, out_found, 1024u,
                        c, pc)) {
@@ -2094,7 +2605,7 @@ static hipError_t launch_lookup_k(const TreeView& t, const LookupArgs& a, hipStr
       t, a.ukey, a.uop, a.gstart, a.npend, a.sidx, a.counters, a.chunk, fill, a.out_vals,
       a.out_found, LEARNED ? a.route_hdr : nullptr, LEARNED ? a.fences : nullptr,
       LEARNED ? a.lids : nullptr, LEARNED ? a.segs : nullptr, a.desc, a.ihint, a.gval, a.fanout,
-      a.fanout_cap);
+      a.fanout_cap, a.split);
   return hipGetLastError();
 }
 
@@ -2120,54 +2631,53 @@ hipError_t launch_lookup(const TreeView& t, const LookupArgs& a, hipStream_t s) 
   STM_DISPATCH_F(t.fanout, launch_lookup_f<F>(t, a, s));
 }
 
-template <int F, int G>
-static hipError_t launch_upsert_fast(const TreeView& t, const UpsertArgs& a, hipStream_t s,
-                                     uint32_t& waves) {
-  // Each wavefront takes an equal contiguous share of the merged INSERTs and works through it
-  // in rounds of WAVE / G: a grid of exactly the wavefronts the chip holds at once finishes
-  // in one generation of rounds instead of two.
+template <int F>
+static hipError_t launch_upsert_f(const TreeView& t, const UpsertArgs& a, hipStream_t s) {
+  // Each wavefront takes an equal contiguous share of the merged INSERTs, at least 64 of them: a
+  // grid of at most the wavefronts the chip holds at once works through them in one generation.
   static std::atomic<int> resident{0};  // blocks of this instantiation the device holds at once
   if (resident.load(std::memory_order_relaxed) == 0) {
     int dev = 0, cus = 0, per_cu = 0;
     hipError_t e = hipGetDevice(&dev);
     if (e == hipSuccess) e = hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     if (e == hipSuccess)
-      e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_upsert_fast<F, G>, 256, 0);
+      e = hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_upsert_runs<F>, 256, 0);
     if (e != hipSuccess) return e;
     resident.store(std::max(1, cus * per_cu), std::memory_order_relaxed);
   }
   const uint32_t blocks = std::min<uint32_t>(
-      std::min<uint32_t>(a.blocks, (uint32_t)resident.load(std::memory_order_relaxed)),
-      FAST_WAVES_MAX / 4);
-  waves = blocks * 4;  // one scount entry per wavefront
-  k_upsert_fast<F, G><<<blocks, 256, 0, s>>>(t, a.ukey, a.uval, a.uop, a.gstart, a.npend, a.sidx,
-                                                a.ilist, a.ihint, a.counters, a.slist,
-                                                a.scount, a.out_vals, a.out_found, a.desc,
-                                                a.fanout, a.fanout_cap, a.gval);
-  return hipGetLastError();
-}
-
-template <int F>
-static hipError_t launch_upsert_f(const TreeView& t, const UpsertArgs& a, hipStream_t s) {
-  hipError_t e = hipSuccess;
-  const bool fast = a.ihint && a.ilist && a.slist && a.scount;
-  uint32_t fast_waves = 0;
-  if (fast) {
-    switch (a.lanes) {
-      case 8: e = launch_upsert_fast<F, (F >= 8 ? 8 : F)>(t, a, s, fast_waves); break;
-      case 16: e = launch_upsert_fast<F, (F >= 16 ? 16 : F)>(t, a, s, fast_waves); break;
-      case 32: e = launch_upsert_fast<F, (F >= 32 ? 32 : F)>(t, a, s, fast_waves); break;
-      default: return hipErrorInvalidValue;
-    }
-    if (e != hipSuccess) return e;
-  }
-  k_upsert<F><<<a.blocks, 256, 0, s>>>(t, a.ukey, a.uval, a.uop, a.gstart, a.npend, a.sidx,
-                                        fast ? a.slist : nullptr, a.scount, fast_waves,
-                                        fast ? a.ihint : nullptr, a.counters, a.dlist,
-                                        a.max_attempts, a.out_vals,
-                                        a.out_found, a.desc);
-  e = hipGetLastError();
+      std::min<uint32_t>((uint32_t)((a.n_max + 255) / 256), (uint32_t)resident.load(std::memory_order_relaxed)),
+      RUN_WAVES_MAX / 4);
+  const uint32_t waves = blocks * 4;  // one rfirst / rcount entry per wavefront
+  k_upsert_runs<F><<<blocks, 256, 0, s>>>(t, a.ukey, a.uval, a.gstart, a.npend, a.sidx, a.ilist,
+                                          a.ihint, a.counters, a.piece, a.split, a.plist, a.rlist,
+                                          a.rlen, a.rfirst,
+                                          a.rcount, a.dlist, a.out_vals, a.out_found, a.desc, a.fanout,
+                                          a.fanout_cap, a.gval);
+  hipError_t e = hipGetLastError();
   if (e != hipSuccess) return e;
+  if (a.piece >= (uint32_t)WAVE) {
+    const uint32_t lb = std::min<uint32_t>((uint32_t)(a.n_max / WAVE), LONG_BLOCKS);
+    if (lb > 0) {  // no run of more than 64 ops in fewer
+      k_upsert_long<F><<<lb, 1024, 0, s>>>(t, a.ukey, a.uval, a.sidx, a.ilist, a.ihint, a.counters,
+                                           a.split, a.plist, a.rlist, a.rlen, a.dlist, a.out_vals,
+                                           a.out_found, a.desc);
+      if ((e = hipGetLastError()) != hipSuccess) return e;
+    }
+  }
+  const bool few = a.n_max <= FEW_INSERTS;
+  if (!few) {
+    k_upsert_parents<F><<<PARENT_BLOCKS, 256, 0, s>>>(t, a.split, a.plist, a.plist2);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
+  k_upsert_upper<F><<<1, 1024, 0, s>>>(t, a.split, a.plist, a.plist2, few ? 1u : 2u);
+  if ((e = hipGetLastError()) != hipSuccess) return e;
+  if (a.piece < (uint32_t)WAVE) {
+    k_upsert<F><<<a.blocks, 256, 0, s>>>(t, a.ukey, a.uval, a.sidx, a.ilist, a.rlist, a.rlen,
+                                          a.rfirst, a.rcount, waves, a.ihint, a.counters, a.dlist,
+                                          a.max_attempts, a.out_vals, a.out_found, a.desc);
+    if ((e = hipGetLastError()) != hipSuccess) return e;
+  }
   k_upsert_serial<F><<<1, 64, 0, s>>>(t, a.ukey, a.uval, a.gstart, a.npend, a.sidx, a.dlist,
                                       a.counters, a.out_vals, a.out_found, a.desc,
                                       a.host_counters);

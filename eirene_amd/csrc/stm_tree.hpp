@@ -6,9 +6,8 @@
 
 namespace stm {
 
-// Wavefronts of the upsert fast path at most (2048 workgroups of 4); each records how many ops
-// it handed back.
-constexpr uint32_t FAST_WAVES_MAX = 8192;
+// Wavefronts of k_upsert_runs at most (2048 workgroups of 4); each records the runs it leaves.
+constexpr uint32_t RUN_WAVES_MAX = 8192;
 
 // Answers of a GET group with more than FANOUT_DIRECT waiting ops (a hot key) are not written
 // by the one lane that looked the key up: the lookup kernel queues the group's answer range in
@@ -20,7 +19,7 @@ inline uint64_t fanout_capacity(uint64_t n) { return n / FANOUT_CHUNK + n / FANO
 
 // Slot hint of a merged INSERT (written by the lookup kernel): bits 0..7 hold the key's slot
 // in the hinted leaf when the key is there (UPOS_FOUND set); bits 16..23 the leaf's entry
-// count.  Valid while the leaf keeps the version the lookup kernel read.
+// count.  Valid until an upsert kernel writes the leaf.
 constexpr uint32_t UPOS_SLOT = 0xffu;
 constexpr uint32_t UPOS_FOUND = 0x100u;
 constexpr uint32_t UPOS_COUNT_SHIFT = 16;
@@ -30,15 +29,28 @@ constexpr uint32_t UPOS_COUNT_SHIFT = 16;
 // inserts are a sparse subset of the groups, so each array they gathered from instead cost a
 // line per insert.
 struct alignas(32) InsHint {
-  uint64_t ver;   // the hinted leaf's lock word when the lookup kernel ran
   uint32_t leaf;  // the leaf whose fences hold the key
   uint32_t pos;   // slot hint (UPOS_*)
   uint32_t par;   // level-1 node that routed it (NODE_NONE if none)
   uint32_t gs;    // sorted position of the group's first op
   uint32_t np;    // ops of the group waiting for the tree's answer
-  uint32_t pad;
+  uint32_t pad[3];
 };
 static_assert(sizeof(InsHint) == 32, "two 16-byte words");
+
+// Leaves split without a lock in this batch (k_upsert_runs) and the parents they concern.  Reset
+// by the lookup kernel.
+struct SplitState {
+  uint32_t made;     // new leaves asked for, ids from TreeHeader::n_nodes on
+  uint32_t refused;  // the first request the pool could not hold begins here (NODE_NONE: none)
+  uint32_t n_dirty;  // level-1 nodes on the list
+  uint32_t inner;    // new inner nodes, ids after the accepted leaves
+  uint32_t n_dirty2; // level-2 nodes on theirs
+  uint32_t root;     // 1 + the root, when it was split and needs a parent; 0: it was not
+  uint32_t n_long;   // runs left to k_upsert_long
+  uint32_t pad[9];
+};
+static_assert(sizeof(SplitState) == 64, "one 64-byte block");
 
 struct LookupArgs {
   const uint64_t* ukey;
@@ -63,12 +75,12 @@ struct LookupArgs {
   uint64_t* gval;         // a hot GET group's value (per group; GET groups leave uval unused)
   uint64_t* fanout;       // queued answer chunks: group | first op << 32 | found << 63
   uint64_t fanout_cap;    // fanout_capacity(n_max)
+  SplitState* split;      // reset here for the upsert kernels
 };
 
 struct UpsertArgs {
   const uint64_t* ukey;
   const uint64_t* uval;
-  const uint8_t* uop;
   const uint32_t* gstart;
   const uint32_t* npend;
   const uint32_t* sidx;
@@ -79,13 +91,17 @@ struct UpsertArgs {
   uint64_t* out_vals;
   uint8_t* out_found;
   const BatchDesc* desc;
-  const InsHint* ihint;   // the lookup kernel's records of the merged INSERTs; with slist: the
-                          //   fast path runs
-  const uint32_t* ilist;  // the merged INSERT groups (counters->n_upserts)
-  uint32_t* slist;        // ops the fast path hands back (capacity: groups), in the handing
-                          //   wavefront's own range of the insert list
-  uint32_t* scount;       // per fast-path wavefront: ops it handed back (capacity: FAST_WAVES_MAX)
-  uint32_t lanes;         // lanes per op of the fast path: 8, 16 or 32
+  const InsHint* ihint;   // the lookup kernel's records of the merged INSERTs
+  const uint32_t* ilist;  // the merged INSERT groups in key order (counters->n_upserts)
+  uint64_t n_max;         // upper bound of their number (grid sizing)
+  uint32_t piece;         // runs the transactions take are cut into pieces of at most this many ops
+  SplitState* split;
+  uint32_t* plist;        // level-1 nodes with new children (capacity: groups)
+  uint32_t* plist2;       // their level's parents (capacity: groups)
+  uint32_t* rlist;        // per piece: its first list entry (capacity: groups)
+  uint32_t* rlen;         //   and its ops
+  uint32_t* rfirst;       // per wavefront of k_upsert_runs: its first piece's index
+  uint32_t* rcount;       //   and their number (capacity: RUN_WAVES_MAX)
   const uint64_t* fanout; // hot GET groups' answer chunks queued by the lookup kernel (the fast
   uint64_t fanout_cap;    //   path writes them first); null: none queued
   const uint64_t* gval;   // their values (per group)

@@ -63,8 +63,10 @@ typedef struct stm_config {
     int32_t device;       /* HIP device ordinal (default 0) */
     uint32_t lanes_per_op;/* lookup kernel lanes per op: 8, 16, 32 or 64 (default 16) */
     uint32_t ops_per_group;/* sorted ops walked by one lane group (default 16) */
-    uint32_t upsert_ops_per_wave; /* batch ops per upsert wavefront: the upsert grid is
-                                     max_batch / this many wavefronts, at most 8192 (default 512) */
+    uint32_t upsert_ops_per_wave; /* batch ops per upsert wavefront (default 512).  From 64 on the
+                                     inserts of a leaf run together without locks; below, a leaf's
+                                     inserts beyond this many run as transactions that contend for
+                                     it, on a grid of max_batch / this many wavefronts, at most 8192 */
     uint32_t max_attempts;/* STM attempts before an op is deferred to the serial pass (default 64) */
     uint32_t route;       /* STM_ROUTE_* */
     uint32_t timing;      /* 1 = record HIP events around every phase (stm_get_stats) */
@@ -74,10 +76,8 @@ typedef struct stm_config {
                                  keys; default 16) */
     uint32_t use_graphs;  /* stm_run_batches_device: 1 = replay one captured hipGraph per batch
                              size class (default 1), 0 = launch every kernel from the host */
-    uint32_t upsert_lanes;/* lanes per insert on the upsert kernel's lane-group fast path:
-                             8, 16 or 32, at most fanout (64 / this many inserts per
-                             wavefront at once); 0 = automatic (default): 8 up to fanout 64,
-                             16 above */
+    uint32_t upsert_lanes;/* 8, 16 or 32, at most fanout; 0 = automatic (default).  Checked, but
+                             without effect: the upsert kernel gives every insert one lane */
     uint32_t retrain_splits; /* learned routing / static index: also rebuild the directory (and
                                 retrain) before a batch once this many leaves have split since
                                 the last retrain; 0 = automatic (default): a 32nd of the leaves
@@ -105,8 +105,9 @@ typedef struct stm_stats {
     uint64_t ops;             /* ops submitted */
     uint64_t unique_ops;      /* ops after the per-key fold */
     uint64_t upserts;         /* merged INSERT ops executed as transactions */
-    uint64_t commits;         /* committed transactions (upserts + preemptive splits) */
-    uint64_t aborts;          /* aborted transaction attempts */
+    uint64_t commits;         /* committed transactions (a leaf's inserts, or part of them, and splits) */
+    uint64_t aborts;          /* attempts given up and made again: a leaf's inserts that do not fit it
+                                 as it is, a transaction that met a lock or a changed node */
     uint64_t leaf_splits;
     uint64_t inner_splits;
     uint64_t root_splits;

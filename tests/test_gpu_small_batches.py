@@ -97,3 +97,77 @@ def test_misleading_sample_sorts_again(oracle_mod, stream):
         st = t.stats()
         assert st["sort_fallbacks"] == 1 and st["batches"] == 4 and st["ops"] == 4 * n
         assert t.check() == 0
+
+
+def grow(oracle_mod, batches, load, **kw):
+    """Runs (keys, ops) batches on a tree and the oracle; answers, dump and invariants must agree."""
+    from eirene_amd import StmConfig, StmTree
+    rng = np.random.default_rng(3)
+    o = oracle_mod.Oracle()
+    o.bulk_load(load, load)
+    with StmTree(StmConfig(**{**dict(max_keys=1 << 21, max_batch=1 << 19), **kw})) as t:
+        if load.size:
+            t.bulk_load(load, load)
+        for b, (keys, ops) in enumerate(batches):
+            vals = rng.integers(0, 1 << 63, keys.size, dtype=np.uint64)
+            got, want = t.run_batch(keys, vals, ops), o.run_batch(keys, vals, ops)
+            assert np.array_equal(got[1], want[1]) and np.array_equal(got[0], want[0]), b
+            assert t.check() == 0
+        k, v = t.dump()
+        ek, ev = o.dump()
+        assert np.array_equal(k, ek) and np.array_equal(v, ev)
+        return t.stats()
+
+
+@pytest.mark.parametrize("fanout", [32, 64, 128])
+@pytest.mark.parametrize("run", [1, 2, 16, 17, 63, 64, 65, 100, 1024, 1025, 5000])
+def test_runs_of_one_leaf(oracle_mod, fanout, run):
+    """Runs of `run` inserts into single leaves, new keys and present ones, beside leaves without
+    any: leaves that fill exactly, overfill by one, split into two and into hundreds, under
+    parents that overfill in turn."""
+    rng = np.random.default_rng(run * 7 + fanout)
+    load = np.arange(1, 6001, dtype=np.uint64) << np.uint64(40)
+    batches = []
+    for b in range(3):
+        at = rng.choice(5990, 40 if run < 1000 else 6, replace=False)
+        new = (load[at][:, None] + rng.integers(1, 1 << 39, (at.size, run), dtype=np.uint64)).ravel()
+        old = np.concatenate([load[a: a + 3] for a in at])
+        keys = np.concatenate([new, old, rng.choice(load, 500)])
+        ops = np.concatenate([np.zeros(new.size + old.size, np.uint8), np.ones(500, np.uint8)])
+        order = rng.permutation(keys.size)
+        batches.append((keys[order], ops[order]))
+    st = grow(oracle_mod, batches, load, fanout=fanout)
+    assert st["deferred"] == 0
+
+
+@pytest.mark.parametrize("fanout", [32, 64, 128])
+@pytest.mark.parametrize("n", [1, 32, 33, 64, 65, 129, 3000, 200000])
+def test_inserts_into_an_empty_tree(oracle_mod, fanout, n):
+    """Every insert goes into the one leaf: the root splits, for the larger batches into more nodes
+    than one new root holds."""
+    rng = np.random.default_rng(n + fanout)
+    batches = [(rng.integers(0, 1 << 63, m, dtype=np.uint64), np.zeros(m, np.uint8))
+               for m in (n, max(1, n // 3))]
+    st = grow(oracle_mod, batches, np.zeros(0, np.uint64), fanout=fanout)
+    assert st["height"] > 1 or n <= fanout
+
+
+def test_pool_runs_full(oracle_mod):
+    """Batches past what the pool holds: the call reports it, and the tree stays well formed and
+    keeps every key it had."""
+    from eirene_amd import StmConfig, StmError, StmTree
+    rng = np.random.default_rng(9)
+    with StmTree(StmConfig(max_keys=2000, max_batch=1 << 16)) as t:
+        kept = None
+        for _ in range(40):
+            keys = rng.integers(0, 1 << 63, 4000, dtype=np.uint64)
+            try:
+                t.run_batch(keys, keys, np.zeros(keys.size, np.uint8))
+            except StmError as e:
+                assert e.code == 2
+                break
+            kept = t.dump()[0]
+        else:
+            pytest.fail("the pool never ran full")
+        assert t.check() == 0
+        assert np.isin(kept, t.dump()[0]).all()
