@@ -375,7 +375,7 @@ class StmTree:
             out_found.ptr))
 
     def capture_graphs(self) -> None:
-        """Captures every batch size class's graph now (otherwise done on first use)."""
+        """Prepares batch streams now: graphs of the small size classes, the second scratch set."""
         _check(self._lib.stm_capture_graphs(self._h))
 
     def sync(self) -> None:

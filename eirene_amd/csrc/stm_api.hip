@@ -54,69 +54,34 @@ hipError_t dalloc(T** p, size_t count) {
   return hipMalloc((void**)p, count * sizeof(T));
 }
 
-// Totals of a batch stream, accumulated on the device so replays need no host round trip.
-struct StreamAcc {
-  unsigned long long unique;   // groups after the per-key fold
-  unsigned long long bad;      // ops rejected for the reserved key
-  unsigned long long batches;  // batches that ran
-  unsigned long long skipped;  // batches skipped after an error
-  unsigned long long sort_stalls;  // batches whose sort gave up a grid-barrier wait
-  unsigned long long fallbacks;    // batches whose normalized sort fell back to the exact passes
-  unsigned long long leaf_splits;  // leaves the batches split
-  unsigned long long retries;      // a batch whose small-batch sort overflowed a bucket
-};
-
 constexpr uint32_t DESC_TABLE = 4096;  // descriptors uploaded per window of a stream
 constexpr int GRAPH_CLASSES = 12;      // size classes 2^10, 2^12, ..., up to max_batch
+constexpr uint32_t GRAPH_MAX_OPS = 1u << 12;  // classes that are captured
+constexpr uint32_t OVERLAP_MIN_OPS = 2049;    // batches whose front half may run on its own stream
+constexpr uint64_t OVERLAP_BATCHES = 32;      // such batches before that stream is made
 
-// First node of every replayed graph: takes the next descriptor of the window.  Once a batch
-// has failed (reserved key, full node pool) the later batches of the stream run empty, so the
-// tree holds exactly the batches up to the failing one.
+// Waits, for at most a tenth of a millisecond, until k_probe_set has run; says whether it saw it.
+__global__ void k_probe_wait(uint32_t* flag, uint32_t* seen) {
+  if (threadIdx.x != 0) return;
+  const uint64_t until = wall_clock64() + 10000;  // 100 MHz
+  while (!__hip_atomic_load(flag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT)) {
+    if (wall_clock64() > until) return;
+    __builtin_amdgcn_s_sleep(4);
+  }
+  *seen = 1;
+}
+__global__ void k_probe_set(uint32_t* flag) {
+  if (threadIdx.x == 0)
+    __hip_atomic_store(flag, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// First node of every replayed graph: takes the next descriptor of the window.
 __global__ void k_advance(const BatchDesc* __restrict__ table, uint32_t* __restrict__ cursor,
-                          BatchDesc* __restrict__ live, const StreamAcc* __restrict__ acc,
-                          const TreeHeader* __restrict__ hdr) {
+                          BatchDesc* __restrict__ live) {
   if (threadIdx.x != 0) return;
   const uint32_t c = cursor[0];
-  BatchDesc d = table[c];
-  if (acc->bad || acc->sort_stalls || acc->retries || hdr->error) d.n = 0;
-  *live = d;
+  *live = table[c];
   cursor[0] = c + 1;
-}
-
-// Last node of every replayed graph.
-__global__ void k_epilogue(const BatchCounters* __restrict__ cnt, const BatchDesc* __restrict__ live,
-                           StreamAcc* __restrict__ acc) {
-  if (threadIdx.x != 0) return;
-  if (live->n == 0) {
-    acc->skipped += 1;
-    return;
-  }
-  if (cnt->sort_retry) {  // ran empty: the host runs it again and resumes the stream after it
-    acc->retries += 1;
-    return;
-  }
-  acc->unique += cnt->n_unique;
-  acc->bad += cnt->n_bad;
-  acc->sort_stalls += cnt->sort_stall;
-  acc->fallbacks += cnt->sort_fallback;
-  acc->leaf_splits += cnt->leaf_splits;
-  acc->batches += 1;
-}
-
-// First node of a back half: the front half of this batch may have run beside the back half of
-// a batch that failed, so the failure is checked again here, after every earlier back half
-// (same stream).  A batch after a failure keeps no groups: its lookups and upserts do nothing.
-__global__ void k_gate(const StreamAcc* __restrict__ acc, const TreeHeader* __restrict__ hdr,
-                       BatchDesc* __restrict__ live, BatchCounters* __restrict__ cnt) {
-  if (threadIdx.x != 0) return;
-  if (live->n == 0) return;
-  if (acc->bad || acc->sort_stalls || acc->retries || hdr->error) {
-    live->n = 0;
-    cnt->n_unique = 0;
-    cnt->n_upserts = 0;
-    cnt->n_fanout = 0;
-    cnt->n_deferred = 0;
-  }
 }
 
 // Plain streaming copy of n16 16-byte words: the known-size reference kernel for HBM traffic
@@ -264,29 +229,25 @@ struct stm_tree {
   uint32_t batches_since_train = 0;
   uint64_t splits_since_train = 0;  // leaf splits counted since the last directory rebuild
   uint64_t dir_leaves = 0;          // leaves of the directory at the last rebuild
-  // Batch streams (stm_run_batches_device) run each batch as two captured halves on two
-  // scratch sets, so the front half (descriptor, sort, fold) of batch i + 1 runs on
-  // stream_front while the back half (lookups, upserts, counters) of batch i runs on `stream`.
-  // One graph per half, size class and scratch set (null until first needed).
+  // Batch streams (stm_run_batches_device) run each batch as two halves, on two scratch sets, so
+  // that the front half (sort, fold) of batch i + 1 runs on stream_front while the back half
+  // (lookups, upserts, counters) of batch i runs on `stream`.  Captured graphs, one per small size
+  // class, hold both halves for `stream`.
   Scratch scr2;
   bool scr2_alloc = false;
   hipStream_t stream_front = nullptr;
-  hipEvent_t ev_front[2] = {};  // front half of the slot's latest batch done
-  hipEvent_t ev_back[2] = {};   // back half of the slot's latest batch done (its scratch is free)
-  hipEvent_t ev_sync = nullptr;
-  hipGraphExec_t graphs_front[GRAPH_CLASSES][2] = {};
-  hipGraphExec_t graphs_back[GRAPH_CLASSES][2] = {};
+  hipEvent_t ev_front[2] = {};  // front half of the set's latest batch done
+  hipEvent_t ev_back[2] = {};   // the set's latest batch done (its scratch is free)
+  uint64_t overlap_batches = 0;  // batches seen that could have overlapped
+  hipGraphExec_t graphs[GRAPH_CLASSES] = {};
   // Batches above 2^18 ops sort normalized keys unless exact_left > 0: a batch whose normalized
   // sort had to fall back (long buckets of distinct keys: hot keys with neighbours) makes the
-  // next EXACT_HOLD batches use the eight exact passes directly.  graphs_exact: the form the
-  // captured graphs hold.
-  // A smaller batch is sorted by the front half's own sort unless front_hold > 0: one that
-  // overflowed a bucket there makes the next EXACT_HOLD of them use the exact passes too
-  // (graphs_front_exact: the form the captured graphs of those sizes hold).
+  // next EXACT_HOLD batches use the eight exact passes directly.  A smaller batch is sorted by the
+  // front half's own sort unless front_hold > 0: one that overflowed a bucket there makes the next
+  // EXACT_HOLD of them use the exact passes too (launched, not replayed: the captured graphs hold
+  // the front half's sort).
   uint32_t exact_left = 0;
-  bool graphs_exact = false;
   uint32_t front_hold = 0;
-  bool graphs_front_exact = false;
   uint64_t sort_fallbacks = 0;  // batches sorted again with the exact passes (stm_stats)
 };
 
@@ -398,14 +359,10 @@ int init_empty(stm_tree* t) {
 }
 
 void drop_graphs(stm_tree* t) {
-  for (int c = 0; c < GRAPH_CLASSES; ++c)
-    for (int k = 0; k < 2; ++k) {
-      hipGraphExec_t* gs[] = {&t->graphs_front[c][k], &t->graphs_back[c][k]};
-      for (hipGraphExec_t* g : gs) {
-        if (*g) (void)hipGraphExecDestroy(*g);
-        *g = nullptr;
-      }
-    }
+  for (hipGraphExec_t& g : t->graphs) {
+    if (g) (void)hipGraphExecDestroy(g);
+    g = nullptr;
+  }
 }
 
 int alloc_router(stm_tree* t) {
@@ -505,6 +462,8 @@ struct PipeIn {
   uint64_t scan_cap;
   // optional: the last upsert kernel copies the batch counters here (pinned host memory)
   BatchCounters* host_counters;
+  // optional: the batch of a stream: runs empty after a failed one, its counters are added here
+  StreamAcc* acc;
 };
 
 // Front half of a batch: sort and fold.  Reads only the batch and writes only the scratch and
@@ -605,6 +564,7 @@ hipError_t enqueue_back(stm_tree* t, Scratch& s, const PipeIn& in, bool timed) {
   la.fanout = s.fanout;
   la.fanout_cap = fanout_capacity(in.n);
   la.split = s.split;
+  la.acc = in.acc;
   if ((e = launch_lookup(t->view, la, st)) != hipSuccess) return e;
 
   if (in.scans) {  // on the tree as it was before the batch: before the upsert kernel
@@ -647,6 +607,7 @@ hipError_t enqueue_back(stm_tree* t, Scratch& s, const PipeIn& in, bool timed) {
   ua.fanout_cap = fanout_capacity(in.n);
   ua.gval = s.uval;
   ua.host_counters = in.host_counters;
+  ua.acc = in.acc;
   if ((e = launch_upsert(t->view, ua, st)) != hipSuccess) return e;
   if (timed) phase_end(t, STM_PHASE_UPSERT);
   if (in.scans && (e = launch_scan_answers(sa, st)) != hipSuccess) return e;
@@ -691,7 +652,7 @@ int run_chunk(stm_tree* t, const uint64_t* keys, const uint64_t* vals, const uin
   hipStream_t st = t->stream;
   int rc = maybe_retrain(t);
   if (rc) return rc;
-  PipeIn in{keys, vals, ops, n, out_vals, out_found, nullptr, false, nullptr, nullptr, 0, nullptr};
+  PipeIn in{keys, vals, ops, n, out_vals, out_found, nullptr, false, nullptr, nullptr, 0, nullptr, nullptr};
   if (so) {
     in.scans = true;
     in.scan_keys = so->keys;
@@ -753,126 +714,164 @@ int class_of(const stm_tree* t, uint32_t n) {
   return GRAPH_CLASSES - 1;  // max_batch <= 2^30 fits class 10
 }
 
+// A stream whose kernels run beside those of `beside`.  Streams share a few hardware queues, and
+// two streams on one queue run one after the other (a stream of 2^16-op batches then took 65 µs per
+// batch instead of 54), so a candidate is tried: does its kernel reach a kernel that waits on
+// `beside`?  The rejected ones are kept until the choice is made, so that each candidate gets another
+// queue.
+hipError_t stream_beside(hipStream_t beside, uint32_t* words /*2, device*/, hipStream_t* out) {
+  constexpr int TRIES = 4;
+  hipStream_t tried[TRIES] = {};
+  hipError_t e = hipSuccess;
+  int n = 0;
+  uint32_t seen = 0;
+  while (n < TRIES && !seen && e == hipSuccess) {
+    if ((e = hipStreamCreate(&tried[n])) != hipSuccess) break;
+    hipStream_t c = tried[n++];
+    if ((e = hipMemsetAsync(words, 0, 8, beside)) != hipSuccess ||
+        (e = hipStreamSynchronize(beside)) != hipSuccess)
+      break;
+    k_probe_wait<<<1, 64, 0, beside>>>(words, words + 1);
+    k_probe_set<<<1, 64, 0, c>>>(words);
+    if ((e = hipGetLastError()) != hipSuccess || (e = hipStreamSynchronize(c)) != hipSuccess) break;
+    e = hipMemcpyAsync(&seen, words + 1, 4, hipMemcpyDeviceToHost, beside);
+    if (e == hipSuccess) e = hipStreamSynchronize(beside);
+  }
+  const int keep = e == hipSuccess ? n - 1 : -1;
+  for (int i = 0; i < n; ++i)
+    if (i != keep && tried[i]) (void)hipStreamDestroy(tried[i]);
+  if (keep >= 0) *out = tried[keep];
+  return e;
+}
+
 // The second scratch set, the front stream and the pipeline's events, made on first use.
 int ensure_pipeline(stm_tree* t) {
   if (t->scr2_alloc) return STM_OK;
   hipError_t e = t->scr2.alloc(t->cfg.max_batch, Scratch::STREAM);
-  if (e == hipSuccess) e = hipStreamCreate(&t->stream_front);
+  if (e == hipSuccess && !t->stream_front)
+    e = stream_beside(t->stream, reinterpret_cast<uint32_t*>(t->scr2.counters), &t->stream_front);
   for (int k = 0; k < 2 && e == hipSuccess; ++k) {
-    e = hipEventCreateWithFlags(&t->ev_front[k], hipEventDisableTiming);
-    if (e == hipSuccess) e = hipEventCreateWithFlags(&t->ev_back[k], hipEventDisableTiming);
+    if (!t->ev_front[k]) e = hipEventCreateWithFlags(&t->ev_front[k], hipEventDisableTiming);
+    if (e == hipSuccess && !t->ev_back[k])
+      e = hipEventCreateWithFlags(&t->ev_back[k], hipEventDisableTiming);
   }
-  if (e == hipSuccess) e = hipEventCreateWithFlags(&t->ev_sync, hipEventDisableTiming);
-  if (e != hipSuccess) return fail(STM_ERR_NOMEM, "stream pipeline set-up: %s", hipGetErrorString(e));
+  if (e != hipSuccess) {
+    t->scr2.release();
+    return fail(STM_ERR_NOMEM, "stream pipeline set-up: %s", hipGetErrorString(e));
+  }
   t->scr2_alloc = true;
   return STM_OK;
 }
 
 Scratch& slot_scratch(stm_tree* t, int k) { return k ? t->scr2 : t->scr; }
 
-// Captures the two halves of size class c on scratch set k:
-//   front: advance (next descriptor of the window into the set's live descriptor) -> sort -> fold
-//   back:  gate -> lookups -> upserts -> epilogue (counters into the stream's accumulator)
-// The descriptor window, its cursor and the accumulator are the first set's.
-int capture_pair(stm_tree* t, int c, int k) {
-  if (t->graphs_front[c][k] && t->graphs_back[c][k]) return STM_OK;
-  Scratch& s0 = t->scr;
-  Scratch& s = slot_scratch(t, k);
+// Captures the launch sequence of size class c (on the first scratch set): advance (next descriptor
+// of the window into the live descriptor), front half, back half.  Only classes up to
+// GRAPH_MAX_OPS, and only when the caller asks (stm_capture_graphs): one call of the host replaces
+// nine launches, but the kernels read their batch through the descriptor, which costs 6 µs of a
+// 31 µs batch of 2^10 ops; above, the two halves on two streams are faster than any single graph
+// (2^16 ops 69 against 87 µs, 2^18 ops 109 against 137).
+int capture_class(stm_tree* t, int c) {
+  if (t->graphs[c]) return STM_OK;
+  Scratch& s = t->scr;
+  hipStream_t st = t->stream;
   PipeIn in{nullptr, nullptr, nullptr, class_nmax(t, c), nullptr, nullptr, s.desc_live,
-            false, nullptr, nullptr, 0, nullptr};
-  for (int half = 0; half < 2; ++half) {
-    hipStream_t st = half ? t->stream : t->stream_front;
-    HIP_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
-    hipError_t e;
-    if (half == 0) {
-      k_advance<<<1, 64, 0, st>>>(s0.desc_table, s0.cursor, s.desc_live, s0.acc, t->view.hdr);
-      e = hipGetLastError();
-      const bool exact = in.n <= FRONT_MAX_OPS ? t->graphs_front_exact : t->graphs_exact;
-      if (e == hipSuccess) e = enqueue_front(t, s, in, false, exact, st);
-    } else {
-      k_gate<<<1, 64, 0, st>>>(s0.acc, t->view.hdr, s.desc_live, s.counters);
-      e = hipGetLastError();
-      if (e == hipSuccess) e = enqueue_back(t, s, in, false);
-      if (e == hipSuccess) {
-        k_epilogue<<<1, 64, 0, st>>>(s.counters, s.desc_live, s0.acc);
-        e = hipGetLastError();
-      }
-    }
-    hipGraph_t g = nullptr;
-    hipError_t e2 = hipStreamEndCapture(st, &g);
-    if (e == hipSuccess) e = e2;
-    hipGraphExec_t& x = half ? t->graphs_back[c][k] : t->graphs_front[c][k];
-    if (e == hipSuccess) e = hipGraphInstantiate(&x, g, nullptr, nullptr, 0);
-    if (g) (void)hipGraphDestroy(g);
-    if (e != hipSuccess) {
-      x = nullptr;
-      return fail(STM_ERR_DEVICE, "graph capture of size class %d: %s", c, hipGetErrorString(e));
-    }
+            false, nullptr, nullptr, 0, nullptr, s.acc};
+  HIP_TRY(hipStreamBeginCapture(st, hipStreamCaptureModeThreadLocal));
+  k_advance<<<1, 64, 0, st>>>(s.desc_table, s.cursor, s.desc_live);
+  hipError_t e = hipGetLastError();
+  if (e == hipSuccess) e = enqueue_front(t, s, in, false, false, st);
+  if (e == hipSuccess) e = enqueue_back(t, s, in, false);
+  hipGraph_t g = nullptr;
+  const hipError_t e2 = hipStreamEndCapture(st, &g);
+  if (e == hipSuccess) e = e2;
+  if (e == hipSuccess) e = hipGraphInstantiate(&t->graphs[c], g, nullptr, nullptr, 0);
+  if (g) (void)hipGraphDestroy(g);
+  if (e != hipSuccess) {
+    t->graphs[c] = nullptr;
+    return fail(STM_ERR_DEVICE, "graph capture of size class %d: %s", c, hipGetErrorString(e));
   }
   return STM_OK;
 }
 
-int capture_class(stm_tree* t, int c) {
-  int rc = ensure_pipeline(t);
-  for (int k = 0; k < 2 && rc == STM_OK; ++k) rc = capture_pair(t, c, k);
-  return rc;
-}
-
-// Replays the graphs of descs[at..]; ran = how many of them ran.  Fewer than all with STM_OK: the
-// next one's small-batch sort overflowed a bucket, and it and the later ones ran empty.
-int replay_stream(stm_tree* t, const std::vector<BatchDesc>& descs, const std::vector<uint8_t>& cls,
-                  size_t at, size_t& ran) {
+// Runs descs[at..] without a host round trip; ran = how many of them ran.  Fewer than all with
+// STM_OK: the next one's small-batch sort overflowed a bucket, and it and the later ones ran empty.
+//
+// A batch runs in one of three ways, in order of size:
+//   * a captured graph, where stm_capture_graphs made one for its class;
+//   * both halves launched on the tree's stream: up to 2048 ops, whose front half is one short
+//     kernel (per batch of 2^10 ops 31 µs, 41 with two streams), and while the tree has seen too few
+//     larger batches to pay for the second scratch set and stream;
+//   * the front half on stream_front once the back half of the scratch set's previous user is done,
+//     the back half on the tree's stream once its front half is done (against one stream: 2^16 ops
+//     69 / 79 µs, 2^18 109 / 129, 2^20 252 / 268, 2^22 657 / 669).
+// Back halves run in batch order on one stream, so each sees the tree after the previous batch; the
+// learned router retrains on that stream between them.
+int run_descs(stm_tree* t, const std::vector<BatchDesc>& descs, const std::vector<uint8_t>& cls,
+              size_t at, size_t& ran) {
   Scratch& s = t->scr;
   hipStream_t st = t->stream;
   ran = 0;
   int rc = maybe_retrain(t);  // learned routing: the router's buffers exist before capture
   if (rc) return rc;
-  if (t->graphs_exact != (t->exact_left > 0) || t->graphs_front_exact != (t->front_hold > 0)) {
-    drop_graphs(t);  // graphs of the other sort form
-    t->graphs_exact = t->exact_left > 0;
-    t->graphs_front_exact = t->front_hold > 0;
-  }
-  for (size_t i = at; i < descs.size(); ++i) {
-    rc = capture_class(t, cls[i]);
-    if (rc) return rc;
-  }
-  // Batch i runs on scratch set i % 2: its front half on stream_front once the back half of
-  // batch i - 2 (the set's previous user) is done, its back half on the tree's stream once its
-  // front half is done.  Back halves run in batch order on one stream, so each sees the tree
-  // after the previous batch; the learned router retrains on that stream between them.
+  const bool exact_large = t->exact_left > 0, exact_small = t->front_hold > 0;
+  auto replayed = [&](size_t i) {
+    return descs[i].n <= GRAPH_MAX_OPS && t->graphs[cls[i]] && !exact_small;
+  };
+  for (size_t i = at; i < descs.size(); ++i) t->overlap_batches += descs[i].n >= OVERLAP_MIN_OPS;
+  const bool overlap = t->overlap_batches >= OVERLAP_BATCHES;
+  if (overlap && (rc = ensure_pipeline(t))) return rc;
   hipStream_t sf = t->stream_front;
-  bool used[2] = {false, false};
+  bool used[2] = {false, false};  // ev_back[k] marks the end of the set's latest batch
   HIP_TRY(hipMemsetAsync(s.acc, 0, sizeof(StreamAcc), st));
+  std::vector<BatchDesc> table;
+  int k = 0;  // the scratch set of the latest batch
   for (size_t w0 = at; w0 < descs.size(); w0 += DESC_TABLE) {
     const size_t w1 = std::min<size_t>(descs.size(), w0 + DESC_TABLE);
-    // The window's table and cursor are replaced once every front half of the previous window
-    // has taken its descriptor.
-    HIP_TRY(hipEventRecord(t->ev_sync, sf));
-    HIP_TRY(hipStreamWaitEvent(st, t->ev_sync, 0));
-    HIP_TRY(hipMemcpyAsync(s.desc_table, descs.data() + w0, (w1 - w0) * sizeof(BatchDesc),
-                           hipMemcpyHostToDevice, st));
-    HIP_TRY(hipMemsetAsync(s.cursor, 0, sizeof(uint32_t), st));
-    HIP_TRY(hipEventRecord(t->ev_sync, st));
-    HIP_TRY(hipStreamWaitEvent(sf, t->ev_sync, 0));
+    table.clear();
+    for (size_t i = w0; i < w1; ++i)
+      if (replayed(i)) table.push_back(descs[i]);
+    if (!table.empty()) {
+      HIP_TRY(hipMemcpyAsync(s.desc_table, table.data(), table.size() * sizeof(BatchDesc),
+                             hipMemcpyHostToDevice, st));
+      HIP_TRY(hipMemsetAsync(s.cursor, 0, sizeof(uint32_t), st));
+    }
     for (size_t i = w0; i < w1; ++i) {
-      const int k = (int)(i & 1);
-      if (used[k]) HIP_TRY(hipStreamWaitEvent(sf, t->ev_back[k], 0));
-      HIP_TRY(hipGraphLaunch(t->graphs_front[cls[i]][k], sf));
-      HIP_TRY(hipEventRecord(t->ev_front[k], sf));
+      const BatchDesc& d = descs[i];
       rc = maybe_retrain(t);
       if (rc) return rc;
-      HIP_TRY(hipStreamWaitEvent(st, t->ev_front[k], 0));
-      HIP_TRY(hipGraphLaunch(t->graphs_back[cls[i]][k], st));
-      HIP_TRY(hipEventRecord(t->ev_back[k], st));
-      used[k] = true;
+      if (replayed(i)) {
+        HIP_TRY(hipGraphLaunch(t->graphs[cls[i]], st));
+        k = 0;
+      } else {
+        const PipeIn in{d.keys, d.vals, d.ops, d.n, d.out_vals, d.out_found, nullptr,
+                        false, nullptr, nullptr, 0, nullptr, s.acc};
+        const bool exact = d.n <= FRONT_MAX_OPS ? exact_small : exact_large;
+        if (!overlap || d.n < OVERLAP_MIN_OPS) {
+          HIP_TRY(enqueue_front(t, s, in, false, exact, st));
+          HIP_TRY(enqueue_back(t, s, in, false));
+          k = 0;
+        } else {
+          k ^= 1;
+          Scratch& sk = slot_scratch(t, k);
+          if (used[k]) HIP_TRY(hipStreamWaitEvent(sf, t->ev_back[k], 0));
+          HIP_TRY(enqueue_front(t, sk, in, false, exact, sf));
+          HIP_TRY(hipEventRecord(t->ev_front[k], sf));
+          HIP_TRY(hipStreamWaitEvent(st, t->ev_front[k], 0));
+          HIP_TRY(enqueue_back(t, sk, in, false));
+        }
+      }
+      // A later batch's front half may take this scratch set on the other stream.
+      if (overlap) {
+        HIP_TRY(hipEventRecord(t->ev_back[k], st));
+        used[k] = true;
+      }
       t->st.batches += 1;
-      t->st.ops += descs[i].n;
+      t->st.ops += d.n;
       t->batches_since_train += 1;
     }
   }
   StreamAcc acc;
-  HIP_TRY(hipEventRecord(t->ev_sync, sf));
-  HIP_TRY(hipStreamWaitEvent(st, t->ev_sync, 0));
   HIP_TRY(hipMemcpyAsync(&acc, s.acc, sizeof(acc), hipMemcpyDeviceToHost, st));
   HIP_TRY(hipStreamSynchronize(st));
   ran = (size_t)acc.batches;
@@ -885,8 +884,8 @@ int replay_stream(stm_tree* t, const std::vector<BatchDesc>& descs, const std::v
   t->sort_fallbacks += acc.fallbacks;
   t->splits_since_train += acc.leaf_splits;
   if (acc.fallbacks) t->exact_left = EXACT_HOLD;
-  else if (t->graphs_exact) t->exact_left -= (uint32_t)std::min<uint64_t>(t->exact_left, acc.batches);
-  if (t->graphs_front_exact) t->front_hold -= (uint32_t)std::min<uint64_t>(t->front_hold, acc.batches);
+  else if (exact_large) t->exact_left -= (uint32_t)std::min<uint64_t>(t->exact_left, acc.batches);
+  if (exact_small) t->front_hold -= (uint32_t)std::min<uint64_t>(t->front_hold, acc.batches);
   if (acc.sort_stalls)
     return fail(STM_ERR_DEVICE, "a batch sort gave up a grid-barrier wait (%llu later batches skipped)",
                 acc.skipped);
@@ -918,7 +917,7 @@ int run_stream(stm_tree* t, const uint64_t* keys, const uint64_t* vals, const ui
   }
   for (size_t at = 0; at < descs.size();) {
     size_t ran = 0;
-    int rc = replay_stream(t, descs, cls, at, ran);
+    int rc = run_descs(t, descs, cls, at, ran);
     if (rc) return rc;
     at += ran;
     if (at >= descs.size()) break;
@@ -1240,7 +1239,6 @@ int stm_destroy(stm_tree* t) {
     if (t->ev_front[k]) (void)hipEventDestroy(t->ev_front[k]);
     if (t->ev_back[k]) (void)hipEventDestroy(t->ev_back[k]);
   }
-  if (t->ev_sync) (void)hipEventDestroy(t->ev_sync);
   if (t->stream_front) (void)hipStreamDestroy(t->stream_front);
   if (t->pool) (void)hipFree(t->pool);
   for (int p = 0; p < STM_NUM_PHASES; ++p) {
@@ -1498,16 +1496,12 @@ int stm_capture_graphs(stm_tree* t) {
   if (rc) return rc;
   rc = maybe_retrain(t);  // learned routing: the router's buffers exist before capture
   if (rc) return rc;
-  if (t->graphs_exact != (t->exact_left > 0)) {
-    drop_graphs(t);
-    t->graphs_exact = t->exact_left > 0;
-  }
-  const int last = class_of(t, (uint32_t)t->cfg.max_batch);
-  for (int c = 0; c <= last; ++c) {
+  for (int c = 0; c < GRAPH_CLASSES && class_nmax(t, c) <= GRAPH_MAX_OPS; ++c) {
     rc = capture_class(t, c);
     if (rc) return rc;
+    if (class_nmax(t, c) == t->cfg.max_batch) break;
   }
-  return STM_OK;
+  return ensure_pipeline(t);
 }
 
 int stm_run_batch(stm_tree* t, const uint64_t* keys, const uint64_t* vals, const uint8_t* ops,

@@ -81,9 +81,26 @@ struct BatchCounters {
   uint32_t leaf_splits;    // leaves the batch's transactions split
   uint32_t sort_retry;     // a bucket of the small-batch sort overflowed: the batch ran empty and
                            // is to be run again with the exact sort
-  uint32_t pad;
+  uint32_t skipped;        // the batch ran empty because an earlier one of its stream failed
 };
 static_assert(sizeof(BatchCounters) == 64, "one 64-byte block");
+
+// Totals of a batch stream, accumulated on the device so its batches need no host round trip.
+struct StreamAcc {
+  unsigned long long unique;   // groups after the per-key fold
+  unsigned long long bad;      // ops rejected for the reserved key
+  unsigned long long batches;  // batches that ran
+  unsigned long long skipped;  // batches skipped after an error
+  unsigned long long sort_stalls;  // batches whose sort gave up a grid-barrier wait
+  unsigned long long fallbacks;    // batches whose normalized sort fell back to the exact passes
+  unsigned long long leaf_splits;  // leaves the batches split
+  unsigned long long retries;      // a batch whose small-batch sort overflowed a bucket
+};
+// Whether an earlier batch of the stream failed: the later ones then run empty, so the tree holds
+// exactly the batches up to the failing one.
+STM_DEV bool stream_failed(const StreamAcc* acc, const TreeHeader* hdr) {
+  return acc->bad || acc->sort_stalls || acc->retries || hdr->error;
+}
 
 struct FoldArgs {
   const uint64_t* skeys;  // sorted keys

@@ -286,19 +286,32 @@ __global__ __launch_bounds__(256, (lookup_min_waves<F, G>())) void k_lookup(Tree
                                                 uint64_t* __restrict__ gval,
                                                 uint64_t* __restrict__ fanout,
                                                 uint64_t fanout_cap,
-                                                SplitState* __restrict__ split) {
+                                                SplitState* __restrict__ split,
+                                                const StreamAcc* __restrict__ acc) {
   constexpr int K = F / G;
+  const bool skip = acc && stream_failed(acc, t.hdr);
   if (blockIdx.x == 0 && threadIdx.x == 0) {
     SplitState z{};
     z.refused = NODE_NONE;
     *split = z;
+    if (acc) {
+      // Every workgroup sees the earlier failure itself; the later kernels see no groups.
+      BatchCounters* c = const_cast<BatchCounters*>(cnt);
+      c->skipped = skip ? 1u : 0u;
+      if (skip) {
+        c->n_unique = 0;
+        c->n_upserts = 0;
+        c->n_fanout = 0;
+        c->n_deferred = 0;
+      }
+    }
   }
   const int lane = lane_id();
   const int g = lane & (G - 1);
   const int gbase = lane - g;
   const uint64_t grp0 = (blockIdx.x * (uint64_t)blockDim.x + threadIdx.x) / G;
   const uint64_t ngroups = (uint64_t)gridDim.x * blockDim.x / G;
-  const uint32_t U = cnt->n_unique;
+  const uint32_t U = skip ? 0u : cnt->n_unique;
   // Every lane group walks one contiguous span of sorted groups, so its cached leaf, parent and
   // directory cursor carry over for the whole span: at least `chunk` of them once there are
   // enough to give every lane group the device holds at once (`fill`) a chunk, fewer below that.
@@ -2379,7 +2392,7 @@ __global__ __launch_bounds__(64) void k_upsert_serial(TreeView t, const uint64_t
                                                       uint64_t* __restrict__ out_vals,
                                                       uint8_t* __restrict__ out_found,
                                                       const BatchDesc* __restrict__ desc,
-                                                      BatchCounters* host_out) {
+                                                      StreamAcc* acc, BatchCounters* host_out) {
   const uint32_t n = cnt->n_deferred;
   if (desc) {
     out_vals = desc->out_vals;
@@ -2402,7 +2415,24 @@ __global__ __launch_bounds__(64) void k_upsert_serial(TreeView t, const uint64_t
   // The last kernel of a batch: the tree's error bits travel back with the batch counters.
   wave_order();
   const uint64_t err = ld_relaxed(&t.hdr->error);
-  if (lane_id() == 0) const_cast<BatchCounters*>(cnt)->hdr_error = err;
+  if (lane_id() == 0) {
+    BatchCounters* b = const_cast<BatchCounters*>(cnt);
+    b->hdr_error = err;
+    if (acc) {
+      if (b->skipped) {
+        acc->skipped += 1;
+      } else if (b->sort_retry) {  // ran empty: the host runs it again and resumes the stream after it
+        acc->retries += 1;
+      } else {
+        acc->unique += b->n_unique;
+        acc->bad += b->n_bad;
+        acc->sort_stalls += b->sort_stall;
+        acc->fallbacks += b->sort_fallback;
+        acc->leaf_splits += ld_relaxed32(&b->leaf_splits);
+        acc->batches += 1;
+      }
+    }
+  }
   if (host_out) {
     // Lanes 0-7 store the 64-byte block into pinned host memory, which spares the batch a
     // separate copy on the stream.  Agent-scope loads read the other kernels' counter updates
@@ -2605,7 +2635,7 @@ static hipError_t launch_lookup_k(const TreeView& t, const LookupArgs& a, hipStr
       t, a.ukey, a.uop, a.gstart, a.npend, a.sidx, a.counters, a.chunk, fill, a.out_vals,
       a.out_found, LEARNED ? a.route_hdr : nullptr, LEARNED ? a.fences : nullptr,
       LEARNED ? a.lids : nullptr, LEARNED ? a.segs : nullptr, a.desc, a.ihint, a.gval, a.fanout,
-      a.fanout_cap, a.split);
+      a.fanout_cap, a.split, a.acc);
   return hipGetLastError();
 }
 
@@ -2679,7 +2709,7 @@ static hipError_t launch_upsert_f(const TreeView& t, const UpsertArgs& a, hipStr
     if ((e = hipGetLastError()) != hipSuccess) return e;
   }
   k_upsert_serial<F><<<1, 64, 0, s>>>(t, a.ukey, a.uval, a.gstart, a.npend, a.sidx, a.dlist,
-                                      a.counters, a.out_vals, a.out_found, a.desc,
+                                      a.counters, a.out_vals, a.out_found, a.desc, a.acc,
                                       a.host_counters);
   return hipGetLastError();
 }

@@ -76,6 +76,7 @@ struct LookupArgs {
   uint64_t* fanout;       // queued answer chunks: group | first op << 32 | found << 63
   uint64_t fanout_cap;    // fanout_capacity(n_max)
   SplitState* split;      // reset here for the upsert kernels
+  const StreamAcc* acc;   // optional: the batch of a stream, which runs empty after a failed one
 };
 
 struct UpsertArgs {
@@ -105,6 +106,7 @@ struct UpsertArgs {
   const uint64_t* fanout; // hot GET groups' answer chunks queued by the lookup kernel (the fast
   uint64_t fanout_cap;    //   path writes them first); null: none queued
   const uint64_t* gval;   // their values (per group)
+  StreamAcc* acc;                // optional: the stream's totals, to which the last kernel adds
   BatchCounters* host_counters;  // optional: pinned host memory the last kernel copies the
                                  //   counters into (null: the caller copies them back)
 };

@@ -74,8 +74,10 @@ typedef struct stm_config {
     uint32_t train_steps; /* learned routing: Adam steps per segment MLP (default 300) */
     uint32_t sort_tile_items; /* radix sort elements per thread: 8 or 16 (tiles of 2048 or 4096
                                  keys; default 16) */
-    uint32_t use_graphs;  /* stm_run_batches_device: 1 = replay one captured hipGraph per batch
-                             size class (default 1), 0 = launch every kernel from the host */
+    uint32_t use_graphs;  /* stm_run_batches_device: 1 = the host reads nothing back until the
+                             stream ends, and small size classes replay a hipGraph when
+                             stm_capture_graphs made one (default 1); 0 = one synchronous call per
+                             batch */
     uint32_t upsert_lanes;/* 8, 16 or 32, at most fanout; 0 = automatic (default).  Checked, but
                              without effect: the upsert kernel gives every insert one lane */
     uint32_t retrain_splits; /* learned routing / static index: also rebuild the directory (and
@@ -208,24 +210,24 @@ int stm_run_batch_scan_device(stm_tree* tree, const uint64_t* d_keys, const uint
  * [offsets[b], offsets[b+1]) of d_keys / d_vals / d_ops and is answered into the same range of
  * d_out_vals / d_out_found.  offsets is a host array of n_batches + 1 non-decreasing entries;
  * a batch longer than max_batch is chunked as in stm_run_batch_device.  The results equal
- * n_batches calls of stm_run_batch_device, in order.  With use_graphs the launch sequence of a
- * batch is captured once per size class (powers of 4 up to max_batch) as a hipGraph that reads
- * its batch from a device-side descriptor table, and replayed: the host reads nothing back
- * until the stream has run (a reserved key or a full node pool is reported at the end, the
- * tree then holds every batch up to and including the failing one; the outputs of the batches
- * after it are unspecified).  The graphs come in two halves per batch on two scratch sets, so
- * batch b + 1's sort and fold run while batch b's lookups and upserts do (a second batch
- * scratch and a second stream are made on first use).
+ * n_batches calls of stm_run_batch_device, in order.  With use_graphs the host reads nothing back
+ * until the stream has run (a reserved key or a full node pool is reported at the end, the tree
+ * then holds every batch up to and including the failing one; the outputs of the batches after it
+ * are unspecified).  Batches above 2048 ops run in two halves on two scratch sets, so batch b + 1's
+ * sort and fold run while batch b's lookups and upserts do; the second batch scratch and a second
+ * stream are made once the tree's streams have brought 32 such batches (or by
+ * stm_capture_graphs).
  * Replaces the batch loop of GPU_STM_Tree::gpu_work_main (src/gpu-stm-tree-v38/bpt-gpustm.cpp:77-135:
  * transferData, launchKernelBefore, launchKernel, launchKernelAfter, transferAns per batch). */
 int stm_run_batches_device(stm_tree* tree, const uint64_t* d_keys, const uint64_t* d_vals,
                            const uint8_t* d_ops, const uint64_t* offsets, size_t n_batches,
                            uint64_t* d_out_vals, uint8_t* d_out_found);
 
-/* Captures the graphs of every batch size class now (stm_run_batches_device captures a class
- * the first time a batch of that size arrives), so a latency-sensitive caller pays no capture
- * inside its stream.  No reference counterpart (the reference launches every kernel from the
- * host, src/gpu-stm-tree-v38/bpt-gpustm-kernel.cu:264-332). */
+/* Prepares batch streams now: captures the launch sequence of the batch size classes up to 2^12 ops
+ * as hipGraphs, which stm_run_batches_device then replays (one call of the host per batch instead
+ * of one per kernel; each reads its batch from a device-side descriptor), and makes the second
+ * scratch set and stream for larger batches.  No reference counterpart (the reference launches
+ * every kernel from the host, src/gpu-stm-tree-v38/bpt-gpustm-kernel.cu:264-332). */
 int stm_capture_graphs(stm_tree* tree);
 
 /* Stable ascending sort of n device-resident u64 keys on `device`: d_keys_out receives the
