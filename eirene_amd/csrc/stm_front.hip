@@ -145,6 +145,153 @@ STM_DEV void block_sort(uint64_t (&k)[E], uint32_t (&p)[E], uint64_t* s_k, uint3
   }
 }
 
+// LDS of bin_sort beside the elements.
+constexpr uint32_t BIN_BITS = 11;
+constexpr uint32_t BINS = 1u << BIN_BITS;
+constexpr uint32_t BIN_MAX = 32;  // a bin with more elements sends the block to the comparison sort
+struct BinShared {
+  uint32_t bin[BINS];
+  uint64_t mn, mx;  // least and greatest key
+  uint32_t heavy;
+  uint32_t w[FW];
+};
+
+// Before the first barrier ahead of bin_sort.
+template <int NT>
+STM_DEV void bin_sort_open(BinShared& sh) {
+#pragma unroll
+  for (uint32_t q = threadIdx.x; q < BINS; q += NT) sh.bin[q] = 0;
+  if (threadIdx.x == 0) {
+    sh.mn = KEY_EMPTY;
+    sh.mx = 0;
+    sh.heavy = 0;
+  }
+}
+
+// The block's m <= NT * E elements, element r * NT + tid in k[r], p[r], into sorted order in s_k, s_p.
+// They are counted into BINS bins by the leading bits of their key within the block's range (of
+// their tie where all keys are equal), placed by bin and ranked among the few elements of their
+// bin.  Keys that crowd a bin (a hot key, tight clusters) are sorted by comparison.
+// The comparison sort is bound by its arithmetic: 55 steps of some 14 instructions per element at
+// 1024 elements, where a lane of this one executes about 100.  Comparison sort / this, µs:
+// k_front_small of 1000 ops 9.1 / 7.2, k_front_bucket of 40001 ops 11.2 / 7.7, k_front_split of 131075
+// ops (2048 samples) 19.4 / 16.8; with crowded bins (Zipf inserts, 2^14 ops) no difference.
+// Every thread of the workgroup calls it, after bin_sort_open and a barrier.
+template <int NT, int E>
+STM_DEV void bin_sort(uint32_t m, uint64_t (&k)[E], uint32_t (&p)[E], uint64_t* s_k, uint32_t* s_p,
+                      BinShared& sh) {
+  const uint32_t tid = threadIdx.x;
+  const uint32_t wave = tid / WAVE;
+  uint64_t mn = KEY_EMPTY, mx = 0;
+#pragma unroll
+  for (int r = 0; r < E; ++r) {
+    if ((uint32_t)r * NT + tid < m) {
+      mn = k[r] < mn ? k[r] : mn;
+      mx = k[r] > mx ? k[r] : mx;
+    }
+  }
+#pragma unroll
+  for (int off = 1; off < WAVE; off <<= 1) {
+    const uint64_t a = ((uint64_t)lane_xor((uint32_t)(mn >> 32), off) << 32) | lane_xor((uint32_t)mn, off);
+    const uint64_t b = ((uint64_t)lane_xor((uint32_t)(mx >> 32), off) << 32) | lane_xor((uint32_t)mx, off);
+    mn = a < mn ? a : mn;
+    mx = b > mx ? b : mx;
+  }
+  if (lane_id() == 0 && wave * WAVE < m) {
+    atomicMin((unsigned long long*)&sh.mn, (unsigned long long)mn);
+    atomicMax((unsigned long long*)&sh.mx, (unsigned long long)mx);
+  }
+  __syncthreads();
+  mn = sh.mn;
+  mx = sh.mx;
+  const bool same = mn == mx;
+  const uint32_t len = same ? 32u : mx ? 64u - (uint32_t)__clzll((long long)(mx - mn)) : 0u;
+  const uint64_t base = same ? 0ull : mn;
+  const uint32_t shift = len > BIN_BITS ? len - BIN_BITS : 0u;
+  uint32_t bin[E], at[E];
+#pragma unroll
+  for (int r = 0; r < E; ++r) {
+    bin[r] = 0;
+    at[r] = 0;
+    if ((uint32_t)r * NT + tid < m) {
+      bin[r] = (uint32_t)(((same ? (uint64_t)p[r] : k[r]) - base) >> shift);
+      at[r] = atomicAdd(&sh.bin[bin[r]], 1u);
+      if (at[r] >= BIN_MAX) sh.heavy = 1;
+    }
+  }
+  __syncthreads();
+  if (sh.heavy) {
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+      const bool v = (uint32_t)r * NT + tid < m;
+      k[r] = v ? k[r] : KEY_EMPTY;
+      p[r] = v ? p[r] : ~0u;
+    }
+    block_sort<NT * E, E>(k, p, s_k, s_p);
+    __syncthreads();
+#pragma unroll
+    for (int r = 0; r < E; ++r) {
+      s_k[tid * E + r] = k[r];
+      s_p[tid * E + r] = p[r];
+    }
+    __syncthreads();
+    return;
+  }
+  // Exclusive scan of the bins, PER per thread.
+  constexpr uint32_t PER = BINS / NT;
+  uint32_t c[PER], sum = 0;
+#pragma unroll
+  for (uint32_t q = 0; q < PER; ++q) {
+    c[q] = sh.bin[tid * PER + q];
+    sum += c[q];
+  }
+  uint32_t x = sum;
+#pragma unroll
+  for (int off = 1; off < WAVE; off <<= 1) {
+    const uint32_t y = __shfl_up(x, off, WAVE);
+    if (lane_id() >= off) x += y;
+  }
+  if (lane_id() == WAVE - 1) sh.w[wave] = x;
+  __syncthreads();
+  uint32_t run = x - sum;
+#pragma unroll
+  for (int w = 0; w < NT / WAVE; ++w) run += (uint32_t)w < wave ? sh.w[w] : 0u;
+#pragma unroll
+  for (uint32_t q = 0; q < PER; ++q) {
+    sh.bin[tid * PER + q] = run;
+    run += c[q];
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < E; ++r) {
+    if ((uint32_t)r * NT + tid < m) {
+      at[r] += sh.bin[bin[r]];
+      s_k[at[r]] = k[r];
+      s_p[at[r]] = p[r];
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < E; ++r) {
+    if ((uint32_t)r * NT + tid < m) {
+      const uint32_t lo = sh.bin[bin[r]];
+      const uint32_t hi = bin[r] + 1 < BINS ? sh.bin[bin[r] + 1] : m;
+      at[r] = lo;
+      if (hi - lo > 1)
+        for (uint32_t j = lo; j < hi; ++j) at[r] += elem_less(s_k[j], s_p[j], k[r], p[r]) ? 1u : 0u;
+    }
+  }
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < E; ++r) {
+    if ((uint32_t)r * NT + tid < m) {
+      s_k[at[r]] = k[r];
+      s_p[at[r]] = p[r];
+    }
+  }
+  __syncthreads();
+}
+
 // ------------------------------------------------------------------ fold of sorted elements
 // One sorted element as the fold sees it (a thread's own).
 struct FoldElem {
@@ -250,6 +397,7 @@ __global__ __launch_bounds__(FT) void k_front_small(FrontArgs fa) {
   __shared__ uint64_t s_k[N];
   __shared__ uint32_t s_p[N];
   __shared__ Acc s_acc[CHUNKS];
+  __shared__ BinShared s_bin;
   __shared__ uint32_t s_bad;
   const FrontIn in = front_in(fa);
   FoldArgs a = fa.fold;
@@ -268,15 +416,10 @@ __global__ __launch_bounds__(FT) void k_front_small(FrontArgs fa) {
     k[r] = kk;
     p[r] = v ? tie_of(i, op) : ~0u;
   }
-  block_sort<N, E>(k, p, s_k, s_p);
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < E; ++r) {
-    s_k[tid * E + r] = k[r];
-    s_p[tid * E + r] = p[r];
-  }
+  bin_sort_open<FT>(s_bin);
   if (tid == 0) s_bad = 0;
   __syncthreads();
+  bin_sort<FT, E>(n, k, p, s_k, s_p, s_bin);
   FoldElem x[E];
   uint64_t hm[E], im[E];
 #pragma unroll
@@ -332,10 +475,10 @@ __global__ __launch_bounds__(FT) void k_front_split(FrontArgs fa) {
   constexpr uint32_t TILE = FT * E;
   constexpr int B = S / (int)OVERSAMPLE;
   constexpr int SE = S > FT ? S / FT : 1;  // samples per thread
-  __shared__ uint64_t s_k[S];
-  __shared__ uint32_t s_p[S];
-  __shared__ uint64_t s_spk[B];
-  __shared__ uint32_t s_spp[B];
+  constexpr int SN = FT * SE;
+  __shared__ uint64_t s_k[SN];
+  __shared__ uint32_t s_p[SN];
+  __shared__ BinShared s_bin;
   __shared__ uint32_t s_cnt[B], s_off[B + 1];
   __shared__ uint32_t s_w[FW];
   const FrontIn in = front_in(fa);
@@ -361,7 +504,7 @@ __global__ __launch_bounds__(FT) void k_front_split(FrontArgs fa) {
   uint32_t sp[SE];
 #pragma unroll
   for (int r = 0; r < SE; ++r) {
-    const uint32_t j = tid * SE + r;
+    const uint32_t j = (uint32_t)r * FT + tid;
     sk[r] = KEY_EMPTY;
     sp[r] = ~0u;
     if (j < (uint32_t)S) {
@@ -374,16 +517,19 @@ __global__ __launch_bounds__(FT) void k_front_split(FrontArgs fa) {
     }
   }
   if (tid < (uint32_t)B) s_cnt[tid] = 0;
-  block_sort<S, SE>(sk, sp, s_k, s_p);
-#pragma unroll
-  for (int r = 0; r < SE; ++r) {
-    const uint32_t j = tid * SE + r;
-    if (j < (uint32_t)S && j % OVERSAMPLE == 0) {
-      s_spk[j / OVERSAMPLE] = sk[r];
-      s_spp[j / OVERSAMPLE] = sp[r];
+  if constexpr (S < FT) {  // few enough for the comparison sort, and indifferent to crowded keys
+    block_sort<S, 1>(sk, sp, s_k, s_p);
+    __syncthreads();
+    if (tid < (uint32_t)S) {
+      s_k[tid] = sk[0];
+      s_p[tid] = sp[0];
     }
+    __syncthreads();
+  } else {
+    bin_sort_open<FT>(s_bin);
+    __syncthreads();
+    bin_sort<FT, SE>(S, sk, sp, s_k, s_p, s_bin);
   }
-  __syncthreads();
   // Bucket: the splitters 1 .. B - 1 not above the element.
   uint32_t bkt[E], rank[E];
 #pragma unroll
@@ -394,7 +540,7 @@ __global__ __launch_bounds__(FT) void k_front_split(FrontArgs fa) {
 #pragma unroll
     for (int step = B / 2; step > 0; step >>= 1) {
       const uint32_t q = lo + (uint32_t)step;
-      if (!elem_less(ek[r], ep[r], s_spk[q], s_spp[q])) lo = q;
+      if (!elem_less(ek[r], ep[r], s_k[q * OVERSAMPLE], s_p[q * OVERSAMPLE])) lo = q;
     }
     bkt[r] = lo;
     rank[r] = le < tile_n ? atomicAdd(&s_cnt[lo], 1u) : 0u;
@@ -435,7 +581,7 @@ __global__ __launch_bounds__(FT) void k_front_split(FrontArgs fa) {
 // from position start, and back to s_k for the summary.
 template <int E>
 STM_DEV void sort_bucket(const FrontArgs& fa, uint32_t m, uint32_t start, uint64_t* s_k, uint32_t* s_p,
-                         BucketSum& sum, Acc* s_acc) {
+                         BinShared& s_bin, BucketSum& sum, Acc* s_acc) {
   const uint32_t tid = threadIdx.x;
   uint64_t k[E];
   uint32_t p[E];
@@ -445,14 +591,7 @@ STM_DEV void sort_bucket(const FrontArgs& fa, uint32_t m, uint32_t start, uint64
     k[r] = i < m ? s_k[i] : KEY_EMPTY;
     p[r] = i < m ? s_p[i] : ~0u;
   }
-  block_sort<FT * E, E>(k, p, s_k, s_p);
-  __syncthreads();
-#pragma unroll
-  for (int r = 0; r < E; ++r) {
-    s_k[tid * E + r] = k[r];
-    s_p[tid * E + r] = p[r];
-  }
-  __syncthreads();
+  bin_sort<FT, E>(m, k, p, s_k, s_p, s_bin);
 #pragma unroll
   for (int r = 0; r < E; ++r) {
     const uint32_t i = (uint32_t)r * FT + tid;
@@ -480,6 +619,7 @@ __global__ __launch_bounds__(FT) void k_front_bucket(FrontArgs fa, uint32_t tile
   __shared__ uint32_t s_src[TILES_MAX], s_dst[TILES_MAX], s_len[TILES_MAX];
   __shared__ uint32_t s_w[2][2];
   __shared__ Acc s_acc[BUCKET_CAP / WAVE];
+  __shared__ BinShared s_bin;
   static_assert(BUCKET_CAP / WAVE <= WAVE, "one wavefront combines a bucket's states");
   static_assert(TILES_MAX <= 2 * WAVE, "the tiles fit two wavefronts");
   const uint32_t n = front_in(fa).n;
@@ -522,6 +662,7 @@ __global__ __launch_bounds__(FT) void k_front_bucket(FrontArgs fa, uint32_t tile
   if (m > BUCKET_CAP) {
     if (tid == 0) fa.words[FRONT_RETRY] = 1;
   } else if (m > 0) {
+    bin_sort_open<FT>(s_bin);
     // Eight lanes per piece: the mean piece is a few elements.
     for (uint32_t t = tid / 8; t < tiles; t += FT / 8) {
       const uint32_t src = s_src[t], dst = s_dst[t], l = s_len[t];
@@ -531,9 +672,9 @@ __global__ __launch_bounds__(FT) void k_front_bucket(FrontArgs fa, uint32_t tile
       }
     }
     __syncthreads();
-    if (m <= FT) sort_bucket<1>(fa, m, start, s_k, s_p, sum, s_acc);
-    else if (m <= 2 * FT) sort_bucket<2>(fa, m, start, s_k, s_p, sum, s_acc);
-    else sort_bucket<4>(fa, m, start, s_k, s_p, sum, s_acc);
+    if (m <= FT) sort_bucket<1>(fa, m, start, s_k, s_p, s_bin, sum, s_acc);
+    else if (m <= 2 * FT) sort_bucket<2>(fa, m, start, s_k, s_p, s_bin, sum, s_acc);
+    else sort_bucket<4>(fa, m, start, s_k, s_p, s_bin, sum, s_acc);
   }
   if (tid == 0) sums[b] = sum;
 }

@@ -129,8 +129,8 @@ struct FoldArgs {
 // ------------------------------------------------------------------ front half of small batches
 // (stm_front.hip): sort and fold of at most FRONT_MAX_OPS ops in one or three launches, with the
 // results of the radix sort and fold_batch.  A whole call on 2^22 uniform keys, with the radix
-// form and the lookup's longer spans in parentheses: 1000 ops 37 µs (113), 16384 ops 60 (123), 2^16
-// ops 73 (144), 2^18 ops 119 (171).  Above
+// form and the lookup's longer spans in parentheses: 1000 ops 33 µs (113), 16384 ops 58 (123), 2^16
+// ops 70 (144), 2^18 ops 113 (171).  Above
 // 2^18 ops a workgroup's sample sort and the buckets' comparison sorts grow past what they save.
 constexpr uint32_t FRONT_MAX_OPS = 1u << 18;
 struct FrontArgs {
