@@ -501,7 +501,7 @@ hipError_t enqueue_front(stm_tree* t, Scratch& s, const PipeIn& in, bool timed, 
     return hipSuccess;
   }
   e = radix_sort_pairs_desc(in.keys, in.ops, in.desc, in.n, s.skeys_tmp, s.skeys, s.sidx_tmp, s.sidx, 0,
-                            64, s.hist, (int)t->cfg.sort_tile_items, exact, st);
+                            64, s.hist, (int)t->cfg.sort_tile_items, exact, in.out_found, st);
   if (e != hipSuccess) return e;
   if (timed) phase_switch(t, STM_PHASE_SORT, STM_PHASE_MERGE);
   fa.sort_stall = sort_stall_word(s.hist);

@@ -258,8 +258,7 @@ __global__ __launch_bounds__(FOLD_BLOCK) void k_fold_apply(FoldArgs a, const Acc
         if (a.lastins) a.lastins[i] = is_ins ? i : last_before;
         if (a.out_vals && last_before >= 0) {
           const uint32_t pos = pos_of(ch.sx[r]);
-          a.out_vals[pos] = va[q];
-          a.out_found[pos] = 1;
+          a.out_vals[pos] = va[q];  // out_found stays 1
         }
         if (a.gstart && is_ins && last_before < 0) a.npend[g] = (uint32_t)(i - head + 1);
         if (group_end) {

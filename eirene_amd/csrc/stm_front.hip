@@ -317,8 +317,7 @@ STM_DEV void fold_store(const FoldArgs& a, const FoldElem& x, uint32_t* bad) {
   if (!x.valid) return;
   if (a.lastins) a.lastins[x.i] = x.ins ? x.i : x.lb;
   if (x.lb >= 0) {
-    a.out_vals[x.pos] = x.va;
-    a.out_found[x.pos] = 1;
+    a.out_vals[x.pos] = x.va;  // out_found stays 1
   }
   if (x.ins && x.lb < 0) a.npend[x.g] = (uint32_t)(x.i - x.head + 1);
   if (!x.end) return;
@@ -455,7 +454,10 @@ __global__ __launch_bounds__(FT) void k_front_small(FrontArgs fa) {
     fold_gather(a, x[r]);
   }
 #pragma unroll
-  for (int r = 0; r < E; ++r) fold_store(a, x[r], &s_bad);
+  for (int r = 0; r < E; ++r) {
+    if (x[r].valid) a.out_found[x[r].i] = 1;  // the answers' default
+    fold_store(a, x[r], &s_bad);
+  }
   __syncthreads();
   if (tid == 0) reset_counters(a.counters, run.c, run.m & ~ACC_LEAD, s_bad);
 }
@@ -484,6 +486,7 @@ __global__ __launch_bounds__(FT) void k_front_split(FrontArgs fa) {
   const FrontIn in = front_in(fa);
   const uint32_t n = in.n;
   const uint32_t tid = threadIdx.x;
+  uint8_t* found = fa.fold.desc ? fa.fold.desc->out_found : fa.fold.out_found;
   if (blockIdx.x == 0 && tid == 0) {
     reset_counters(fa.fold.counters, 0, 0, 0);
     fa.words[FRONT_RETRY] = 0;
@@ -572,6 +575,7 @@ __global__ __launch_bounds__(FT) void k_front_split(FrontArgs fa) {
       const uint32_t dst = tile0 + s_off[bkt[r]] + rank[r];
       fa.tmp_keys[dst] = ek[r];
       fa.tmp_ties[dst] = ep[r];
+      found[tile0 + le] = 1;  // the answers' default
     }
   }
 }

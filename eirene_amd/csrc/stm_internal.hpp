@@ -52,13 +52,15 @@ hipError_t radix_sort_pairs(const uint64_t* keys_in, uint64_t* keys_tmp, uint64_
 // With desc the keys, op codes and their count are read from the device-side descriptor
 // (keys_in and ops_in unused) and n_max only bounds that count (grid and scratch sizing);
 // without it keys_in holds n_max keys.
+// found (the descriptor's out_found with desc; null: none) is set to 1 throughout on the way: the
+// answers' default.
 // The normalized-key form runs unless `exact` asks for the eight-pass form (the library asks for
 // it after a batch whose normalized sort had to fall back).
 hipError_t radix_sort_pairs_desc(const uint64_t* keys_in, const uint8_t* ops_in,
                                  const BatchDesc* desc, uint32_t n_max,
                                  uint64_t* keys_tmp, uint64_t* keys_out, uint32_t* idx_tmp,
                                  uint32_t* idx_out, int begin_bit, int end_bit, uint32_t* hist_words,
-                                 int tile_items, bool exact, hipStream_t stream);
+                                 int tile_items, bool exact, uint8_t* found, hipStream_t stream);
 // Non-zero after a normalized-key sort that found a long bucket of distinct keys and re-sorted
 // the batch with the eight exact passes inside one launch (correct, but slower); cleared when
 // the next sort on the same scratch starts.
@@ -111,7 +113,7 @@ struct FoldArgs {
   const BatchDesc* desc;  // optional: n, vals, ops and outputs come from here
   // outputs
   uint64_t* out_vals;     // per original op (may be null for bulk load)
-  uint8_t* out_found;
+  uint8_t* out_found;     // holds 1s already (the sort writes them); not written by the fold
   uint64_t* ukey;         // per group
   uint64_t* uval;
   uint8_t* uop;           // OP_GET, OP_INSERT or UOP_SKIP

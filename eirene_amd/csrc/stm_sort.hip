@@ -309,7 +309,7 @@ STM_DEV void scatter_body(
     const BatchDesc* __restrict__ desc, uint32_t n_host, int first_pass, int shift,
     const uint32_t* __restrict__ hist, uint32_t stride, const uint32_t* __restrict__ totals,
     uint64_t* __restrict__ keys_out, uint32_t* __restrict__ idx_out,
-    const uint32_t* __restrict__ norm, int npass) {
+    const uint32_t* __restrict__ norm, int npass, uint8_t* __restrict__ found) {
   constexpr int TILE = SORT_BLOCK * ITEMS;
   constexpr int SEG = TILE / SORT_WAVES;  // contiguous elements owned by one wavefront
   __shared__ uint32_t s_wcnt[SORT_WAVES][RADIX];  // running per-wave digit counts, then wave bases
@@ -332,6 +332,8 @@ STM_DEV void scatter_body(
   const uint32_t ntiles = (rg.n + TILE - 1) / TILE;
   const uint64_t* kin = rg.keys;
   const uint8_t* ops = (first_pass && desc) ? desc->ops : ops_in;  // read on the first pass only
+  if (desc) found = desc->out_found;
+  if (!first_pass) found = nullptr;
   const int lane = lane_id();
   const int wave = threadIdx.x / WAVE;
   {
@@ -428,6 +430,11 @@ STM_DEV void scatter_body(
 #pragma unroll
       for (int r = 0; r < ITEMS; ++r) id[r] = (uint32_t)tile0 + lane0 + (uint32_t)r * WAVE;
     }
+    if (found) {
+#pragma unroll
+      for (int r = 0; r < ITEMS; ++r)
+        if (lane0 + (uint32_t)r * WAVE < tile_n) found[tile0 + lane0 + (uint32_t)r * WAVE] = 1;
+    }
     __syncthreads();
     // The digit of every position a thread writes, four to a register, for the payload phase.
     uint32_t dg[(ITEMS + 3) / 4];
@@ -471,9 +478,9 @@ __global__ __launch_bounds__(SORT_BLOCK) void k_scatter(
     const BatchDesc* __restrict__ desc, uint32_t n_host, int first_pass, int shift,
     const uint32_t* __restrict__ hist, uint32_t stride, const uint32_t* __restrict__ totals,
     uint64_t* __restrict__ keys_out, uint32_t* __restrict__ idx_out,
-    const uint32_t* __restrict__ norm, int npass) {
+    const uint32_t* __restrict__ norm, int npass, uint8_t* __restrict__ found) {
   scatter_body<ITEMS>(keys_in, idx_in, ops_in, desc, n_host, first_pass, shift, hist, stride,
-                      totals, keys_out, idx_out, norm, npass);
+                      totals, keys_out, idx_out, norm, npass, found);
 }
 
 // ================================================================ normalized-key form
@@ -710,7 +717,7 @@ __global__ __launch_bounds__(SORT_BLOCK) void k_sort_exact(
     scan_hist_body<ITEMS>(hist, stride, desc, n_host, totals);
     grid_barrier(words, (++arrivals) * gridDim.x);
     scatter_body<ITEMS>(kin, iin, first ? ops_in : nullptr, desc, n_host, first, 8 * p, hist,
-                        stride, totals, kout, iout, nullptr, 0);
+                        stride, totals, kout, iout, nullptr, 0, nullptr);
     grid_barrier(words, (++arrivals) * gridDim.x);
     kin = kout;
     iin = iout;
@@ -772,7 +779,8 @@ template <int ITEMS>
 static hipError_t sort_normalized(const uint64_t* keys_in, const uint8_t* ops_in,
                                   const BatchDesc* desc, uint32_t n_host, uint32_t n_max,
                                   uint64_t* keys_tmp, uint64_t* keys_out, uint32_t* idx_tmp,
-                                  uint32_t* idx_out, uint32_t* words, hipStream_t stream) {
+                                  uint32_t* idx_out, uint32_t* words, uint8_t* found,
+                                  hipStream_t stream) {
   const uint32_t tile = sort_tile(ITEMS);
   const uint32_t stride = (n_max + tile - 1) / tile;
   const uint32_t grid = std::max<uint32_t>(1, std::min<uint32_t>(stride, SORT_GRID_CAP));
@@ -795,7 +803,7 @@ static hipError_t sort_normalized(const uint64_t* keys_in, const uint8_t* ops_in
     k_scan_hist<ITEMS><<<RADIX, SORT_BLOCK, 0, stream>>>(hist, stride, desc, n_host, totals);
     k_scatter<ITEMS><<<grid, SORT_BLOCK, 0, stream>>>(kin, iin, first ? ops_in : nullptr, desc,
                                                       n_host, first, 8 * p, hist, stride, totals,
-                                                      kout, iout, words, npass);
+                                                      kout, iout, words, npass, found);
     e = hipGetLastError();
     if (e != hipSuccess) return e;
     kin = kout;
@@ -815,7 +823,7 @@ static hipError_t sort_passes(const uint64_t* keys_in, const uint8_t* ops_in, co
                               uint32_t n_host,
                               uint32_t n_max, uint64_t* keys_tmp, uint64_t* keys_out,
                               uint32_t* idx_tmp, uint32_t* idx_out, int begin_bit, int end_bit,
-                              uint32_t* words, bool exact, hipStream_t stream) {
+                              uint32_t* words, bool exact, uint8_t* found, hipStream_t stream) {
   const uint32_t tile = sort_tile(ITEMS);
   const uint32_t stride = (n_max + tile - 1) / tile;  // tiles of the largest batch
   const int passes = (end_bit - begin_bit + 7) / 8;
@@ -827,7 +835,7 @@ static hipError_t sort_passes(const uint64_t* keys_in, const uint8_t* ops_in, co
   if (passes > MAX_PASSES) return hipErrorInvalidValue;
   if (!exact && begin_bit == 0 && end_bit == 64)
     return sort_normalized<ITEMS>(keys_in, ops_in, desc, n_host, n_max, keys_tmp, keys_out,
-                                  idx_tmp, idx_out, words, stream);
+                                  idx_tmp, idx_out, words, found, stream);
   // The exact form: eight 8-bit passes of three kernels each.
   const uint64_t* kin = keys_in;
   const uint32_t* iin = nullptr;
@@ -845,7 +853,7 @@ static hipError_t sort_passes(const uint64_t* keys_in, const uint8_t* ops_in, co
     k_scan_hist<ITEMS><<<RADIX, SORT_BLOCK, 0, stream>>>(hist, stride, desc, n_host, totals);
     k_scatter<ITEMS><<<grid, SORT_BLOCK, 0, stream>>>(kin, iin, first ? ops_in : nullptr, desc,
                                                       n_host, first, shift, hist, stride,
-                                                      totals, kout, iout, nullptr, 0);
+                                                      totals, kout, iout, nullptr, 0, found);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return e;
     kin = kout;
@@ -858,14 +866,14 @@ hipError_t radix_sort_pairs_desc(const uint64_t* keys_in, const uint8_t* ops_in,
                                  const BatchDesc* desc, uint32_t n_max,
                                  uint64_t* keys_tmp, uint64_t* keys_out, uint32_t* idx_tmp,
                                  uint32_t* idx_out, int begin_bit, int end_bit, uint32_t* hist_words,
-                                 int tile_items, bool exact, hipStream_t stream) {
+                                 int tile_items, bool exact, uint8_t* found, hipStream_t stream) {
   if (n_max == 0) return hipSuccess;
   const uint32_t n_host = desc ? 0u : n_max;
   if (tile_items == 8)
     return sort_passes<8>(keys_in, ops_in, desc, n_host, n_max, keys_tmp, keys_out, idx_tmp,
-                          idx_out, begin_bit, end_bit, hist_words, exact, stream);
+                          idx_out, begin_bit, end_bit, hist_words, exact, found, stream);
   return sort_passes<16>(keys_in, ops_in, desc, n_host, n_max, keys_tmp, keys_out, idx_tmp,
-                         idx_out, begin_bit, end_bit, hist_words, exact, stream);
+                         idx_out, begin_bit, end_bit, hist_words, exact, found, stream);
 }
 
 hipError_t radix_sort_pairs(const uint64_t* keys_in, uint64_t* keys_tmp, uint64_t* keys_out,
@@ -873,7 +881,7 @@ hipError_t radix_sort_pairs(const uint64_t* keys_in, uint64_t* keys_tmp, uint64_
                             int end_bit, uint32_t* hist_words, hipStream_t stream) {
   if (n == 0) return hipSuccess;
   return sort_passes<16>(keys_in, nullptr, nullptr, n, n, keys_tmp, keys_out, idx_tmp, idx_out,
-                         begin_bit, end_bit, hist_words, false, stream);
+                         begin_bit, end_bit, hist_words, false, nullptr, stream);
 }
 
 const uint32_t* sort_exact_word(const uint32_t* words) { return words + CTL_NEED_EXACT; }

@@ -485,7 +485,11 @@ __global__ __launch_bounds__(256, (lookup_min_waves<F, G>())) void k_lookup(Tree
       h->gs = gs_l;
       h->np = np_l;
     }
-    // The answers.
+    // The answers.  out_found holds 1s already (the front half writes them in input order, whole
+    // lines at a time), so only an absent key's op is written here: a byte scattered to its input
+    // position is a memory request of its own, as its value is.  With every byte scattered (2^26
+    // keys, 2^22 ops at 95/5): this kernel 356 µs instead of 342, k_fold_apply 46.8 instead of 41.7,
+    // k_upsert_runs 39.2 instead of 35.7.
     if (mine) {
       if (np_l > FANOUT_DIRECT) {
         // A hot key: its waiting ops are answered by the whole grid (fanout_answers), in
@@ -500,12 +504,12 @@ __global__ __launch_bounds__(256, (lookup_min_waves<F, G>())) void k_lookup(Tree
       } else {
         if (np_l) {
           out_vals[pos_l] = val;
-          out_found[pos_l] = found_l ? 1 : 0;
+          if (!found_l) out_found[pos_l] = 0;
         }
         for (uint32_t p = 1; p < np_l; ++p) {
           const uint32_t pos = pos_of(sidx[gs_l + p]);
           out_vals[pos] = val;
-          out_found[pos] = found_l ? 1 : 0;
+          if (!found_l) out_found[pos] = 0;
         }
       }
     }
@@ -1443,14 +1447,14 @@ STM_DEV void fanout_answers(const uint64_t* __restrict__ fanout, uint64_t cap,
     const uint64_t e = fanout[c];
     const uint32_t g = (uint32_t)e;
     const uint32_t first = (uint32_t)(e >> 32) & 0x7fffffffu;
-    const uint8_t found = (uint8_t)(e >> 63);
+    const bool found = e >> 63;
     const uint32_t gs = gstart[g];
     const uint32_t end = min(npend[g], first + FANOUT_CHUNK);
     const uint64_t v = gval[g];
     for (uint32_t p = first + threadIdx.x; p < end; p += blockDim.x) {
       const uint32_t pos = pos_of(sidx[gs + p]);
       out_vals[pos] = v;
-      out_found[pos] = found;
+      if (!found) out_found[pos] = 0;
     }
   }
 }
@@ -1466,7 +1470,7 @@ STM_DEV void write_upsert_answers(bool ans, bool found, uint64_t old, uint32_t g
     for (uint32_t p = 0; p < np; ++p) {
       const uint32_t pos = p == 0 ? p0 : pos_of(sidx[gs + p]);
       out_vals[pos] = old;
-      out_found[pos] = found ? 1 : 0;
+      if (!found) out_found[pos] = 0;
     }
   }
   for (uint64_t bm = ballot(many); bm; bm &= bm - 1) {
@@ -1474,11 +1478,11 @@ STM_DEV void write_upsert_answers(bool ans, bool found, uint64_t old, uint32_t g
     const uint32_t gsb = __builtin_amdgcn_readlane(gs, b);
     const uint32_t npb = __builtin_amdgcn_readlane(np, b);
     const uint64_t ob = readlane64(old, b);
-    const uint8_t fb = (uint8_t)__builtin_amdgcn_readlane(found ? 1 : 0, b);
+    const bool fb = __builtin_amdgcn_readlane(found ? 1 : 0, b) != 0;
     for (uint32_t p = lane_id(); p < npb; p += WAVE) {
       const uint32_t pos = pos_of(sidx[gsb + p]);
       out_vals[pos] = ob;
-      out_found[pos] = fb;
+      if (!fb) out_found[pos] = 0;
     }
   }
 }
