@@ -38,6 +38,12 @@ constexpr uint32_t SCAN_REG = 8;               // tiles per thread the histogram
 
 constexpr int MAX_PASSES = 8;
 
+// Up to this many elements (384 tiles of 4096, three for every two CUs) the smaller tile is the
+// faster one whatever the configuration says: a pass is then as long as one tile's chain of
+// steps.  k_scatter with tiles of 4096 / 2048, µs: 2^19 elements 15.5 / 11.7, 2^20 16.0 / 14.2, 1.5 M
+// 18.0 / 15.9, 2^21 18.9 / 19.7 (and k_hist 7.0 / 7.6), 2^22 28.2 / 35.6.
+constexpr uint32_t SMALL_TILE_OPS = 3u << 19;
+
 // Sort scratch (u32 words): control words, k_range's partials, then the histogram region (per-tile
 // histograms and digit totals).
 constexpr uint32_t CTL_STALL = 0;
@@ -869,7 +875,7 @@ hipError_t radix_sort_pairs_desc(const uint64_t* keys_in, const uint8_t* ops_in,
                                  int tile_items, bool exact, uint8_t* found, hipStream_t stream) {
   if (n_max == 0) return hipSuccess;
   const uint32_t n_host = desc ? 0u : n_max;
-  if (tile_items == 8)
+  if (tile_items == 8 || n_max <= SMALL_TILE_OPS)
     return sort_passes<8>(keys_in, ops_in, desc, n_host, n_max, keys_tmp, keys_out, idx_tmp,
                           idx_out, begin_bit, end_bit, hist_words, exact, found, stream);
   return sort_passes<16>(keys_in, ops_in, desc, n_host, n_max, keys_tmp, keys_out, idx_tmp,
@@ -880,6 +886,9 @@ hipError_t radix_sort_pairs(const uint64_t* keys_in, uint64_t* keys_tmp, uint64_
                             uint32_t* idx_tmp, uint32_t* idx_out, uint32_t n, int begin_bit,
                             int end_bit, uint32_t* hist_words, hipStream_t stream) {
   if (n == 0) return hipSuccess;
+  if (n <= SMALL_TILE_OPS)
+    return sort_passes<8>(keys_in, nullptr, nullptr, n, n, keys_tmp, keys_out, idx_tmp, idx_out,
+                          begin_bit, end_bit, hist_words, false, nullptr, stream);
   return sort_passes<16>(keys_in, nullptr, nullptr, n, n, keys_tmp, keys_out, idx_tmp, idx_out,
                          begin_bit, end_bit, hist_words, false, nullptr, stream);
 }
