@@ -8,7 +8,8 @@
 //   k_route_root          root line segment ~ a*key + b through the first and last fence
 //   k_route_segments      segment s = ranks whose root prediction falls in bucket s
 //   k_route_train         one wavefront per segment: full-batch Adam on the MSE of a
-//                         1 -> 16 -> 1 ReLU MLP (hand-written forward and backward)
+//                         1 -> 16 -> 1 ReLU MLP (hand-written forward and backward; a pair or a
+//                         hidden unit per lane)
 // k_mlp_grad exposes one forward/backward pass for the gradient check against the CPU.
 #include <cmath>
 
@@ -376,30 +377,159 @@ STM_DEV void broadcast_params(float pv, float* p) {
     p[q] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(pv), lane_of_param(q)));
 }
 
+// Few pairs: one hidden unit per lane instead of one pair.  Lane 16 q + j keeps unit j's three
+// parameters (and b2), and the four rows of 16 lanes take the pairs q, q + 4, ...: the units'
+// contributions to y are summed within the row by four rotations.  A row of lanes that holds pairs
+// instead leaves most lanes idle when there are few (a tree of 2^22 keys has about 20 leaves per
+// segment), and pays for the broadcast and the reduction of all 49 parameters in every step.
+constexpr uint32_t UNIT_MAX_PAIRS = 128;
+static_assert(MLP_HIDDEN == 16 && WAVE == 64, "a row of lanes per pair, four rows");
+struct UnitParams {
+  float w1, b1, w2, b2;
+};
+struct UnitGrad {
+  float w1, b1, w2, b2;
+};
+
+// Sum over the 16 lanes of a row, in every one of them.
+STM_DEV float row_sum(float v) {
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x128, 0xF, 0xF, true));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x124, 0xF, 0xF, true));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x122, 0xF, 0xF, true));
+  v += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(v), 0x121, 0xF, 0xF, true));
+  return v;
+}
+
+// One pair per row of lanes: adds its gradient to the lane's, returns its loss (in every lane).
+STM_DEV float unit_accumulate(const UnitParams& p, float x, float t, float scale, UnitGrad& g) {
+  const float z = p.w1 * x + p.b1;
+  const float h = fmaxf(z, 0.0f);
+  const float e = row_sum(p.w2 * h) + p.b2 - t;
+  const float dy = e * scale;
+  const float dz = z > 0.0f ? dy * p.w2 : 0.0f;
+  g.b2 += dy;
+  g.w2 += dy * h;
+  g.w1 += dz * x;
+  g.b1 += dz;
+  return 0.5f * e * e * scale;
+}
+
+// The four rows' gradients summed: row 0 gets w1's, row 1 b1's, row 2 w2's, row 3 b2's; so lane L
+// holds that of parameter min(L, 48), in the order of SegModel::p.
+STM_DEV float unit_reduce(const UnitGrad& g) {
+  const bool up32 = (lane_id() & 32) != 0, up16 = (lane_id() & 16) != 0;
+  const float a = (up32 ? g.w2 : g.w1) + __shfl_xor(up32 ? g.w1 : g.w2, 32, WAVE);
+  const float b = (up32 ? g.b2 : g.b1) + __shfl_xor(up32 ? g.b1 : g.b2, 32, WAVE);
+  return (up16 ? b : a) + __shfl_xor(up16 ? a : b, 16, WAVE);
+}
+
+// The lane's unit from the parameters by lane (lane L holds parameter min(L, 48)).
+STM_DEV UnitParams unit_params(float pv) {
+  const int j = lane_id() & 15;
+  return UnitParams{__shfl(pv, j, WAVE), __shfl(pv, 16 + j, WAVE), __shfl(pv, 32 + j, WAVE),
+                    __shfl(pv, 48, WAVE)};
+}
+
 constexpr int TRAIN_WAVES = 4;
 constexpr int TRAIN_CACHE = 8;  // pairs per lane kept in registers
 constexpr uint32_t TRAIN_MAX_PAIRS = WAVE * TRAIN_CACHE;  // 512 pairs per segment and step
 
-// One wavefront per segment: full-batch Adam for `steps` steps.  Lane L owns parameter
-// param_of_lane(L): its Adam moments and its value; the forward and backward passes read the
-// parameters as wave-uniform values.
+// b^n.
+STM_DEV double power(double b, uint32_t n) {
+  double r = 1.0;
+  for (; n; n >>= 1, b *= b)
+    if (n & 1u) r *= b;
+  return r;
+}
+
+// What Adam's steps base .. base + 63 do not compute from gradients, step base + L in lane L: the
+// learning rate over 1 - beta1^t and 1 / (1 - beta2^t).
+constexpr float ADAM_B1 = 0.9f, ADAM_B2 = 0.999f, ADAM_EPS = 1e-8f;
+struct AdamSchedule {
+  float lr1, c2;
+};
+STM_DEV AdamSchedule adam_schedule(uint32_t base, uint32_t steps, float lr) {
+  const uint32_t it = base + (uint32_t)lane_id();
+  const double rate = (double)lr * (1.0 - 0.9 * (double)it / (double)steps);
+  return AdamSchedule{(float)(rate / (1.0 - power((double)ADAM_B1, it + 1))),
+                      (float)(1.0 / (1.0 - power((double)ADAM_B2, it + 1)))};
+}
+STM_DEV float lane_value(float v, uint32_t lane) {
+  return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), (int)lane));
+}
+
+// Adam's moments of one parameter; step returns its new value.
+struct Adam {
+  float am = 0.0f, av = 0.0f;
+  STM_DEV float step(float p, float g, const AdamSchedule& sched, uint32_t r) {
+    am = ADAM_B1 * am + (1.0f - ADAM_B1) * g;
+    av = ADAM_B2 * av + (1.0f - ADAM_B2) * g * g;
+    return p - lane_value(sched.lr1, r) * am / (sqrtf(av * lane_value(sched.c2, r)) + ADAM_EPS);
+  }
+};
+
+// Training of a segment of cnt (wave-uniform) leaves, at most UNIT_MAX_PAIRS, by one wavefront, a
+// hidden unit per lane.  s_x: UNIT_MAX_PAIRS words of the wavefront's own.
+STM_DEV void train_units(SegModel& m, uint32_t cnt, const uint64_t* __restrict__ fences,
+                         uint32_t steps, float lr, float* s_x) {
+  const uint32_t lane = (uint32_t)lane_id();
+  const uint32_t q = lane / 16;
+  const float scale = 1.0f / (float)cnt;
+  for (uint32_t i = lane; i < UNIT_MAX_PAIRS; i += WAVE)
+    s_x[i] = i < cnt ? seg_x(m, fences[m.r0 + i]) : 0.0f;
+  __builtin_amdgcn_s_waitcnt(0);
+  __builtin_amdgcn_wave_barrier();
+  float pv = m.p[min(lane, (uint32_t)MLP_PARAMS - 1)];
+  Adam adam;
+  for (uint32_t base = 0; base < steps; base += WAVE) {
+    const AdamSchedule sched = adam_schedule(base, steps, lr);
+    const uint32_t here = min(steps - base, (uint32_t)WAVE);
+    for (uint32_t r = 0; r < here; ++r) {
+      const UnitParams p = unit_params(pv);
+      UnitGrad g{0.0f, 0.0f, 0.0f, 0.0f};
+      const float* x = s_x + q;
+      float fi = (float)q;
+#pragma unroll 4
+      for (uint32_t k = cnt / 4; k > 0; --k) {
+        unit_accumulate(p, *x, fi * scale, scale, g);
+        x += 4;
+        fi += 4.0f;
+      }
+      // The last pairs: a row without one adds nothing.
+      if (cnt % 4) unit_accumulate(p, *x, fi * scale, q < cnt % 4 ? scale : 0.0f, g);
+      pv = adam.step(pv, unit_reduce(g), sched, r);
+    }
+  }
+  if (lane < (uint32_t)MLP_PARAMS) m.p[lane] = pv;
+}
+
+// One wavefront per segment: full-batch Adam for `steps` steps.  Up to UNIT_MAX_PAIRS pairs a lane
+// owns a hidden unit (train_units), above it lane L owns parameter param_of_lane(L), its Adam
+// moments and its value, and the forward and backward passes read the parameters as wave-uniform
+// values.  Bound by instruction issue: 4096 wavefronts are one per SIMD slot of four, and a step
+// costs about 450 instructions plus 150 per 64 pairs with a pair per lane, 120 plus 18 per four
+// pairs with a unit per lane (the same at some 130 pairs).  Cold build of 2^22 keys (21 pairs per
+// segment, 300 steps): 992 / 374 µs.
 __global__ __launch_bounds__(TRAIN_WAVES * WAVE) void k_route_train(
     const RouteHeader* __restrict__ rh, const uint64_t* __restrict__ fences,
     SegModel* __restrict__ segs, uint32_t steps, float lr, uint32_t salt) {
+  __shared__ float s_x[TRAIN_WAVES][UNIT_MAX_PAIRS];
   const int wave = threadIdx.x / WAVE;
   const int lane = lane_id();
   const uint32_t s = blockIdx.x * TRAIN_WAVES + wave;
   if (s >= rh->S) return;  // whole wavefront leaves together
   SegModel& m = segs[s];
-  const uint32_t cnt = m.cnt;
+  const uint32_t cnt = uniform32(m.cnt);
   if (cnt < 2 || m.inv_w == 0.0f) return;
+  if (cnt <= UNIT_MAX_PAIRS) {
+    train_units(m, cnt, fences, steps, lr, s_x[wave]);
+    return;
+  }
   const int own = param_of_lane(lane);
   const bool owner = own < MLP_PARAMS;
   float pv = owner ? m.p[own] : 0.0f;
-  float am = 0.0f, av = 0.0f;  // Adam moments of the owned parameter
+  Adam adam;
   const float inv_n = 1.0f / (float)cnt;
-  const float beta1 = 0.9f, beta2 = 0.999f, eps = 1e-8f;
-  float b1t = 1.0f, b2t = 1.0f;
   // The training pairs sit in registers for all steps.  A segment of at most TRAIN_MAX_PAIRS
   // leaves trains on all of them; a larger one (the linear root leaves dense key ranges with
   // several times the mean) on every span-th pair, from an offset that differs between builds
@@ -417,22 +547,21 @@ __global__ __launch_bounds__(TRAIN_WAVES * WAVE) void k_route_train(
     xc[c] = j < used ? seg_x(m, fences[m.r0 + i]) : 0.0f;
     tc[c] = (float)i * inv_n;
   }
-  for (uint32_t it = 0; it < steps; ++it) {
-    float p[MLP_PARAMS];
-    broadcast_params(pv, p);
-    float g[MLP_PARAMS];
+  for (uint32_t base = 0; base < steps; base += WAVE) {
+    const AdamSchedule sched = adam_schedule(base, steps, lr);
+    const uint32_t here = min(steps - base, (uint32_t)WAVE);
+    for (uint32_t r = 0; r < here; ++r) {
+      float p[MLP_PARAMS];
+      broadcast_params(pv, p);
+      float g[MLP_PARAMS];
 #pragma unroll
-    for (int q = 0; q < MLP_PARAMS; ++q) g[q] = 0.0f;
+      for (int q = 0; q < MLP_PARAMS; ++q) g[q] = 0.0f;
 #pragma unroll
-    for (int c = 0; c < TRAIN_CACHE; ++c)
-      if ((uint32_t)lane + (uint32_t)c * WAVE < used) mlp_accumulate(p, xc[c], tc[c], scale, g);
-    const float gr = wave_reduce_scatter(g);
-    b1t *= beta1;
-    b2t *= beta2;
-    am = beta1 * am + (1.0f - beta1) * gr;
-    av = beta2 * av + (1.0f - beta2) * gr * gr;
-    const float step_lr = lr * (1.0f - 0.9f * (float)it / (float)steps);
-    if (owner) pv = pv - step_lr * (am / (1.0f - b1t)) / (sqrtf(av / (1.0f - b2t)) + eps);
+      for (int c = 0; c < TRAIN_CACHE; ++c)
+        if ((uint32_t)lane + (uint32_t)c * WAVE < used) mlp_accumulate(p, xc[c], tc[c], scale, g);
+      const float moved = adam.step(pv, wave_reduce_scatter(g), sched, r);
+      if (owner) pv = moved;
+    }
   }
   if (owner) m.p[own] = pv;
 }
@@ -441,13 +570,28 @@ __global__ __launch_bounds__(TRAIN_WAVES * WAVE) void k_route_train(
 __global__ __launch_bounds__(WAVE) void k_mlp_grad(const float* __restrict__ x, const float* __restrict__ t,
                                                    uint32_t n, const float* __restrict__ params,
                                                    float* __restrict__ grad, float* __restrict__ loss) {
+  const float inv_n = n ? 1.0f / (float)n : 0.0f;
+  float l = 0.0f;
+  if (n <= UNIT_MAX_PAIRS) {  // as in training
+    const uint32_t lane = (uint32_t)lane_id(), q = lane / 16;
+    const UnitParams up = unit_params(params[min(lane, (uint32_t)MLP_PARAMS - 1)]);
+    UnitGrad ug{0.0f, 0.0f, 0.0f, 0.0f};
+    for (uint32_t i = q; i - q < n; i += 4) {
+      const uint32_t ic = min(i, n - 1);
+      l += unit_accumulate(up, x[ic], t[ic], i < n ? inv_n : 0.0f, ug);
+    }
+    const float gr = unit_reduce(ug);
+    if (lane < (uint32_t)MLP_PARAMS) grad[lane] = gr;
+    l += __shfl_xor(l, 16, WAVE);
+    l += __shfl_xor(l, 32, WAVE);
+    if (lane == 0) *loss = l;
+    return;
+  }
   const int own = param_of_lane(lane_id());
   float p[MLP_PARAMS];
   broadcast_params(own < MLP_PARAMS ? params[own] : 0.0f, p);
   float g[MLP_PARAMS];
   for (int q = 0; q < MLP_PARAMS; ++q) g[q] = 0.0f;
-  float l = 0.0f;
-  const float inv_n = n ? 1.0f / (float)n : 0.0f;
   for (uint32_t i = lane_id(); i < n; i += WAVE) l += mlp_accumulate(p, x[i], t[i], inv_n, g);
   const float gr = wave_reduce_scatter(g);
   if (own < MLP_PARAMS) grad[own] = gr;

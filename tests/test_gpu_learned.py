@@ -25,6 +25,25 @@ def test_mlp_gradients_match_cpu():
         assert abs(loss - want_loss) <= 2e-5 * max(want_loss, 1e-6) + 1e-7
 
 
+@pytest.mark.parametrize("n", [2, 3, 4, 5, 16, 17, 127, 128, 129])
+def test_mlp_gradients_of_few_pairs(n):
+    """Up to 128 pairs a lane computes one hidden unit instead of one pair: the rows' remainders and
+    both sides of that limit, against float64 with the same tolerance as above."""
+    import eirene_amd as ea
+    from oracle import mlp
+    rng = np.random.default_rng(n)
+    for _ in range(4):
+        p = rng.normal(0, 1, size=49).astype(np.float32)
+        x = rng.uniform(0, 1, size=n).astype(np.float32)
+        t = np.sort(rng.uniform(0, 1, size=n)).astype(np.float32)
+        loss, g = ea.mlp_gradients(x, t, p)
+        want_loss, want_g = mlp.loss_and_grad(p.astype(np.float64), x.astype(np.float64),
+                                              t.astype(np.float64))
+        scale = max(np.abs(want_g).max(), 1e-3)
+        np.testing.assert_allclose(g, want_g, rtol=0, atol=2e-5 * scale + 1e-7)
+        assert abs(loss - want_loss) <= 2e-5 * max(want_loss, 1e-6) + 1e-7
+
+
 def gamma_tree(ea, w, n, seed, **kw):
     load = w.gamma_keys(n, seed, 2.0, 2.0 ** 56)
     vals = w.values_for(load)
