@@ -240,9 +240,10 @@ struct stm_tree {
   hipEvent_t ev_back[2] = {};   // the set's latest batch done (its scratch is free)
   uint64_t overlap_batches = 0;  // batches seen that could have overlapped
   hipGraphExec_t graphs[GRAPH_CLASSES] = {};
-  // Batches above 2^18 ops sort normalized keys unless exact_left > 0: a batch whose normalized
-  // sort had to fall back (long buckets of distinct keys: hot keys with neighbours) makes the
-  // next EXACT_HOLD batches use the eight exact passes directly.  A smaller batch is sorted by the
+  // Batches above 2^18 ops outside the sample sort's sizes sort normalized keys unless exact_left > 0:
+  // a batch whose normalized sort had to fall back (long buckets of distinct keys: hot keys with
+  // neighbours) makes the next EXACT_HOLD batches use the eight exact passes directly.  (A sample
+  // that misled says nothing of the next batch.)  A batch up to 2^18 ops is sorted by the
   // front half's own sort unless front_hold > 0: one that overflowed a bucket there makes the next
   // EXACT_HOLD of them use the exact passes too (launched, not replayed: the captured graphs hold
   // the front half's sort).
@@ -663,7 +664,8 @@ int run_chunk(stm_tree* t, const uint64_t* keys, const uint64_t* vals, const uin
   }
   const bool small = n <= FRONT_MAX_OPS;
   uint32_t& hold = small ? t->front_hold : t->exact_left;
-  bool exact = hold > 0;
+  const bool sampled = sample_sorted(n);
+  bool exact = hold > 0 && !sampled;
   BatchCounters bc;
   for (;;) {
     HIP_TRY(enqueue_pipeline(t, s, in, true, exact));
@@ -681,7 +683,7 @@ int run_chunk(stm_tree* t, const uint64_t* keys, const uint64_t* vals, const uin
   phase_collect(t);
   if (bc.sort_stall) return fail(STM_ERR_DEVICE, "batch sort: a grid-barrier wait gave up");
   if (bc.sort_fallback) {
-    t->exact_left = EXACT_HOLD;
+    if (!sampled) t->exact_left = EXACT_HOLD;
     t->sort_fallbacks += 1;
   } else if (exact) {
     hold -= 1;
@@ -818,7 +820,11 @@ int run_descs(stm_tree* t, const std::vector<BatchDesc>& descs, const std::vecto
   auto replayed = [&](size_t i) {
     return descs[i].n <= GRAPH_MAX_OPS && t->graphs[cls[i]] && !exact_small;
   };
-  for (size_t i = at; i < descs.size(); ++i) t->overlap_batches += descs[i].n >= OVERLAP_MIN_OPS;
+  bool normalized = false;  // batches whose sort may fall back for what the next ones hold too
+  for (size_t i = at; i < descs.size(); ++i) {
+    t->overlap_batches += descs[i].n >= OVERLAP_MIN_OPS;
+    normalized |= descs[i].n > FRONT_MAX_OPS && !sample_sorted(descs[i].n);
+  }
   const bool overlap = t->overlap_batches >= OVERLAP_BATCHES;
   if (overlap && (rc = ensure_pipeline(t))) return rc;
   hipStream_t sf = t->stream_front;
@@ -846,7 +852,7 @@ int run_descs(stm_tree* t, const std::vector<BatchDesc>& descs, const std::vecto
       } else {
         const PipeIn in{d.keys, d.vals, d.ops, d.n, d.out_vals, d.out_found, nullptr,
                         false, nullptr, nullptr, 0, nullptr, s.acc};
-        const bool exact = d.n <= FRONT_MAX_OPS ? exact_small : exact_large;
+        const bool exact = d.n <= FRONT_MAX_OPS ? exact_small : exact_large && !sample_sorted(d.n);
         if (!overlap || d.n < OVERLAP_MIN_OPS) {
           HIP_TRY(enqueue_front(t, s, in, false, exact, st));
           HIP_TRY(enqueue_back(t, s, in, false));
@@ -883,7 +889,7 @@ int run_descs(stm_tree* t, const std::vector<BatchDesc>& descs, const std::vecto
   t->st.unique_ops += acc.unique;
   t->sort_fallbacks += acc.fallbacks;
   t->splits_since_train += acc.leaf_splits;
-  if (acc.fallbacks) t->exact_left = EXACT_HOLD;
+  if (acc.fallbacks && normalized) t->exact_left = EXACT_HOLD;
   else if (exact_large) t->exact_left -= (uint32_t)std::min<uint64_t>(t->exact_left, acc.batches);
   if (exact_small) t->front_hold -= (uint32_t)std::min<uint64_t>(t->front_hold, acc.batches);
   if (acc.sort_stalls)

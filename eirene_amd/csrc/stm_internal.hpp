@@ -66,6 +66,25 @@ hipError_t radix_sort_pairs_desc(const uint64_t* keys_in, const uint8_t* ops_in,
 // the next sort on the same scratch starts.
 const uint32_t* sort_exact_word(const uint32_t* words);
 
+// ------------------------------------------------------------------ sample sort (stm_sample.hip)
+// The sort of full 64-bit keys between these sizes, called by the radix entry points.  Below, the
+// normalized radix form stays: there a hot key with neighbours still shows in sort_fallbacks, which
+// callers of those sizes watch, and the difference is smallest (30 µs of a 2^19-op call).  Above, a
+// tile of FT * 16 keys per workgroup no longer covers the batch with TILES_MAX tiles.
+constexpr uint32_t SAMPLE_SORT_MIN = (3u << 17) + 1;
+constexpr uint32_t SAMPLE_SORT_MAX = 1u << 22;
+inline bool sample_sorted(uint64_t n) { return n >= SAMPLE_SORT_MIN && n <= SAMPLE_SORT_MAX; }
+struct SampleControl {
+  uint32_t* words;    // sample_sort_words(n) of scratch, 8-byte aligned
+  uint32_t* need;     // set to 1 when the batch is to be sorted by the exact passes, else 0
+  uint32_t* stall;    // words of the exact passes, cleared
+  uint32_t* barrier;
+};
+size_t sample_sort_words(uint64_t n);
+hipError_t sample_sort(const uint64_t* keys, const uint8_t* ops, uint32_t n, uint64_t* tmp_keys,
+                       uint32_t* tmp_ties, uint64_t* keys_out, uint32_t* idx_out,
+                       const SampleControl& ctl, uint8_t* found, hipStream_t stream);
+
 // ------------------------------------------------------------------ per-key fold (stm_fold.hip)
 // Per-batch counters written by the fold and the tree kernels (one 64-byte block).
 struct BatchCounters {

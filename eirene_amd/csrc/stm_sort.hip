@@ -16,7 +16,8 @@
 //               digit order (keys, then payloads, through one buffer), then coalesced runs
 //               to global memory.
 // Batches of at most FRONT_MAX_OPS ops are sorted elsewhere (stm_front.hip): a dozen launches of
-// a few microseconds each would set their time.
+// a few microseconds each would set their time.  From SAMPLE_SORT_MIN to SAMPLE_SORT_MAX keys the
+// sample sort of stm_sample.hip takes the place of the normalized form, with k_sort_exact behind it.
 //
 // The element count and the input keys can come from a device-side batch descriptor, and the
 // grids are sized for the largest batch, so one launch sequence (and one captured hipGraph)
@@ -746,7 +747,8 @@ size_t sort_hist_words(uint64_t n) {
   // the histogram region, sized for the smallest tile (the most tiles)
   uint64_t ntiles = (n + sort_tile(8) - 1) / sort_tile(8);
   if (ntiles == 0) ntiles = 1;
-  return (size_t)CTL_WORDS + (size_t)ntiles * RADIX + RADIX;
+  return (size_t)CTL_WORDS + std::max((size_t)ntiles * RADIX + RADIX,
+                                      sample_sort_words(std::min<uint64_t>(n, SAMPLE_SORT_MAX)));
 }
 
 hipError_t sort_scratch_init(uint32_t* words) {
@@ -839,6 +841,19 @@ static hipError_t sort_passes(const uint64_t* keys_in, const uint8_t* ops_in, co
     return hipGetLastError();
   }
   if (passes > MAX_PASSES) return hipErrorInvalidValue;
+  // The sample sort reads its count and arrays on the host (no descriptor).
+  if (!exact && !desc && begin_bit == 0 && end_bit == 64 && sample_sorted(n_host)) {
+    uint32_t xgrid = 0;
+    hipError_t e = exact_grid<ITEMS>(xgrid);
+    if (e != hipSuccess) return e;
+    const SampleControl ctl{words + CTL_WORDS, words + CTL_NEED_EXACT, words + CTL_STALL,
+                            words + CTL_BARRIER};
+    e = sample_sort(keys_in, ops_in, n_host, keys_tmp, idx_tmp, keys_out, idx_out, ctl, found, stream);
+    if (e != hipSuccess) return e;
+    k_sort_exact<ITEMS><<<xgrid, SORT_BLOCK, 0, stream>>>(keys_in, ops_in, nullptr, n_host, keys_tmp,
+                                                         keys_out, idx_tmp, idx_out, words, stride);
+    return hipGetLastError();
+  }
   if (!exact && begin_bit == 0 && end_bit == 64)
     return sort_normalized<ITEMS>(keys_in, ops_in, desc, n_host, n_max, keys_tmp, keys_out,
                                   idx_tmp, idx_out, words, found, stream);

@@ -124,10 +124,11 @@ typedef struct stm_stats {
                                  routing after leaf splits; the reference's leaf traversal steps,
                                  src/gpu-stm-tree-v38/bpt-gpustm.cpp:142-160) */
     uint64_t sort_fallbacks;  /* batches sorted a second time with the exact passes: above 2^18
-                                 ops, one whose normalized keys met a long run of close, distinct
-                                 keys (hot keys with neighbours); up to there, one whose keys
-                                 misled the sample its buckets are cut by.  The next 16 such
-                                 batches then sort exactly at once */
+                                 and up to 3 * 2^17 ops, and above 2^22, one whose normalized keys
+                                 met a long run of close, distinct keys (hot keys with neighbours);
+                                 at the other sizes, one whose keys misled the sample its buckets
+                                 are cut by.  The next 16 such batches then sort exactly at once,
+                                 but for those between 3 * 2^17 and 2^22 ops */
 } stm_stats;
 
 typedef struct stm_tree stm_tree;
