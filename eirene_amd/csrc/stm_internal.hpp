@@ -193,7 +193,7 @@ struct ScanArgs {
   const int32_t* lastins;
   BatchCounters* counters;
   // scratch
-  uint64_t* soff;       // per input position: output offset, then pair count
+  uint64_t* soff;       // per input position: output offset, and pair count above it
   uint64_t* tile_sums;  // scan_tile_words(n)
 };
 size_t scan_tile_words(uint64_t n);

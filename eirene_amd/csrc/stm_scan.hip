@@ -9,7 +9,8 @@
 // SCAN(k, L) at input position i returns the first L pairs (x, v) with x >= k in the state
 // before op i.  That state is the tree before the batch plus the batch's inserts at input
 // positions < i.  Scans therefore run after the per-key fold and before the upsert kernel:
-//   * the tree part is read from the unmodified pre-batch tree (leaf, then right siblings);
+//   * the tree part is read from the unmodified pre-batch tree (leaf, then right siblings; where the
+//     batch inserts nothing, the leaves a level-1 node lists, without the merge);
 //   * the batch part is read from the fold's output, one group per unique key in key order:
 //     a group contributes key x iff its first insert precedes i; its value is the latest
 //     insert of x before i, found by a binary search over the group's input positions
@@ -37,12 +38,15 @@ constexpr int OFF_TILE = OFF_BLOCK * OFF_ITEMS;
 constexpr uint32_t OFF_SUM_TILES = 1024;
 constexpr uint32_t SCAN_GRID_CAP = 2048;
 // Wavefronts that share the scans of one 64-op window: at least SCAN_SPLIT, and up to one per scan
-// while the batch is too short to give the device SCAN_WAVES wavefronts otherwise.  A scan is a
-// chain of dependent leaf reads, so a window holding several scans sets the kernel's time when
-// few wavefronts run them all (4099 ops, half of them scans of 500..8000 pairs: 3.91 ms a call
-// with four wavefronts per window and no load ahead, 0.41 ms now).
+// while the batch is too short to give the device SCAN_WAVES wavefronts otherwise; a batch still
+// shorter (below 8192 ops) gives every scan SCAN_PARTS of them.  A scan is a chain of round trips, so
+// a window holding several scans, or one long scan, sets the kernel's time when few wavefronts run
+// them.  4099 ops, half of them scans of 500..8000 pairs, µs a call: 3910 with four wavefronts per window
+// and the sibling links, 317 with a wavefront per scan, 196 with whole nodes at a time (scan_plain),
+// 157 with four wavefronts per scan.
 constexpr uint32_t SCAN_SPLIT = 4;
 constexpr uint32_t SCAN_WAVES = 8192;
+constexpr uint32_t SCAN_PARTS = 4;
 constexpr uint32_t SCAN_ROUND_CAP = 1u << 24;
 
 STM_DEV uint64_t scan_len(uint8_t op, uint64_t v) {
@@ -205,35 +209,72 @@ STM_DEV uint32_t lanes_below(uint64_t v, uint32_t n, uint64_t x) {
 
 STM_DEV uint64_t mask_below(uint32_t r) { return r >= 64 ? ~0ull : ((1ull << r) - 1); }
 
-// The leaf that holds key, by a root-to-leaf descent (each level one round trip: a node's keys and
-// children are loaded together).
+// The children of a level-1 node: child j * WAVE + lane and its separator in id[j], sep[j].
 template <int F>
-STM_DEV uint32_t wave_find_leaf(const TreeView& t, uint64_t key) {
-  constexpr int SPL = (F + WAVE - 1) / WAVE;
+struct Kids {
+  static constexpr int SPL = (F + WAVE - 1) / WAVE;
+  uint64_t sep[SPL];
+  uint32_t id[SPL];
+  uint32_t n;     // children
+  uint32_t at;    // the one the scan goes on with
+  uint32_t up;    // the level-1 node after this one (NODE_NONE: none)
+  uint64_t high;  // the node's high fence
+};
+
+// Element at (uniform, below F) of a lane-distributed array.
+template <int F>
+STM_DEV uint32_t lane_at(const uint32_t (&x)[(F + WAVE - 1) / WAVE], uint32_t at) {
+  uint32_t r = 0;
+#pragma unroll
+  for (int j = 0; j < (F + WAVE - 1) / WAVE; ++j)
+    if ((at >> 6) == (uint32_t)j) r = (uint32_t)__builtin_amdgcn_readlane((int)x[j], (int)(at & 63));
+  return r;
+}
+
+template <int F>
+STM_DEV void load_kids(const TreeView& t, uint32_t node, Kids<F>& kids) {
+  const int lane = lane_id();
+#pragma unroll
+  for (int j = 0; j < Kids<F>::SPL; ++j) {
+    const uint64_t at = (uint64_t)node * F + (uint32_t)min(j * WAVE + lane, F - 1);
+    kids.sep[j] = t.keys[at];
+    kids.id[j] = (uint32_t)t.vals[at];
+  }
+  const NodeMeta* m = t.meta + node;
+  const uint64_t info = uniform64(m->info), next = uniform64(m->next);
+  kids.high = uniform64(m->high);
+  kids.n = min(meta_count(info), (uint32_t)F);
+  kids.at = 0;
+  kids.up = next < t.capacity ? (uint32_t)next : NODE_NONE;
+}
+
+// The level-1 node whose child kids.at holds key, by a root-to-leaf descent (each level one round
+// trip: a node's keys, children and metadata are loaded together).  A root that is a leaf is its
+// own only child.
+template <int F>
+STM_DEV void wave_find_kids(const TreeView& t, uint64_t key, Kids<F>& kids) {
   const uint32_t cap = t.capacity;
   uint32_t node = (uint32_t)min<uint64_t>(uniform64(t.hdr->root), cap - 1);
   const uint32_t height = (uint32_t)min<uint64_t>(uniform64(t.hdr->height), 64);
   const int lane = lane_id();
-  for (uint32_t lvl = height; lvl > 1; --lvl) {
-    uint64_t k[SPL], v[SPL];
 #pragma unroll
-    for (int j = 0; j < SPL; ++j) {
-      const uint64_t at = (uint64_t)node * F + (uint32_t)min(j * WAVE + lane, F - 1);
-      k[j] = t.keys[at];
-      v[j] = t.vals[at];
-    }
+  for (int j = 0; j < Kids<F>::SPL; ++j) {
+    kids.sep[j] = 0;
+    kids.id[j] = node;
+  }
+  kids.n = 1;
+  kids.at = 0;
+  kids.up = NODE_NONE;
+  kids.high = KEY_EMPTY;
+  for (uint32_t lvl = height; lvl > 1; --lvl) {
+    load_kids<F>(t, node, kids);
     uint32_t cnt = 0;
 #pragma unroll
-    for (int j = 0; j < SPL; ++j)
-      cnt += (uint32_t)__popcll(ballot(j * WAVE + lane < F && k[j] <= key));
-    const uint32_t slot = cnt ? cnt - 1 : 0;
-    uint64_t child = 0;
-#pragma unroll
-    for (int j = 0; j < SPL; ++j)
-      if ((slot >> 6) == (uint32_t)j) child = readlane64(v[j], (int)(slot & 63));
-    node = (uint32_t)min<uint64_t>(child, cap - 1);
+    for (int j = 0; j < Kids<F>::SPL; ++j)
+      cnt += (uint32_t)__popcll(ballot(j * WAVE + lane < F && kids.sep[j] <= key));
+    kids.at = cnt ? cnt - 1 : 0;
+    node = min(lane_at<F>(kids.id, kids.at), cap - 1);
   }
-  return node;
 }
 
 // First of the n ascending keys that is not below x: every lane probes one key of the range per
@@ -254,27 +295,29 @@ STM_DEV uint32_t wave_lower_bound(const uint64_t* __restrict__ keys, uint32_t n,
   return lo + (n ? (uint32_t)__popcll(ballot(at < hi && keys[min(at, n - 1)] < x)) : 0u);
 }
 
-// A leaf on its way into registers: slot j * WAVE + lane of its keys and values, and its right
-// sibling.  Free slots hold KEY_EMPTY, so the entry count need not be known to load it.
+// A leaf in registers: slot j * WAVE + lane of its keys and values.  Free slots hold KEY_EMPTY, so
+// the entry count need not be known to load it.  As loaded, lanes past a leaf of 32 slots hold its
+// last one: a select on a key here would wait for the load (mask_slots does it later).
 template <int F>
 struct LeafLoad {
   static constexpr int SPL = (F + WAVE - 1) / WAVE;
   uint64_t k[SPL], v[SPL];
-  uint64_t next;
 };
 
 template <int F>
 STM_DEV void load_leaf(const TreeView& t, uint32_t leaf, LeafLoad<F>& b) {
   const int lane = lane_id();
-  b.next = t.meta[leaf].next;
 #pragma unroll
   for (int j = 0; j < LeafLoad<F>::SPL; ++j) {
-    const int sl = j * WAVE + lane;
-    const uint64_t at = (uint64_t)leaf * F + (uint32_t)min(sl, F - 1);
-    const uint64_t k = t.keys[at];
+    const uint64_t at = (uint64_t)leaf * F + (uint32_t)min(j * WAVE + lane, F - 1);
+    b.k[j] = t.keys[at];
     b.v[j] = t.vals[at];
-    b.k[j] = sl < F ? k : KEY_EMPTY;
   }
+}
+
+template <int F>
+STM_DEV void mask_slots(LeafLoad<F>& b) {
+  if constexpr (F < WAVE) b.k[0] = lane_id() < F ? b.k[0] : KEY_EMPTY;
 }
 
 // Element p (lane-dependent, p < F) of a leaf held in registers.
@@ -364,21 +407,154 @@ STM_DEV void leaf_in_key_order(LeafLoad<F>& b) {
   for (int j = 0; j < SPL; ++j) b.v[j] = sv[j];
 }
 
-// One scan op, run by the whole wavefront; returns the pairs written.  The leaf chain is walked one
-// leaf ahead: the right sibling's load goes out before the current leaf is ordered and written, so
-// a step costs the longer of the two instead of their sum.  Bound by that chain's latency (about
-// 1 µs a leaf), not by bytes.
+// Leaves of the fast form read in one round trip, and 64-group windows of the batch it looks
+// through for inserts before it gives up.
 template <int F>
+constexpr uint32_t scan_chunk() {
+  return F > WAVE ? 4 : 8;
+}
+constexpr uint32_t SCAN_GROUP_WINDOWS = 4;
+
+// A scan over stretches of the tree into which the batch inserts nothing: a level-1 node's leaves
+// and their entry counts are known at once, so every leaf's place in the output is too, and the
+// leaves are read a chunk at a time (a step along the sibling links, load, order and store, took
+// about 1.9 µs a leaf, whatever was loaded ahead).  Goes on from node to node; returns true when the scan is
+// complete, false when a node's stretch meets an insert (kids.at: the leaf to go on with; first: it
+// is still the leaf of k).  Of PARTS wavefronts that run the scan, the part-th takes every PARTS-th
+// chunk.
+template <int F, uint32_t PARTS>
+STM_DEV bool scan_plain(const TreeView& t, const ScanArgs& a, const ScanIn& in, uint32_t U, uint64_t k,
+                        uint32_t L, uint64_t off, uint32_t part, Kids<F>& kids,
+                        uint32_t& bg, uint32_t& cnt, bool& first) {
+  constexpr int SPL = (F + WAVE - 1) / WAVE;
+  constexpr uint32_t C = scan_chunk<F>();
+  const uint32_t lane = (uint32_t)lane_id();
+  const uint32_t cap = t.capacity;
+  uint32_t turn = part;  // chunks until this wavefront's next one
+  for (uint32_t node = 0; node < cap; ++node) {
+    const uint32_t room = L - cnt;
+    const uint32_t avail = kids.n - kids.at;
+    LeafLoad<F> b[C];
+    auto load_chunk = [&](uint32_t q, uint32_t m) {
+#pragma unroll
+      for (uint32_t e = 0; e < C; ++e)
+        if (q + e < m) load_leaf<F>(t, min(lane_at<F>(kids.id, kids.at + q + e), cap - 1), b[e]);
+    };
+    // In one round trip: the entry counts of the node's leaves, the first chunk (as many leaves as
+    // the scan may take where they are half full), the batch's next groups.
+    uint32_t c[SPL];
+#pragma unroll
+    for (int j = 0; j < SPL; ++j) {
+      const uint32_t at = (uint32_t)(j * WAVE) + lane;
+      const bool v = at >= kids.at && at < kids.n;
+      c[j] = v ? meta_count(t.meta[min(kids.id[j], cap - 1)].info) : 0u;
+    }
+    const uint32_t early = max(min(min(room / (F / 2) + 2, C), avail), 1u);
+    load_chunk(0, turn == 0 ? early : first ? 1u : 0u);  // every wavefront looks at k's own leaf
+    uint64_t gk = bg + lane < U ? a.ukey[bg + lane] : KEY_EMPTY;
+    uint32_t gop = bg + lane < U ? a.uop[bg + lane] : 0u;
+    // Entries before each leaf (from kids.at on), and how many leaves the scan needs.
+    uint32_t start[SPL], sum = 0;
+#pragma unroll
+    for (int j = 0; j < SPL; ++j) {
+      uint32_t x = c[j];
+#pragma unroll
+      for (int o = 1; o < WAVE; o <<= 1) {
+        const uint32_t y = (uint32_t)__shfl_up((int)x, o, WAVE);
+        if (lane >= (uint32_t)o) x += y;
+      }
+      start[j] = sum + x - c[j];
+      sum += (uint32_t)__builtin_amdgcn_readlane((int)x, WAVE - 1);
+    }
+    uint32_t below = 0;  // entries of the first leaf before k
+    if (first) {
+      mask_slots<F>(b[0]);
+#pragma unroll
+      for (int j = 0; j < SPL; ++j) below += (uint32_t)__popcll(ballot(b[0].k[j] < k));
+    }
+    uint32_t m = 0;
+#pragma unroll
+    for (int j = 0; j < SPL; ++j) {
+      const uint32_t at = (uint32_t)(j * WAVE) + lane;
+      m += (uint32_t)__popcll(ballot(at >= kids.at && at < kids.n && start[j] < room + below));
+    }
+    m = max(m, 1u);
+    uint64_t end = kids.high;
+    if (kids.at + m < kids.n) {
+#pragma unroll
+      for (int j = 0; j < SPL; ++j)
+        if (((kids.at + m) >> 6) == (uint32_t)j) end = readlane64(kids.sep[j], (int)((kids.at + m) & 63));
+    }
+    // The groups below the stretch's end: any insert among them ends the fast form.
+    uint32_t gw = bg;
+    for (uint32_t w = 0;; ++w) {
+      const bool inside = gw + lane < U && gk < end;
+      if (ballot(inside && gop == OP_INSERT)) return false;
+      const uint32_t n = (uint32_t)__popcll(ballot(inside));
+      gw += n;
+      if (n < (uint32_t)WAVE) break;
+      if (w + 1 >= SCAN_GROUP_WINDOWS) return false;
+      gk = gw + lane < U ? a.ukey[gw + lane] : KEY_EMPTY;
+      gop = gw + lane < U ? a.uop[gw + lane] : 0u;
+    }
+    uint32_t have = early;  // leaves of the current chunk
+    for (uint32_t q = 0; q < m; q += have) {
+      if (q > 0) have = C;
+      if (turn-- > 0) continue;
+      turn = PARTS - 1;
+      if (q > 0) load_chunk(q, m);
+#pragma unroll
+      for (uint32_t e = 0; e < C; ++e) {
+        if (e < have && q + e < m) {
+          LeafLoad<F>& x = b[e];
+          mask_slots<F>(x);
+          leaf_in_key_order<F>(x);
+          const uint32_t s0 = lane_at<F>(start, kids.at + q + e);
+#pragma unroll
+          for (int j = 0; j < SPL; ++j) {
+            const uint32_t p = s0 + (uint32_t)(j * WAVE) + lane;  // entries from the first leaf's on
+            if (x.k[j] != KEY_EMPTY && p >= below && p - below < room) {
+              in.scan_keys[off + cnt + (p - below)] = x.k[j];
+              in.scan_vals[off + cnt + (p - below)] = x.v[j];
+            }
+          }
+        }
+      }
+    }
+    // Entries of the leaves taken, less those before k.
+    const uint32_t held = (kids.at + m < kids.n ? lane_at<F>(start, kids.at + m) : sum) - below;
+    cnt += min(held, room);
+    kids.at += m;
+    bg = gw;
+    if (cnt >= L) return true;
+    first = false;
+    if (kids.up == NODE_NONE) return true;
+    load_kids<F>(t, kids.up, kids);
+  }
+  return true;
+}
+
+// One scan op, run by the whole wavefront; returns the pairs written.  Where the batch inserts into
+// its range the leaf chain is walked along the sibling links instead, merged with the batch.
+template <int F, uint32_t PARTS>
 STM_DEV uint32_t run_scan(const TreeView& t, const ScanArgs& a, const ScanIn& in, uint32_t U,
-                          uint64_t k, uint32_t i, uint32_t L, uint64_t off) {
+                          uint64_t k, uint32_t i, uint32_t L, uint64_t off, uint32_t part) {
   const int lane = lane_id();
   const uint32_t cap = t.capacity;
   constexpr int SPL = (F + WAVE - 1) / WAVE;
-  LeafLoad<F> cur, ahead;
-  load_leaf<F>(t, wave_find_leaf<F>(t, k), cur);
+  Kids<F> kids;
+  wave_find_kids<F>(t, k, kids);
   // First group with key >= k (groups are in ascending key order).
-  uint32_t bg = wave_lower_bound(a.ukey, U, k);
+  uint32_t bg = uniform32(wave_lower_bound(a.ukey, U, k));
   uint32_t cnt = 0;
+  bool first = true;
+  if (scan_plain<F, PARTS>(t, a, in, U, k, L, off, part, kids, bg, cnt, first) || part > 0)
+    return cnt;
+  LeafLoad<F> cur, ahead;
+  uint64_t cur_next, ahead_next = NODE_NONE;
+  const uint32_t leaf0 = min(lane_at<F>(kids.id, kids.at), cap - 1);
+  load_leaf<F>(t, leaf0, cur);
+  cur_next = t.meta[leaf0].next;
   uint32_t tl = NODE_NONE;  // the next leaf of the chain, NODE_NONE at its end
   bool loaded = false;      // `ahead` holds it
   uint32_t ts = 0, tcount = 0;  // key-order positions [ts, tcount) of cur are left
@@ -386,7 +562,8 @@ STM_DEV uint32_t run_scan(const TreeView& t, const ScanArgs& a, const ScanIn& in
   // Makes the leaf in `cur` current: its entries into key order, its right sibling under way when
   // the scan will go past it.
   auto enter = [&](uint64_t from) {
-    const uint64_t nx = uniform64(cur.next);
+    mask_slots<F>(cur);
+    const uint64_t nx = uniform64(cur_next);
     tl = nx < cap ? (uint32_t)nx : NODE_NONE;
     tcount = 0;
     ts = 0;
@@ -396,10 +573,13 @@ STM_DEV uint32_t run_scan(const TreeView& t, const ScanArgs& a, const ScanIn& in
       ts += (uint32_t)__popcll(ballot(cur.k[j] < from));
     }
     loaded = tl != NODE_NONE && L - cnt > tcount - ts;
-    if (loaded) load_leaf<F>(t, tl, ahead);
+    if (loaded) {
+      load_leaf<F>(t, tl, ahead);
+      ahead_next = t.meta[tl].next;
+    }
     leaf_in_key_order<F>(cur);
   };
-  enter(k);
+  enter(first ? k : 0);
   // The groups [bg, bg + 64) as the scan sees them, loaded when bg moves: key, whether the group
   // inserts before op i, and the value it then holds.
   uint32_t bn = 0, bg_at = NODE_NONE;
@@ -412,8 +592,12 @@ STM_DEV uint32_t run_scan(const TreeView& t, const ScanArgs& a, const ScanIn& in
       if (tl == NODE_NONE || hop >= SCAN_ROUND_CAP) {
         t_done = true;
       } else {
-        if (!loaded) load_leaf<F>(t, tl, ahead);
+        if (!loaded) {
+          load_leaf<F>(t, tl, ahead);
+          ahead_next = t.meta[tl].next;
+        }
         cur = ahead;
+        cur_next = ahead_next;
         enter(0);
       }
     }
@@ -509,8 +693,10 @@ STM_DEV uint32_t run_scan(const TreeView& t, const ScanArgs& a, const ScanIn& in
 }
 
 // One wavefront per window of 64 input positions: the window's scan ops run one after the
-// other, each by the whole wavefront.  soff[i] becomes the pair count of scan op i.
-template <int F>
+// other, each by the whole wavefront.  soff[i] gets the pair count of scan op i in its upper bits
+// (another part's wavefront may read the offset after that; it is below 2^47: 2^30 ops of 2^16 pairs).
+constexpr int SCAN_OFF_BITS = 47;
+template <int F, uint32_t PARTS>
 __global__ __launch_bounds__(256) void k_range_scan(TreeView t, ScanArgs a, uint32_t split) {
   const ScanIn in = scan_in(a);
   const uint32_t U = a.counters->n_unique;
@@ -519,12 +705,13 @@ __global__ __launch_bounds__(256) void k_range_scan(TreeView t, ScanArgs a, uint
   const uint64_t nwaves = (uint64_t)gridDim.x * blockDim.x / WAVE;
   const uint64_t nwin = ((uint64_t)in.n + WAVE - 1) / WAVE;
   const uint64_t lt = lanemask_lt();
-  // Work item p = (window p / split, share p % split): the wavefront runs the scans of the window
-  // whose rank among the window's scans is p % split modulo split, so a window with several scans
+  // Work item p = (window, share, part): the wavefront runs the scans of the window
+  // whose rank among the window's scans is its share modulo split, so a window with several scans
   // spreads them over split wavefronts.
-  for (uint64_t p = wave0; p < nwin * split; p += nwaves) {
-    const uint64_t w = p / split;
-    const uint32_t share = (uint32_t)(p % split);
+  for (uint64_t p = wave0; p < nwin * split * PARTS; p += nwaves) {
+    const uint32_t part = (uint32_t)(p % PARTS);
+    const uint64_t w = p / PARTS / split;
+    const uint32_t share = (uint32_t)(p / PARTS % split);
     const uint64_t i_l = w * WAVE + lane;
     const bool is_scan = i_l < in.n && in.ops[i_l] == OP_RANGE;
     const uint32_t rank = (uint32_t)__popcll(ballot(is_scan) & lt);
@@ -534,7 +721,7 @@ __global__ __launch_bounds__(256) void k_range_scan(TreeView t, ScanArgs a, uint
     if (mine) {
       k_l = in.keys[i_l];
       v_l = in.vals[i_l];
-      off_l = a.soff[i_l];
+      off_l = a.soff[i_l] & ((1ull << SCAN_OFF_BITS) - 1);
     }
     while (todo) {
       const int src = __builtin_ctzll(todo);
@@ -546,11 +733,11 @@ __global__ __launch_bounds__(256) void k_range_scan(TreeView t, ScanArgs a, uint
       uint32_t c = 0;
       const bool ok = L >= 1 && L <= SCAN_MAX_LEN && off + L <= in.scan_cap && k != KEY_EMPTY;
       if (ok) {
-        c = run_scan<F>(t, a, in, U, k, i, (uint32_t)L, off);
-      } else if (lane == 0) {
+        c = run_scan<F, PARTS>(t, a, in, U, k, i, (uint32_t)L, off, part);
+      } else if (lane == 0 && part == 0) {
         atomicAdd(&a.counters->scan_bad, 1u);
       }
-      if (lane == src) a.soff[i_l] = c;
+      if (lane == src && part == 0) a.soff[i_l] = off | ((uint64_t)c << SCAN_OFF_BITS);
     }
   }
 }
@@ -560,7 +747,7 @@ __global__ __launch_bounds__(256) void k_scan_answers(ScanArgs a) {
   const ScanIn in = scan_in(a);
   for (uint64_t i = blockIdx.x * 256ull + threadIdx.x; i < in.n; i += (uint64_t)gridDim.x * 256ull) {
     if (in.ops[i] == OP_RANGE) {
-      const uint64_t c = a.soff[i];
+      const uint64_t c = a.soff[i] >> SCAN_OFF_BITS;
       in.out_vals[i] = c;
       in.out_found[i] = c ? 1 : 0;
     }
@@ -588,9 +775,11 @@ static hipError_t launch_range_scan_f(const TreeView& t, const ScanArgs& a, hipS
   const uint64_t windows = ((uint64_t)a.n + WAVE - 1) / WAVE;
   uint32_t split = SCAN_SPLIT;
   while (split < (uint32_t)WAVE && windows * split < SCAN_WAVES) split *= 2;
-  const uint64_t waves = windows * split;
-  const uint32_t blocks = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((waves + 3) / 4, SCAN_GRID_CAP));
-  k_range_scan<F><<<blocks, 256, 0, s>>>(t, a, split);
+  const bool parts = split == (uint32_t)WAVE && windows * split < SCAN_WAVES;
+  const uint64_t waves = windows * split * (parts ? SCAN_PARTS : 1u);
+  const uint32_t blocks = (uint32_t)std::max<uint64_t>(1, std::min<uint64_t>((waves + 3) / 4, SCAN_WAVES));
+  if (parts) k_range_scan<F, SCAN_PARTS><<<blocks, 256, 0, s>>>(t, a, split);
+  else k_range_scan<F, 1><<<blocks, 256, 0, s>>>(t, a, split);
   return hipGetLastError();
 }
 
