@@ -2062,6 +2062,13 @@ __global__ __launch_bounds__(1024) void k_upsert_long(TreeView t, UpsertArgs a) 
 // through its parent's lock.  Upsert kernels per batch, before / now: 2^22 ops at 95/5 (210 K
 // inserts) 73 / 57 µs; 2^19 ops at 50/50 (262 K inserts, most leaves split) 517 / 99 µs; 2^14 ops
 // at 50/50 beside Zipf-hot keys 830 / 72 µs.
+// Entries of the insert list a wavefront owns at least.  It looks at 64 in any case; owning all of
+// them saves reads where the chip is full, but a wavefront splits its overfull leaves one after the
+// other, some 4 µs each, so lists of up to RUN_SPREAD_OPS are dealt out in parts of RUN_PART.  16
+// batches of 2^14 ops at 50/50 beside Zipf-hot keys, µs: parts of 64 entries 2850, 16 2440, 8 2385; lists of 2^18 in parts of 32 gained nothing.  A list of
+// up to 64 stays with one wavefront (1000-op call with 50 inserts 30.0 µs, dealt out 30.3).
+constexpr uint32_t RUN_PART = 8;
+constexpr uint32_t RUN_SPREAD_OPS = 1u << 16;
 template <int F>
 STM_DEV void leaf_runs(const TreeView& t, const UpsertArgs& a, uint64_t* __restrict__ out_vals,
                        uint8_t* __restrict__ out_found) {
@@ -2082,7 +2089,7 @@ STM_DEV void leaf_runs(const TreeView& t, const UpsertArgs& a, uint64_t* __restr
     fanout_answers(a.fanout, a.fanout_cap, cnt, a.gstart, a.npend, a.gval, sidx, out_vals, out_found);
   const uint32_t nw = gridDim.x * (blockDim.x / WAVE);
   const uint32_t w = uniform32((blockIdx.x * blockDim.x + threadIdx.x) / WAVE);
-  const uint32_t per = max((N + nw - 1) / nw, (uint32_t)WAVE);
+  const uint32_t per = max((N + nw - 1) / nw, N > (uint32_t)WAVE && N <= RUN_SPREAD_OPS ? RUN_PART : (uint32_t)WAVE);
   const uint32_t e0 = (uint32_t)min<uint64_t>((uint64_t)w * per, N);
   const uint32_t e1 = min(e0 + per, N);
   const uint32_t lane = (uint32_t)lane_id();
@@ -2723,8 +2730,9 @@ hipError_t launch_lookup(const TreeView& t, const LookupArgs& a, hipStream_t s) 
 
 template <int F>
 static hipError_t launch_upsert_f(const TreeView& t, const UpsertArgs& a, hipStream_t s) {
-  // Each wavefront takes an equal contiguous share of the merged INSERTs, at least 64 of them: a
-  // grid of at most the wavefronts the chip holds at once works through them in one generation.
+  // Each wavefront takes an equal contiguous share of the merged INSERTs, at least 64 of them (8 of
+  // a short list): a grid of at most the wavefronts the chip holds at once works through them in one
+  // generation.
   static std::atomic<int> resident{0};  // blocks of this instantiation the device holds at once
   if (resident.load(std::memory_order_relaxed) == 0) {
     int dev = 0, cus = 0, per_cu = 0;
@@ -2736,7 +2744,7 @@ static hipError_t launch_upsert_f(const TreeView& t, const UpsertArgs& a, hipStr
     resident.store(std::max(1, cus * per_cu), std::memory_order_relaxed);
   }
   const uint32_t blocks = std::min<uint32_t>(
-      std::min<uint32_t>((uint32_t)((a.n_max + 255) / 256), (uint32_t)resident.load(std::memory_order_relaxed)),
+      std::min<uint32_t>((uint32_t)((a.n_max + 63) / 64), (uint32_t)resident.load(std::memory_order_relaxed)),
       RUN_WAVES_MAX / 4);
   const uint32_t waves = blocks * 4;  // one rfirst / rcount entry per wavefront
   const bool runs_only = a.piece >= (uint32_t)WAVE;
