@@ -13,8 +13,9 @@
 // Buckets are cut between samples of (key, position), so the ops of a hot key are shared by as many
 // buckets as they fill and no normalization is needed.  A bucket holds 1024 elements in the mean
 // (2048 above 2^21); one with more than BUCKET_CAP is taken in groups of the eight intervals between
-// its own samples.  Only an interval (an eighth of a bucket in the mean) of more than BUCKET_CAP
-// elements, at most about once in 500 batches of the largest size, asks for the exact sort.
+// its own samples, and an interval (an eighth of a bucket in the mean) that holds more, as happens
+// about once in 500 batches of the largest size, in halves of its key range.  Only a half that
+// is still too large, which takes keys built to mislead the sample, asks for the exact sort.
 //
 // Bound by the round trips of a workgroup (k_sample_pick: 4 to 16 workgroups on the chip;
 // k_sample_bucket: about 13 µs of row words, elements and barriers per bucket, two buckets on a CU) and,
@@ -384,11 +385,40 @@ __global__ __launch_bounds__(FT, 8) void k_sample_bucket(uint32_t n, uint32_t ti
     }
     __syncthreads();
   }
+  // An interval of its own that is too large is cut once more, between its bounds.
+  uint32_t half = 0, upper = 0;  // half 1, 2: the pass takes the elements below (mk, mt), the others
+  uint64_t mk = 0;
+  uint32_t mt = 0;
 #pragma unroll 1
-  for (uint32_t i0 = 0, i1; i0 < PER_BUCKET; i0 = i1) {
+  for (uint32_t i0 = 0, i1; i0 < PER_BUCKET; i0 = half == 1 ? i0 : i1) {
     uint32_t gm = one ? m : uniform32(s_sub[i0]);
     i1 = one ? PER_BUCKET : i0 + 1;
-    while (i1 < PER_BUCKET && gm + uniform32(s_sub[i1]) <= BUCKET_CAP) gm += uniform32(s_sub[i1++]);
+    if (half == 1) {
+      half = 2;
+      gm = upper;
+    } else {
+      half = 0;
+      while (i1 < PER_BUCKET && gm + uniform32(s_sub[i1]) <= BUCKET_CAP) gm += uniform32(s_sub[i1++]);
+      if (gm > BUCKET_CAP && !(b == 0 && i0 == 0) && !(b + 1 == B && i1 == PER_BUCKET)) {
+        const uint64_t k0 = uniform64(bk[i0]), k1 = uniform64(bk[i1]);
+        const uint32_t t0 = uniform32(bt[i0]), t1 = uniform32(bt[i1]);
+        mk = k0 + (k1 - k0) / 2;
+        mt = k0 == k1 ? t0 + (t1 - t0) / 2 : 0u;
+        __syncthreads();
+        if (tid == 0) s_fill = 0;
+        __syncthreads();
+        for (uint32_t i = tid; i < m; i += FT) {
+          const uint32_t src = source(i);
+          const uint64_t key = tmp_keys[src];
+          const uint32_t t = tmp_ties[src];
+          if (interval(key, t) == i0 && elem_less(key, t, mk, mt)) atomicAdd(&s_fill, 1u);
+        }
+        __syncthreads();
+        half = 1;
+        upper = gm - uniform32(s_fill);
+        gm -= upper;
+      }
+    }
     const uint32_t out = start;
     start += gm;
     if (gm == 0) continue;
@@ -425,7 +455,7 @@ __global__ __launch_bounds__(FT, 8) void k_sample_bucket(uint32_t n, uint32_t ti
         const uint64_t key = tmp_keys[src];
         const uint32_t t = tmp_ties[src];
         const uint32_t v = interval(key, t);
-        if (v >= i0 && v < i1) {
+        if (v >= i0 && v < i1 && (half == 0 || elem_less(key, t, mk, mt) == (half == 1))) {
           const uint32_t to = atomicAdd(&s_fill, 1u);
           s_k[to] = key;
           s_p[to] = t;
@@ -449,6 +479,10 @@ __global__ __launch_bounds__(FT, 8) void k_sample_bucket(uint32_t n, uint32_t ti
       khi = uniform64(bk[end]);
       tlo = uniform32(bt[i0]);
       thi = uniform32(bt[end]);
+      if (half) {
+        if (klo == khi) (half == 1 ? thi : tlo) = mt;
+        else (half == 1 ? khi : klo) = mk;
+      }
     }
     if (last || (b == 0 && i0 == 0)) {
       uint64_t mn = KEY_EMPTY, mx = 0;

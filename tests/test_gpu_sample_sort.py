@@ -27,13 +27,13 @@ def sample_positions(n):
     return (lo + ((x * (hi - lo)) >> np.uint64(32))).astype(np.int64)
 
 
-def crafted(n, rng, width):
-    """Evenly spread samples; 12000 of the other keys within `width` intervals from the 800th on."""
+def crafted(n, rng, width, many=12000):
+    """Evenly spread samples; `many` of the other keys within `width` intervals from the 800th on."""
     s = samples_of(n)
     keys = rng.integers(0, s << 40, n, dtype=np.uint64)
     at = sample_positions(n)
     rest = np.setdiff1d(np.arange(n), at)
-    dense = rng.choice(rest, 12000, replace=False)
+    dense = rng.choice(rest, many, replace=False)
     keys[dense] = np.uint64(800 << 40) + rng.integers(0, width << 40, dense.size, dtype=np.uint64)
     keys[at] = rng.permutation(s).astype(np.uint64) << np.uint64(40)
     return keys
@@ -98,3 +98,35 @@ def test_batches_count_the_exact_sort(oracle_mod, dist, fallbacks):
         ek, ev = o.dump()
         assert np.array_equal(k, ek) and np.array_equal(v, ev)
         assert t.check() == 0
+
+
+@pytest.mark.parametrize("n", [400000, MAX])
+@pytest.mark.parametrize("equal", [False, True])
+def test_one_large_interval_is_halved(n, equal):
+    """6000 keys between two samples, spread or all equal to the lower one: no exact sort, checked by
+    its results alone where the keys go through sort_pairs."""
+    from eirene_amd import sort_pairs
+    rng = np.random.default_rng(n + equal)
+    keys = crafted(n, rng, 1, 6000)
+    if equal:
+        inside = (keys >= np.uint64(800 << 40)) & (keys < np.uint64(801 << 40))
+        keys[inside] = np.uint64(800 << 40)
+    got_k, got_i = sort_pairs(keys)
+    want = np.argsort(keys, kind="stable")
+    assert np.array_equal(got_i, want.astype(np.uint32))
+    assert np.array_equal(got_k, keys[want])
+
+
+def test_one_large_interval_needs_no_exact_sort(oracle_mod):
+    from eirene_amd import StmConfig, StmTree
+    rng = np.random.default_rng(4)
+    n = 400000
+    keys = crafted(n, rng, 1, 6000)
+    vals = rng.integers(0, 1 << 63, n, dtype=np.uint64)
+    ops = (rng.random(n) < 0.5).astype(np.uint8)
+    o = oracle_mod.Oracle()
+    want = o.run_batch(keys, vals, ops)
+    with StmTree(StmConfig(max_keys=1 << 20, max_batch=1 << 19)) as t:
+        got = t.run_batch(keys, vals, ops)
+        assert np.array_equal(got[0], want[0]) and np.array_equal(got[1], want[1])
+        assert t.stats()["sort_fallbacks"] == 0
