@@ -54,8 +54,9 @@ hipError_t radix_sort_pairs(const uint64_t* keys_in, uint64_t* keys_tmp, uint64_
 // without it keys_in holds n_max keys.
 // found (the descriptor's out_found with desc; null: none) is set to 1 throughout on the way: the
 // answers' default.
-// The normalized-key form runs unless `exact` asks for the eight-pass form (the library asks for
-// it after a batch whose normalized sort had to fall back).
+// Full 64-bit keys without desc go through the sample sort at its sizes, else through the
+// normalized-key form, unless `exact` asks for the eight-pass form (the library asks for it after a
+// batch whose normalized sort had to fall back).
 hipError_t radix_sort_pairs_desc(const uint64_t* keys_in, const uint8_t* ops_in,
                                  const BatchDesc* desc, uint32_t n_max,
                                  uint64_t* keys_tmp, uint64_t* keys_out, uint32_t* idx_tmp,

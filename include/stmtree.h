@@ -73,7 +73,9 @@ typedef struct stm_config {
     uint32_t retrain_every; /* learned routing: rebuild + retrain after this many batches (default 8) */
     uint32_t train_steps; /* learned routing: Adam steps per segment MLP (default 300) */
     uint32_t sort_tile_items; /* radix sort elements per thread: 8 or 16 (tiles of 2048 or 4096
-                                 keys; default 16); 8 up to 3 * 2^19 keys in any case */
+                                 keys; default 16); 8 up to 3 * 2^19 keys in any case.  Batches
+                                 of up to 2^18 and of 3 * 2^17 + 1 .. 2^22 ops use it only where
+                                 they are sorted a second time (stm_stats.sort_fallbacks) */
     uint32_t use_graphs;  /* stm_run_batches_device: 1 = the host reads nothing back until the
                              stream ends, and small size classes replay a hipGraph when
                              stm_capture_graphs made one (default 1); 0 = one synchronous call per
