@@ -14,13 +14,16 @@
 #include <cstdarg>
 #include <cstdio>
 #include <cstring>
+#include <memory>
 #include <mutex>
+#include <new>
 #include <string>
 #include <vector>
 
 #include "../../include/stmtree.h"
 #include "stm_common.hpp"
 #include "stm_internal.hpp"
+#include "stm_pairs.hpp"
 #include "stm_tree.hpp"
 
 using namespace stm;
@@ -1412,6 +1415,8 @@ int stm_run_batch_scan(stm_tree* t, const uint64_t* keys, const uint64_t* vals, 
   // Scan lengths: checked here, and each chunk's output area sized from them.
   const uint64_t mb = t->cfg.max_batch;
   std::vector<uint64_t> chunk_pairs;
+  std::vector<ScanOp> scans;
+  std::vector<size_t> chunk_scans{0};  // a chunk's scan ops begin here in `scans`
   uint64_t total = 0;
   for (size_t off = 0; off < n; off += mb) {
     const size_t m = (size_t)std::min<uint64_t>(mb, n - off);
@@ -1422,8 +1427,10 @@ int stm_run_batch_scan(stm_tree* t, const uint64_t* keys, const uint64_t* vals, 
         return fail(STM_ERR_INVALID, "scan op %zu has length %llu, not in [1, %u]", i,
                     (unsigned long long)vals[i], STM_SCAN_MAX_LEN);
       c += vals[i];
+      scans.push_back(ScanOp{i, vals[i]});
     }
     chunk_pairs.push_back(c);
+    chunk_scans.push_back(scans.size());
     total += c;
   }
   if (total > scan_cap)
@@ -1437,6 +1444,7 @@ int stm_run_batch_scan(stm_tree* t, const uint64_t* keys, const uint64_t* vals, 
     return fail(STM_ERR_NOMEM, "scan output area of %llu pairs", (unsigned long long)most);
   }
   Scratch& s = t->scr;
+  std::unique_ptr<uint64_t[]> part;  // the area on the host, where scans left slots unwritten
   uint64_t base = 0;
   size_t ci = 0;
   for (size_t off = 0; off < n && rc == STM_OK; off += mb, ++ci) {
@@ -1454,9 +1462,32 @@ int stm_run_batch_scan(stm_tree* t, const uint64_t* keys, const uint64_t* vals, 
     const uint64_t c = chunk_pairs[ci];
     e = hipMemcpyAsync(out_vals + off, s.out_vals, m * 8, hipMemcpyDeviceToHost, t->stream);
     if (e == hipSuccess) e = hipMemcpyAsync(out_found + off, s.out_found, m, hipMemcpyDeviceToHost, t->stream);
-    if (e == hipSuccess && c) e = hipMemcpyAsync(scan_keys + base, dsk, c * 8, hipMemcpyDeviceToHost, t->stream);
-    if (e == hipSuccess && c) e = hipMemcpyAsync(scan_vals + base, dsv, c * 8, hipMemcpyDeviceToHost, t->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(t->stream);
+    if (e == hipSuccess && c) {
+      // The caller's slots past a scan's pairs stay as they are: straight into the caller's arrays
+      // only when every slot was written.
+      const ScanOp* sc = scans.data() + chunk_scans[ci];
+      const size_t nsc = chunk_scans[ci + 1] - chunk_scans[ci];
+      uint64_t wrote = 0;
+      for (size_t q = 0; q < nsc; ++q) wrote += out_vals[sc[q].op];
+      const bool whole = wrote == c;
+      if (!whole && !part) part.reset(new (std::nothrow) uint64_t[most]);
+      if (!whole && !part) {
+        rc = fail(STM_ERR_NOMEM, "host copy of %llu scan pairs", (unsigned long long)most);
+        break;
+      }
+      const uint64_t* from[] = {dsk, dsv};
+      uint64_t* to[] = {scan_keys + base, scan_vals + base};
+      for (int k = 0; k < 2 && e == hipSuccess; ++k) {
+        e = hipMemcpyAsync(whole ? to[k] : part.get(), from[k], c * 8, hipMemcpyDeviceToHost, t->stream);
+        if (e != hipSuccess || whole) continue;
+        if ((e = hipStreamSynchronize(t->stream)) != hipSuccess) continue;
+        written_pairs(sc, nsc, out_vals, [&](uint64_t at, uint64_t pairs) {
+          std::memcpy(to[k] + at, part.get() + at, pairs * 8);
+        });
+      }
+      if (e == hipSuccess) e = hipStreamSynchronize(t->stream);
+    }
     if (e != hipSuccess) rc = fail(STM_ERR_DEVICE, "result copy: %s", hipGetErrorString(e));
     base += c;
   }

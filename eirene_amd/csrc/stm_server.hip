@@ -17,8 +17,8 @@
 //              forming), copies it to HBM on its own stream, runs it as one batch (scan mode
 //              when it holds scans) and queues the answer copies on a third stream.
 //   completer  waits for a slot's answers, scatters them into the requests' buffers (split
-//              over helper threads for large slots), marks the requests done and returns the
-//              slot.
+//              over helper threads for large slots; of a scan's slots only those it wrote),
+//              marks the requests done and returns the slot.
 // Requests of one batch are concatenated in admission order, and batches run in order, so
 // every request sees exactly the state it would see if the requests ran one by one in
 // admission order: a result is the same alone and in the mix.
@@ -42,6 +42,7 @@
 #include <vector>
 
 #include "../../include/stmtree.h"
+#include "stm_pairs.hpp"
 
 namespace {
 
@@ -159,7 +160,7 @@ struct Req {
   uint64_t* scan_keys = nullptr;
   uint64_t* scan_vals = nullptr;
   uint64_t pairs = 0;  // sum of its scan lengths
-  uint64_t scans = 0;
+  std::vector<stm::ScanOp> scans;
   double t_arrival = 0, t_admit = 0, t_done = 0;
   uint64_t off = 0, poff = 0;  // place in its slot (ops, scan pairs)
   int status = STM_OK;
@@ -241,7 +242,7 @@ struct stm_server {
       r->poff = s->pairs;
       s->n += r->n;
       s->pairs += r->pairs;
-      s->scans += r->scans;
+      s->scans += r->scans.size();
       s->copies += 1;
       r->t_admit = now_s();
       s->reqs.push_back(r);
@@ -364,10 +365,11 @@ struct stm_server {
             Req* r = s->reqs[i];
             std::memcpy(r->out_vals, s->h_ovals + r->off, r->n * 8);
             std::memcpy(r->out_found, s->h_ofound + r->off, r->n);
-            if (r->pairs) {
-              std::memcpy(r->scan_keys, s->h_skeys + r->poff, r->pairs * 8);
-              std::memcpy(r->scan_vals, s->h_svals + r->poff, r->pairs * 8);
-            }
+            stm::written_pairs(r->scans.data(), r->scans.size(), r->out_vals,
+                               [&](uint64_t at, uint64_t m) {
+                                 std::memcpy(r->scan_keys + at, s->h_skeys + r->poff + at, m * 8);
+                                 std::memcpy(r->scan_vals + at, s->h_svals + r->poff + at, m * 8);
+                               });
           }
         };
         if (k == 1) scatter(0);
@@ -384,7 +386,7 @@ struct stm_server {
           r->done = true;
           st_requests += 1;
           st_ops += r->n;
-          st_scans += r->scans;
+          st_scans += r->scans.size();
           st_pairs += r->pairs;
           outstanding -= 1;
         }
@@ -562,7 +564,8 @@ int stm_server_submit(stm_server* s, const uint64_t* keys, const uint64_t* vals,
   *ticket = 0;
   if (n == 0) return sfail(STM_ERR_INVALID, "empty request");
   if (!keys || !vals || !ops || !out_vals || !out_found) return sfail(STM_ERR_INVALID, "null array");
-  uint64_t pairs = 0, scans = 0;
+  uint64_t pairs = 0;
+  std::vector<stm::ScanOp> scans;
   for (size_t i = 0; i < n; ++i) {
     if (keys[i] == STM_KEY_RESERVED)
       return sfail(STM_ERR_INVALID, "op %zu uses the reserved key 0xffffffffffffffff", i);
@@ -572,7 +575,7 @@ int stm_server_submit(stm_server* s, const uint64_t* keys, const uint64_t* vals,
         return sfail(STM_ERR_INVALID, "scan op %zu has length %llu, not in [1, %u]", i,
                      (unsigned long long)vals[i], STM_SCAN_MAX_LEN);
       pairs += vals[i];
-      scans += 1;
+      scans.push_back(stm::ScanOp{i, vals[i]});
     }
   }
   if (pairs > scan_cap || (pairs && (!scan_keys || !scan_vals)))
@@ -592,7 +595,7 @@ int stm_server_submit(stm_server* s, const uint64_t* keys, const uint64_t* vals,
   r->scan_keys = scan_keys;
   r->scan_vals = scan_vals;
   r->pairs = pairs;
-  r->scans = scans;
+  r->scans = std::move(scans);
   r->t_arrival = arrival_s >= 0 ? arrival_s : now_s();
   std::vector<std::pair<Slot*, Req*>> adm;
   {
