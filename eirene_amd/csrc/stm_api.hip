@@ -239,6 +239,7 @@ struct stm_tree {
   Scratch scr2;
   bool scr2_alloc = false;
   hipStream_t stream_front = nullptr;
+  hipEvent_t ev_open = nullptr;  // what was queued on `stream` before the stream of batches
   hipEvent_t ev_front[2] = {};  // front half of the set's latest batch done
   hipEvent_t ev_back[2] = {};   // the set's latest batch done (its scratch is free)
   uint64_t overlap_batches = 0;  // batches seen that could have overlapped
@@ -755,6 +756,7 @@ int ensure_pipeline(stm_tree* t) {
   hipError_t e = t->scr2.alloc(t->cfg.max_batch, Scratch::STREAM);
   if (e == hipSuccess && !t->stream_front)
     e = stream_beside(t->stream, reinterpret_cast<uint32_t*>(t->scr2.counters), &t->stream_front);
+  if (e == hipSuccess && !t->ev_open) e = hipEventCreateWithFlags(&t->ev_open, hipEventDisableTiming);
   for (int k = 0; k < 2 && e == hipSuccess; ++k) {
     if (!t->ev_front[k]) e = hipEventCreateWithFlags(&t->ev_front[k], hipEventDisableTiming);
     if (e == hipSuccess && !t->ev_back[k])
@@ -811,9 +813,11 @@ int capture_class(stm_tree* t, int c) {
 //     the back half on the tree's stream once its front half is done (against one stream: 2^16 ops
 //     69 / 79 µs, 2^18 109 / 129, 2^20 252 / 268, 2^22 657 / 669).
 // Back halves run in batch order on one stream, so each sees the tree after the previous batch; the
-// learned router retrains on that stream between them.
-int run_descs(stm_tree* t, const std::vector<BatchDesc>& descs, const std::vector<uint8_t>& cls,
-              size_t at, size_t& ran) {
+// learned router retrains on that stream between them.  The first front half starts after
+// whatever the caller had queued on the tree's stream: a copy into the batches' arrays, or out of
+// the answers'.
+int enqueue_descs(stm_tree* t, const std::vector<BatchDesc>& descs, const std::vector<uint8_t>& cls,
+                  size_t at, size_t& ran) {
   Scratch& s = t->scr;
   hipStream_t st = t->stream;
   ran = 0;
@@ -833,6 +837,10 @@ int run_descs(stm_tree* t, const std::vector<BatchDesc>& descs, const std::vecto
   hipStream_t sf = t->stream_front;
   bool used[2] = {false, false};  // ev_back[k] marks the end of the set's latest batch
   HIP_TRY(hipMemsetAsync(s.acc, 0, sizeof(StreamAcc), st));
+  if (overlap) {
+    HIP_TRY(hipEventRecord(t->ev_open, st));
+    HIP_TRY(hipStreamWaitEvent(sf, t->ev_open, 0));
+  }
   std::vector<BatchDesc> table;
   int k = 0;  // the scratch set of the latest batch
   for (size_t w0 = at; w0 < descs.size(); w0 += DESC_TABLE) {
@@ -906,6 +914,18 @@ int run_descs(stm_tree* t, const std::vector<BatchDesc>& descs, const std::vecto
     char buf[64];
     snprintf(buf, sizeof(buf), " (%llu later batches skipped)", acc.skipped);
     g_last_error += buf;
+  }
+  return rc;
+}
+
+// enqueue_descs; after an error both streams are idle, as after success: what they still ran uses
+// the scratch sets and the caller's arrays.
+int run_descs(stm_tree* t, const std::vector<BatchDesc>& descs, const std::vector<uint8_t>& cls,
+              size_t at, size_t& ran) {
+  const int rc = enqueue_descs(t, descs, cls, at, ran);
+  if (rc != STM_OK) {
+    (void)hipStreamSynchronize(t->stream);
+    if (t->stream_front) (void)hipStreamSynchronize(t->stream_front);
   }
   return rc;
 }
@@ -1244,6 +1264,7 @@ int stm_destroy(stm_tree* t) {
   drop_graphs(t);
   t->scr.release();
   if (t->scr2_alloc) t->scr2.release();
+  if (t->ev_open) (void)hipEventDestroy(t->ev_open);
   for (int k = 0; k < 2; ++k) {
     if (t->ev_front[k]) (void)hipEventDestroy(t->ev_front[k]);
     if (t->ev_back[k]) (void)hipEventDestroy(t->ev_back[k]);

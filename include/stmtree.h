@@ -257,7 +257,10 @@ int stm_check(stm_tree* tree, uint64_t* bad);
 int stm_get_stats(stm_tree* tree, stm_stats* out);
 int stm_reset_stats(stm_tree* tree);
 
-/* The hipStream_t every kernel of this tree runs on. */
+/* The tree's hipStream_t.  Every call's kernels and copies start after what is queued on it when
+ * the call is made.  They run on it, but for the sorts and folds of a batch stream, which run on a
+ * second stream of the library's own beside it, by the same rule; both are done when the call
+ * returns. */
 int stm_get_stream(stm_tree* tree, void** stream);
 
 /* Learned routing (no reference counterpart; the reference always descends from the root).
