@@ -817,7 +817,7 @@ int capture_class(stm_tree* t, int c) {
 // whatever the caller had queued on the tree's stream: a copy into the batches' arrays, or out of
 // the answers'.
 int enqueue_descs(stm_tree* t, const std::vector<BatchDesc>& descs, const std::vector<uint8_t>& cls,
-                  size_t at, size_t& ran) {
+                  size_t at, size_t& ran, std::vector<BatchDesc>& table, StreamAcc& acc) {
   Scratch& s = t->scr;
   hipStream_t st = t->stream;
   ran = 0;
@@ -828,7 +828,9 @@ int enqueue_descs(stm_tree* t, const std::vector<BatchDesc>& descs, const std::v
     return descs[i].n <= GRAPH_MAX_OPS && t->graphs[cls[i]] && !exact_small;
   };
   bool normalized = false;  // batches whose sort may fall back for what the next ones hold too
+  size_t replays = 0;
   for (size_t i = at; i < descs.size(); ++i) {
+    replays += replayed(i);
     t->overlap_batches += descs[i].n >= OVERLAP_MIN_OPS;
     normalized |= descs[i].n > FRONT_MAX_OPS && !sample_sorted(descs[i].n);
   }
@@ -841,16 +843,18 @@ int enqueue_descs(stm_tree* t, const std::vector<BatchDesc>& descs, const std::v
     HIP_TRY(hipEventRecord(t->ev_open, st));
     HIP_TRY(hipStreamWaitEvent(sf, t->ev_open, 0));
   }
-  std::vector<BatchDesc> table;
+  // The replayed batches' descriptors, window after window: a queued copy may still read those of
+  // an earlier window.
+  table.reserve(replays);
   int k = 0;  // the scratch set of the latest batch
   for (size_t w0 = at; w0 < descs.size(); w0 += DESC_TABLE) {
     const size_t w1 = std::min<size_t>(descs.size(), w0 + DESC_TABLE);
-    table.clear();
+    const size_t first = table.size();
     for (size_t i = w0; i < w1; ++i)
       if (replayed(i)) table.push_back(descs[i]);
-    if (!table.empty()) {
-      HIP_TRY(hipMemcpyAsync(s.desc_table, table.data(), table.size() * sizeof(BatchDesc),
-                             hipMemcpyHostToDevice, st));
+    if (table.size() > first) {
+      HIP_TRY(hipMemcpyAsync(s.desc_table, table.data() + first,
+                             (table.size() - first) * sizeof(BatchDesc), hipMemcpyHostToDevice, st));
       HIP_TRY(hipMemsetAsync(s.cursor, 0, sizeof(uint32_t), st));
     }
     for (size_t i = w0; i < w1; ++i) {
@@ -888,7 +892,6 @@ int enqueue_descs(stm_tree* t, const std::vector<BatchDesc>& descs, const std::v
       t->batches_since_train += 1;
     }
   }
-  StreamAcc acc;
   HIP_TRY(hipMemcpyAsync(&acc, s.acc, sizeof(acc), hipMemcpyDeviceToHost, st));
   HIP_TRY(hipStreamSynchronize(st));
   ran = (size_t)acc.batches;
@@ -919,10 +922,12 @@ int enqueue_descs(stm_tree* t, const std::vector<BatchDesc>& descs, const std::v
 }
 
 // enqueue_descs; after an error both streams are idle, as after success: what they still ran uses
-// the scratch sets and the caller's arrays.
+// the scratch sets, the caller's arrays and the two copies' host memory here.
 int run_descs(stm_tree* t, const std::vector<BatchDesc>& descs, const std::vector<uint8_t>& cls,
               size_t at, size_t& ran) {
-  const int rc = enqueue_descs(t, descs, cls, at, ran);
+  std::vector<BatchDesc> table;
+  StreamAcc acc;
+  const int rc = enqueue_descs(t, descs, cls, at, ran, table, acc);
   if (rc != STM_OK) {
     (void)hipStreamSynchronize(t->stream);
     if (t->stream_front) (void)hipStreamSynchronize(t->stream_front);
