@@ -243,6 +243,7 @@ struct stm_tree {
   hipEvent_t ev_front[2] = {};  // front half of the set's latest batch done
   hipEvent_t ev_back[2] = {};   // the set's latest batch done (its scratch is free)
   uint64_t overlap_batches = 0;  // batches seen that could have overlapped
+  bool pipeline_failed = false;  // and that nothing of this could be made for
   hipGraphExec_t graphs[GRAPH_CLASSES] = {};
   // Batches above 2^18 ops outside the sample sort's sizes sort normalized keys unless exact_left > 0:
   // a batch whose normalized sort had to fall back (long buckets of distinct keys: hot keys with
@@ -750,9 +751,9 @@ hipError_t stream_beside(hipStream_t beside, uint32_t* words /*2, device*/, hipS
   return e;
 }
 
-// The second scratch set, the front stream and the pipeline's events, made on first use.
-int ensure_pipeline(stm_tree* t) {
-  if (t->scr2_alloc) return STM_OK;
+// The second scratch set, the front stream and the pipeline's events.
+hipError_t make_pipeline(stm_tree* t) {
+  if (t->scr2_alloc) return hipSuccess;
   hipError_t e = t->scr2.alloc(t->cfg.max_batch, Scratch::STREAM);
   if (e == hipSuccess && !t->stream_front)
     e = stream_beside(t->stream, reinterpret_cast<uint32_t*>(t->scr2.counters), &t->stream_front);
@@ -762,12 +763,23 @@ int ensure_pipeline(stm_tree* t) {
     if (e == hipSuccess && !t->ev_back[k])
       e = hipEventCreateWithFlags(&t->ev_back[k], hipEventDisableTiming);
   }
-  if (e != hipSuccess) {
+  if (e == hipSuccess) t->scr2_alloc = true;
+  else {
     t->scr2.release();
-    return fail(STM_ERR_NOMEM, "stream pipeline set-up: %s", hipGetErrorString(e));
+    (void)hipGetLastError();  // or the next launch's check would find it
   }
-  t->scr2_alloc = true;
-  return STM_OK;
+  return e;
+}
+
+// Whether batches may overlap: the pipeline is there (stm_capture_graphs makes it at once), or the
+// tree has seen enough batches for it to pay.  Making it takes 250 µs, and freeing it at the
+// tree's end some 500 at a max_batch of 2^18 and more; a batch then gains 8 µs at 2^18 ops, 10 at
+// 2^20, 15 at 2^22 (lookups on 2^22 keys).  Without the memory for it streams go on as before.
+bool pipeline_ready(stm_tree* t) {
+  if (t->scr2_alloc) return true;
+  if (t->overlap_batches < OVERLAP_BATCHES || t->pipeline_failed) return false;
+  t->pipeline_failed = make_pipeline(t) != hipSuccess;
+  return t->scr2_alloc;
 }
 
 Scratch& slot_scratch(stm_tree* t, int k) { return k ? t->scr2 : t->scr; }
@@ -807,8 +819,8 @@ int capture_class(stm_tree* t, int c) {
 // A batch runs in one of three ways, in order of size:
 //   * a captured graph, where stm_capture_graphs made one for its class;
 //   * both halves launched on the tree's stream: up to 2048 ops, whose front half is one short
-//     kernel (per batch of 2^10 ops 31 µs, 41 with two streams), and while the tree has seen too few
-//     larger batches to pay for the second scratch set and stream;
+//     kernel (per batch of 2^10 ops 31 µs, 41 with two streams), and while there is no second
+//     scratch set and stream (pipeline_ready);
 //   * the front half on stream_front once the back half of the scratch set's previous user is done,
 //     the back half on the tree's stream once its front half is done (against one stream: 2^16 ops
 //     69 / 79 µs, 2^18 109 / 129, 2^20 252 / 268, 2^22 657 / 669).
@@ -828,14 +840,14 @@ int enqueue_descs(stm_tree* t, const std::vector<BatchDesc>& descs, const std::v
     return descs[i].n <= GRAPH_MAX_OPS && t->graphs[cls[i]] && !exact_small;
   };
   bool normalized = false;  // batches whose sort may fall back for what the next ones hold too
-  size_t replays = 0;
+  size_t replays = 0, large = 0;
   for (size_t i = at; i < descs.size(); ++i) {
     replays += replayed(i);
-    t->overlap_batches += descs[i].n >= OVERLAP_MIN_OPS;
+    large += descs[i].n >= OVERLAP_MIN_OPS;
     normalized |= descs[i].n > FRONT_MAX_OPS && !sample_sorted(descs[i].n);
   }
-  const bool overlap = t->overlap_batches >= OVERLAP_BATCHES;
-  if (overlap && (rc = ensure_pipeline(t))) return rc;
+  t->overlap_batches += large;
+  const bool overlap = large > 0 && pipeline_ready(t);
   hipStream_t sf = t->stream_front;
   bool used[2] = {false, false};  // ev_back[k] marks the end of the set's latest batch
   HIP_TRY(hipMemsetAsync(s.acc, 0, sizeof(StreamAcc), st));
@@ -1564,7 +1576,8 @@ int stm_capture_graphs(stm_tree* t) {
     if (rc) return rc;
     if (class_nmax(t, c) == t->cfg.max_batch) break;
   }
-  return ensure_pipeline(t);
+  const hipError_t e = make_pipeline(t);
+  return e == hipSuccess ? STM_OK : fail(STM_ERR_NOMEM, "stream pipeline set-up: %s", hipGetErrorString(e));
 }
 
 int stm_run_batch(stm_tree* t, const uint64_t* keys, const uint64_t* vals, const uint8_t* ops,

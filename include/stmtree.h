@@ -217,9 +217,9 @@ int stm_run_batch_scan_device(stm_tree* tree, const uint64_t* d_keys, const uint
  * until the stream has run (a reserved key or a full node pool is reported at the end, the tree
  * then holds every batch up to and including the failing one; the outputs of the batches after it
  * are unspecified).  Batches above 2048 ops run in two halves on two scratch sets, so batch b + 1's
- * sort and fold run while batch b's lookups and upserts do; the second batch scratch and a second
- * stream are made once the tree's streams have brought 32 such batches (or by
- * stm_capture_graphs).
+ * sort and fold run while batch b's lookups and upserts do, once there is a second batch scratch
+ * and a second stream: stm_capture_graphs makes them, or the first stream after the tree's streams
+ * have brought 32 such batches, if the GPU has the memory (else they stay on one stream).
  * Replaces the batch loop of GPU_STM_Tree::gpu_work_main (src/gpu-stm-tree-v38/bpt-gpustm.cpp:77-135:
  * transferData, launchKernelBefore, launchKernel, launchKernelAfter, transferAns per batch). */
 int stm_run_batches_device(stm_tree* tree, const uint64_t* d_keys, const uint64_t* d_vals,
