@@ -1,5 +1,7 @@
 """Batch streams on a tree for whose second batch scratch the GPU has no memory: they run on one
 stream, as they did before the tree had seen enough batches for two."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -9,7 +11,6 @@ GIB = 1 << 30
 
 
 def test_streams_without_memory_for_the_second_scratch(oracle_mod):
-    import torch
     from eirene_amd import DeviceBuffer, StmError, StmTree
     rng = np.random.default_rng(13)
     load = np.unique(rng.integers(0, 1 << 40, 20000, dtype=np.uint64))
@@ -25,8 +26,9 @@ def test_streams_without_memory_for_the_second_scratch(oracle_mod):
         t.bulk_load(load, load)
         dk, dv, do = (DeviceBuffer.from_array(x) for x in (keys, keys, ops))
         ov, of = DeviceBuffer(n, np.uint64), DeviceBuffer(n, np.uint8)
-        free = torch.cuda.mem_get_info()[0]
-        ballast = torch.empty(max(free - 64 * GIB, 1), dtype=torch.uint8, device="cuda")
+        free, total = C.c_size_t(), C.c_size_t()
+        assert t._lib.hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+        ballast = DeviceBuffer(max(free.value - 64 * GIB, 1), np.uint8)
         for _ in range(2):
             t.run_batches_device(dk, dv, do, ov, of, offsets)
             want = [o.run_batch(keys[a:z], keys[a:z], ops[a:z])
@@ -38,5 +40,4 @@ def test_streams_without_memory_for_the_second_scratch(oracle_mod):
         assert e.value.code == 2
         v, f = t.run_batch(load[:100], load[:100], np.ones(100, np.uint8))
         assert f.all()
-        del ballast
-        torch.cuda.empty_cache()
+        ballast.free()

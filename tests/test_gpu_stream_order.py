@@ -1,28 +1,19 @@
 """A batch stream starts after whatever the caller has queued on the tree's stream, also once its
 sorts run on a second stream: inputs that a queued copy has yet to bring, answers that a queued copy
 has yet to take away."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
 pytestmark = pytest.mark.gpu
 
-
-class Array:
-    """A torch tensor in the place of a DeviceBuffer."""
-
-    def __init__(self, tensor):
-        self.tensor, self.ptr, self.n = tensor, tensor.data_ptr(), tensor.numel()
-
-
-def device(x):
-    import torch
-    return torch.from_numpy(x.view(np.int64) if x.dtype == np.uint64 else x).cuda()
+DEVICE_TO_DEVICE = 3
 
 
 @pytest.mark.parametrize("size", [2049, 40000])
 def test_stream_waits_for_queued_copies(oracle_mod, size):
-    import torch
-    from eirene_amd import StmTree
+    from eirene_amd import DeviceBuffer, StmTree
     rng = np.random.default_rng(size)
     load = np.unique(rng.integers(0, 1 << 50, 60000, dtype=np.uint64))
     n = 4 * size
@@ -43,36 +34,36 @@ def test_stream_waits_for_queued_copies(oracle_mod, size):
 
     with StmTree(max_keys=1 << 20, max_batch=1 << 16) as t:
         t.bulk_load(load, load)
-        stream = torch.cuda.ExternalStream(t.stream())
-        busy = torch.zeros(2, 1 << 28, dtype=torch.uint8, device="cuda")
-        cur = [Array(device(x)) for x in batch()]
-        cur[2].tensor.fill_(1)  # lookups only: they leave the tree as it is
-        out = Array(torch.zeros(n, dtype=torch.int64, device="cuda"))
-        found = Array(torch.zeros(n, dtype=torch.uint8, device="cuda"))
-        torch.cuda.synchronize()
+
+        def queue_copy(dst, src):
+            item = np.dtype(src.dtype).itemsize
+            assert t._lib.hipMemcpyAsync(C.c_void_p(dst.ptr), C.c_void_p(src.ptr),
+                                         C.c_size_t(src.n * item), DEVICE_TO_DEVICE,
+                                         C.c_void_p(t.stream())) == 0
+
+        busy = DeviceBuffer(1 << 28, np.uint8), DeviceBuffer(1 << 28, np.uint8)
+        first = batch()
+        first[2][:] = 1  # lookups only: they leave the tree as it is
+        cur = [DeviceBuffer.from_array(x) for x in first]
+        out = DeviceBuffer(n, np.uint64), DeviceBuffer(n, np.uint8)
         for _ in range(8):  # enough batches for the second stream
-            t.run_batches_device(*cur, out, found, offsets)
+            t.run_batches_device(*cur, *out, offsets)
         before = None
         for _ in range(3):
             b = batch()
-            new = [device(x) for x in b]
-            kept = torch.zeros_like(out.tensor), torch.zeros_like(found.tensor)
-            torch.cuda.synchronize()
-            with torch.cuda.stream(stream):
-                for _ in range(40):  # some milliseconds
-                    busy[0].copy_(busy[1])
-                kept[0].copy_(out.tensor)
-                kept[1].copy_(found.tensor)
-                for a, x in zip(cur, new):
-                    a.tensor.copy_(x)
-            t.run_batches_device(*cur, out, found, offsets)
+            new = [DeviceBuffer.from_array(x) for x in b]
+            kept = DeviceBuffer(n, np.uint64), DeviceBuffer(n, np.uint8)
+            for _ in range(40):  # some milliseconds
+                queue_copy(*busy)
+            for dst, src in list(zip(kept, out)) + list(zip(cur, new)):
+                queue_copy(dst, src)
+            t.run_batches_device(*cur, *out, offsets)
             want = replay(b)
-            got = out.tensor.cpu().numpy().view(np.uint64), found.tensor.cpu().numpy()
-            np.testing.assert_array_equal(got[0], want[0])
-            np.testing.assert_array_equal(got[1], want[1])
+            for x, w in zip(out, want):
+                np.testing.assert_array_equal(x.download(), w)
             if before is not None:
-                np.testing.assert_array_equal(kept[0].cpu().numpy().view(np.uint64), before[0])
-                np.testing.assert_array_equal(kept[1].cpu().numpy(), before[1])
+                for x, w in zip(kept, before):
+                    np.testing.assert_array_equal(x.download(), w)
             before = want
         k, v = t.dump()
         ek, ev = o.dump()
