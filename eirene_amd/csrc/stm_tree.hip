@@ -1393,7 +1393,11 @@ STM_DEV bool run_upsert(const TreeView& t, uint64_t key, uint64_t val, uint32_t 
     const TxResult r = tx_upsert_attempt<F>(t, key, val, found, old, c, pc,
                                             aborts + restarts == 0 ? par_hint : NODE_NONE);
     if (r == TX_DONE) break;
-    if (r == TX_FAIL) return true;  // pool exhausted: error bit raised, op dropped
+    if (r == TX_FAIL) {  // pool exhausted: error bit raised, op dropped, answered as absent
+      found = false;
+      old = 0;
+      break;
+    }
     if (r == TX_ABORT) {
       c.aborts++;
       if (++aborts >= max_attempts) return false;
@@ -1911,7 +1915,7 @@ STM_DEV void long_runs(const TreeView& t, const UpsertArgs& a, uint64_t* __restr
   const uint32_t tid = threadIdx.x;
   const uint32_t wave = uniform32(tid / WAVE);
   TxCounters c;
-  uint32_t upserts = 0, deferred = 0;
+  uint32_t upserts = 0;
   for (uint32_t q = blockIdx.x; q < runs; q += gridDim.x) {
     const uint32_t e0 = uniform32(ld_relaxed32(a.rlist + q)), len = uniform32(ld_relaxed32(a.rlen + q));
     const InsHint h0 = ihint[ilist[e0]];
@@ -1972,8 +1976,15 @@ STM_DEV void long_runs(const TreeView& t, const UpsertArgs& a, uint64_t* __restr
       const uint64_t key = ukey[gi], val = uval[gi];
       uint32_t total;
       const uint32_t idx = block_rank_1024(fresh, s_w, total);
-      if (base == NODE_NONE) {  // the pool is all but full: the serial pass takes the new keys
-        if (fresh) dlist[atomicAdd(&cnt->n_deferred, 1u)] = gi;
+      if (base == NODE_NONE) {  // the pool refused: transactions take the keys past a full leaf
+        const uint32_t at = count + before + idx;
+        if (fresh && at < (uint32_t)F) {
+          t.keys[nb + at] = key;
+          t.vals[nb + at] = val;
+        } else if (fresh) {
+          dlist[atomicAdd(&cnt->n_deferred, 1u)] = gi;
+        }
+        before += total;
         continue;
       }
       if (fresh) s_new[idx] = key;
@@ -1986,18 +1997,16 @@ STM_DEV void long_runs(const TreeView& t, const UpsertArgs& a, uint64_t* __restr
     if (base != NODE_NONE) {
       if (tid < count) spread_entry<F>(t, sp, tid + xr, xk, xv);
       spread_finish<F>(t, sp, 0, count, high, next, wave, BT / WAVE);
+    } else if (tid == 0) {  // (more entries than slots, or no request would have been made)
+      st_relaxed(&t.meta[leaf].info, make_info(F, 0));
     }
     __syncthreads();  // LDS is the next run's
     if (wave == 0) {
-      upserts += len;
+      upserts += base == NODE_NONE ? len - (T - F) : len;
       c.node_reads += len;
       c.commits++;
-      if (base == NODE_NONE) {
-        deferred += news;
-      } else {
-        c.new_keys += news;
-        c.leaf_splits += nl - 1;
-      }
+      c.new_keys += base == NODE_NONE ? F - count : news;
+      if (base != NODE_NONE) c.leaf_splits += nl - 1;
       if (nl > 1 && base != NODE_NONE) {
         uint32_t par = NODE_NONE;
         const uint32_t p = h0.par;
@@ -2018,10 +2027,7 @@ STM_DEV void long_runs(const TreeView& t, const UpsertArgs& a, uint64_t* __restr
   }
   if (wave == 0) {
     flush_counters(t, c, cnt);
-    if (lane_id() == 0) {
-      stat_add(t.stats, ST_UPSERTS, blockIdx.x, upserts);
-      stat_add(t.stats, ST_DEFERRED, blockIdx.x, deferred);
-    }
+    if (lane_id() == 0) stat_add(t.stats, ST_UPSERTS, blockIdx.x, upserts);
   }
 }
 
@@ -2095,7 +2101,7 @@ STM_DEV void leaf_runs(const TreeView& t, const UpsertArgs& a, uint64_t* __restr
   const uint32_t lane = (uint32_t)lane_id();
   const uint64_t lt = lanemask_lt();
   TxCounters c;
-  uint32_t upserts = 0, deferred = 0;
+  uint32_t upserts = 0;
   uint32_t first = NODE_NONE;  // the first run owned
   uint32_t recs = 0;
   uint32_t base = e0;
@@ -2159,23 +2165,28 @@ STM_DEV void leaf_runs(const TreeView& t, const UpsertArgs& a, uint64_t* __restr
       nb0 = at + incl - want;
     }
     const bool splits = mine && ((splitm >> hl) & 1ull);
-    const size_t nb = (size_t)(fits || splits ? leaf : 0u) * F;
+    // A run that the pool refused: what needs no node is done here, up to a full leaf.
+    const bool refused = mine && !fits && !splits && !(badm & run) && piece >= (uint32_t)WAVE;
+    const bool placed = fits || splits || refused;
+    const size_t nb = (size_t)(placed ? leaf : 0u) * F;
+    const uint32_t at = count + (uint32_t)__popcll(newm & lt);  // of a new key
+    const bool answered = fits || splits || (refused && (hfound || at < (uint32_t)F));
     uint64_t old = 0;
-    if (fits || splits) {
+    if (answered) {
       if (hfound) {
         old = t.vals[nb + slot];
         t.vals[nb + slot] = val;
-      } else if (fits) {
-        const uint32_t at = count + (uint32_t)__popcll(newm & lt);
+      } else if (!splits) {
         t.keys[nb + at] = key;
         t.vals[nb + at] = val;
       }
-      if (fits && lane == hl && news) st_relaxed(&t.meta[leaf].info, make_info(count + news, 0));
     }
-    write_upsert_answers(fits || splits, hfound, old, h.gs, h.np, p0, sidx, out_vals, out_found);
-    const uint64_t okm = ballot(fits || splits);
+    if (placed && !splits && lane == hl && news)
+      st_relaxed(&t.meta[leaf].info, make_info(min(count + news, (uint32_t)F), 0));
+    write_upsert_answers(answered, hfound, old, h.gs, h.np, p0, sidx, out_vals, out_found);
+    const uint64_t okm = ballot(answered);
     c.commits += (uint32_t)__popcll(okm & hm);
-    c.new_keys += (uint32_t)__popcll(ballot((fits || splits) && !hfound));
+    c.new_keys += (uint32_t)__popcll(ballot(answered && !hfound));
     c.node_reads += (uint32_t)__popcll(okm);
     upserts += (uint32_t)__popcll(okm);
     if (splitm) {
@@ -2211,16 +2222,14 @@ STM_DEV void leaf_runs(const TreeView& t, const UpsertArgs& a, uint64_t* __restr
     // again (a split here, or by one of the kernels after this one).
     const uint64_t again = ballot(mine && !fits);
     c.aborts += (uint32_t)__popcll(again & hm);
-    const uint64_t leave = ballot(mine && !fits && !splits);
+    const uint64_t leave = ballot(mine && !answered);
     if (piece >= (uint32_t)WAVE) {
-      // Refused by the pool (or a hint out of range): op by op in the serial pass.
+      // Refused by the pool, for want of a node (or a hint out of range): transactions at the end.
       if (leave) {
         uint32_t at = 0;
         if (lane == 0) at = atomicAdd(&cnt->n_deferred, (uint32_t)__popcll(leave));
         at = uniform32(at);
         if ((leave >> lane) & 1ull) dlist[at + (uint32_t)__popcll(leave & lt)] = gi;
-        deferred += (uint32_t)__popcll(leave);
-        upserts += (uint32_t)__popcll(leave);
       }
     } else {
       for (uint64_t lm = leave & hm; lm; lm &= lm - 1) {
@@ -2270,10 +2279,7 @@ STM_DEV void leaf_runs(const TreeView& t, const UpsertArgs& a, uint64_t* __restr
     a.rcount[w] = recs;
   }
   flush_counters(t, c, cnt);
-  if (lane == 0) {
-    stat_add(t.stats, ST_UPSERTS, wave_stripe(), upserts);
-    stat_add(t.stats, ST_DEFERRED, wave_stripe(), deferred);
-  }
+  if (lane == 0) stat_add(t.stats, ST_UPSERTS, wave_stripe(), upserts);
 }
 
 template <int F>
@@ -2282,33 +2288,83 @@ __global__ __launch_bounds__(256) void k_upsert_runs(TreeView t, UpsertArgs a) {
   leaf_runs<F>(t, a, o.vals, o.found);
 }
 
-// Wave-wide transactions for the runs that k_upsert_runs left: many inserts into one leaf.
+// Wave-wide transactions for a round of ops, group gi per lane with `mine`.  Ops of the round whose
+// keys share a leaf commit together (tx_merge_attempt): a hot leaf takes one transaction per round
+// instead of one per op.  Ops that exhaust their attempts go to `later` (*n_later of them).
+template <int F>
+STM_DEV void tx_ops(const TreeView& t, const UpsertArgs& a, uint32_t gi, bool mine,
+                    uint64_t* __restrict__ out_vals, uint8_t* __restrict__ out_found,
+                    uint32_t* later, uint32_t* n_later, TxCounters& c, ParentCache<F>& pc,
+                    uint32_t& upserts, uint32_t& deferred) {
+  // The round's op data, loaded together and read lane by lane.
+  uint64_t todo = ballot(mine);
+  const InsHint h = a.ihint[gi];
+  const uint64_t k_l = a.ukey[gi];
+  const uint64_t v_l = a.uval[gi];
+  const uint32_t gs_l = h.gs, np_l = h.np, par_l = h.par, leaf_l = h.leaf;
+  const uint32_t p0_l = pos_of(a.sidx[gs_l]);
+  while (todo) {
+    const int l = __builtin_ctzll(todo);
+    const uint64_t key = readlane64(k_l, l);
+    const uint32_t ph = __builtin_amdgcn_readlane(par_l, l);
+    const uint32_t lh = __builtin_amdgcn_readlane(leaf_l, l);
+    uint32_t aborts = 0, restarts = 0;
+    uint64_t done = 0;
+    bool found_l = false;
+    uint64_t old_l = 0;
+    bool gave_up = false;
+    for (;;) {
+      // The hint is only tried on the first attempt; retries descend from the root.
+      const bool first = aborts + restarts == 0;
+      const TxResult r = tx_merge_attempt<F>(t, key, todo, k_l, v_l, c, pc,
+                                             first ? ph : NODE_NONE, first ? lh : NODE_NONE,
+                                             done, found_l, old_l);
+      if (r == TX_DONE) break;
+      if (r == TX_FAIL) {  // pool exhausted: error bit raised, the op is dropped
+        done = 1ull << l;
+        found_l = false;
+        old_l = 0;
+        break;
+      }
+      if (r == TX_ABORT) {
+        c.aborts++;
+        if (++aborts >= a.max_attempts) {
+          gave_up = true;
+          break;
+        }
+        backoff(aborts);
+      } else if (++restarts >= 4 * a.max_attempts) {  // TX_RESTART after a preemptive split
+        gave_up = true;
+        break;
+      }
+    }
+    if (gave_up) {  // the op of lane l goes to the serial pass
+      const uint32_t g = __builtin_amdgcn_readlane(gi, l);
+      if (lane_id() == 0)
+        __hip_atomic_store(later + atomicAdd(n_later, 1u), g, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      deferred++;
+      upserts++;
+      todo &= ~(1ull << l);
+      continue;
+    }
+    write_upsert_answers(((done >> lane_id()) & 1ull) != 0, found_l, old_l, gs_l, np_l, p0_l, a.sidx,
+                         out_vals, out_found);
+    upserts += (uint32_t)__popcll(done);
+    todo &= ~done;
+  }
+}
+
+// The runs that k_upsert_runs left for transactions: many inserts into one leaf.
 // Wavefront f of that kernel recorded rcount[f] pieces from index rfirst[f] of rlist / rlen on.
 // With r = nw / run_waves wavefronts here per wavefront there, each takes every r-th of its pieces;
 // with fewer, wavefront w takes all pieces of wavefronts w, w + nw, ...  A piece is the ops of one
 // leaf in key order, so the ops of a round mostly commit in one transaction, and only the parent is
 // shared with other wavefronts (and the leaf, when its run was cut into pieces).
 template <int F>
-__global__ __launch_bounds__(256) void k_upsert(TreeView t, const uint64_t* __restrict__ ukey,
-                                                const uint64_t* __restrict__ uval,
-                                                const uint32_t* __restrict__ sidx,
-                                                const uint32_t* __restrict__ ilist,
-                                                const uint32_t* __restrict__ rlist,
-                                                const uint32_t* __restrict__ rlen,
-                                                const uint32_t* __restrict__ rfirst,
-                                                const uint32_t* __restrict__ rcount,
-                                                uint32_t run_waves,
-                                                const InsHint* __restrict__ ihint,
-                                                BatchCounters* cnt, uint32_t* __restrict__ dlist,
-                                                uint32_t max_attempts,
-                                                uint64_t* __restrict__ out_vals,
-                                                uint8_t* __restrict__ out_found,
-                                                const BatchDesc* __restrict__ desc) {
+__global__ __launch_bounds__(256) void k_upsert(TreeView t, UpsertArgs a, uint32_t run_waves) {
+  BatchCounters* cnt = a.counters;
   if (cnt->n_upserts == 0) return;
-  if (desc) {
-    out_vals = desc->out_vals;
-    out_found = desc->out_found;
-  }
+  const OutArrays o = out_arrays(a);
   const uint32_t nw = gridDim.x * (blockDim.x / WAVE);
   const uint32_t w = uniform32((blockIdx.x * blockDim.x + threadIdx.x) / WAVE);
   const uint32_t r = max(nw / run_waves, 1u);
@@ -2316,78 +2372,18 @@ __global__ __launch_bounds__(256) void k_upsert(TreeView t, const uint64_t* __re
   ParentCache<F> pc;
   uint32_t upserts = 0, deferred = 0;
   for (uint32_t f = w / r; f < run_waves; f += nw / r) {
-  const uint32_t pieces = uniform32(rcount[f]);
-  const uint32_t at = uniform32(rfirst[f]);
-  for (uint32_t q = w % r; q < pieces; q += r) {
-  const uint32_t s0 = uniform32(rlist[at + q]);
-  const uint32_t s1 = s0 + uniform32(rlen[at + q]);
-  for (uint32_t base = s0; base < s1; base += WAVE) {
-    // Op data of the round's upserts, loaded together and read lane by lane.
-    const uint32_t e = base + lane_id();
-    const bool mine = e < s1;
-    const uint32_t gi = ilist[min(e, s1 - 1)];
-    uint64_t todo = ballot(mine);
-    const InsHint h = ihint[gi];
-    const uint64_t k_l = ukey[gi];
-    const uint64_t v_l = uval[gi];
-    const uint32_t gs_l = h.gs, np_l = h.np, par_l = h.par, leaf_l = h.leaf;
-    const uint32_t p0_l = pos_of(sidx[gs_l]);
-    // Ops of the round whose keys share a leaf commit together (tx_merge_attempt): a hot
-    // leaf takes one transaction per round instead of one per op.
-    while (todo) {
-      const int l = __builtin_ctzll(todo);
-      const uint64_t key = readlane64(k_l, l);
-      const uint32_t ph = __builtin_amdgcn_readlane(par_l, l);
-      const uint32_t lh = __builtin_amdgcn_readlane(leaf_l, l);
-      uint32_t aborts = 0, restarts = 0;
-      uint64_t done = 0;
-      bool found_l = false;
-      uint64_t old_l = 0;
-      bool gave_up = false;
-      for (;;) {
-        // The hint is only tried on the first attempt; retries descend from the root.
-        const bool first = aborts + restarts == 0;
-        const TxResult r = tx_merge_attempt<F>(t, key, todo, k_l, v_l, c, pc,
-                                               first ? ph : NODE_NONE, first ? lh : NODE_NONE,
-                                               done, found_l, old_l);
-        if (r == TX_DONE) break;
-        if (r == TX_FAIL) {  // pool exhausted: error bit raised, the op is dropped
-          done = 1ull << l;
-          found_l = false;
-          old_l = 0;
-          break;
-        }
-        if (r == TX_ABORT) {
-          c.aborts++;
-          if (++aborts >= max_attempts) {
-            gave_up = true;
-            break;
-          }
-          backoff(aborts);
-        } else if (++restarts >= 4 * max_attempts) {  // TX_RESTART after a preemptive split
-          gave_up = true;
-          break;
-        }
+    const uint32_t pieces = uniform32(a.rcount[f]);
+    const uint32_t at = uniform32(a.rfirst[f]);
+    for (uint32_t q = w % r; q < pieces; q += r) {
+      const uint32_t s0 = uniform32(a.rlist[at + q]);
+      const uint32_t s1 = s0 + uniform32(a.rlen[at + q]);
+      for (uint32_t base = s0; base < s1; base += WAVE) {
+        const uint32_t e = base + lane_id();
+        tx_ops<F>(t, a, a.ilist[min(e, s1 - 1)], e < s1, o.vals, o.found, a.dlist, &cnt->n_deferred, c,
+                  pc, upserts, deferred);
       }
-      if (gave_up) {  // the op of lane l goes to the serial pass
-        uint32_t slot = 0;
-        if (lane_id() == 0) slot = atomicAdd(&cnt->n_deferred, 1u);
-        slot = uniform32(__shfl(slot, 0, WAVE));
-        const uint32_t g = __builtin_amdgcn_readlane(gi, l);
-        if (lane_id() == 0) dlist[slot] = g;
-        deferred++;
-        upserts++;
-        todo &= ~(1ull << l);
-        continue;
-      }
-      write_upsert_answers(((done >> lane_id()) & 1ull) != 0, found_l, old_l, gs_l, np_l, p0_l, sidx,
-                           out_vals, out_found);
-      upserts += (uint32_t)__popcll(done);
-      todo &= ~done;
     }
   }
-  }  // pieces
-  }  // wavefronts of k_upsert_runs
   flush_counters(t, c, cnt);
   if (lane_id() == 0) {
     stat_add(t.stats, ST_UPSERTS, wave_stripe(), upserts);
@@ -2395,9 +2391,30 @@ __global__ __launch_bounds__(256) void k_upsert(TreeView t, const uint64_t* __re
   }
 }
 
-// Serial pass over the ops that exhausted their attempts or that the all but full pool refused as
-// a run: one wavefront, no competitors,
-// so every transaction commits on its first attempt.
+// The n ops of the runs that the all but full pool refused, in dlist: a wavefront takes 64 at a
+// time (they were listed run by run, so the ops of a leaf are mostly together).
+template <int F>
+STM_DEV void refused_ops(const TreeView& t, const UpsertArgs& a, uint32_t n,
+                         uint64_t* __restrict__ out_vals, uint8_t* __restrict__ out_found) {
+  TxCounters c;
+  ParentCache<F> pc;
+  uint32_t upserts = 0, deferred = 0;
+  for (;;) {
+    uint32_t at = 0;
+    if (lane_id() == 0) at = atomicAdd(&a.split->head, (uint32_t)WAVE);
+    at = uniform32(at);
+    if (at >= n) break;
+    const uint32_t e = at + lane_id();
+    tx_ops<F>(t, a, ld_relaxed32(a.dlist + min(e, n - 1)), e < n, out_vals, out_found, a.rlist,
+              &a.split->n_redo, c, pc, upserts, deferred);
+  }
+  flush_counters(t, c, a.counters);
+  if (lane_id() == 0) {
+    stat_add(t.stats, ST_UPSERTS, wave_stripe(), upserts);
+    stat_add(t.stats, ST_DEFERRED, wave_stripe(), deferred);
+  }
+}
+
 // The batch's counters and the tree's error bits: lane l below 8 holds 64-bit word l of the block.
 // Agent-scope loads see the other kernels' and wavefronts' updates past this CU's cache.
 struct CounterWords {
@@ -2414,20 +2431,18 @@ STM_DEV CounterWords load_counters(const TreeView& t, const BatchCounters* cnt) 
                       ld_relaxed(&t.hdr->error)};
 }
 
+// Serial pass over the n ops of `list`, which exhausted their attempts: one wavefront, no
+// competitors, so every transaction commits on its first attempt.  Then the batch's counters.
 template <int F>
-STM_DEV void serial_pass(const TreeView& t, const UpsertArgs& a, CounterWords cw,
-                         uint64_t* __restrict__ out_vals, uint8_t* __restrict__ out_found) {
+STM_DEV void serial_pass(const TreeView& t, const UpsertArgs& a, CounterWords cw, const uint32_t* list,
+                         uint32_t n, uint64_t* __restrict__ out_vals,
+                         uint8_t* __restrict__ out_found) {
   BatchCounters* cnt = a.counters;
-  const uint32_t n = cw.at(offsetof(BatchCounters, n_deferred));
   if (n) {
     TxCounters c;
     ParentCache<F> pc;
-    // Once the pool is full the batch fails; the rest then gets a bounded number of tries (an op
-    // that needs no node still succeeds), so that a long list cannot hold the device for seconds.
-    uint32_t tries = 4096;
-    for (uint32_t e = 0; e < n && tries; ++e) {
-      if (uniform64(ld_relaxed(&t.hdr->error)) & ERR_POOL_FULL) --tries;
-      const uint32_t g = uniform32(ld_relaxed32(a.dlist + e));
+    for (uint32_t e = 0; e < n; ++e) {
+      const uint32_t g = uniform32(ld_relaxed32(list + e));
       if (!run_upsert<F>(t, a.ukey[g], a.uval[g], a.gstart[g], a.npend[g], a.sidx, out_vals, out_found,
                          1024u, c, pc)) {
         if (lane_id() == 0) atomicOr((unsigned long long*)&t.hdr->error, (unsigned long long)ERR_LIVELOCK);
@@ -2473,46 +2488,89 @@ STM_DEV void serial_pass(const TreeView& t, const UpsertArgs& a, CounterWords cw
   }
 }
 
-// The end of a batch's upserts, by one workgroup: the upper levels of the tree, then one wavefront
-// for the serial pass and the counters.  A batch of at most ONE_BLOCK_OPS ops has its leaf runs,
-// short and long, done here too.  Each phase sees the writes of the ones before: every wavefront
-// has its stores acknowledged before the barrier, and the words they share are read past the
-// scalar cache.
+// The end of a batch's upserts: one workgroup brings the upper levels of the tree up to date, the
+// ops that the pool refused run as transactions, and one wavefront does the serial pass and the
+// counters.  A batch of at most ONE_BLOCK_OPS ops has its leaf runs, short and long, done here
+// too.  Each phase sees the writes of the ones before: every wavefront has its stores acknowledged
+// before the barrier, and the words they share are read past the scalar cache.
 // A small batch pays for launches and round trips: what the phases need to know (long runs, splits,
-// deferred ops, counters) comes in one.  As four launches (runs, long runs, upper levels, serial
+// refused ops, counters) comes in one.  As four launches (runs, long runs, upper levels, serial
 // pass) a 1000-op call took 33.3 µs, as one 29.5; with the upper levels and the serial pass in one
 // launch a 40001-op call takes 81 µs instead of 84.  Above ONE_BLOCK_OPS one workgroup would take its
 // runs in turns: the grid of k_upsert_runs takes them at once.
+// Only a pool that is all but full refuses runs, and then tens of thousands of ops at once may wait
+// for transactions, which the other workgroups of the grid are for (they leave at once otherwise).
+// Those wait, for a bounded time, until the first has the upper levels done; the ops are dealt out
+// from a counter, so a workgroup that gave up is not missed.  The last to arrive goes on alone.
 constexpr uint32_t FIN_RUNS = 1, FIN_UPPER = 2, FIN_SERIAL = 4;
-template <int F>
-__global__ __launch_bounds__(1024) void k_upsert_finish(TreeView t, UpsertArgs a, uint32_t phases,
-                                                        uint32_t first_level) {
+constexpr uint32_t FIN_BLOCKS = 32;
+constexpr uint32_t UPPER_POLLS = 1u << 18;  // of 64 clocks of sleep and a load each
+template <int F, uint32_t PHASES>
+__global__ __launch_bounds__(1024) void k_upsert_finish(TreeView t, UpsertArgs a, uint32_t first_level) {
+  __shared__ uint32_t s_flag;
   const OutArrays o = out_arrays(a);
-  if (phases & FIN_RUNS) {
+  SplitState* split = a.split;
+  if constexpr ((PHASES & FIN_RUNS) != 0) {  // (one workgroup)
     leaf_runs<F>(t, a, o.vals, o.found);
     wave_order();
     __syncthreads();
   }
-  const uint32_t n_long = ld_relaxed32(&a.split->n_long);
-  uint32_t made = ld_relaxed32(&a.split->made);
+  const uint32_t n_long = PHASES & FIN_RUNS ? ld_relaxed32(&split->n_long) : 0u;
+  uint32_t made = ld_relaxed32(&split->made);
   CounterWords cw = load_counters(t, a.counters);
+  uint32_t listed = cw.at(offsetof(BatchCounters, n_deferred));  // in dlist
   bool changed = false;
-  if ((phases & FIN_RUNS) && n_long) {
+  if ((PHASES & FIN_RUNS) && n_long) {
     long_runs<F>(t, a, o.vals, o.found);
     wave_order();
     __syncthreads();
-    made = ld_relaxed32(&a.split->made);
+    made = ld_relaxed32(&split->made);
+    listed = ld_relaxed32(&a.counters->n_deferred);
     changed = true;
   }
-  if ((phases & FIN_UPPER) && made) {
-    upper_pass<F>(t, a.split, a.plist, a.plist2, first_level);
+  bool go = true;
+  if (blockIdx.x > 0) {
+    if (listed == 0) return;
+    if (threadIdx.x == 0) {
+      uint32_t done = 0;
+      for (uint32_t p = 0; !done && p < UPPER_POLLS; ++p) {
+        done = ld_relaxed32(&split->upper);
+        if (!done) __builtin_amdgcn_s_sleep(1);
+      }
+      s_flag = done;
+    }
+    __syncthreads();
+    go = s_flag != 0;
+  } else if ((PHASES & FIN_UPPER) && made) {
+    upper_pass<F>(t, split, a.plist, a.plist2, first_level);
     wave_order();
     __syncthreads();
     changed = true;
   }
-  if ((phases & FIN_SERIAL) && threadIdx.x < (uint32_t)WAVE) {
+  const uint32_t* list = a.dlist;
+  if ((PHASES & FIN_UPPER) && (PHASES & FIN_SERIAL) && listed) {
+    if (blockIdx.x == 0) {
+      // The nodes' plain stores leave this XCD's cache before the transactions read them.
+      __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+      __syncthreads();
+      if (threadIdx.x == 0)
+        __hip_atomic_store(&split->upper, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    }
+    if (go) refused_ops<F>(t, a, listed, o.vals, o.found);
+    wave_order();
+    __syncthreads();
+    if (gridDim.x > 1) {
+      if (threadIdx.x == 0) s_flag = atomicAdd(&split->arrived, 1u) + 1 == gridDim.x;
+      __syncthreads();
+      if (!s_flag) return;
+    }
+    list = a.rlist;
+    listed = ld_relaxed32(&split->n_redo);
+    changed = true;
+  }
+  if ((PHASES & FIN_SERIAL) && threadIdx.x < (uint32_t)WAVE) {
     if (changed) cw = load_counters(t, a.counters);
-    serial_pass<F>(t, a, cw, o.vals, o.found);
+    serial_pass<F>(t, a, cw, list, listed, o.vals, o.found);
   }
 }
 
@@ -2750,7 +2808,7 @@ static hipError_t launch_upsert_f(const TreeView& t, const UpsertArgs& a, hipStr
   const bool runs_only = a.piece >= (uint32_t)WAVE;
   hipError_t e;
   if (runs_only && a.n_max <= ONE_BLOCK_OPS) {
-    k_upsert_finish<F><<<1, 1024, 0, s>>>(t, a, FIN_RUNS | FIN_UPPER | FIN_SERIAL, 1u);
+    k_upsert_finish<F, FIN_RUNS | FIN_UPPER | FIN_SERIAL><<<1, 1024, 0, s>>>(t, a, 1u);
     return hipGetLastError();
   }
   k_upsert_runs<F><<<blocks, 256, 0, s>>>(t, a);
@@ -2769,16 +2827,15 @@ static hipError_t launch_upsert_f(const TreeView& t, const UpsertArgs& a, hipStr
   }
   const uint32_t first_level = few ? 1u : 2u;
   if (runs_only) {
-    k_upsert_finish<F><<<1, 1024, 0, s>>>(t, a, FIN_UPPER | FIN_SERIAL, first_level);
+    const uint32_t fb = std::max<uint32_t>(1, std::min<uint32_t>((uint32_t)(a.n_max / 1024), FIN_BLOCKS));
+    k_upsert_finish<F, FIN_UPPER | FIN_SERIAL><<<fb, 1024, 0, s>>>(t, a, first_level);
     return hipGetLastError();
   }
-  k_upsert_finish<F><<<1, 1024, 0, s>>>(t, a, FIN_UPPER, first_level);
+  k_upsert_finish<F, FIN_UPPER><<<1, 1024, 0, s>>>(t, a, first_level);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  k_upsert<F><<<a.blocks, 256, 0, s>>>(t, a.ukey, a.uval, a.sidx, a.ilist, a.rlist, a.rlen,
-                                        a.rfirst, a.rcount, waves, a.ihint, a.counters, a.dlist,
-                                        a.max_attempts, a.out_vals, a.out_found, a.desc);
+  k_upsert<F><<<a.blocks, 256, 0, s>>>(t, a, waves);
   if ((e = hipGetLastError()) != hipSuccess) return e;
-  k_upsert_finish<F><<<1, 64, 0, s>>>(t, a, FIN_SERIAL, first_level);
+  k_upsert_finish<F, FIN_SERIAL><<<1, 64, 0, s>>>(t, a, first_level);
   return hipGetLastError();
 }
 

@@ -48,7 +48,12 @@ struct SplitState {
   uint32_t n_dirty2; // level-2 nodes on theirs
   uint32_t root;     // 1 + the root, when it was split and needs a parent; 0: it was not
   uint32_t n_long;   // runs left to k_upsert_long
-  uint32_t pad[9];
+  // The last launch, where the pool refused runs (k_upsert_finish):
+  uint32_t head;     // refused ops handed to a wavefront
+  uint32_t upper;    // 1: the upper levels are done
+  uint32_t arrived;  // workgroups past the refused ops
+  uint32_t n_redo;   // refused ops left to the serial pass
+  uint32_t pad[5];
 };
 static_assert(sizeof(SplitState) == 64, "one 64-byte block");
 
@@ -99,7 +104,8 @@ struct UpsertArgs {
   SplitState* split;
   uint32_t* plist;        // level-1 nodes with new children (capacity: groups)
   uint32_t* plist2;       // their level's parents (capacity: groups)
-  uint32_t* rlist;        // per piece: its first list entry (capacity: groups)
+  uint32_t* rlist;        // per piece: its first list entry (capacity: groups); at the end the
+                          //   refused ops for the serial pass
   uint32_t* rlen;         //   and its ops
   uint32_t* rfirst;       // per wavefront of k_upsert_runs: its first piece's index
   uint32_t* rcount;       //   and their number (capacity: RUN_WAVES_MAX)

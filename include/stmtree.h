@@ -108,7 +108,7 @@ typedef struct stm_stats {
     uint64_t batches;         /* device passes run */
     uint64_t ops;             /* ops submitted */
     uint64_t unique_ops;      /* ops after the per-key fold */
-    uint64_t upserts;         /* merged INSERT ops executed as transactions */
+    uint64_t upserts;         /* merged INSERT ops executed */
     uint64_t commits;         /* committed transactions (a leaf's inserts, or part of them, and splits) */
     uint64_t aborts;          /* attempts given up and made again: a leaf's inserts that do not fit it
                                  as it is, a transaction that met a lock or a changed node */
