@@ -1541,16 +1541,20 @@ int stm_sort_pairs_device(int device, const uint64_t* d_keys, size_t n, uint64_t
   if (!d_keys || !d_keys_out || !d_idx_out) return fail(STM_ERR_INVALID, "null device array");
   if (n > (1ull << 30)) return fail(STM_ERR_INVALID, "sort of %zu keys exceeds 2^30", n);
   HIP_TRY(hipSetDevice(device));
-  uint64_t* ktmp = nullptr;
+  uint64_t *ktmp = nullptr, *kin = nullptr;
   uint32_t *itmp = nullptr, *words = nullptr;
   int rc = STM_OK;
+  // In place: the passes write the output before they have read the input for the last time.
+  const bool apart = d_keys_out + n <= d_keys || d_keys + n <= d_keys_out;
   if (dalloc(&ktmp, n) != hipSuccess || dalloc(&itmp, n) != hipSuccess ||
-      dalloc(&words, sort_hist_words(n)) != hipSuccess) {
+      dalloc(&words, sort_hist_words(n)) != hipSuccess || (!apart && dalloc(&kin, n) != hipSuccess)) {
     rc = fail(STM_ERR_NOMEM, "sort scratch for %zu keys", n);
   } else {
     hipError_t e = sort_scratch_init(words);
+    if (e == hipSuccess && kin)
+      e = hipMemcpyAsync(kin, d_keys, n * 8, hipMemcpyDeviceToDevice, nullptr);
     if (e == hipSuccess)
-      e = radix_sort_pairs(d_keys, ktmp, d_keys_out, itmp, d_idx_out, (uint32_t)n, 0, 64, words,
+      e = radix_sort_pairs(kin ? kin : d_keys, ktmp, d_keys_out, itmp, d_idx_out, (uint32_t)n, 0, 64, words,
                            nullptr);
     uint32_t stalled = 0;
     if (e == hipSuccess)
@@ -1559,7 +1563,7 @@ int stm_sort_pairs_device(int device, const uint64_t* d_keys, size_t n, uint64_t
     else if (stalled) rc = fail(STM_ERR_DEVICE, "sort: a bounded wait between workgroups gave up");
   }
   (void)hipDeviceSynchronize();
-  void* ps[] = {ktmp, itmp, words};
+  void* ps[] = {ktmp, kin, itmp, words};
   for (void* q : ps)
     if (q) (void)hipFree(q);
   return rc;

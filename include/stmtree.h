@@ -234,8 +234,9 @@ int stm_run_batches_device(stm_tree* tree, const uint64_t* d_keys, const uint64_
 int stm_capture_graphs(stm_tree* tree);
 
 /* Stable ascending sort of n device-resident u64 keys on `device`: d_keys_out receives the
- * keys in order, d_idx_out the input position of each (ties keep input order).  The batch
- * path's own sort, exposed for callers and tests; it allocates its scratch per call.
+ * keys in order, d_idx_out the input position of each (ties keep input order).  d_keys_out may be
+ * d_keys.  The batch path's own sort, exposed for callers and tests; it allocates its scratch per
+ * call.
  * Replaces cub::DeviceRadixSort::SortPairs of (key, position)
  * (src/gpu-stm-tree-v38/bpt-gpustm-kernel.cu:293). */
 int stm_sort_pairs_device(int device, const uint64_t* d_keys, size_t n, uint64_t* d_keys_out,
