@@ -153,8 +153,9 @@ struct Scratch {
     n = cap;
 #define A_(p, c) p = static_cast<decltype(p)>(cur.take(sizeof(*p) * (size_t)(c)))
     const bool staging = use == CALLS;
+    if (use != LOAD) A_(in_ops, cap);
     if (staging) {
-      A_(in_keys, cap); A_(in_vals, cap); A_(in_ops, cap); A_(out_vals, cap); A_(out_found, cap);
+      A_(in_keys, cap); A_(in_vals, cap); A_(out_vals, cap); A_(out_found, cap);
     }
     A_(skeys_tmp, cap); A_(skeys, cap); A_(sidx_tmp, cap); A_(sidx, cap);
     A_(hist, sort_hist_words(cap));
@@ -641,6 +642,11 @@ int maybe_retrain(stm_tree* t) {
   return train_router(t, t->cfg.train_steps, true);
 }
 
+// Whether found flags and op codes of n ops share memory.
+bool overlaps(const uint8_t* found, const uint8_t* ops, size_t n) {
+  return found < ops + n && ops < found + n;
+}
+
 // Scan output area of a chunk (device pointers); null = op 3 runs as GET.
 struct ScanOut {
   uint64_t* keys;
@@ -666,6 +672,10 @@ int run_chunk(stm_tree* t, const uint64_t* keys, const uint64_t* vals, const uin
     in.scan_cap = so->cap;
   } else {
     in.host_counters = s.h_counters;  // the scan answers kernel runs after the upsert kernels
+  }
+  if (overlaps(out_found, ops, n)) {  // the flags' default is written before the last look at the ops
+    HIP_TRY(hipMemcpyAsync(s.in_ops, ops, n, hipMemcpyDeviceToDevice, st));
+    in.ops = s.in_ops;
   }
   const bool small = n <= FRONT_MAX_OPS;
   uint32_t& hold = small ? t->front_hold : t->exact_left;
@@ -1403,7 +1413,10 @@ int stm_run_batches_device(stm_tree* t, const uint64_t* d_keys, const uint64_t* 
     return fail(STM_ERR_INVALID, "null device array (device batches always carry values)");
   int rc = set_device(t);
   if (rc) return rc;
-  if (!t->cfg.use_graphs) {
+  // Flags in the place of op codes: a batch that has to be sorted again would find the ops of the
+  // ones behind it gone.
+  if (!t->cfg.use_graphs || overlaps(d_out_found + offsets[0], d_ops + offsets[0],
+                                     offsets[n_batches] - offsets[0])) {
     for (size_t b = 0; b < n_batches; ++b) {
       const uint64_t o = offsets[b];
       rc = run_device(t, d_keys + o, d_vals + o, d_ops + o, offsets[b + 1] - o, d_out_vals + o,

@@ -160,7 +160,8 @@ int stm_bulk_load_device(stm_tree* tree, const uint64_t* d_keys, const uint64_t*
 int stm_run_batch(stm_tree* tree, const uint64_t* keys, const uint64_t* vals, const uint8_t* ops,
                   size_t n, uint64_t* out_vals, uint8_t* out_found);
 
-/* Same with device-resident inputs and outputs (d_vals is required).  Work is queued on
+/* Same with device-resident inputs and outputs (d_vals is required; d_out_found may be d_ops, here
+ * and in the calls below: a batch stream then runs batch by batch).  Work is queued on
  * the tree's stream (stm_get_stream); the call returns after the batch has completed.
  * The exact re-sort of a batch (stm_stats.sort_fallbacks) waits between workgroups, for a bounded
  * time; a sort that gives up such a wait fails the call with STM_ERR_DEVICE, and that batch then
