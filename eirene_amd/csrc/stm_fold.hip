@@ -260,6 +260,11 @@ __global__ __launch_bounds__(FOLD_BLOCK) void k_fold_apply(FoldArgs a, const Acc
           const uint32_t pos = pos_of(ch.sx[r]);
           a.out_vals[pos] = va[q];  // out_found stays 1
         }
+        if (a.out_vals && key == KEY_EMPTY) {
+          const uint32_t pos = pos_of(ch.sx[r]);
+          a.out_vals[pos] = 0;
+          a.out_found[pos] = 0;
+        }
         if (a.gstart && is_ins && last_before < 0) a.npend[g] = (uint32_t)(i - head + 1);
         if (group_end) {
           a.ukey[g] = key;

@@ -76,12 +76,16 @@ STM_DEV void fold_gather(const FoldArgs& a, FoldElem& x) {
   x.vb = need_b ? a.vals[x.pos] : 0ull;
 }
 
-// Writes the element's outputs.  Ops with the reserved key are added to bad.
+// Writes the element's outputs.  Ops with the reserved key are added to bad, and answered as absent.
 STM_DEV void fold_store(const FoldArgs& a, const FoldElem& x, uint32_t* bad) {
   if (!x.valid) return;
   if (a.lastins) a.lastins[x.i] = x.ins ? x.i : x.lb;
   if (x.lb >= 0) {
     a.out_vals[x.pos] = x.va;  // out_found stays 1
+  }
+  if (x.key == KEY_EMPTY) {
+    a.out_vals[x.pos] = 0;
+    a.out_found[x.pos] = 0;
   }
   if (x.ins && x.lb < 0) a.npend[x.g] = (uint32_t)(x.i - x.head + 1);
   if (!x.end) return;
@@ -174,6 +178,7 @@ __global__ __launch_bounds__(FT) void k_front_small(FrontArgs fa) {
     const uint32_t op = v ? gload(in.ops + i) : 0u;
     k[r] = kk;
     p[r] = v ? tie_of(i, op) : ~0u;
+    if (v) a.out_found[i] = 1;  // the answers' default
   }
   bin_sort_open<FT>(s_bin);
   if (tid == 0) s_bad = 0;
@@ -214,10 +219,7 @@ __global__ __launch_bounds__(FT) void k_front_small(FrontArgs fa) {
     fold_gather(a, x[r]);
   }
 #pragma unroll
-  for (int r = 0; r < E; ++r) {
-    if (x[r].valid) a.out_found[x[r].i] = 1;  // the answers' default
-    fold_store(a, x[r], &s_bad);
-  }
+  for (int r = 0; r < E; ++r) fold_store(a, x[r], &s_bad);
   __syncthreads();
   if (tid == 0) reset_counters(a.counters, run.c, run.m & ~ACC_LEAD, s_bad);
 }
