@@ -8,8 +8,7 @@ same distribution.  A step is one batch.  All batches are generated on the host 
 to HBM before the timed region.  Each route (plain descent, learned routing, the static leaf
 index; at the library defaults and at the launch parameters of the tuning record) runs them
 back to back through stm_run_batch_device, one synchronous call per batch; the learned and
-descent routes also run them as one device-resident stream (stm_run_batches_device, graph
-replay).
+descent routes also run them as one device-resident stream (stm_run_batches_device).
 
 Prints one JSON line.  `value` is Mops/s over the K timed batches of the learned route at
 the tuned parameters, as a stream (wall clock from the first launch to the last batch's
@@ -165,9 +164,9 @@ def copy_ceiling_gbs(ea, mib=4096, reps=4):
 
 def run_uneven(args, ea, w):
     """Uneven batching: 2^load_log2 Normal(2^62, 2^58) keys, a stream of batches with sizes
-    log-uniform in [2^10, 2^22] at 95/5, replayed from captured graphs with the autotuned
-    launch parameters, against the same stream launched batch by batch from the host with the
-    library defaults."""
+    log-uniform in [2^10, 2^22] at 95/5, as one device-resident stream (batches of up to 2^12 ops
+    replayed from captured graphs, larger ones on two streams) with the autotuned launch
+    parameters, against the same batches one synchronous call each with the library defaults."""
     from eirene_amd import autotune as at
     n_load = 1 << args.load_log2
     t0 = time.time()
@@ -214,15 +213,15 @@ def run_uneven(args, ea, w):
     m_dh, dt_dh, _, out_dh = timed(base, False)
     same = bool(all(np.array_equal(a, b) for a, b in zip(out_tg[:2], out_dh[:2]))
                 and all(np.array_equal(a, b) for a, b in zip(out_tg[2], out_dh[2])))
-    log(f"[uneven] graphs+tuned {m_tg:.1f}, graphs+default {m_dg:.1f}, host+default {m_dh:.1f} "
+    log(f"[uneven] stream+tuned {m_tg:.1f}, stream+default {m_dg:.1f}, calls+default {m_dh:.1f} "
         f"Mops/s; identical={same}")
     sample.free()
     return {
         "workload": f"bulk-load 2^{args.load_log2} Normal(2^62, 2^58) keys; {args.uneven_batches} "
                     f"batches log-uniform in [2^10, 2^22] ({n_ops} ops), 95% lookup / 5% insert",
-        "mops_graphs_tuned": round(m_tg, 2), "mops_graphs_default": round(m_dg, 2),
-        "mops_host_default": round(m_dh, 2),
-        "ms_graphs_tuned": round(dt_tg * 1e3, 2), "ms_host_default": round(dt_dh * 1e3, 2),
+        "mops_stream_tuned": round(m_tg, 2), "mops_stream_default": round(m_dg, 2),
+        "mops_calls_default": round(m_dh, 2),
+        "ms_stream_tuned": round(dt_tg * 1e3, 2), "ms_calls_default": round(dt_dh * 1e3, 2),
         "tuned_config": rec["best"], "tuned_from": tuned_from,
         "autotune_trials": len(rec.get("trials", [])),
         "results_identical_tuned_vs_default": same,
@@ -489,8 +488,9 @@ def main():
 
     def run_stream(route):
         """The same batches through stm_run_batches_device: the warm-up batches as one stream,
-        then the timed batches as one device-resident stream (one captured graph per size class,
-        replayed; retrains between replays), on a fresh tree from the same bulk load."""
+        then the timed batches as one device-resident stream (a batch's sort and fold beside the
+        lookups and upserts of the one before; retrains between), on a fresh tree from the same
+        bulk load."""
         cfg = route_config(route)
         cfg.timing = False
         tree = ea.StmTree(cfg)
@@ -514,7 +514,7 @@ def main():
     def small_batch_routes():
         """Routing at small batch sizes (the sizes of the uneven stream and of serving
         requests): per route, on a fresh tree from the same bulk load, streams of batches of
-        2^12, 2^14 and 2^16 ops (2^21 ops each, 95/5, Gamma keys) replayed from graphs.  The
+        2^12 (replayed from a graph), 2^14 and 2^16 ops (2^21 ops each, 95/5, Gamma keys).  The
         router is trained once before the streams (no periodic retrain inside them), so the
         comparison is the routing itself."""
         sizes = [(12, 512), (14, 128), (16, 32)]
@@ -714,7 +714,7 @@ def main():
                                f"(90% hits) / 5% insert, router retrained every 8 batches",
                    "global_batch": n_batch, "value_route": head_name,
                    "value_api": ("stm_run_batches_device: the timed batches as one device-resident "
-                                 "stream (graph replay)" if head_name in streams else
+                                 "stream" if head_name in streams else
                                  "stm_run_batch_device: one synchronous call per batch"),
                    "defaults": {"fanout": args.fanout, "lanes_per_op": args.lanes,
                                 "ops_per_group": args.group},

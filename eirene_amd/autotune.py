@@ -8,7 +8,7 @@ Search space (every point is a valid StmConfig):
 
 Method: for each fanout (the tree must be rebuilt for it), coordinate descent over the other
 parameters from the library defaults, two sweeps, keeping a change only when it is faster by
-more than `min_gain`.  A trial bulk-loads a fresh tree from device-resident keys and replays the
+more than `min_gain`.  A trial bulk-loads a fresh tree from device-resident keys and runs the
 sample stream once untimed (first touch), then times the stream on fresh trees loaded from the
 same keys, so every trial starts from the same tree.  Each timed tree captures its graphs and
 (with learned routing) trains its router before the clock starts; throughput is ops / wall

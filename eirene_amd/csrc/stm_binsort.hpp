@@ -247,7 +247,8 @@ STM_DEV void bin_sort(uint32_t m, uint64_t (&k)[E], uint32_t (&p)[E], uint64_t* 
 STM_DEV uint32_t tie_of(uint32_t i, uint32_t op) { return (i << 2) | (op > 3u ? 1u : op); }
 STM_DEV uint32_t payload_of(uint32_t tie) { return (tie >> 2) | (tie << POS_BITS); }
 
-// Where within its stretch of the input a sample is drawn.
+// Where within its stretch of the input a sample is drawn: lowbias32, the 32-bit integer hash that
+// Chris Wellons published with his hash-prospector (public domain).
 STM_DEV uint32_t hash32(uint32_t x) {
   x = (x ^ (x >> 16)) * 0x7feb352du;
   x = (x ^ (x >> 15)) * 0x846ca68bu;

@@ -126,7 +126,8 @@ struct TreeView {
 // inserts into a leaf are neighbours in its sorted list), and the kernels that bring the new
 // leaves to their parents (one wavefront per parent, one launch or one workgroup step per level).
 // No other wavefront of the launch reads or writes those nodes, so the plain loads return what
-// earlier kernels left, and the launch boundary publishes the plain stores.  Metadata words, which
+// earlier kernels left, and the launch boundary publishes the plain stores (in k_upsert_finish,
+// where transactions may follow in the same launch, a release fence does).  Metadata words, which
 // share lines with other nodes' words, are stored at agent scope there too.
 // Plain load through a pointer known to address device global memory.  Pointers read from
 // memory (a batch descriptor's) are generic to the compiler, which then emits flat loads; this

@@ -3,9 +3,9 @@
 //
 // A batch of this size is bound by latency, not by bytes: each launch costs 2-4 µs and each
 // dependent round trip to memory about 1 µs, whatever they move.  So the front half is built for
-// few launches and few round trips, and sorts by comparison in LDS, where the exact key and the
-// input position are one 96-bit value: no normalization, no second pass over near-equal keys, and
-// equal keys need no special care.
+// few launches and few round trips, and sorts in LDS (stm_binsort.hpp), where the exact key and
+// the input position are one 96-bit value: no normalization, no second pass over near-equal keys,
+// and equal keys need no special care.
 //
 //   up to FRONT_SMALL ops, one workgroup:
 //     k_front_small   sort in LDS, fold, outputs
@@ -18,9 +18,9 @@
 //
 // The radix form this replaces took ten or eleven launches: k_range, the digit histograms and
 // their scan, two or three single-sweep passes, the bucket fix-up, the exact-sort check and three
-// fold kernels.  Kernel times, replaced / now: 1000 ops 52 / 9.1 µs, 40001 ops 86 / 29 µs, 131075 ops
-// 101 / 46 µs; most of what is left is the compare-exchanges (a sort of 1024 elements by one
-// workgroup is 55 steps, about 3 µs) and three round trips to memory per kernel.
+// fold kernels.  Kernel times, replaced / now: 1000 ops 52 / 7.0 µs, 40001 ops 86 / 26 µs, 131075 ops
+// 101 / 38 µs; most of what is left is three round trips to memory per kernel and the barriers
+// between the steps of a workgroup's sort.
 //
 // Buckets are cut between samples of (key, position), so a hot key's ops are shared by as many
 // buckets as they fill.  With OVERSAMPLE samples per bucket drawn at hashed positions, one per

@@ -70,8 +70,9 @@ const uint32_t* sort_exact_word(const uint32_t* words);
 // ------------------------------------------------------------------ sample sort (stm_sample.hip)
 // The sort of full 64-bit keys between these sizes, called by the radix entry points.  Below, the
 // normalized radix form stays: there a hot key with neighbours still shows in sort_fallbacks, which
-// callers of those sizes watch, and the difference is smallest (30 µs of a 2^19-op call).  Above, a
-// tile of FT * 16 keys per workgroup no longer covers the batch with TILES_MAX tiles.
+// callers of those sizes watch.  It costs them a step up and one down: a call on 2^22 uniform keys
+// takes 93 µs at 2^18 ops (stm_front.hip), 132 at 2^18 + 1, 142 at 3 * 2^17, 113 at 3 * 2^17 + 1.
+// Above, a tile of FT * 16 keys per workgroup no longer covers the batch with TILES_MAX tiles.
 constexpr uint32_t SAMPLE_SORT_MIN = (3u << 17) + 1;
 constexpr uint32_t SAMPLE_SORT_MAX = 1u << 22;
 inline bool sample_sorted(uint64_t n) { return n >= SAMPLE_SORT_MIN && n <= SAMPLE_SORT_MAX; }
@@ -150,10 +151,10 @@ struct FoldArgs {
 };
 // ------------------------------------------------------------------ front half of small batches
 // (stm_front.hip): sort and fold of at most FRONT_MAX_OPS ops in one or three launches, with the
-// results of the radix sort and fold_batch.  A whole call on 2^22 uniform keys, with the radix
-// form and the lookup's longer spans in parentheses: 1000 ops 33 µs (113), 16384 ops 58 (123), 2^16
-// ops 70 (144), 2^18 ops 113 (171).  Above
-// 2^18 ops a workgroup's sample sort and the buckets' comparison sorts grow past what they save.
+// results of the radix sort and fold_batch.  A whole call on 2^22 uniform keys with 5 % inserts, in
+// parentheses that of the tree whose batches all went through the radix form: 1000 ops 30 µs (116),
+// 16384 ops 53 (128), 2^16 ops 63 (144), 2^18 ops 93 (175).  Above 2^18 ops the sample that every
+// workgroup of k_front_split sorts grows past what it saves.
 constexpr uint32_t FRONT_MAX_OPS = 1u << 18;
 struct FrontArgs {
   const uint64_t* keys;  // the batch (or fold.desc)
