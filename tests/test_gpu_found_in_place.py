@@ -35,9 +35,13 @@ def crowded_interval(n, rng):
     return crafted(n, rng, 1)
 
 
-CASES = pytest.mark.parametrize("n,keys_of,again", [
-    (1000, uniform, 0), (12000, uniform, 0), (12000, misleading, 1), (300000, hot_neighbours, 1),
-    (400000, uniform, 0), (400000, crowded_interval, 1)])
+NOALLOC_MOST = 65536
+CASES = pytest.mark.parametrize("n,keys_of,again,call", [
+    (n, keys_of, again, call)
+    for n, keys_of, again in [(1000, uniform, 0), (12000, uniform, 0), (12000, misleading, 1),
+                              (300000, hot_neighbours, 1), (400000, uniform, 0),
+                              (400000, crowded_interval, 1)]
+    for call in ("batch", "stream", "noalloc") if call != "noalloc" or n <= NOALLOC_MOST])
 
 
 def batch(n, keys_of, rng):
@@ -56,11 +60,8 @@ def check_tree(t, o):
 
 
 @CASES
-@pytest.mark.parametrize("call", ["batch", "noalloc", "stream"])
 def test_found_flags_in_place_of_op_codes(oracle_mod, n, keys_of, again, call):
-    from eirene_amd import DeviceBuffer, NOALLOC_MAX_OPS, StmTree
-    if call == "noalloc" and n > NOALLOC_MAX_OPS:
-        pytest.skip("larger than that call takes")
+    from eirene_amd import DeviceBuffer, StmTree
     rng = np.random.default_rng(n)
     load, keys, vals, ops = batch(n, keys_of, rng)
     o = oracle_mod.Oracle()
