@@ -489,8 +489,18 @@ STM_DEV void train_units(SegModel& m, uint32_t cnt, const uint64_t* __restrict__
       UnitGrad g{0.0f, 0.0f, 0.0f, 0.0f};
       const float* x = s_x + q;
       float fi = (float)q;
-#pragma unroll 4
-      for (uint32_t k = cnt / 4; k > 0; --k) {
+      // Four at a time by hand: the compiler does not unroll a loop over lane exchanges, and one
+      // pair after the other is a chain of four of them.
+      for (uint32_t k = cnt / 16; k > 0; --k) {
+        const float x0 = x[0], x1 = x[4], x2 = x[8], x3 = x[12];
+        unit_accumulate(p, x0, fi * scale, scale, g);
+        unit_accumulate(p, x1, (fi + 4.0f) * scale, scale, g);
+        unit_accumulate(p, x2, (fi + 8.0f) * scale, scale, g);
+        unit_accumulate(p, x3, (fi + 12.0f) * scale, scale, g);
+        x += 16;
+        fi += 16.0f;
+      }
+      for (uint32_t k = cnt % 16 / 4; k > 0; --k) {
         unit_accumulate(p, *x, fi * scale, scale, g);
         x += 4;
         fi += 4.0f;
@@ -506,10 +516,11 @@ STM_DEV void train_units(SegModel& m, uint32_t cnt, const uint64_t* __restrict__
 // One wavefront per segment: full-batch Adam for `steps` steps.  Up to UNIT_MAX_PAIRS pairs a lane
 // owns a hidden unit (train_units), above it lane L owns parameter param_of_lane(L), its Adam
 // moments and its value, and the forward and backward passes read the parameters as wave-uniform
-// values.  Bound by instruction issue: 4096 wavefronts are one per SIMD slot of four, and a step
-// costs about 450 instructions plus 150 per 64 pairs with a pair per lane, 120 plus 18 per four
-// pairs with a unit per lane (the same at some 130 pairs).  Cold build of 2^22 keys (21 pairs per
-// segment, 300 steps): 992 / 374 µs.
+// values.  Bound by instruction issue where every segment has leaves (4096 wavefronts are one per
+// SIMD slot of four), by one wavefront's chain of steps where few have most of them.  A step costs
+// about 450 instructions plus 150 per 64 pairs with a pair per lane, 120 plus 18 per four pairs with a
+// unit per lane (the same at some 130 pairs).  300 steps on 2^22 keys, a pair / a unit per lane:
+// uniform (21 pairs per segment) 960 / 362 µs, Normal (up to 88) 634 / 612, Gamma 801 / 508.
 __global__ __launch_bounds__(TRAIN_WAVES * WAVE) void k_route_train(
     const RouteHeader* __restrict__ rh, const uint64_t* __restrict__ fences,
     SegModel* __restrict__ segs, uint32_t steps, float lr, uint32_t salt) {
