@@ -1558,13 +1558,24 @@ int stm_sort_pairs_device(int device, const uint64_t* d_keys, size_t n, uint64_t
   HIP_TRY(hipSetDevice(device));
   uint64_t *ktmp = nullptr, *kin = nullptr;
   uint32_t *itmp = nullptr, *words = nullptr;
+  void* slab = nullptr;
   int rc = STM_OK;
   // In place: the passes write the output before they have read the input for the last time.
   const bool apart = d_keys_out + n <= d_keys || d_keys + n <= d_keys_out;
-  if (dalloc(&ktmp, n) != hipSuccess || dalloc(&itmp, n) != hipSuccess ||
-      dalloc(&words, sort_hist_words(n)) != hipSuccess || (!apart && dalloc(&kin, n) != hipSuccess)) {
+  auto layout = [&](SlabCursor& cur) {
+    ktmp = (uint64_t*)cur.take(n * 8);
+    itmp = (uint32_t*)cur.take(n * 4);
+    words = (uint32_t*)cur.take(sort_hist_words(n) * 4);
+    if (!apart) kin = (uint64_t*)cur.take(n * 8);
+  };
+  SlabCursor size{nullptr};
+  layout(size);
+  if (hipMalloc(&slab, size.at) != hipSuccess) {
+    slab = nullptr;
     rc = fail(STM_ERR_NOMEM, "sort scratch for %zu keys", n);
   } else {
+    SlabCursor place{static_cast<uint8_t*>(slab)};
+    layout(place);
     hipError_t e = sort_scratch_init(words);
     if (e == hipSuccess && kin)
       e = hipMemcpyAsync(kin, d_keys, n * 8, hipMemcpyDeviceToDevice, nullptr);
@@ -1578,9 +1589,7 @@ int stm_sort_pairs_device(int device, const uint64_t* d_keys, size_t n, uint64_t
     else if (stalled) rc = fail(STM_ERR_DEVICE, "sort: a bounded wait between workgroups gave up");
   }
   (void)hipDeviceSynchronize();
-  void* ps[] = {ktmp, kin, itmp, words};
-  for (void* q : ps)
-    if (q) (void)hipFree(q);
+  if (slab) (void)hipFree(slab);
   return rc;
 }
 
@@ -1638,22 +1647,31 @@ int stm_dump(stm_tree* t, uint64_t* keys, uint64_t* vals, size_t cap, size_t* n)
   uint32_t *ids = nullptr, *order = nullptr, *order_tmp = nullptr, *sorted_ids = nullptr,
            *counts = nullptr, *counter = nullptr, *hist = nullptr;
   uint64_t *ok = nullptr, *ov = nullptr;
+  void *slab = nullptr, *out = nullptr;
   auto cleanup = [&]() {
-    void* ps[] = {lows, slows, slows_tmp, offs, ids, order, order_tmp, sorted_ids, counts, counter,
-                  hist, ok, ov};
-    for (void* p : ps)
-      if (p) (void)hipFree(p);
+    if (slab) (void)hipFree(slab);
+    if (out) (void)hipFree(out);
   };
   auto err = [&](int code, const char* what) {
     (void)hipStreamSynchronize(st);
     cleanup();
     return fail(code, "dump: %s", what);
   };
-  if (dalloc(&lows, nn) || dalloc(&slows, nn) || dalloc(&slows_tmp, nn) || dalloc(&ids, nn) ||
-      dalloc(&order, nn) || dalloc(&order_tmp, nn) || dalloc(&sorted_ids, nn) ||
-      dalloc(&counts, nn) || dalloc(&counter, 1) || dalloc(&offs, (size_t)nn + 1) ||
-      dalloc(&hist, sort_hist_words(nn)))
+  auto layout = [&](SlabCursor& cur) {
+#define A_(p, c) p = static_cast<decltype(p)>(cur.take(sizeof(*p) * (size_t)(c)))
+    A_(lows, nn); A_(slows, nn); A_(slows_tmp, nn); A_(ids, nn); A_(order, nn); A_(order_tmp, nn);
+    A_(sorted_ids, nn); A_(counts, nn); A_(counter, 1); A_(offs, (size_t)nn + 1);
+    A_(hist, sort_hist_words(nn));
+#undef A_
+  };
+  SlabCursor size{nullptr};
+  layout(size);
+  if (hipMalloc(&slab, size.at) != hipSuccess) {
+    slab = nullptr;
     return err(STM_ERR_NOMEM, "scratch");
+  }
+  SlabCursor place{static_cast<uint8_t*>(slab)};
+  layout(place);
   if (sort_scratch_init(hist) != hipSuccess) return err(STM_ERR_DEVICE, "sort scratch");
   if (hipMemsetAsync(counter, 0, 4, st) != hipSuccess) return err(STM_ERR_DEVICE, "memset");
   if (launch_collect_leaves(t->view, nn, lows, ids, counter, st) != hipSuccess)
@@ -1684,7 +1702,12 @@ int stm_dump(stm_tree* t, uint64_t* keys, uint64_t* vals, size_t cap, size_t* n)
     if (!keys && !vals && cap == 0) return STM_OK;  // size query
     return fail(STM_ERR_INVALID, "dump needs room for %llu pairs, got %zu", (unsigned long long)total, cap);
   }
-  if (dalloc(&ok, total) || dalloc(&ov, total)) return err(STM_ERR_NOMEM, "output");
+  if (total && hipMalloc(&out, total * 16) != hipSuccess) {
+    out = nullptr;
+    return err(STM_ERR_NOMEM, "output");
+  }
+  ok = static_cast<uint64_t*>(out);
+  ov = ok + total;
   if (hipMemcpyAsync(offs, ho.data(), 8ull * (n_leaves + 1), hipMemcpyHostToDevice, st) != hipSuccess ||
       launch_dump_copy(t->view, sorted_ids, offs, n_leaves, ok, ov, st) != hipSuccess)
     return err(STM_ERR_DEVICE, "copy");

@@ -15,6 +15,8 @@
 //     k_front_bucket  one workgroup per bucket collects its pieces from the tiles and sorts them
 //     k_front_fold    one workgroup per bucket: the bucket's place among the groups from the
 //                     other buckets' summaries, then the fold's outputs
+// Sorts outside of batches (front_sort: a tree's leaves, loads, stm_sort_pairs_device) take the same
+// kernels without the fold, k_front_keys in the place of k_front_small.
 //
 // The radix form this replaces took ten or eleven launches: k_range, the digit histograms and
 // their scan, two or three single-sweep passes, the bucket fix-up, the exact-sort check and three
@@ -129,6 +131,40 @@ STM_DEV Acc wave_combine(Acc v) {
   return v;
 }
 
+// Up to FT * E keys without op codes, sorted by one workgroup.
+template <int E>
+__global__ __launch_bounds__(FT) void k_front_keys(FrontSort fs) {
+  constexpr uint32_t N = FT * E;
+  __shared__ uint64_t s_k[N];
+  __shared__ uint32_t s_p[N];
+  __shared__ BinShared s_bin;
+  const uint32_t n = min(fs.n, N);
+  const uint32_t tid = threadIdx.x;
+  uint64_t k[E];
+  uint32_t p[E];
+#pragma unroll
+  for (int r = 0; r < E; ++r) {
+    const uint32_t i = (uint32_t)r * FT + tid;
+    k[r] = i < n ? gload(fs.keys + i) : KEY_EMPTY;
+    p[r] = i < n ? i : ~0u;
+  }
+  if (tid == 0) {
+    *fs.need = 0;
+    *fs.stall = 0;
+  }
+  bin_sort_open<FT>(s_bin);
+  __syncthreads();
+  bin_sort<FT, E>(n, k, p, s_k, s_p, s_bin);
+#pragma unroll
+  for (int r = 0; r < E; ++r) {
+    const uint32_t i = (uint32_t)r * FT + tid;
+    if (i < n) {
+      fs.keys_out[i] = s_k[i];
+      fs.idx_out[i] = s_p[i];
+    }
+  }
+}
+
 struct FrontIn {
   const uint64_t* keys;
   const uint8_t* ops;
@@ -228,7 +264,8 @@ __global__ __launch_bounds__(FT) void k_front_small(FrontArgs fa) {
 // Tile blockIdx.x of FT * E elements, ordered by bucket into tmp (the order within a bucket does
 // not matter: the bucket sort compares positions too).  Every workgroup sorts the same S samples
 // itself, which costs less than a launch for it and the round trip that reads the result.
-template <int E, int S>
+// BATCH: with op codes, found flags to set to their default and counters to reset.
+template <int E, int S, bool BATCH>
 __global__ __launch_bounds__(FT) void k_front_split(FrontArgs fa) {
   constexpr uint32_t TILE = FT * E;
   constexpr int B = S / (int)OVERSAMPLE;
@@ -244,8 +281,13 @@ __global__ __launch_bounds__(FT) void k_front_split(FrontArgs fa) {
   const uint32_t tid = threadIdx.x;
   uint8_t* found = fa.fold.desc ? fa.fold.desc->out_found : fa.fold.out_found;
   if (blockIdx.x == 0 && tid == 0) {
-    reset_counters(fa.fold.counters, 0, 0, 0);
-    fa.words[FRONT_RETRY] = 0;
+    if constexpr (BATCH) {
+      reset_counters(fa.fold.counters, 0, 0, 0);
+    } else {
+      *fa.stall = 0;
+      *fa.barrier = 0;
+    }
+    *fa.retry = 0;
   }
   if ((uint64_t)blockIdx.x * TILE >= n) return;
   const uint32_t tile0 = blockIdx.x * TILE;
@@ -257,7 +299,7 @@ __global__ __launch_bounds__(FT) void k_front_split(FrontArgs fa) {
   for (int r = 0; r < E; ++r) {
     const uint32_t le = min((uint32_t)r * FT + tid, tile_n - 1);
     ek[r] = gload(in.keys + tile0 + le);
-    ep[r] = gload(in.ops + tile0 + le);
+    ep[r] = BATCH ? gload(in.ops + tile0 + le) : 0u;
   }
   uint64_t sk[SE];
   uint32_t sp[SE];
@@ -331,7 +373,7 @@ __global__ __launch_bounds__(FT) void k_front_split(FrontArgs fa) {
       const uint32_t dst = tile0 + s_off[bkt[r]] + rank[r];
       fa.tmp_keys[dst] = ek[r];
       fa.tmp_ties[dst] = ep[r];
-      found[tile0 + le] = 1;  // the answers' default
+      if constexpr (BATCH) found[tile0 + le] = 1;  // the answers' default
     }
   }
 }
@@ -420,7 +462,7 @@ __global__ __launch_bounds__(FT) void k_front_bucket(FrontArgs fa, uint32_t tile
   __syncthreads();
   BucketSum sum{start, acc_identity()};
   if (m > BUCKET_CAP) {
-    if (tid == 0) fa.words[FRONT_RETRY] = 1;
+    if (tid == 0) *fa.retry = 1;
   } else if (m > 0) {
     bin_sort_open<FT>(s_bin);
     // Eight lanes per piece: the mean piece is a few elements.
@@ -449,7 +491,7 @@ __global__ __launch_bounds__(FT) void k_front_fold(FrontArgs fa, uint32_t B) {
   const uint32_t b = blockIdx.x;
   const uint32_t tid = threadIdx.x;
   const uint32_t wave = tid / WAVE;
-  if (fa.words[FRONT_RETRY]) {
+  if (*fa.retry) {
     if (b == 0 && tid == 0) a.counters->sort_retry = 1;  // no groups: the batch runs empty
     return;
   }
@@ -518,22 +560,31 @@ __global__ __launch_bounds__(FT) void k_front_fold(FrontArgs fa, uint32_t B) {
 }
 
 // ------------------------------------------------------------------ launcher
-template <int E, int S>
-static hipError_t launch_split(const FrontArgs& a, uint32_t n_max, hipStream_t s) {
+template <int E, int S, bool BATCH>
+static hipError_t launch_shape(const FrontArgs& a, uint32_t n_max, hipStream_t s) {
   constexpr uint32_t B = S / OVERSAMPLE;
   const uint32_t tile = FT * E;
-  k_front_split<E, S><<<(n_max + tile - 1) / tile, FT, 0, s>>>(a);
+  k_front_split<E, S, BATCH><<<(n_max + tile - 1) / tile, FT, 0, s>>>(a);
   k_front_bucket<<<B, FT, 0, s>>>(a, tile, B);
-  k_front_fold<<<B, FT, 0, s>>>(a, B);
+  if constexpr (BATCH) k_front_fold<<<B, FT, 0, s>>>(a, B);
   return hipGetLastError();
 }
 
-// a.fold.n is the op count, or with a.fold.desc the largest count (at most FRONT_MAX_OPS).  About
-// 512 ops per bucket: a bucket then mostly sorts in one element per thread.
-hipError_t front_batch(const FrontArgs& a, hipStream_t s) {
+// About 512 ops per bucket: a bucket then mostly sorts in one element per thread.
+template <bool BATCH>
+static hipError_t launch_split(const FrontArgs& a, uint32_t n, hipStream_t s) {
+  if (n <= (1u << 14)) return launch_shape<1, 256, BATCH>(a, n, s);
+  if (n <= (1u << 15)) return launch_shape<1, 512, BATCH>(a, n, s);
+  if (n <= (1u << 16)) return launch_shape<1, 1024, BATCH>(a, n, s);
+  return launch_shape<2, 2048, BATCH>(a, n, s);
+}
+
+// a.fold.n is the op count, or with a.fold.desc the largest count (at most FRONT_MAX_OPS).
+hipError_t front_batch(FrontArgs a, hipStream_t s) {
   const uint32_t n = a.fold.n;
   if (n == 0) return hipSuccess;
   if (n > FRONT_MAX_OPS) return hipErrorInvalidValue;
+  a.retry = a.words + FRONT_RETRY;
   if (n <= FT) {
     k_front_small<1><<<1, FT, 0, s>>>(a);
     return hipGetLastError();
@@ -542,10 +593,42 @@ hipError_t front_batch(const FrontArgs& a, hipStream_t s) {
     k_front_small<2><<<1, FT, 0, s>>>(a);
     return hipGetLastError();
   }
-  if (n <= (1u << 14)) return launch_split<1, 256>(a, n, s);
-  if (n <= (1u << 15)) return launch_split<1, 512>(a, n, s);
-  if (n <= (1u << 16)) return launch_split<1, 1024>(a, n, s);
-  return launch_split<2, 2048>(a, n, s);
+  return launch_split<true>(a, n, s);
+}
+
+size_t front_sort_words(uint32_t n) {
+  if (n <= FRONT_SMALL) return 0;
+  const uint32_t tiles = n <= (1u << 16) ? (n + FT - 1) / FT : (n + 2 * FT - 1) / (2 * FT);
+  const uint32_t B = n <= (1u << 14) ? 32u : n <= (1u << 15) ? 64u : n <= (1u << 16) ? 128u : 256u;
+  return FRONT_OFFS + (size_t)tiles * (B + 1);
+}
+
+// Stable sort of fs.n keys.  *fs.need is 1 afterwards where a bucket overflowed, and the output then
+// incomplete.  stm_sort_pairs_device with the normalized radix passes and their dozen launches, before
+// its allocations became one, and now: 1000 keys 95 / 36 µs, 16384 keys 103 / 48, 2^18 keys 145 / 95.
+hipError_t front_sort(const FrontSort& fs, hipStream_t s) {
+  if (fs.n == 0) return hipSuccess;
+  if (fs.n > FRONT_MAX_OPS) return hipErrorInvalidValue;
+  if (fs.n <= FT) {
+    k_front_keys<1><<<1, FT, 0, s>>>(fs);
+    return hipGetLastError();
+  }
+  if (fs.n <= FRONT_SMALL) {
+    k_front_keys<2><<<1, FT, 0, s>>>(fs);
+    return hipGetLastError();
+  }
+  FrontArgs a{};
+  a.keys = fs.keys;
+  a.fold.n = fs.n;
+  a.fold.skeys = fs.keys_out;
+  a.fold.sidx = fs.idx_out;
+  a.tmp_keys = fs.tmp_keys;
+  a.tmp_ties = fs.tmp_ties;
+  a.words = fs.words;
+  a.retry = fs.need;
+  a.stall = fs.stall;
+  a.barrier = fs.barrier;
+  return launch_split<false>(a, fs.n, s);
 }
 
 }  // namespace stm

@@ -54,9 +54,10 @@ hipError_t radix_sort_pairs(const uint64_t* keys_in, uint64_t* keys_tmp, uint64_
 // without it keys_in holds n_max keys.
 // found (the descriptor's out_found with desc; null: none) is set to 1 throughout on the way: the
 // answers' default.
-// Full 64-bit keys without desc go through the sample sort at its sizes, else through the
-// normalized-key form, unless `exact` asks for the eight-pass form (the library asks for it after a
-// batch whose normalized sort had to fall back).
+// Full 64-bit keys without desc go through the sample sort at its sizes, keys without op codes
+// through front_sort up to FRONT_MAX_OPS of them, the others through the normalized-key form, unless
+// `exact` asks for the eight-pass form (the library asks for it after a batch whose normalized sort
+// had to fall back).
 hipError_t radix_sort_pairs_desc(const uint64_t* keys_in, const uint8_t* ops_in,
                                  const BatchDesc* desc, uint32_t n_max,
                                  uint64_t* keys_tmp, uint64_t* keys_out, uint32_t* idx_tmp,
@@ -163,9 +164,27 @@ struct FrontArgs {
   uint64_t* tmp_keys;    // scratch of the batch's size
   uint32_t* tmp_ties;
   uint32_t* words;       // front_scratch_words()
+  // set by the launchers: the flag of an overflowed bucket; the radix sort's words to clear
+  uint32_t *retry, *stall, *barrier;
 };
 size_t front_scratch_words();
-hipError_t front_batch(const FrontArgs& a, hipStream_t stream);
+hipError_t front_batch(FrontArgs a, hipStream_t stream);
+
+// The sort alone, of at most FRONT_MAX_OPS keys without op codes.
+struct FrontSort {
+  const uint64_t* keys;
+  uint32_t n;
+  uint64_t* tmp_keys;
+  uint32_t* tmp_ties;
+  uint64_t* keys_out;
+  uint32_t* idx_out;
+  uint32_t* words;    // front_sort_words(n)
+  uint32_t* need;     // as SampleControl
+  uint32_t* stall;
+  uint32_t* barrier;
+};
+size_t front_sort_words(uint32_t n);
+hipError_t front_sort(const FrontSort& fs, hipStream_t stream);
 
 constexpr uint8_t UOP_SKIP = 0xff;
 constexpr uint8_t OP_RANGE = 3;

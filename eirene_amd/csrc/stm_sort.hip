@@ -15,8 +15,8 @@
 //               segment, so (wave, round, lane) order is input order), LDS staging into
 //               digit order (keys, then payloads, through one buffer), then coalesced runs
 //               to global memory.
-// Batches of at most FRONT_MAX_OPS ops are sorted elsewhere (stm_front.hip): a dozen launches of
-// a few microseconds each would set their time.  From SAMPLE_SORT_MIN to SAMPLE_SORT_MAX keys the
+// At most FRONT_MAX_OPS ops or keys are sorted elsewhere (stm_front.hip): a dozen launches of a few
+// microseconds each would set their time.  From SAMPLE_SORT_MIN to SAMPLE_SORT_MAX keys the
 // sample sort of stm_sample.hip takes the place of the normalized form, with k_sort_exact behind it.
 //
 // The element count and the input keys can come from a device-side batch descriptor, and the
@@ -747,8 +747,9 @@ size_t sort_hist_words(uint64_t n) {
   // the histogram region, sized for the smallest tile (the most tiles)
   uint64_t ntiles = (n + sort_tile(8) - 1) / sort_tile(8);
   if (ntiles == 0) ntiles = 1;
-  return (size_t)CTL_WORDS + std::max((size_t)ntiles * RADIX + RADIX,
-                                      sample_sort_words(std::min<uint64_t>(n, SAMPLE_SORT_MAX)));
+  return (size_t)CTL_WORDS +
+         std::max({(size_t)ntiles * RADIX + RADIX, sample_sort_words(std::min<uint64_t>(n, SAMPLE_SORT_MAX)),
+                   front_sort_words((uint32_t)std::min<uint64_t>(n, FRONT_MAX_OPS))});
 }
 
 hipError_t sort_scratch_init(uint32_t* words) {
@@ -850,6 +851,17 @@ static hipError_t sort_passes(const uint64_t* keys_in, const uint8_t* ops_in, co
                             words + CTL_BARRIER};
     e = sample_sort(keys_in, ops_in, n_host, keys_tmp, idx_tmp, keys_out, idx_out, ctl, found, stream);
     if (e != hipSuccess) return e;
+    k_sort_exact<ITEMS><<<xgrid, SORT_BLOCK, 0, stream>>>(keys_in, ops_in, nullptr, n_host, keys_tmp,
+                                                         keys_out, idx_tmp, idx_out, words, stride);
+    return hipGetLastError();
+  }
+  if (!exact && !desc && !ops_in && !found && begin_bit == 0 && end_bit == 64 && n_host <= FRONT_MAX_OPS) {
+    uint32_t xgrid = 0;
+    hipError_t e = exact_grid<ITEMS>(xgrid);
+    if (e != hipSuccess) return e;
+    const FrontSort fs{keys_in, n_host, keys_tmp, idx_tmp, keys_out, idx_out, words + CTL_WORDS,
+                       words + CTL_NEED_EXACT, words + CTL_STALL, words + CTL_BARRIER};
+    if ((e = front_sort(fs, stream)) != hipSuccess || front_sort_words(n_host) == 0) return e;
     k_sort_exact<ITEMS><<<xgrid, SORT_BLOCK, 0, stream>>>(keys_in, ops_in, nullptr, n_host, keys_tmp,
                                                          keys_out, idx_tmp, idx_out, words, stride);
     return hipGetLastError();
